@@ -136,8 +136,12 @@ def _arrived(case):
 
 
 def _rows(case):
-    """Expected expanded rows, the padding of every expert's segment among them."""
-    return _pairs(case) + case['experts'] * (case['align'] - 1) / 2
+    """Expected expanded rows, the padding of every expert's segment among them: an expert's entries are close to Poisson
+    distributed, and its segment has one block of `align` rows more for every multiple of `align` that they exceed."""
+    mean, blocks = _pairs(case) / case['experts'], 0.0
+    for j in range(int((mean + 8 * math.sqrt(mean)) / case['align']) + 1):
+        blocks += 0.5 * math.erfc((j * case['align'] + 0.5 - mean) / math.sqrt(2 * mean)) if j else 1 - math.exp(-mean)
+    return case['experts'] * case['align'] * blocks
 
 
 def _route(case, g):
@@ -292,8 +296,8 @@ def work(case):
         b = a * 5 + d * 3 + _sf_bytes(case['tokens'] // case['group'], case['inner'] + case['hidden'], 1)
         f = 8.0 * a + 3.0 * d
     elif kind == 'swiglu_backward':
-        r, h = _rows(case), case['hidden']
-        b = r * h * (2 + 2 + 2 + 2 + 4) + 2 * _sf_bytes(r, 2 * h, case['group']) + 4 * r + 12 * _arrived(case) * case['topk']
+        r, p, h = _rows(case), _pairs(case), case['hidden']             # rows of padding are written, not read
+        b = p * h * (2 + 2) + r * h * (2 + 2 + 4) + _sf_bytes(p + r, 2 * h, case['group']) + 4 * r + 12 * _arrived(case) * case['topk']
         f = 24.0 * _pairs(case) * h
     elif kind == 'channel_requant':
         r, t, h = _rows(case), _arrived(case), case['hidden']
