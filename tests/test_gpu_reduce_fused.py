@@ -88,3 +88,21 @@ def test_reduce_fused_e4m3_output_beyond_the_format_range():
     assert_same(got, want, 'codes')
     codes = want.view(torch.uint8)[0, :8].tolist()
     assert codes[0] == 0x7F and codes[1] == 0xFF and codes[3] == 0x7F and codes[2] != 0x7F      # 600, -600, 894 -> NaN; 200 is finite
+
+
+@pytest.mark.parametrize('hidden', [256, 768, 1024, 1280, 2048])
+@pytest.mark.parametrize('dtype', [torch.float32, torch.bfloat16], ids=['f32', 'bf16'])
+@pytest.mark.parametrize('T,K', [(5, 1), (9, 15), (3, 64), (4, 67), (2, 130)])
+def test_reduce_fused_with_few_and_many_live_terms(T, K, dtype, hidden):
+    """Every count of live terms, at every place of the list, for lists beyond one ballot and for rows of one to four
+    pieces of 512 columns (the last one half): the sums keep the order of k whatever is skipped."""
+    tk = _tk()
+    g = torch.Generator().manual_seed(T * K + hidden)
+    R = 40
+    x = torch.randn((R, hidden), generator=g).to(dtype)
+    t2p = torch.randint(0, R, (T, K), generator=g, dtype=torch.int32)
+    drop = torch.rand((T, K), generator=g) < torch.linspace(0, 1, T)[:, None]      # none of the first token's, all of the last's
+    t2p = t2p.masked_fill(drop, -1)
+    w = torch.rand((T, K), generator=g)
+    want = torch_ref.reduce_fused(x, w, t2p)
+    assert_same(tk.moe.reduce_fused(x.cuda(), w.cuda(), t2p.cuda()), want, 'reduced')

@@ -420,13 +420,21 @@ __global__ __launch_bounds__(kThreads) void expand_short_rows_kernel(const uint8
 // reduce_fused: the inverse of the expansion.  out[t] = sum over k of x[pos(t, k)] * s(t, k), accumulated in fp32 with
 // one fused multiply-add per term, in the order k = 0, 1, ... (so that results are reproducible bit for bit), where
 // s = topk_weights[t, k] (or 1) times x_sf[pos] (if given); positions < 0 are skipped.  The sum is scaled by *sf (if
-// given) and rounded to the output type.  A thread owns 8 consecutive elements of one token: up to 8 rows' pieces are
-// loaded before the first is used, and there is one store per thread.
-constexpr int kReduceUnroll = 8;
-
+// given) and rounded to the output type.
+//
+// What bounds it is the gather of whole rows from HBM.  A wave owns 512 columns of one token.  Lane k fetches position and
+// factor of term k, a ballot says which terms are live, and only those are loaded, 8 (fp32: 4) of them before the first
+// is used (v_readlane hands a live term's row and factor to the whole wave as scalars).  A rank of an expert-parallel
+// group holds few of a token's experts, one or two of eight on average; loading place-holders for the others (row 0, so
+// that there is no branch around a load) took as long as loading rows.  Measured on MI355X, us, place-holders / this:
+//   bf16 [34816, 7168] -> [21616, 7168], 1.6 live terms of 8: 226 / 130 (6.0 TB/s);  [.., 2560]: 102 / 44;  [.., 1280]: 39 / 26
+//   bf16 [48128, 4096] -> [4096, 4096], 8 of 8: 49.0 / 48.7;  [.., 1280], 8 of 8: 16.0 / 17.0;  [.., 2560], 6 of 6: 27.3 / 24.3
+//   fp32 [81792, 4096], 8 of 8: 209.9 / 211.4 (to E4M3 175.3 / 177.2);  [.., 2304], 9 of 9: 103 / 76
+// Positions and factors through the scalar path instead (eight loads each, put into lanes one by one): 163 and 54 us where 132
+// and 45; two pieces of 512 columns per wave and four terms at a time: 133 and 52.5 us, 8.0 instead of 4.4 us for 300 tokens.
 // fp32 rows whose length is a multiple of 512: a thread's 8 elements are two runs of 4, 256 columns apart, so that each
 // of its 16-byte loads (and of its fp32 stores) is, over the wave, 1024 consecutive bytes.  With the 8 elements in one
-// run, every instruction touches half of each cache line it names (fp32 [81792, 4096] -> fp32, top-8: 220.2 us that way).
+// run, every instruction touches half of each cache line it names (fp32 [81792, 4096] -> fp32, top-8: 220 instead of 210 us).
 struct SplitF32 {};
 struct Raw8SplitF32 {
     u32x4 a, b;
@@ -437,33 +445,29 @@ struct Raw8SplitF32 {
     }
 };
 template <typename InT> struct ReduceIn;
-template <> struct ReduceIn<bf16_t> { typedef Raw8<bf16_t> raw; typedef bf16_t elem; static constexpr bool split = false; };
-template <> struct ReduceIn<float> { typedef Raw8<float> raw; typedef float elem; static constexpr bool split = false; };
-template <> struct ReduceIn<SplitF32> { typedef Raw8SplitF32 raw; typedef float elem; static constexpr bool split = true; };
+template <> struct ReduceIn<bf16_t> { typedef Raw8<bf16_t> raw; typedef bf16_t elem; static constexpr bool split = false; static constexpr int unroll = 8; };
+template <> struct ReduceIn<float> { typedef Raw8<float> raw; typedef float elem; static constexpr bool split = false; static constexpr int unroll = 4; };
+template <> struct ReduceIn<SplitF32> { typedef Raw8SplitF32 raw; typedef float elem; static constexpr bool split = true; static constexpr int unroll = 4; };
 
-// U terms k0 .. k0 + U - 1 of one token: all U rows' pieces are loaded before the first is used
+// the first U terms of `live`, which has at least that many: all pieces are loaded before the first is used
 template <typename InT, int U>
-__device__ __forceinline__ void reduce_terms(float (&acc)[8], const typename ReduceIn<InT>::elem *x, const int32_t *pos_row, int k0, int t, int num_topk, int hidden,
-                                             int num_expanded, int col, const float *topk_weights, const float *x_sf) {
+__device__ __forceinline__ void reduce_terms(float (&acc)[8], const typename ReduceIn<InT>::elem *x, int hidden, unsigned long long &live, int pos,
+                                             float factor) {
     typename ReduceIn<InT>::raw raw[U];
     float s[U];
-    bool live[U];
 #pragma unroll
     for (int j = 0; j < U; ++j) {
-        const int k = k0 + j;
-        const int p = uniform_load(pos_row + k);
-        live[j] = p >= 0 && p < num_expanded;
-        // a skipped term reads row 0 (no branch around the loads) and is not added
-        const int row = live[j] ? p : 0;
-        raw[j].load(x + (int64_t)row * hidden + col);
+        const int k = __builtin_ctzll(live);
+        live &= live - 1;
+        raw[j].load(x + (int64_t)__builtin_amdgcn_readlane(pos, k) * hidden);
         vmem_issue_gap();
-        s[j] = 1.0f;
-        if (topk_weights) s[j] = live[j] ? uniform_load(topk_weights + (int64_t)t * num_topk + k) : 0.0f;
-        if (x_sf) s[j] = s[j] * uniform_load(x_sf + row);
+        s[j] = u2f((uint32_t)__builtin_amdgcn_readlane((int)f2u(factor), k));
     }
+    // without this the arithmetic on the first piece moves in front of the later loads, which then wait for it
+    // (bf16 [16384, 256], 8 of 8 terms: 20.2 -> 12.5 us)
+    __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
     for (int j = 0; j < U; ++j) {
-        if (!live[j]) continue;      // wave-uniform
         float v[8];
         raw[j].get(v);
 #pragma unroll
@@ -473,33 +477,9 @@ __device__ __forceinline__ void reduce_terms(float (&acc)[8], const typename Red
 
 // OUT: 0 bf16, 1 fp32, 2 E4M3
 template <typename InT, int OUT>
-__global__ __launch_bounds__(kThreads) void reduce_fused_kernel(const typename ReduceIn<InT>::elem *x, const int32_t *token_topk_to_pos, int num_topk,
-                                                                int hidden, int num_expanded, const float *topk_weights, const float *x_sf,
-                                                                const float *sf, void *out) {
+__device__ __forceinline__ void reduce_store(const float (&acc)[8], void *out, int64_t idx) {
     typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
     constexpr bool SPLIT = ReduceIn<InT>::split;
-    const int t = blockIdx.y;
-    // SPLIT: elements col .. col + 3 and col + 256 .. col + 259 (the wave's 512 columns are all inside the row or all outside)
-    const int col = SPLIT ? (blockIdx.x * kThreads + (threadIdx.x & ~63)) * 8 + (threadIdx.x & 63) * 4 : (blockIdx.x * kThreads + threadIdx.x) * 8;
-    if (col >= hidden) return;
-    const int32_t *pos_row = token_topk_to_pos + (int64_t)t * num_topk;
-    float acc[8];
-#pragma unroll
-    for (int i = 0; i < 8; ++i) acc[i] = 0.0f;
-    // whole groups of 8 terms, then the rest in steps of 4, 2 and 1: padding a short list to 8 with skipped terms would
-    // still issue their loads (top-2 of bf16 [8576, 7168]: 46.7 us that way)
-    int k0 = 0;
-    for (; k0 + kReduceUnroll <= num_topk; k0 += kReduceUnroll)
-        reduce_terms<InT, kReduceUnroll>(acc, x, pos_row, k0, t, num_topk, hidden, num_expanded, col, topk_weights, x_sf);
-    if ((num_topk - k0) & 4) { reduce_terms<InT, 4>(acc, x, pos_row, k0, t, num_topk, hidden, num_expanded, col, topk_weights, x_sf); k0 += 4; }
-    if ((num_topk - k0) & 2) { reduce_terms<InT, 2>(acc, x, pos_row, k0, t, num_topk, hidden, num_expanded, col, topk_weights, x_sf); k0 += 2; }
-    if ((num_topk - k0) & 1) reduce_terms<InT, 1>(acc, x, pos_row, k0, t, num_topk, hidden, num_expanded, col, topk_weights, x_sf);
-    if (sf) {
-        const float f = uniform_load(sf);
-#pragma unroll
-        for (int i = 0; i < 8; ++i) acc[i] = acc[i] * f;
-    }
-    const int64_t idx = (int64_t)t * hidden + col;
     if (OUT == 1) {
         u32x4 *o = reinterpret_cast<u32x4 *>(reinterpret_cast<float *>(out) + idx);
         __builtin_nontemporal_store(u32x4{f2u(acc[0]), f2u(acc[1]), f2u(acc[2]), f2u(acc[3])}, o);
@@ -520,6 +500,48 @@ __global__ __launch_bounds__(kThreads) void reduce_fused_kernel(const typename R
     } else {
         st_stream8(reinterpret_cast<uint8_t *>(out) + idx, pack_e4m3x8<false>(acc));
     }
+}
+
+// (Registers for eight waves per SIMD: the gather needs them all in flight, bf16 [34816, 7168] at six waves 142 us.)
+// A workgroup is kWaves >> side_log2 tokens high and 1 << side_log2 pieces of 512 columns wide.
+template <typename InT, int OUT>
+__global__ __launch_bounds__(kThreads, 8) void reduce_fused_kernel(const typename ReduceIn<InT>::elem *x, const int32_t *token_topk_to_pos, int64_t num_tokens,
+                                                                int num_topk, int hidden, int num_expanded, int side_log2, int one_col,
+                                                                const float *topk_weights, const float *x_sf, const float *sf, void *out) {
+    constexpr bool SPLIT = ReduceIn<InT>::split;
+    const int lane = threadIdx.x & 63, wave = wave_id();
+    const int64_t t = ((int64_t)tile_grid_row(one_col) << (2 - side_log2)) + (wave >> side_log2);
+    static_assert(kWaves == 4, "side_log2 is 0 to 2");
+    const int piece = (tile_grid_col(one_col) << side_log2) + (wave & ((1 << side_log2) - 1));
+    // SPLIT: elements col .. col + 3 and col + 256 .. col + 259
+    const int col = piece * kStripCols + lane * (SPLIT ? 4 : 8);
+    if (t >= num_tokens) return;
+    const bool inside = col < hidden;
+    x += inside ? col : 0;
+    float acc[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) acc[i] = 0.0f;
+    for (int k0 = 0; k0 < num_topk; k0 += 64) {
+        const int k = k0 + lane;
+        const int64_t at = t * num_topk + (k < num_topk ? k : k0);
+        const int pos = token_topk_to_pos[at];
+        float factor = topk_weights ? topk_weights[at] : 1.0f;
+        const bool ok = k < num_topk && pos >= 0 && pos < num_expanded;
+        if (x_sf) factor = factor * x_sf[ok ? pos : 0];
+        unsigned long long live = __builtin_amdgcn_ballot_w64(ok);
+        int n = __popcll(live);
+        constexpr int U = ReduceIn<InT>::unroll;
+        for (; n >= U; n -= U) reduce_terms<InT, U>(acc, x, hidden, live, pos, factor);
+        if (U > 4 && (n & 4)) reduce_terms<InT, 4>(acc, x, hidden, live, pos, factor);
+        if (n & 2) reduce_terms<InT, 2>(acc, x, hidden, live, pos, factor);
+        if (n & 1) reduce_terms<InT, 1>(acc, x, hidden, live, pos, factor);
+    }
+    if (sf) {
+        const float f = uniform_load(sf);
+#pragma unroll
+        for (int i = 0; i < 8; ++i) acc[i] = acc[i] * f;
+    }
+    if (inside) reduce_store<InT, OUT>(acc, out, t * hidden + col);
 }
 
 // reduce_fused without a single expanded row: every term is skipped, the result is zeros.  (The reduction kernel
@@ -739,29 +761,28 @@ extern "C" int tk_reduce_fused(const void *x, int x_dtype, int64_t num_expanded,
                            static_cast<uint64_t *>(out), words);
         return (int)hipGetLastError();
     }
-    const unsigned chunks = (unsigned)((hidden + kThreads * 8 - 1) / (kThreads * 8));
-    // tokens ride on grid.y (at most 65535 per launch)
-    for (int64_t t0 = 0; t0 < num_tokens; t0 += 65535) {
-        const unsigned nt = (unsigned)(num_tokens - t0 < 65535 ? num_tokens - t0 : 65535);
-        const dim3 grid(chunks, nt);
-        const int32_t *pos = token_topk_to_pos + t0 * num_topk;
-        const float *w = topk_weights ? topk_weights + t0 * num_topk : nullptr;
-        const int64_t out_bytes = out_dtype == TK_F32 ? 4 : (out_dtype == TK_BF16 ? 2 : 1);
-        void *o = static_cast<uint8_t *>(out) + t0 * hidden * out_bytes;
+    const int strips = (int)((hidden + kStripCols - 1) / kStripCols);
+    // Two pieces side by side where the row has an even number of them (300 tokens of 4096 columns 4.9 -> 4.3 us, nothing
+    // lost at larger sizes), four of fp32 (344 tokens of 4096 4.5 -> 3.7, 65536 terms of 4096 columns 213.5 -> 211); with an odd
+    // number the last workgroup of a row would be half idle (3 pieces: 26 -> 32 us).
+    const int side_log2 = strips % 4 == 0 && x_dtype == TK_F32 ? 2 : (strips % 2 == 0 ? 1 : 0);
+    const int64_t rows = kWaves >> side_log2;
+    const int cols = strips >> side_log2;
+    const dim3 grid = tile_grid(cols, (int)((num_tokens + rows - 1) / rows));
 #define TK_REDUCE_LAUNCH(T, O)                                                                                              \
-    hipLaunchKernelGGL((reduce_fused_kernel<T, O>), grid, dim3(kThreads), 0, s, static_cast<const ReduceIn<T>::elem *>(x), pos, num_topk, \
-                       (int)hidden, (int)num_expanded, w, x_sf, sf, o)
-        if (x_dtype == TK_BF16) {
-            if (out_dtype == TK_OUT_E4M3) TK_REDUCE_LAUNCH(bf16_t, 2);
-            else TK_REDUCE_LAUNCH(bf16_t, 0);
-        } else if (hidden % 512 == 0) {
-            if (out_dtype == TK_OUT_E4M3) TK_REDUCE_LAUNCH(SplitF32, 2);
-            else TK_REDUCE_LAUNCH(SplitF32, 1);
-        } else {
-            if (out_dtype == TK_OUT_E4M3) TK_REDUCE_LAUNCH(float, 2);
-            else TK_REDUCE_LAUNCH(float, 1);
-        }
-#undef TK_REDUCE_LAUNCH
+    hipLaunchKernelGGL((reduce_fused_kernel<T, O>), grid, dim3(kThreads), 0, s, static_cast<const ReduceIn<T>::elem *>(x),  \
+                       token_topk_to_pos, num_tokens, num_topk, (int)hidden, (int)num_expanded, side_log2, (int)(cols == 1), \
+                       topk_weights, x_sf, sf, out)
+    if (x_dtype == TK_BF16) {
+        if (out_dtype == TK_OUT_E4M3) TK_REDUCE_LAUNCH(bf16_t, 2);
+        else TK_REDUCE_LAUNCH(bf16_t, 0);
+    } else if (hidden % 512 == 0) {
+        if (out_dtype == TK_OUT_E4M3) TK_REDUCE_LAUNCH(SplitF32, 2);
+        else TK_REDUCE_LAUNCH(SplitF32, 1);
+    } else {
+        if (out_dtype == TK_OUT_E4M3) TK_REDUCE_LAUNCH(float, 2);
+        else TK_REDUCE_LAUNCH(float, 1);
     }
+#undef TK_REDUCE_LAUNCH
     return (int)hipGetLastError();
 }
