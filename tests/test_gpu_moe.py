@@ -97,3 +97,44 @@ def test_moe_chain_mapping_expand_swiglu_cast():
     xe = tk.moe.expand_to_fused(x.cuda(), m[3], m[0])
     got = tk.quant.swiglu_forward_and_per_token_cast(xe, 'e4m3', 128, m[2], w.cuda().contiguous(), m[0])
     check_fused(got, want, H // 128, False, 'chain')
+
+
+@pytest.mark.parametrize('K', [1, 8, 11, 70])
+@pytest.mark.parametrize('T,dim,dtype', [(37, 16, torch.bfloat16), (37, 1024, torch.bfloat16), (37, 1032, torch.bfloat16), (9, 2048, torch.float8_e4m3fn),
+                                         (9, 7168, torch.float8_e4m3fn), (33, 4096, torch.bfloat16)])
+@pytest.mark.parametrize('live', [0.0, 0.15, 1.0])
+def test_expand_to_fused_sparse_and_full_lists(T, K, dim, dtype, live):
+    """One workgroup per token: lists with no, few and all positions set, beyond one ballot, rows shorter than, equal to and
+    longer than a chunk (4 KB)."""
+    tk = _tk()
+    g = torch.Generator().manual_seed(T * K + dim)
+    here = torch.rand((T, K), generator=g) < live
+    R = int(here.sum()) + 5
+    t2p = torch.full((T, K), -1, dtype=torch.int32)
+    t2p[here] = torch.randperm(R, generator=g)[:int(here.sum())].to(torch.int32)
+    p2e = torch.full((R,), -1, dtype=torch.int32)
+    p2e[t2p[here].long()] = 3
+    x = torch.randn((T, dim), generator=g).to(dtype)
+    want = torch_ref.expand_to_fused(x.view(torch.uint8), t2p, p2e)
+    got = tk.moe.expand_to_fused(x.cuda(), t2p.cuda(), p2e.cuda())
+    assert torch.equal(got.cpu().view(torch.uint8), want)
+
+
+@pytest.mark.parametrize('dim', [512, 8192])
+def test_expand_to_fused_long_output_with_full_lists(dim):
+    """Outputs beyond 160 MB with several positions per token take a workgroup per list entry."""
+    tk = _tk()
+    T, K = (170 << 20) // (dim * 2) // 4, 4
+    g = torch.Generator().manual_seed(dim)
+    t2p = torch.randperm(T * K, generator=g).to(torch.int32).view(T, K)
+    t2p[::7, 1] = -1
+    p2e = torch.full((T * K,), -1, dtype=torch.int32)
+    p2e[t2p[t2p >= 0].long()] = 0
+    x = torch.randn((T, dim), generator=g).to(torch.bfloat16).cuda()
+    got = tk.moe.expand_to_fused(x, t2p.cuda(), p2e.cuda())
+    assert T * K * dim * 2 >= 160 << 20
+    want = torch.zeros_like(got)
+    for k in range(K):
+        here = (t2p[:, k] >= 0).cuda()
+        want[t2p[:, k].cuda()[here].long()] = x[here]
+    assert torch.equal(got.view(torch.int16), want.view(torch.int16))

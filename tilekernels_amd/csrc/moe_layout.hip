@@ -6,6 +6,7 @@
 // tile_kernels/moe/expand_to_fused_kernel.py:16-200, tile_kernels/torch/expand_to_fused.py,
 // tile_kernels/moe/reduce_fused_kernel.py:12-135, tile_kernels/torch/reduce_fused.py.
 #include <atomic>
+#include <algorithm>
 
 #include "tk_device.hpp"
 #include "tk_host.hpp"
@@ -350,6 +351,15 @@ __device__ __forceinline__ void expand_zero_padding(int pb, int pad_rows, int nu
     }
 }
 
+// EVERY: a workgroup per list entry, one store per thread, as described above.  That pays for full lists that fill
+// a long buffer.  Otherwise one workgroup serves every live entry of a token's chunk: it reads the list with one load per lane, a
+// ballot says which entries have a position, and there is one store per thread for each of them.  What bounds an
+// expert-parallel rank's expansion with EVERY is the dispatch of workgroups that find no position (0.7 ns each, whatever
+// they do).  us per call on MI355X, EVERY / one per token (codes with scales, top-8 unless said):
+//   [4096, 7168] of 8 ranks, [21504] tokens -> [34816]  218 / 62      340 tokens -> [3232, 4096] (worst-case buffer)  5.4 / 4.4
+//   [512, 4096] -> [6144]   7.0 / 6.2                  [2048, 7168] -> [18432]  30.6 / 28.5       top-2 of [4096, 7168]  17.3 / 17.3
+//   [4096, 4096] -> [48128]  38.1 / 39.2               bf16 [4096, 4096] -> [48128]  64.4 / 73.5
+template <bool EVERY>
 __global__ __launch_bounds__(kThreads) void expand_to_fused_kernel(const uint8_t *x, int64_t row_bytes, const int32_t *token_topk_to_pos,
                                                                    int num_topk, int chunks, int copy_blocks, int num_tokens,
                                                                    int num_expanded, uint8_t *out, const int32_t *pos_to_expert,
@@ -357,20 +367,34 @@ __global__ __launch_bounds__(kThreads) void expand_to_fused_kernel(const uint8_t
                                                                    int64_t out_sf_ld, int sf_col_major, int pad_rows) {
     const int b = blockIdx.x;
     if (b < copy_blocks) {
-        // b = 8 * ((token group * chunks + chunk) * num_topk + k) + token within its group of 8
+        // b = 8 * ((token group * chunks + chunk) * entries + entry) + token within its group of 8
         const int q = b >> 3;
-        const int k = q % num_topk, q2 = q / num_topk;
+        const int k = EVERY ? q % num_topk : 0, q2 = EVERY ? q / num_topk : q;
         const int c = q2 % chunks, t = (q2 / chunks) * 8 + (b & 7);
         if (t >= num_tokens) return;
-        const int p = uniform_load(token_topk_to_pos + (int64_t)t * num_topk + k);
         const int64_t off = (int64_t)c * kExpandChunk + threadIdx.x * 16;
+        const u32x4 *src = reinterpret_cast<const u32x4 *>(x + (int64_t)t * row_bytes + off);
+        const int32_t *list = token_topk_to_pos + (int64_t)t * num_topk;
         u32x4 v = u32x4{0u, 0u, 0u, 0u};
-        if (off < row_bytes) v = *reinterpret_cast<const u32x4 *>(x + (int64_t)t * row_bytes + off);   // cached: read num_topk times
-        if (p < 0 || p >= num_expanded) return;
-        if (off < row_bytes) expand_store16(out + (int64_t)p * row_bytes + off, v);
-        if (x_sf && c == 0)
-            for (int j = threadIdx.x; j < sf_cols; j += kThreads)
-                out_sf[sf_col_major ? (int64_t)j * out_sf_ld + p : (int64_t)p * out_sf_ld + j] = x_sf[(int64_t)t * sf_cols + j];
+        auto copy_to = [&](int p) {
+            if (off < row_bytes) expand_store16(out + (int64_t)p * row_bytes + off, v);
+            if (x_sf && c == 0)
+                for (int j = threadIdx.x; j < sf_cols; j += kThreads)
+                    out_sf[sf_col_major ? (int64_t)j * out_sf_ld + p : (int64_t)p * out_sf_ld + j] = x_sf[(int64_t)t * sf_cols + j];
+        };
+        if (EVERY) {
+            const int p = uniform_load(list + k);
+            if (off < row_bytes) v = *src;   // cached: read num_topk times
+            if (p >= 0 && p < num_expanded) copy_to(p);
+            return;
+        }
+        for (int k0 = 0; k0 < num_topk; k0 += 64) {
+            const int kk = k0 + (threadIdx.x & 63);
+            const int pos = list[kk < num_topk ? kk : 0];
+            if (k0 == 0 && off < row_bytes) v = *src;      // a token without any position is rare: not waited for
+            unsigned long long live = __builtin_amdgcn_ballot_w64(kk < num_topk && pos >= 0 && pos < num_expanded);
+            for (; live; live &= live - 1) copy_to(__builtin_amdgcn_readlane(pos, __builtin_ctzll(live)));
+        }
     } else {
         const int r0 = (b - copy_blocks) * pad_rows;
         for (int r = r0; r < r0 + pad_rows && r < num_expanded; ++r) {
@@ -387,6 +411,9 @@ __global__ __launch_bounds__(kThreads) void expand_to_fused_kernel(const uint8_t
 // threads form kpw groups of tpr threads (tpr * 16 >= row_bytes), and group g copies the row to position kg * kpw + g
 // of the token, still one load and one store per thread.  (With one position per workgroup half or more of the
 // threads had nothing to copy: bf16 [32768, 1024], top-8: 198.7 us, 124.6 us this way.)
+// EVERY as above; without it kpw counts tokens, and group g serves all entries of token b * kpw + g (us, EVERY / per token:
+// codes [21504, 1280] of 8 ranks 47 / 17.5; top-8 of [8192, 1024] codes 26.2 / 24.8; of bf16 [32768, 1024] 133.5 / 138.9).
+template <bool EVERY>
 __global__ __launch_bounds__(kThreads) void expand_short_rows_kernel(const uint8_t *x, int64_t row_bytes, const int32_t *token_topk_to_pos,
                                                                      int num_topk, int kpw, int tpr, int copy_blocks, int num_tokens,
                                                                      int num_expanded, uint8_t *out, const int32_t *pos_to_expert,
@@ -394,22 +421,44 @@ __global__ __launch_bounds__(kThreads) void expand_short_rows_kernel(const uint8
                                                                      int64_t out_sf_ld, int sf_col_major, int pad_rows) {
     const int b = blockIdx.x;
     if (b < copy_blocks) {
-        // b = 8 * ((token group * groups of positions) + kg) + token within its group of 8
-        const int kgroups = (num_topk + kpw - 1) / kpw;
-        const int q = b >> 3;
-        const int kg = q % kgroups, t = (q / kgroups) * 8 + (b & 7);
         const int g = (int)threadIdx.x / tpr, i = (int)threadIdx.x - g * tpr;
-        const int k = kg * kpw + g;
         const int64_t off = (int64_t)i * 16;
+        int k = 0, t;
+        if (EVERY) {
+            // b = 8 * ((token group * groups of positions) + kg) + token within its group of 8
+            const int kgroups = (num_topk + kpw - 1) / kpw;
+            const int q = b >> 3;
+            k = (q % kgroups) * kpw + g;
+            t = (q / kgroups) * 8 + (b & 7);
+        } else {
+            t = b * kpw + g;
+        }
         if (t >= num_tokens || g >= kpw || k >= num_topk) return;
-        const int p = token_topk_to_pos[(int64_t)t * num_topk + k];
+        const u32x4 *src = reinterpret_cast<const u32x4 *>(x + (int64_t)t * row_bytes + off);
+        const int32_t *list = token_topk_to_pos + (int64_t)t * num_topk;
         u32x4 v = u32x4{0u, 0u, 0u, 0u};
-        if (off < row_bytes) v = *reinterpret_cast<const u32x4 *>(x + (int64_t)t * row_bytes + off);   // cached: read num_topk times
-        if (p < 0 || p >= num_expanded) return;
-        if (off < row_bytes) expand_store16(out + (int64_t)p * row_bytes + off, v);
-        if (x_sf)
-            for (int j = i; j < sf_cols; j += tpr)
-                out_sf[sf_col_major ? (int64_t)j * out_sf_ld + p : (int64_t)p * out_sf_ld + j] = x_sf[(int64_t)t * sf_cols + j];
+        auto copy_to = [&](int p) {
+            if (p < 0 || p >= num_expanded) return;
+            if (off < row_bytes) expand_store16(out + (int64_t)p * row_bytes + off, v);
+            if (x_sf)
+                for (int j = i; j < sf_cols; j += tpr)
+                    out_sf[sf_col_major ? (int64_t)j * out_sf_ld + p : (int64_t)p * out_sf_ld + j] = x_sf[(int64_t)t * sf_cols + j];
+        };
+        if (EVERY) {
+            const int p = list[k];
+            if (off < row_bytes) v = *src;   // cached: read num_topk times
+            copy_to(p);
+            return;
+        }
+        if (off < row_bytes) v = *src;
+        for (int k0 = 0; k0 < num_topk; k0 += 8) {
+            int p[8];
+#pragma unroll
+            for (int j = 0; j < 8; ++j) p[j] = list[k0 + j < num_topk ? k0 + j : k0];
+#pragma unroll
+            for (int j = 0; j < 8; ++j)
+                if (k0 + j < num_topk) copy_to(p[j]);
+        }
     } else {
         expand_zero_padding(b - copy_blocks, pad_rows, num_expanded, row_bytes, out, pos_to_expert, x_sf != nullptr, sf_cols, out_sf, out_sf_ld,
                             sf_col_major);
@@ -707,25 +756,39 @@ extern "C" int tk_expand_to_fused(const void *x, int64_t num_tokens, int64_t row
                                             x_sf, sf_cols, out_sf, out_sf_ld, sf_col_major);
     if (rc != TK_OK) return rc;
     const int64_t chunks = (row_bytes + kExpandChunk - 1) / kExpandChunk;
-    // rows of at most half a chunk: several positions of a token per workgroup
+    // A workgroup per list entry only for long outputs with many positions per token, see the kernel's comment.  num_expanded
+    // bounds the live entries; a buffer sized for the worst case looks like a full list here and loses nothing against before.
+    const bool many = num_expanded >= 4 * num_tokens;
+    const bool every = many && num_expanded * row_bytes >= (int64_t)160 << 20;
+    // rows of at most half a chunk: several positions of a token, or several tokens, per workgroup
     const int tpr = (int)((row_bytes + 15) / 16);
-    const int kpw = tpr * 2 <= kThreads ? (kThreads / tpr < num_topk ? kThreads / tpr : num_topk) : 1;
-    const int64_t copy_blocks = (num_tokens + 7) / 8 * 8 * (kpw > 1 ? (num_topk + kpw - 1) / kpw : num_topk * chunks);
+    const bool short_rows = tpr * 2 <= kThreads;
+    const int kpw = !short_rows ? 1 : (every && kThreads / tpr > num_topk ? num_topk : kThreads / tpr);
+    const int64_t token_groups = (num_tokens + 7) / 8 * 8;
+    const int64_t copy_blocks = every ? token_groups * (short_rows ? (num_topk + kpw - 1) / kpw : num_topk * chunks)
+                                      : (short_rows ? (num_tokens + kpw - 1) / kpw : token_groups * chunks);
     // padding workgroups take 8 KB of consecutive rows each, two stores per thread.  Measured (us per call, 1 / 2 / 4
     // rows per workgroup): 8 KB rows 64.4 / 69.7 / 71.0; 4 KB rows with scales 41.4 / 36.0 / 37.0
-    const int pad_rows = row_bytes >= 8192 ? 1 : (int)(8192 / row_bytes > 8 ? 8 : 8192 / row_bytes);
+    int pad_rows = row_bytes >= 8192 ? 1 : (int)(8192 / row_bytes > 8 ? 8 : 8192 / row_bytes);
+    // Most rows of a long buffer are live where tokens have few positions: four times the rows per padding workgroup (codes
+    // of [34816, 7168]: 68.7 -> 62.2 us; with a third of the rows padding it costs 1 to 3 %, and below 16384 rows nothing is won)
+    if (!many && num_expanded >= 16384) pad_rows *= 4;
     const int64_t grid = copy_blocks + (num_expanded + pad_rows - 1) / pad_rows;
     if (grid == 0) return TK_OK;
-    if (kpw > 1)
-        hipLaunchKernelGGL(expand_short_rows_kernel, dim3((unsigned)grid), dim3(kThreads), 0, static_cast<hipStream_t>(stream),
-                           static_cast<const uint8_t *>(x), row_bytes, token_topk_to_pos, num_topk, kpw, tpr, (int)copy_blocks,
-                           (int)num_tokens, (int)num_expanded, static_cast<uint8_t *>(out), pos_to_expert,
-                           static_cast<const uint32_t *>(x_sf), sf_cols, static_cast<uint32_t *>(out_sf), out_sf_ld, sf_col_major, pad_rows);
-    else
-        hipLaunchKernelGGL(expand_to_fused_kernel, dim3((unsigned)grid), dim3(kThreads), 0, static_cast<hipStream_t>(stream),
-                           static_cast<const uint8_t *>(x), row_bytes, token_topk_to_pos, num_topk, (int)chunks, (int)copy_blocks,
-                           (int)num_tokens, (int)num_expanded, static_cast<uint8_t *>(out), pos_to_expert,
-                           static_cast<const uint32_t *>(x_sf), sf_cols, static_cast<uint32_t *>(out_sf), out_sf_ld, sf_col_major, pad_rows);
+    hipStream_t s = static_cast<hipStream_t>(stream);
+#define TK_EXPAND_LAUNCH(KERNEL, ...)                                                                                       \
+    hipLaunchKernelGGL(KERNEL, dim3((unsigned)grid), dim3(kThreads), 0, s, static_cast<const uint8_t *>(x), row_bytes,      \
+                       token_topk_to_pos, num_topk, __VA_ARGS__, (int)copy_blocks, (int)num_tokens, (int)num_expanded,      \
+                       static_cast<uint8_t *>(out), pos_to_expert, static_cast<const uint32_t *>(x_sf), sf_cols,            \
+                       static_cast<uint32_t *>(out_sf), out_sf_ld, sf_col_major, pad_rows)
+    if (short_rows) {
+        if (every) TK_EXPAND_LAUNCH(expand_short_rows_kernel<true>, kpw, tpr);
+        else TK_EXPAND_LAUNCH(expand_short_rows_kernel<false>, kpw, tpr);
+    } else {
+        if (every) TK_EXPAND_LAUNCH(expand_to_fused_kernel<true>, (int)chunks);
+        else TK_EXPAND_LAUNCH(expand_to_fused_kernel<false>, (int)chunks);
+    }
+#undef TK_EXPAND_LAUNCH
     return (int)hipGetLastError();
 }
 
