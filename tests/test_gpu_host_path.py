@@ -1,0 +1,182 @@
+"""The native call path of the ops against their Python code: the same results in the same layout for every form both accept,
+and None (so that the Python code takes the call) for the forms it leaves alone."""
+import itertools
+
+import pytest
+import torch
+
+
+class Recorder:
+    """Stands in for the native functions: counts the calls they took, or leaves all of them to the Python code."""
+
+    def __init__(self, native):
+        self.native, self.taken = native, 0
+
+    def __getattr__(self, name):
+        def call(*args):
+            if self.native is None:
+                return None
+            r = getattr(self.native, name)(*args)
+            self.taken += r is not None
+            return r
+        return call
+
+
+def _flat(r):
+    return [v for item in r for v in _flat(item)] if isinstance(r, (tuple, list)) else [r]
+
+
+def _bytes(t):
+    return t.cpu().clone(memory_format=torch.contiguous_format).view(-1).view(torch.uint8)
+
+
+def _compare(monkeypatch, calls, native=True):
+    from tilekernels_amd import _ffi
+    _ffi.host.per_token_cast        # load
+    host = _ffi.host
+    for name, call in calls:
+        recorder = Recorder(host)
+        monkeypatch.setattr(_ffi, 'host', recorder)
+        got = call()
+        assert bool(recorder.taken) == native, (name, recorder.taken)
+        monkeypatch.setattr(_ffi, 'host', Recorder(None))
+        want = call()
+        monkeypatch.setattr(_ffi, 'host', host)
+        for g, w in zip(_flat(got), _flat(want), strict=True):
+            if isinstance(w, int):
+                assert g == w, name
+                continue
+            assert (g.dtype, g.shape, g.stride(), g.device, g.requires_grad) == (w.dtype, w.shape, w.stride(), w.device, w.requires_grad), name
+            assert g.untyped_storage().nbytes() == w.untyped_storage().nbytes(), name
+            assert torch.equal(_bytes(g), _bytes(w)), name
+
+
+LAYOUTS = [(False, False, False), (False, True, False), (True, False, False), (True, True, True)]
+
+
+def _x(rows, cols, dtype=torch.bfloat16, scale=1.0):
+    g = torch.Generator().manual_seed(rows * 131 + cols)
+    return (torch.randn((rows, cols), generator=g) * scale).to(dtype).cuda()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize('rows', [1, 3, 65])
+def test_casts_and_dequantisation(monkeypatch, rows):
+    import tilekernels_amd as tk
+    q, calls = tk.quant, []
+    for dtype, layout in itertools.product((torch.bfloat16, torch.float32), LAYOUTS):
+        for cols, fmt, group in ((512, 'e4m3', 128), (576, 'e4m3', 64), (704, 'e2m1', 32), (64, 'e4m3', 16), (576, 'e4m3', 576), (584, 'e5m6', 584)):
+            x = _x(rows, cols, dtype)
+            calls.append(((dtype, layout, cols, fmt), lambda x=x, f=fmt, g=group, l=layout: q.per_token_cast(x, f, g, None, *l)))
+            wide = _x(rows, cols + 64, dtype)[:, :cols]
+            calls.append(((dtype, layout, cols, fmt, 'strided'), lambda x=wide, f=fmt, g=group, l=layout: q.per_token_cast(x, f, g, None, *l)))
+        for fmt, block in (('e4m3', (128, 128)), ('e2m1', (32, 32)), ('e4m3', (32, 128))):
+            x = _x(rows, 320, dtype)
+            calls.append(((dtype, layout, fmt, block), lambda x=x, f=fmt, b=block, l=layout: q.per_block_cast(x, f, b, *l)))
+    for fmt, group, layout in (('e4m3', 128, LAYOUTS[0]), ('e4m3', 32, LAYOUTS[2]), ('e2m1', 32, LAYOUTS[3]), ('e4m3', 64, LAYOUTS[3]),
+                               ('e2m1', 128, LAYOUTS[0])):
+        for cols in (128, 1088):
+            codes = q.per_token_cast_with_sf_only(_x(rows, cols), fmt, group, None, *layout), q.per_token_cast(_x(rows, cols), fmt, group, None, *layout)
+            codes = (codes[1][0], codes[0])
+            for back in ('bf16', 'fp32'):
+                calls.append(((fmt, group, layout, cols, back), lambda c=codes, b=back, g=group: q.per_token_cast_back(c, b, g)))
+            for out in LAYOUTS:
+                calls.append(((fmt, group, layout, cols, out), lambda c=codes, g=group, l=out: q.per_token_cast(c, 'e4m3', 32, (1, g), *l)))
+    codes = q.per_token_cast(_x(rows, 584), 'e5m6', 584)
+    calls.append(('e5m6', lambda: q.per_token_cast_back(codes, 'bf16', 584, 'e5m6')))
+    _compare(monkeypatch, calls)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize('tokens,hidden', [(1, 256), (97, 768)])
+def test_expanded_ops(monkeypatch, tokens, hidden):
+    import tilekernels_amd as tk
+    q, moe, calls = tk.quant, tk.moe, []
+    g = torch.Generator().manual_seed(tokens)
+    idx = torch.topk(torch.rand((tokens, 16), generator=g), 4, dim=-1).indices
+    idx = idx.masked_fill(idx > 7, -1)
+    idx[0, 0] = 3
+    idx, weights = idx.cuda(), torch.rand((tokens, 4), generator=g).cuda()
+    for args in ((8, 0, 16), (8, 0, 64), (8, 2048, 16), (8, 0, 16, True)):
+        def mapping(args=args):
+            m = moe.get_fused_mapping(idx, *args)
+            return m if args[1] == 0 and len(args) == 3 else (m[3:7], m[7])     # (buffers longer than the live rows have an unwritten end)
+        calls.append((args, mapping))
+    maps = moe.get_fused_mapping(idx, 8, 0, 16)
+    p2e, p2t, p2tk, t2p = maps[:4]
+    rows = p2e.shape[0]
+    x = _x(tokens, hidden)
+    calls.append(('expand', lambda: moe.expand_to_fused(x, t2p, p2e)))
+    for layout in (LAYOUTS[0], LAYOUTS[3]):
+        codes, sf = q.per_token_cast(x, 'e4m3', 128, None, *layout)
+        for col in ((True,) if sf.dtype == torch.int32 else (False, True)):
+            calls.append((('expand', layout, col), lambda c=codes, s=sf.contiguous(), col=col: moe.expand_to_fused_with_sf((c, s), 128, t2p, p2e, col)))
+    y = _x(rows, hidden)
+    row_sf, one = torch.rand((rows,), generator=g).cuda(), torch.full((1,), 0.5, device='cuda')
+    for dtype in (torch.bfloat16, torch.float32):
+        for args in ((y.to(dtype), None, t2p), (y.to(dtype), weights, t2p), ((y.to(dtype), row_sf), weights, t2p), (y.to(dtype), weights, t2p, 'e4m3', one)):
+            calls.append((('reduce', dtype, len(args)), lambda args=args: moe.reduce_fused(*args)))
+        z = _x(rows, 2 * hidden, dtype, 2.0)
+        for layout, clamp in itertools.product(LAYOUTS, (None, 1.5)):
+            calls.append((('swiglu', dtype, layout, clamp),
+                          lambda z=z, l=layout, c=clamp: q.swiglu_forward_and_per_token_cast(z, 'e4m3', 128, p2tk, weights, p2e, *l, swiglu_clamp_value=c)))
+        calls.append((('swiglu row', dtype), lambda z=z: q.swiglu_forward_and_per_token_cast(z, 'e4m3', hidden, sf_clamp_min=1e-3)))
+    for group, clamp in ((32, None), (128, 1.5)):
+        codes = q.per_token_cast(_x(rows, 2 * hidden, scale=2.0), 'e4m3', group)
+        calls.append((('backward', group), lambda c=codes, g=group, cl=clamp: q.swiglu_backward_and_per_token_cast(c, y, weights, p2tk, t2p, g,
+                                                                                                                   swiglu_clamp_value=cl)))
+    t = _x(128, hidden)
+    quantised = q.per_token_cast(_x(tokens, hidden), 'e4m3', 128)
+    calls += [('channel', lambda: q.per_channel_cast(t, 'e4m3', 128, True)), ('transpose', lambda: q.per_channel_cast_and_transpose(t, 'e4m3', 32)),
+              ('gather', lambda: q.per_channel_cast_fused(quantised, 'e4m3', 128, num_per_channels=128, pos_to_token=p2t)),
+              ('swiglu channel', lambda: q.swiglu_forward_and_per_channel_cast_and_transpose(t, 'e4m3', 128, swiglu_clamp_value=1.5))]
+    _compare(monkeypatch, calls)
+
+
+@pytest.mark.gpu
+def test_calls_the_python_code_takes(monkeypatch):
+    """Empty inputs, modes, number types and options the native path leaves alone: the result is that of the Python code."""
+    import tilekernels_amd as tk
+    from torch.utils._python_dispatch import TorchDispatchMode
+    q = tk.quant
+    x = _x(8, 512)
+
+    class Seen(TorchDispatchMode):
+        calls = 0
+
+        def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+            Seen.calls += 1
+            return func(*args, **(kwargs or {}))
+
+    def in_mode():
+        with Seen():
+            return q.per_token_cast(x, 'e4m3', 128)
+
+    _compare(monkeypatch, [('mode', in_mode), ('empty', lambda: q.per_token_cast(x[:0], 'e4m3', 128)),
+                           ('options as numbers', lambda: q.per_token_cast(x, 'e4m3', 128, None, 1, 1, 1)),
+                           ('integer clamp', lambda: q.swiglu_forward_and_per_token_cast(x, 'e4m3', 128, swiglu_clamp_value=2))], native=False)
+    assert Seen.calls > 0
+    for bad in (lambda: q.per_token_cast(x, 'e4m3', 48), lambda: q.per_token_cast(x, 'e3m4', 128), lambda: q.per_token_cast(x.half(), 'e4m3', 128),
+                lambda: q.per_block_cast(x.T, 'e4m3', (128, 128)), lambda: q.per_token_cast(x, 'e4m3', 128, None, False, False, True),
+                lambda: tk.moe.reduce_fused(x[:, :128], None, torch.zeros((1, 1), dtype=torch.int32, device='cuda'))):
+        with pytest.raises(AssertionError):
+            bad()
+    from tilekernels_amd._ffi import TkError
+    with pytest.raises(TkError):                     # misaligned rows
+        q.per_token_cast(_x(8, 513)[:, 1:], 'e4m3', 128)
+
+
+@pytest.mark.parametrize('op', ['per_token_cast', 'per_block_cast', 'cast_back', 'swiglu_forward', 'reduce_fused', 'expand_to_fused', 'get_fused_mapping'])
+def test_cpu_tensors_are_left_alone(op):
+    from tilekernels_amd import _ffi
+    x, sf = torch.zeros((4, 512), dtype=torch.bfloat16), torch.ones((4, 4))
+    t2p, e = torch.zeros((4, 2), dtype=torch.int32), torch.zeros((8,), dtype=torch.int32)
+    args = {'per_token_cast': (x, 'e4m3', 128, None, False, False, False), 'per_block_cast': (x, 'e4m3', (128, 128), False, False, False),
+            'cast_back': ((x.to(torch.float8_e4m3fn), sf), 'bf16', 1, 128, None), 'reduce_fused': (x, None, t2p, '', None),
+            'swiglu_forward': (x, 'e4m3', 128, None, None, None, False, False, False, None, None),
+            'expand_to_fused': (x, None, None, t2p, e, False), 'get_fused_mapping': (t2p.long(), 8, 0, 16, False)}[op]
+    fn = getattr(_ffi.host, op)
+    assert fn(*args) is None
+    assert fn(*[None] * len(args)) is None and fn(*[object()] * len(args)) is None
+    with pytest.raises(TypeError):
+        fn()

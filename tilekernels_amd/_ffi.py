@@ -3,12 +3,14 @@
 There is deliberately no fallback: if the library has not been built, importing the ops raises.
 """
 import ctypes
+import importlib.util
 import os
 
 import torch  # noqa: F401  (loads the HIP runtime the library links against before the library itself)
 
 _PKG = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_PKG, 'lib', 'libtk_quant.so')
+HOST_PATH = os.path.join(_PKG, 'lib', '_host.so')
 
 TK_BF16, TK_F32, TK_OUT_E4M3 = 0, 1, 2
 TK_E4M3, TK_E2M1, TK_E5M6 = 0, 1, 2
@@ -77,6 +79,25 @@ def load() -> ctypes.CDLL:
             fn.argtypes = args
         _lib = lib
     return _lib
+
+
+class _UnloadedHost:
+    """Stands in `host` until the first op is called: importing the package does not need the built libraries."""
+
+    def __getattr__(self, name):
+        global host
+        load()
+        if not os.path.exists(HOST_PATH):
+            raise ImportError(f'{HOST_PATH} not found: build it with `python -m tilekernels_amd.build`')
+        spec = importlib.util.spec_from_file_location('tilekernels_amd._host', HOST_PATH)
+        module = importlib.util.module_from_spec(spec)
+        spec.loader.exec_module(module)
+        host = module
+        return getattr(module, name)
+
+
+# the native call path (csrc/host.cpp): each function gives an op's result, or None for calls that its Python code is to take
+host = _UnloadedHost()
 
 
 class TkError(RuntimeError):

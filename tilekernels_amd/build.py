@@ -1,19 +1,21 @@
-"""Ahead-of-time build of libtk_quant.so (hipcc, gfx950 only).
+"""Ahead-of-time build of libtk_quant.so (hipcc, gfx950 only) and of _host.so, the ops' native call path (host code on torch).
 
     python -m tilekernels_amd.build [--force]
 
-The library is written to tilekernels_amd/lib/ inside the source tree so that it travels with
+The libraries are written to tilekernels_amd/lib/ inside the source tree so that they travel with
 the checkout; nothing is JIT-compiled at run time.
 """
 import os
 import subprocess
 import sys
+import sysconfig
 from concurrent.futures import ThreadPoolExecutor
 
 PKG = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(PKG, 'csrc')
 LIB_DIR = os.path.join(PKG, 'lib')
 LIB_PATH = os.path.join(LIB_DIR, 'libtk_quant.so')
+HOST_PATH = os.path.join(LIB_DIR, '_host.so')
 SOURCES = ['api.hip', 'per_token_cast.hip', 'per_block_cast.hip', 'swiglu_cast.hip', 'cast_back.hip', 'moe_layout.hip',
            'swiglu_backward.hip', 'per_channel_cast.hip', 'lossless_cast.hip', 'stream_floor.hip', 'swiglu_cast_variants.hip']
 
@@ -43,9 +45,20 @@ def _compile(src: str) -> str:
     return obj
 
 
+def _build_host() -> None:
+    import torch
+    root = os.path.dirname(torch.__file__)
+    cmd = [os.environ.get('CXX', 'g++'), '-O2', '-std=c++17', '-fPIC', '-shared', '-Wall', '-D__HIP_PLATFORM_AMD__=1', '-DUSE_ROCM=1',
+           f'-I{root}/include', f'-I{sysconfig.get_paths()["include"]}', '-I/opt/rocm/include', os.path.join(CSRC, 'host.cpp'), '-o', HOST_PATH,
+           f'-L{LIB_DIR}', '-l:libtk_quant.so', f'-L{root}/lib', '-lc10', '-lc10_hip', '-ltorch_cpu', '-ltorch_python', '-Wl,-rpath,$ORIGIN']
+    r = subprocess.run(cmd, capture_output=True, text=True)
+    if r.returncode != 0:
+        raise RuntimeError(f'the build of _host.so failed:\n{r.stderr}')
+
+
 def build_library(force: bool = True) -> str:
-    """Compile every HIP source and link libtk_quant.so.  Returns its path."""
-    if not force and os.path.exists(LIB_PATH):
+    """Compile every HIP source, link libtk_quant.so and build _host.so beside it.  Returns the path of libtk_quant.so."""
+    if not force and os.path.exists(LIB_PATH) and os.path.exists(HOST_PATH):
         return LIB_PATH
     os.makedirs(LIB_DIR, exist_ok=True)
     with ThreadPoolExecutor(max_workers=min(len(SOURCES), 8)) as ex:
@@ -56,6 +69,7 @@ def build_library(force: bool = True) -> str:
         raise RuntimeError(f'link failed:\n{r.stderr}')
     for o in objs:
         os.remove(o)
+    _build_host()
     return LIB_PATH
 
 

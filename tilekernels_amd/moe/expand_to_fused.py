@@ -9,6 +9,9 @@ from ..utils import align, ceil_div
 def expand_to_fused(x: torch.Tensor, token_topk_to_pos: torch.Tensor, pos_to_expert: torch.Tensor) -> torch.Tensor:
     """Copy row ``t`` of ``x`` to every expanded position ``token_topk_to_pos[t, k] >= 0``; padding rows
     (``pos_to_expert < 0``) are zero."""
+    done = _ffi.host.expand_to_fused(x, None, None, token_topk_to_pos, pos_to_expert, False)
+    if done is not None:
+        return done
     assert x.is_contiguous() and token_topk_to_pos.is_contiguous()
     assert x.dim() == 2 and token_topk_to_pos.dim() == 2
     assert token_topk_to_pos.dtype == torch.int32 and pos_to_expert.dtype == torch.int32 and pos_to_expert.is_contiguous()
@@ -33,6 +36,10 @@ def expand_to_fused_with_sf(x: QuantTensor, num_per_channels: int, token_topk_to
     """:func:`expand_to_fused` for codes plus their (contiguous, row-per-token) scale rows; the expanded
     scales are row-major or, with ``use_tma_aligned_col_major_sf``, column-major over a 4-row-aligned buffer."""
     x, x_sf = x
+    if x_sf is not None:
+        done = _ffi.host.expand_to_fused(x, x_sf, num_per_channels, token_topk_to_pos, pos_to_expert, use_tma_aligned_col_major_sf)
+        if done is not None:
+            return done
     assert x.is_contiguous() and x_sf.is_contiguous() and token_topk_to_pos.is_contiguous() and pos_to_expert.is_contiguous()
     assert x.dim() == 2 and token_topk_to_pos.dim() == 2 and pos_to_expert.dim() == 1
     assert x_sf.dtype in (torch.float32, torch.int32)

@@ -15,6 +15,9 @@ def get_fused_mapping(topk_idx: torch.Tensor, num_experts: int, num_expanded_tok
     Returns ``(pos_to_expert, pos_to_token, pos_to_token_topk, token_topk_to_pos, expert_start, expert_end,
     num_tokens_per_expert, num_tokens_per_expert_list)``; the list is empty unless a sync happened.
     """
+    done = _ffi.host.get_fused_mapping(topk_idx, num_experts, num_expanded_tokens, alignment, force_no_sync)
+    if done is not None:
+        return done
     num_tokens, num_topk = topk_idx.shape
     assert topk_idx.is_contiguous() and topk_idx.dtype == torch.int64
     dev = _ffi.require_gpu(topk_idx)

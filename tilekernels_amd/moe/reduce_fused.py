@@ -21,6 +21,10 @@ def reduce_fused(
     """``out[t] = sum_k x[token_topk_to_pos[t, k]] * topk_weights[t, k]`` (positions < 0 skipped), accumulated in
     fp32; ``x`` may be ``(data, x_sf)`` with one fp32 factor per expanded row.  ``fp8_format='e4m3'`` gives an FP8
     result, scaled by the one-element tensor ``sf`` if given; otherwise the result has the dtype of ``x``."""
+    if out is None:
+        done = _ffi.host.reduce_fused(x, topk_weights, token_topk_to_pos, fp8_format, sf)
+        if done is not None:
+            return done
     x_sf = None
     if isinstance(x, tuple):
         x, x_sf = x

@@ -14,6 +14,10 @@ from .types import QuantTensor
 def cast_back(x: QuantTensor, fmt: str, x_block_size: tuple, x_special_fmt: Optional[str] = None) -> torch.Tensor:
     """Dequantise ``(data, sf)`` to ``'bf16'`` or ``'fp32'``; ``x_block_size`` is the
     ``(rows, channels)`` extent that shares one scale."""
+    if isinstance(x_block_size, tuple) and len(x_block_size) == 2:
+        done = _ffi.host.cast_back(x, fmt, x_block_size[0], x_block_size[1], x_special_fmt)
+        if done is not None:
+            return done
     assert fmt in ('bf16', 'fp32')
     out_dtype = torch.bfloat16 if fmt == 'bf16' else torch.float32
     data, x_sf = x

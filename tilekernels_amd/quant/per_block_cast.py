@@ -60,6 +60,9 @@ def per_block_cast(
 ) -> QuantTensor:
     """Cast contiguous ``x[num_tokens, hidden]`` to FP8/FP4 with one scale per ``block_size`` block.
     Returns ``(out, out_sf)``."""
+    done = _ffi.host.per_block_cast(x, fmt, block_size, use_tma_aligned_col_major_sf, round_sf, use_packed_ue8m0)
+    if done is not None:
+        return done
     return per_block_cast_impl(x, fmt, block_size, use_tma_aligned_col_major_sf, round_sf, use_packed_ue8m0)
 
 

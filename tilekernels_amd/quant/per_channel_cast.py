@@ -15,6 +15,10 @@ from .types import QuantTensor
 
 def _launch(x, x_sf, num_tokens, hidden, pos_to_token, num_tokens_out, num_per_tokens, round_sf, transpose,
             swiglu=False, swiglu_clamp_value=None):
+    done = _ffi.host.per_channel_cast(x, x_sf, num_tokens, hidden, pos_to_token, num_tokens_out, num_per_tokens, round_sf, transpose, swiglu,
+                                      swiglu_clamp_value)
+    if done is not None:
+        return done
     dev = _ffi.require_gpu(x, x_sf, pos_to_token)
     lib = _ffi.load()
     out_shape = (hidden, num_tokens_out) if transpose else (num_tokens_out, hidden)

@@ -123,6 +123,9 @@ def per_token_cast(
     """Cast ``x[num_tokens, hidden]`` to FP8 (``'e4m3'``) or packed FP4 (``'e2m1'``) with one scale per
     ``num_per_channels`` consecutive channels of a token, or to packed 12-bit ``'e5m6'`` (uint8
     ``[num_tokens, hidden * 3 // 2]``) with one scale per token.  Returns ``(out, out_sf)``."""
+    done = _ffi.host.per_token_cast(x, fmt, num_per_channels, x_block_size, use_tma_aligned_col_major_sf, round_sf, use_packed_ue8m0)
+    if done is not None:
+        return done
     return per_token_cast_impl(x, fmt, num_per_channels, x_block_size, use_tma_aligned_col_major_sf, round_sf, use_packed_ue8m0)
 
 

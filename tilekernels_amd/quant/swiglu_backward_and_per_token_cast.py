@@ -29,6 +29,9 @@ def swiglu_backward_and_per_token_cast(
     input gradient quantised per token in groups of ``num_per_channels`` (32 or 128), the same gradient
     in bf16, and the fp32 gradient of the routing weights ``[num_tokens, num_topk]``.
     """
+    done = _ffi.host.swiglu_backward(x, grad_out, weight, pos_to_token_topk, token_topk_to_pos, num_per_channels, round_sf, swiglu_clamp_value)
+    if done is not None:
+        return done
     assert num_per_channels in (32, 128)
     x, x_sf = x
 

@@ -33,6 +33,11 @@ def swiglu_forward_and_per_token_cast(
     Rows whose ``pos_to_expert`` entry is negative are padding: their codes and scales are zeros.
     ``clamped_count`` (int64[3]) is incremented in place.  Returns ``(out, out_sf)``.
     """
+    if clamped_count is None:
+        done = _ffi.host.swiglu_forward(x, fmt, num_per_channels, pos_to_token_topk, topk_weights, pos_to_expert, use_tma_aligned_col_major_sf,
+                                        round_sf, use_packed_ue8m0, swiglu_clamp_value, sf_clamp_min)
+        if done is not None:
+            return done
     assert x.dim() == 2 and x.is_contiguous()
     assert x.dtype in (torch.bfloat16, torch.float32)
     num_expanded_tokens, hidden = x.shape
