@@ -138,3 +138,23 @@ def test_expand_to_fused_long_output_with_full_lists(dim):
         here = (t2p[:, k] >= 0).cuda()
         want[t2p[:, k].cuda()[here].long()] = x[here]
     assert torch.equal(got.view(torch.int16), want.view(torch.int16))
+
+
+@pytest.mark.parametrize('T,K,E,drop,alignment', [(65536, 1, 1, 0.0, 128), (65537, 1, 512, 0.0, 16), (8200, 8, 3, 0.9, 128), (12000, 6, 9, 1.0, 16),
+                                                  (95000, 8, 256, 0.9, 128), (100001, 9, 4, 0.5, 64)])
+def test_mapping_of_long_lists(T, K, E, drop, alignment):
+    """Lists from 64 Ki pairs on, which are counted into a table first (95000 x 8 of 256 experts: too long for it, three launches);
+    buffers that are longer, and shorter, than the expanded rows."""
+    tk = _tk()
+    g = torch.Generator().manual_seed(T)
+    idx = torch.randint(0, E, (T, K), generator=g)
+    idx = idx.masked_fill(torch.rand(idx.shape, generator=g) < drop, -1).contiguous()
+    want = torch_ref.get_fused_mapping(idx, E, alignment)
+    rows = want[0].numel()
+    for extra in (0, 1000, -(rows // 3)):
+        got = tk.moe.get_fused_mapping(idx.cuda(), E, rows + extra, alignment, force_no_sync=True)
+        n = min(rows, rows + extra)
+        for name, a, b in zip(('pos_to_expert', 'pos_to_token', 'pos_to_token_topk'), got[:3], want[:3]):
+            assert torch.equal(a.cpu()[:n], b[:n]) and bool((a.cpu()[n:] == -1).all()), (name, extra)
+        for a, b, name in zip(got[3:7], want[3:7], ('token_topk_to_pos', 'expert_start', 'expert_end', 'num_tokens_per_expert')):
+            assert_same(a, b, name)

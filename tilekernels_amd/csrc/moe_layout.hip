@@ -15,10 +15,10 @@ namespace tk {
 
 // ------------------------------------------------------------------------------------------------
 // get_fused_mapping: a stable counting sort of the flat (token, k) list by expert, every expert's
-// segment padded to a multiple of `alignment`.  Lists of more than 64 Ki pairs take three launches, no grid-wide
-// barrier (a single workgroup doing all of it was measured at 70 us for 32 Ki pairs against 18 us for the three
-// launches: one CU cannot absorb the scattered 4-byte stores of the hand-out); shorter lists take the single
-// launch of several workgroups further down:
+// segment padded to a multiple of `alignment`.  Lists of up to 64 Ki pairs take a single launch of
+// several workgroups, longer ones two launches (both further down), the longest, and those of more than 512 experts, three, with no
+// grid-wide barrier (a single workgroup doing all of it was measured at 70 us for 32 Ki pairs against 18 us for the three
+// launches: one CU cannot absorb the scattered 4-byte stores of the hand-out):
 //   count  : each wave histograms its own 256-element slice            -> ws[slice][expert]
 //   scan   : one workgroup turns the histograms into exclusive offsets  -> ws[slice][expert], expert_start/end
 //   assign : each wave walks its slice again in order and hands out positions
@@ -171,6 +171,26 @@ __global__ __launch_bounds__(1024) void fused_mapping_scan_kernel(int32_t *ws, i
     }
 }
 
+// Row b of the table: how many of the entries 1024 b .. 1024 b + 1023 each expert has.
+__global__ __launch_bounds__(kThreads) void fused_mapping_table_kernel(const int64_t *topk_idx, int numel, int num_experts, int32_t *table) {
+    extern __shared__ int32_t hist[];   // [num_experts]
+    constexpr int U = 1024 / kThreads;
+    const int base = blockIdx.x * 1024;
+    int64_t ids[U];
+#pragma unroll
+    for (int j = 0; j < U; ++j) {
+        const int i = base + j * kThreads + (int)threadIdx.x;
+        ids[j] = topk_idx[i < numel ? i : base];
+    }
+    for (int e = threadIdx.x; e < num_experts; e += kThreads) hist[e] = 0;
+    __syncthreads();
+#pragma unroll
+    for (int j = 0; j < U; ++j)
+        if (base + j * kThreads + (int)threadIdx.x < numel && ids[j] >= 0 && ids[j] < num_experts) atomicAdd(&hist[(int)ids[j]], 1);
+    __syncthreads();
+    for (int e = threadIdx.x; e < num_experts; e += kThreads) table[(int64_t)blockIdx.x * num_experts + e] = hist[e];
+}
+
 // The whole mapping in one launch, for lists of up to kSingleLaunchPairs (token, k) pairs: no launch has to wait for
 // another, and no table in global memory is needed.  A workgroup of 16 waves owns 16 consecutive slices of 64, and instead
 // of being told how many entries of every expert precede them it counts them itself: every workgroup reads the whole
@@ -186,27 +206,58 @@ constexpr int kSingleSlice = 64;            // entries a wave hands out: 1024 pe
                                             // hand-out spread over many CUs (256 per wave, 8 workgroups for 32 Ki pairs: 13.6 us)
 constexpr int kSingleMaxExperts = 512;      // (1 + kSingleWaves) histograms of 4-byte counters must fit the LDS of a workgroup
 
+// TABLE: longer lists, in two launches.  fused_mapping_table_kernel counts the entries of every 1024 into one row of a table, and
+// the workgroups of this kernel sum the table's columns (all rows, and the rows before their own) in place of reading the list.
+// What the three launches spent their time on is the scan in the middle: one workgroup, two walks over a table with a row per
+// 256 entries, 8.3 of 20 us for 172160 pairs.  A workgroup reads the whole table here, so the table is held short: see
+// table_mapping_pays.
+template <bool TABLE>
 __global__ __launch_bounds__(64 * kSingleWaves) void fused_mapping_single_kernel(const int64_t *topk_idx, int numel, int num_topk,
                                                                                 int num_experts, int expert_bits, int alignment,
                                                                                 int32_t *pos_to_expert, int32_t *pos_to_token,
                                                                                 int32_t *pos_to_token_topk, int32_t *token_topk_to_pos,
                                                                                 int32_t *expert_start, int32_t *expert_end,
-                                                                                int32_t *num_tokens_per_expert, int num_expanded) {
+                                                                                int32_t *num_tokens_per_expert, int num_expanded,
+                                                                                const int32_t *table) {
     // counts[e]: entries of expert e in the whole list (low half) and before this workgroup's range (high half): one
     // LDS atomic per entry for both, which is what this pass spends its time on (a list of fewer than 64 Ki pairs
-    // cannot overflow a half); slice[w][e]: entries of expert e in slice w of the workgroup's own range
-    extern __shared__ int32_t hist[];        // counts[E], slice[kSingleWaves][E]
+    // cannot overflow a half; TABLE: two words); slice[w][e]: entries of expert e in slice w of the workgroup's own range
+    extern __shared__ int32_t hist[];        // counts[E] (TABLE: all[E], before[E]), slice[kSingleWaves][E]
     __shared__ int32_t padded[kSingleMaxExperts];
     __shared__ int32_t ends[kSingleMaxExperts];
     __shared__ int32_t wave_total[kSingleMaxExperts / 64];
     uint32_t *counts = reinterpret_cast<uint32_t *>(hist);
-    int32_t *slice = hist + num_experts;
+    constexpr int kCounts = TABLE ? 2 : 1;
+    int32_t *slice = hist + kCounts * num_experts;
     const int tid = threadIdx.x, lane = tid & 63, wave = wave_id();
     const int nthreads = 64 * kSingleWaves;
     const int own_base = blockIdx.x * (kSingleWaves * kSingleSlice), own_end = own_base + kSingleWaves * kSingleSlice;
 
-    for (int i = tid; i < (1 + kSingleWaves) * num_experts; i += nthreads) hist[i] = 0;
+    auto all_of = [&](int e) { return (int32_t)(TABLE ? counts[e] : counts[e] & 0xFFFFu); };
+    auto before_of = [&](int e) { return (int32_t)(TABLE ? counts[num_experts + e] : counts[e] >> 16); };
+
+    for (int i = tid; i < (kCounts + kSingleWaves) * num_experts; i += nthreads) hist[i] = 0;
     __syncthreads();
+    if constexpr (TABLE) {
+        static_assert(kSingleSlice == 64, "one entry per thread");
+        const int i = own_base + tid;
+        const int64_t v = topk_idx[i < numel ? i : 0];
+        // threads beyond the last whole table row of the 1024 words idle; the others read consecutive words
+        const int lead = nthreads / num_experts * num_experts, words = (int)gridDim.x * num_experts, own_word = (int)blockIdx.x * num_experts;
+        if (tid < lead) {
+            int32_t all = 0, before = 0;
+#pragma unroll 8
+            for (int w = tid; w < words; w += lead) {
+                const int32_t n = table[w];
+                all += n;
+                before += w < own_word ? n : 0;
+            }
+            const int e = tid % num_experts;
+            if (all) atomicAdd(&hist[e], all);
+            if (before) atomicAdd(&hist[num_experts + e], before);
+        }
+        if (i < numel && v >= 0 && v < num_experts) atomicAdd(&slice[wave * num_experts + (int)v], 1);
+    }
     auto count = [&](int i, int64_t v) {
         if (v >= 0 && v < num_experts) {
             const int e = (int)v;
@@ -216,8 +267,8 @@ __global__ __launch_bounds__(64 * kSingleWaves) void fused_mapping_single_kernel
     };
     // The list is read in 16-byte pieces (two ids), 16 of them per thread in flight at a time: with a load or four at a
     // time the pass took as many memory round trips as it has iterations (24 us for 32 Ki pairs).
-    const int head = (int)((reinterpret_cast<uintptr_t>(topk_idx) >> 3) & 1);      // ids before the first 16-byte boundary
-    const int pairs = (numel - head) / 2;
+    const int head = TABLE ? 0 : (int)((reinterpret_cast<uintptr_t>(topk_idx) >> 3) & 1);      // ids before the first 16-byte boundary
+    const int pairs = TABLE ? 0 : (numel - head) / 2;
     const u32x4 *wide = reinterpret_cast<const u32x4 *>(topk_idx + head);
     constexpr int U = 16;
     for (int p0 = 0; p0 < pairs; p0 += U * nthreads) {
@@ -238,12 +289,12 @@ __global__ __launch_bounds__(64 * kSingleWaves) void fused_mapping_single_kernel
         }
     }
     if (tid == 0 && head) count(0, topk_idx[0]);
-    if (tid == 1 && head + 2 * pairs < numel) count(numel - 1, topk_idx[numel - 1]);
+    if (!TABLE && tid == 1 && head + 2 * pairs < numel) count(numel - 1, topk_idx[numel - 1]);
     __syncthreads();
     // prefix sum over the padded expert sizes: inside each wave by shuffles, across the (at most 8) waves through LDS
     int32_t mine = 0, incl = 0;
     if (tid < kSingleMaxExperts) {
-        mine = tid < num_experts ? (int32_t)(((counts[tid] & 0xFFFFu) + alignment - 1) / alignment * alignment) : 0;
+        mine = tid < num_experts ? (int32_t)(((uint32_t)all_of(tid) + alignment - 1) / alignment * alignment) : 0;
         incl = mine;
 #pragma unroll
         for (int d = 1; d < 64; d <<= 1) {
@@ -265,7 +316,7 @@ __global__ __launch_bounds__(64 * kSingleWaves) void fused_mapping_single_kernel
             num_tokens_per_expert[tid] = mine;
         }
         // first position of every slice of this workgroup inside the expert
-        int32_t run = start + (int32_t)(counts[tid] >> 16);
+        int32_t run = start + before_of(tid);
         for (int w = 0; w < kSingleWaves; ++w) {
             const int32_t n = slice[w * num_experts + tid];
             slice[w * num_experts + tid] = run;
@@ -278,11 +329,29 @@ __global__ __launch_bounds__(64 * kSingleWaves) void fused_mapping_single_kernel
     if (base < numel)
         assign_range<kSingleSlice / 64>(topk_idx, base, numel, num_topk, num_experts, expert_bits, slice + wave * num_experts, nullptr,
                                         pos_to_token, pos_to_token_topk, token_topk_to_pos, num_expanded);
+    if constexpr (TABLE) {
+        // Every position's expert by bisection of the ends, and the padding marks, in one stride over the buffers.
+        for (int64_t i = (int)blockIdx.x * nthreads + tid; i < num_expanded; i += (int)gridDim.x * nthreads) {
+            int lo = 0, hi = num_experts - 1;              // the first expert that ends behind i (experts without entries end where they start)
+            while (lo < hi) {
+                const int mid = (lo + hi) >> 1;
+                if (ends[mid] > i) hi = mid;
+                else lo = mid + 1;
+            }
+            const bool live = i < total && i < ends[lo] - padded[lo] + all_of(lo);
+            pos_to_expert[i] = live ? lo : -1;
+            if (!live) {
+                pos_to_token[i] = -1;
+                pos_to_token_topk[i] = -1;
+            }
+        }
+        return;
+    }
     // The experts this workgroup looks after, a wave per expert: pos_to_expert of the whole segment (it follows from the
     // offsets, and written here it leaves as whole lines instead of one scattered word per entry: the hand-out above
     // is bound by the rate at which one CU issues scattered stores) and the padding marks at the segment's end.
     for (int e = (int)blockIdx.x + wave * (int)gridDim.x; e < num_experts; e += kSingleWaves * (int)gridDim.x) {
-        const int end = ends[e], start = end - padded[e], first = start + (int)(counts[e] & 0xFFFFu);
+        const int end = ends[e], start = end - padded[e], first = start + all_of(e);
         for (int i = start + lane; i < end && i < num_expanded; i += 64) pos_to_expert[i] = i < first ? e : -1;
         for (int i = first + lane; i < end && i < num_expanded; i += 64) {
             pos_to_token[i] = -1;
@@ -628,7 +697,14 @@ extern "C" int tk_check_get_fused_mapping(const int64_t *topk_idx, int64_t num_t
     return TK_OK;
 }
 
-// the three launches; `ws` holds at least tk_fused_mapping_workspace_bytes() bytes
+// Whether the two launches around a table (a row per 1024 pairs) beat the three: every workgroup reads the whole table, groups^2 *
+// experts words in all.  us on MI355X, three launches / table: 172160 pairs of 32 experts (0.9 Mi words) 15.5 / 8.5, 73728 of 256
+// (1.3 Mi) 23.0 / 10.2, 1048576 of 64 (64 Mi) 64 / 30, 2097152 of 32 (128 Mi) 56 / 45; beyond that not measured.
+static bool table_mapping_pays(int64_t groups, int64_t num_experts) {
+    return num_experts <= kSingleMaxExperts && groups <= (1 << 13) && groups * groups * num_experts <= (1 << 27);
+}
+
+// `ws` holds at least tk_fused_mapping_workspace_bytes() bytes
 static int launch_fused_mapping(const int64_t *topk_idx, int64_t num_tokens, int num_topk, int num_experts, int alignment,
                                 int64_t num_expanded, int32_t *pos_to_expert, int32_t *pos_to_token, int32_t *pos_to_token_topk,
                                 int32_t *token_topk_to_pos, int32_t *expert_start, int32_t *expert_end,
@@ -641,10 +717,20 @@ static int launch_fused_mapping(const int64_t *topk_idx, int64_t num_tokens, int
     while ((1 << bits) < num_experts) ++bits;
     if (numel > 0 && numel <= kSingleLaunchPairs && num_experts <= kSingleMaxExperts) {
         const int groups = (numel + kSingleWaves * kSingleSlice - 1) / (kSingleWaves * kSingleSlice);
-        hipLaunchKernelGGL(fused_mapping_single_kernel, dim3(groups), dim3(64 * kSingleWaves),
+        hipLaunchKernelGGL(fused_mapping_single_kernel<false>, dim3(groups), dim3(64 * kSingleWaves),
                            (size_t)(1 + kSingleWaves) * num_experts * sizeof(int32_t), s, topk_idx, numel, num_topk, num_experts, bits,
                            alignment, pos_to_expert, pos_to_token, pos_to_token_topk, token_topk_to_pos, expert_start, expert_end,
-                           num_tokens_per_expert, (int)num_expanded);
+                           num_tokens_per_expert, (int)num_expanded, nullptr);
+        return (int)hipGetLastError();
+    }
+    const int groups = (numel + 1023) / 1024;
+    if (numel > 0 && table_mapping_pays(groups, num_experts)) {
+        hipLaunchKernelGGL(fused_mapping_table_kernel, dim3(groups), dim3(kThreads), (size_t)num_experts * sizeof(int32_t), s, topk_idx, numel,
+                           num_experts, ws);
+        hipLaunchKernelGGL(fused_mapping_single_kernel<true>, dim3(groups), dim3(64 * kSingleWaves),
+                           (size_t)(2 + kSingleWaves) * num_experts * sizeof(int32_t), s, topk_idx, numel, num_topk, num_experts, bits,
+                           alignment, pos_to_expert, pos_to_token, pos_to_token_topk, token_topk_to_pos, expert_start, expert_end,
+                           num_tokens_per_expert, (int)num_expanded, ws);
         return (int)hipGetLastError();
     }
     // the count launch also fills the padding markers, so it runs even when there are no tokens
