@@ -2,16 +2,16 @@
 // reference offers around it: row gather (pos_to_token), dequantisation of an E4M3 input with 1 x 128
 // scales, SwiGLU in front, and a transposed ([K, M]) output.
 //
-// A workgroup of 8 waves owns a 128-token x 256-column tile and keeps it in registers between the
-// amax and the conversion, so HBM is read once.  Half a wave (32 lanes x 8 columns = 256 columns)
-// takes 8 consecutive tokens: wave w, half h holds tokens 16 w + 8 h + p, p = 0..7.  A lane
-// therefore owns 8 columns over 8 tokens and reduces |x| down its columns without any cross-lane
-// step; the 16 partial maxima per column (8 waves x 2 halves) meet in LDS, thread c < 256 derives
+// A workgroup of 8 waves owns a 128-token x 256-column tile (of 4 waves a 128 x 128 tile where the wide tiles are too few
+// for the GPU) and keeps it in registers between the amax and the conversion, so HBM is read once.  A run of LANES = 32 (16)
+// lanes x 8 columns = 256 (128) columns takes 8 consecutive tokens: run i of the workgroup holds tokens 8 i + p, p = 0..7.
+// A lane therefore owns 8 columns over 8 tokens and reduces |x| down its columns without any cross-lane
+// step; the 16 partial maxima per column (one per run) meet in LDS, one thread per column derives
 // the scale(s) of column c (one division per scale in the whole workgroup, stored as one coalesced
 // run) and hands the multipliers back through LDS.
-//   plain output      : a lane converts 8 columns of a token -> one 8-byte store, 256 bytes per half-wave
+//   plain output      : a lane converts 8 columns of a token -> one 8-byte store, 256 (128) bytes per run
 //   transposed output : a lane converts 8 tokens of a column -> 8 bytes of an output row; the tile is
-//                       turned in LDS ([256 columns][128 tokens] bytes) and leaves as 128-byte row pieces
+//                       turned in LDS ([columns][128 tokens] bytes) and leaves as 128-byte row pieces
 //
 // Reference semantics: tile_kernels/quant/per_channel_cast_fused_kernel.py:16-203,
 // per_channel_cast_and_transpose_kernel.py:8-123,
@@ -25,18 +25,18 @@ namespace tk {
 
 typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
 
-constexpr int kPcTileM = 128, kPcTileK = 256;
+constexpr int kPcTileM = 128;
 // Consecutive tokens per lane.  With 4 (1024 threads per tile) every mode measured slower on MI355X at
 // [8192, 4096]: plain 17.7 -> 18.3 us, FP8 input 13.4 -> 14.6, transposed 21.1 -> 24.0, SwiGLU 17.3 -> 18.0.
 constexpr int kPcRows = 8;
-constexpr int kPcParts = kPcTileM / kPcRows;             // half-waves per tile = partial maxima per column: 16
-constexpr int kPcThreads = 32 * kPcParts;                // 512
+constexpr int kPcParts = kPcTileM / kPcRows;             // runs of lanes per tile = partial maxima per column: 16
 // Turned tile in LDS: one row of 128 token bytes per column, rows 144 bytes apart.  A lane writes the 8
 // tokens it holds of column 8 hl + j as one 8-byte word; left at its natural place (8 part) the 32
-// lanes of a half-wave would meet in two of the 32 8-byte bank pairs (rows 8 x 144 bytes apart).  So
+// lanes of a half-wave would meet in two (LANES = 16: four) of the 32 8-byte bank pairs (rows 8 x 144 bytes apart).  So
 // the 16-byte unit of a row is rotated by (hl >> 1) & 7 and the two halves of the unit are exchanged
-// when hl >= 16: with the row pitch supplying hl & 1, the five bits of hl land in five different bits
-// of the bank-pair index and a half-wave's writes touch every bank pair once.  Units stay whole, so
+// when hl >= 16: with the row pitch supplying hl & 1, the five bits of hl (LANES = 16: its four bits and the parity of the run,
+// which chooses the half of the unit) land in five different bits of the bank-pair index and a half-wave's writes touch every
+// bank pair once.  Units stay whole, so
 // the reader still takes 16 bytes at a time.
 constexpr int kPcPitch = kPcTileM + 16;
 
@@ -76,16 +76,17 @@ __device__ __forceinline__ uint32_t pack_bf16x2(float a, float b) {
     return __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2{a, b}), bf16x2));
 }
 
-template <int MODE, int NPT, bool TRANS, bool GATHER>
-__global__ __launch_bounds__(kPcThreads, 4) void per_channel_cast_kernel(TK_PC_KERNEL_ARGS) {
+template <int MODE, int NPT, bool TRANS, bool GATHER, int LANES>
+__global__ __launch_bounds__(LANES * kPcParts, 4) void per_channel_cast_kernel(TK_PC_KERNEL_ARGS) {
     TK_PC_KERNEL_UNPACK;
+    constexpr int kPcTileK = LANES * 8, kPcThreads = LANES * kPcParts;
     constexpr int NB = kPcTileM / NPT;          // scale blocks per tile along the tokens: 1 or 4
     typedef typename PcRaw<MODE>::type Raw;
     // the partial maxima are dead once the scales exist (second barrier), so the turned tile reuses their space
     constexpr int kPartBytes = kPcParts * kPcTileK * 4, kTurnedBytes = TRANS ? kPcTileK * kPcPitch : 0;
     __shared__ __attribute__((aligned(16))) uint8_t lds[kPartBytes > kTurnedBytes ? kPartBytes : kTurnedBytes];
     __shared__ __attribute__((aligned(16))) float inv_s[NB][kPcTileK];
-    float (*part)[kPcTileK] = reinterpret_cast<float (*)[kPcTileK]>(lds);    // [wave * 2 + half][column]
+    float (*part)[kPcTileK] = reinterpret_cast<float (*)[kPcTileK]>(lds);    // [run][column]
     uint8_t *turned = lds;
 
     // 2-D grid (x = column tile, y = token tile); the FP8-input mode runs on a 1-D grid that it reorders
@@ -103,11 +104,10 @@ __global__ __launch_bounds__(kPcThreads, 4) void per_channel_cast_kernel(TK_PC_K
             tile_m = (q / p.tiles_k) * 8 + (blockIdx.x & 7);
         }
     }
-    const int lane = threadIdx.x & 63, wave = wave_id();
-    const int half = lane >> 5, hl = lane & 31;
+    const int run = (int)threadIdx.x / LANES, hl = (int)threadIdx.x % LANES;
     const int col0 = tile_k * kPcTileK, col = col0 + hl * 8;
     const bool col_ok = col < p.K;
-    const int tok0 = tile_m * kPcTileM + (wave * 2 + half) * kPcRows;
+    const int tok0 = tile_m * kPcTileM + run * kPcRows;
     const bool rows_ok = tok0 < p.M;            // M is a multiple of 16: all 8 tokens of a lane or none
     const int64_t in_ld = MODE == PC_SWIGLU ? 2 * (int64_t)p.K : p.K;
 
@@ -209,7 +209,7 @@ __global__ __launch_bounds__(kPcThreads, 4) void per_channel_cast_kernel(TK_PC_K
 #pragma unroll
     for (int r = 0; r < kPcRows; ++r) forget_unpacked(raw[r]);
     {
-        u32x4 *dst = reinterpret_cast<u32x4 *>(&part[wave * 2 + half][hl * 8]);
+        u32x4 *dst = reinterpret_cast<u32x4 *>(&part[run][hl * 8]);
         dst[0] = u32x4{f2u(m[0]), f2u(m[1]), f2u(m[2]), f2u(m[3])};
         dst[1] = u32x4{f2u(m[4]), f2u(m[5]), f2u(m[6]), f2u(m[7])};
     }
@@ -233,7 +233,7 @@ __global__ __launch_bounds__(kPcThreads, 4) void per_channel_cast_kernel(TK_PC_K
 
     float inv[8];
     {
-        const u32x4 *src = reinterpret_cast<const u32x4 *>(&inv_s[NB == 1 ? 0 : (wave * 2 * kPcRows) / 32][hl * 8]);
+        const u32x4 *src = reinterpret_cast<const u32x4 *>(&inv_s[NB == 1 ? 0 : (run * kPcRows) / 32][hl * 8]);
         const u32x4 a = src[0], b = src[1];
         inv[0] = u2f(a.x); inv[1] = u2f(a.y); inv[2] = u2f(a.z); inv[3] = u2f(a.w);
         inv[4] = u2f(b.x); inv[5] = u2f(b.y); inv[6] = u2f(b.z); inv[7] = u2f(b.w);
@@ -265,8 +265,7 @@ __global__ __launch_bounds__(kPcThreads, 4) void per_channel_cast_kernel(TK_PC_K
             }
         }
         {
-            const int part = wave * 2 + half;
-            const int unit = ((part >> 1) + (hl >> 1)) & 7, low = (part & 1) ^ (hl >> 4);
+            const int unit = ((run >> 1) + (hl >> 1)) & 7, low = (run & 1) ^ (hl >> 4);
             uint8_t *dst = &turned[hl * 8 * kPcPitch + unit * 16 + low * 8];
 #pragma unroll
             for (int j = 0; j < 8; ++j) *reinterpret_cast<u32x2 *>(dst + j * kPcPitch) = u32x2{acc[j][0], acc[j][1]};
@@ -281,7 +280,7 @@ __global__ __launch_bounds__(kPcThreads, 4) void per_channel_cast_kernel(TK_PC_K
             if (col0 + h < p.K && tok < p.M) {
                 const int unit = (chunk + (h >> 4)) & 7;
                 u32x4 d = *reinterpret_cast<const u32x4 *>(&turned[h * kPcPitch + unit * 16]);
-                if (i >= 2) d = u32x4{d.z, d.w, d.x, d.y};          // rows of the lanes hl >= 16: h >= 128
+                if (LANES == 32 && i >= 2) d = u32x4{d.z, d.w, d.x, d.y};          // rows of the lanes hl >= 16: h >= 128
                 // (write-through stores against non-temporal ones, bf16 [8192, 4096] on MI355X: plain and FP8 input 19.6 -> 19.2 us,
                 // behind the SwiGLU 16.7 -> 16.9 us; ordinary stores 19.6 and 18.4 us)
                 if constexpr (MODE != PC_SWIGLU) st_stream16(p.out + (int64_t)(col0 + h) * p.M + tok, d);
@@ -296,11 +295,11 @@ __global__ __launch_bounds__(kPcThreads, 4) void per_channel_cast_kernel(TK_PC_K
 // load and store instruction of a lane moves 16 bytes (8 bytes per lane make a half-wave's instruction 256 bytes
 // long; measured on MI355X at [8192, 4096]: 13.8 us that way, 12.8 us this way).  The rest is the kernel above: maxima down the lane's columns, the 16 partial maxima per column meet in LDS,
 // thread c derives the scale(s) of column c and hands the multipliers back.
-constexpr int kPcWideK = 512;
-
-template <int NPT, bool GATHER>
-__global__ __launch_bounds__(kPcThreads, 4) void per_channel_cast_fp8in_kernel(TK_PC_KERNEL_ARGS) {
+// LANES = 16: 256 threads, 128 x 256 tiles, where the wide tiles are too few for the GPU.
+template <int NPT, bool GATHER, int LANES>
+__global__ __launch_bounds__(LANES * kPcParts, 4) void per_channel_cast_fp8in_kernel(TK_PC_KERNEL_ARGS) {
     TK_PC_KERNEL_UNPACK;
+    constexpr int kPcWideK = LANES * 16;
     constexpr int NB = kPcTileM / NPT;
     __shared__ __attribute__((aligned(16))) float part[kPcParts][kPcWideK];
     __shared__ __attribute__((aligned(16))) float inv_s[NB][kPcWideK];
@@ -314,11 +313,10 @@ __global__ __launch_bounds__(kPcThreads, 4) void per_channel_cast_fp8in_kernel(T
         tile_k = q % p.tiles_k;
         tile_m = (q / p.tiles_k) * 8 + (blockIdx.x & 7);
     }
-    const int lane = threadIdx.x & 63, wave = wave_id();
-    const int half = lane >> 5, hl = lane & 31;
+    const int run = (int)threadIdx.x / LANES, hl = (int)threadIdx.x % LANES;
     const int col0 = tile_k * kPcWideK, col = col0 + hl * 16;
     const bool col_ok = col < p.K;              // K is a multiple of 128: all 16 columns of a lane or none
-    const int tok0 = tile_m * kPcTileM + (wave * 2 + half) * kPcRows;
+    const int tok0 = tile_m * kPcTileM + run * kPcRows;
     const bool rows_ok = tok0 < p.M;            // M is a multiple of 16: all 8 tokens of a lane or none
 
     Raw8<e4m3in_t> lo[kPcRows], hi[kPcRows];
@@ -373,14 +371,14 @@ __global__ __launch_bounds__(kPcThreads, 4) void per_channel_cast_fp8in_kernel(T
 #pragma unroll
     for (int r = 0; r < kPcRows; ++r) { forget_unpacked(lo[r]); forget_unpacked(hi[r]); }
     {
-        u32x4 *dst = reinterpret_cast<u32x4 *>(&part[wave * 2 + half][hl * 16]);
+        u32x4 *dst = reinterpret_cast<u32x4 *>(&part[run][hl * 16]);
 #pragma unroll
         for (int q = 0; q < 4; ++q) dst[q] = u32x4{f2u(m[4 * q]), f2u(m[4 * q + 1]), f2u(m[4 * q + 2]), f2u(m[4 * q + 3])};
     }
     __syncthreads();
 
     {
-        const int c = threadIdx.x;               // 512 threads, 512 columns
+        const int c = threadIdx.x;               // as many threads as columns
 #pragma unroll
         for (int b = 0; b < NB; ++b) {
             float a = 0.0f;
@@ -396,7 +394,7 @@ __global__ __launch_bounds__(kPcThreads, 4) void per_channel_cast_fp8in_kernel(T
 
     float inv[16];
     {
-        const u32x4 *src = reinterpret_cast<const u32x4 *>(&inv_s[NB == 1 ? 0 : (wave * 2 * kPcRows) / 32][hl * 16]);
+        const u32x4 *src = reinterpret_cast<const u32x4 *>(&inv_s[NB == 1 ? 0 : (run * kPcRows) / 32][hl * 16]);
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
             const u32x4 v = src[q];
@@ -419,26 +417,35 @@ __global__ __launch_bounds__(kPcThreads, 4) void per_channel_cast_fp8in_kernel(T
     }
 }
 
-template <int MODE, int NPT>
-static void launch_per_channel_2(const PerChannelParams &p, bool transpose, hipStream_t stream) {
+// Narrow tiles (16 lanes per run, twice as many workgroups of half the size) where wide ones leave compute units without
+// work; from one wide tile per compute unit on their longer rows are the better traffic.  Measured on MI355X, us per call, wide / narrow:
+//   SwiGLU transposed [128, 4096] 7.4 / 5.1, [1024, 2048] (64 wide tiles) 7.9 / 5.6, [4096, 1408] (192) 9.0 / 8.9, [16256, 1024] (508)
+//   16.6 / 16.4, [12800, 3072] (1200) 37.4 / 39.9; bf16 transposed [1024, 7168] (224) 5.3 / 4.65, [2304, 2560] (180) 5.05 / 4.45,
+//   [16256, 1024] (508) 9.2 / 9.65; E4M3 input [4608, 1408] (108) 6.2 / 5.1, [2048, 7168] (224) 6.7 / 6.6, [4096, 4096] (256) 7.25 / 7.6,
+//   [13120, 2560] (515) 13.8 / 15.0.
+// (Runs of 8 lanes: [128, 4096] 4.9, [1024, 7168] 5.7; 4 tokens per lane instead of 8, E4M3 input: [10112, 7168] 29.0 / 32.0.)
+constexpr int64_t kPcWideMinTiles = 256;      // the compute units of an MI355X
+
+template <int MODE, int NPT, int LANES>
+static void launch_per_channel_3(const PerChannelParams &a, bool transpose, hipStream_t stream) {
+    PerChannelParams p = a;
     const int tiles_m = (p.M + kPcTileM - 1) / kPcTileM;
-    const dim3 block(kPcThreads);
+    const dim3 block(LANES * kPcParts);
     if constexpr (MODE == PC_E4M3) {
         if (!transpose && aligned_to(p.x, 16) && aligned_to(p.out, 16)) {
-            const int wide_k = (p.K + kPcWideK - 1) / kPcWideK;
-            PerChannelParams q = p;
-            q.tiles_k = wide_k;
-            const dim3 wide_grid((unsigned)(tiles_m * wide_k));
-            if (p.pos_to_token) hipLaunchKernelGGL((per_channel_cast_fp8in_kernel<NPT, true>), wide_grid, block, 0, stream, TK_PC_LAUNCH_ARGS(q));
-            else hipLaunchKernelGGL((per_channel_cast_fp8in_kernel<NPT, false>), wide_grid, block, 0, stream, TK_PC_LAUNCH_ARGS(q));
+            p.tiles_k = (p.K + LANES * 16 - 1) / (LANES * 16);
+            const dim3 grid((unsigned)(tiles_m * p.tiles_k));
+            if (p.pos_to_token) hipLaunchKernelGGL((per_channel_cast_fp8in_kernel<NPT, true, LANES>), grid, block, 0, stream, TK_PC_LAUNCH_ARGS(p));
+            else hipLaunchKernelGGL((per_channel_cast_fp8in_kernel<NPT, false, LANES>), grid, block, 0, stream, TK_PC_LAUNCH_ARGS(p));
             return;
         }
     }
+    p.tiles_k = (p.K + LANES * 8 - 1) / (LANES * 8);
     // (token tiles on x, so that successive workgroups write neighbouring pieces of the same transposed rows,
     // measured slower: 19.7 -> 21.1 us transposed, 17.4 -> 20.3 us with SwiGLU)
     const dim3 grid = MODE == PC_E4M3 ? dim3((unsigned)(tiles_m * p.tiles_k)) : dim3((unsigned)p.tiles_k, (unsigned)tiles_m);
 #define TK_PC_LAUNCH(T, G) \
-    hipLaunchKernelGGL((per_channel_cast_kernel<MODE, NPT, T, G>), grid, block, 0, stream, TK_PC_LAUNCH_ARGS(p))
+    hipLaunchKernelGGL((per_channel_cast_kernel<MODE, NPT, T, G, LANES>), grid, block, 0, stream, TK_PC_LAUNCH_ARGS(p))
     if constexpr (MODE == PC_SWIGLU) {
         if (transpose) TK_PC_LAUNCH(true, false);
         else TK_PC_LAUNCH(false, false);
@@ -453,6 +460,14 @@ static void launch_per_channel_2(const PerChannelParams &p, bool transpose, hipS
         else TK_PC_LAUNCH(false, false);
     }
 #undef TK_PC_LAUNCH
+}
+
+template <int MODE, int NPT>
+static void launch_per_channel_2(const PerChannelParams &p, bool transpose, hipStream_t stream) {
+    const int wide_cols = MODE == PC_E4M3 && !transpose ? 512 : 256;
+    const int64_t tiles = (int64_t)((p.M + kPcTileM - 1) / kPcTileM) * ((p.K + wide_cols - 1) / wide_cols);
+    if (tiles < kPcWideMinTiles) launch_per_channel_3<MODE, NPT, 16>(p, transpose, stream);
+    else launch_per_channel_3<MODE, NPT, 32>(p, transpose, stream);
 }
 
 template <int MODE>
@@ -488,7 +503,7 @@ extern "C" int tk_check_per_channel_cast(const void *x, int x_dtype, const float
     if (!x || !out || !out_sf) return TK_ERR_NULL_POINTER;
     if (!aligned_to(x, x_sf ? 8 : 16) || !aligned_to(out, transpose ? 16 : 8) || !aligned_to(out_sf, 4) || !aligned_to(x_sf, 4))
         return TK_ERR_MISALIGNED;
-    const int64_t tiles = ((M + kPcTileM - 1) / kPcTileM) * ((K + kPcTileK - 1) / kPcTileK);
+    const int64_t tiles = ((M + kPcTileM - 1) / kPcTileM) * ((K + 255) / 256);
     if (tiles > INT32_MAX - 8 || (M + kPcTileM - 1) / kPcTileM > 65535) return TK_ERR_TOO_LARGE;   // token tiles ride on grid.y
     return TK_OK;
 }
@@ -508,7 +523,7 @@ extern "C" int tk_per_channel_cast(const void *x, int x_dtype, const float *x_sf
     p.num_tokens = (int)num_tokens;
     p.K = (int)K;
     p.M = (int)M;
-    p.tiles_k = (int)((K + kPcTileK - 1) / kPcTileK);
+    p.tiles_k = 0;      // set with the tile width
     p.round_sf = round_sf;
     p.use_clamp = use_clamp;
     p.clamp = clamp;
