@@ -455,10 +455,18 @@ __global__ __launch_bounds__(TILE == T_ROW ? 64 * kMaxWideWaves : kThreads) void
                 // before the first row is evaluated): a padding row, and a lane beyond the last row or column,
                 // reads the first bytes of the matrix, which every wave shares, and is cleared by value
                 const bool ok = live[r] && piece_ok;
-                const InT *src = ok ? xr : reinterpret_cast<const InT *>(p.x);
-                rg[r].load(src);
-                vmem_issue_gap();
-                ru[r].load(ok ? xr + uh : src);
+                if constexpr (XB != 0) {      // (whole lines: fp32 [4001, 2 x 2560] 18.5 us with each lane reading its own bytes)
+                    const int first = (strip + r * (ROW ? 1 : 0)) * kStripCols, n = live[r] ? p.H - first : 0;
+                    const InT *run = xr - lane * 8;
+                    rg[r].template load_run_part<64>(run, lane, n, p.x);
+                    vmem_issue_gap();
+                    ru[r].template load_run_part<64>(run + uh, lane, n, p.x);
+                } else {
+                    const InT *src = ok ? xr : reinterpret_cast<const InT *>(p.x);
+                    rg[r].load(src);
+                    vmem_issue_gap();
+                    ru[r].load(ok ? xr + uh : src);
+                }
                 if (r + 1 < RPW) vmem_issue_gap();
                 unused[r] = !ok;
                 if constexpr (sizeof(InT) != 4) {
@@ -469,20 +477,19 @@ __global__ __launch_bounds__(TILE == T_ROW ? 64 * kMaxWideWaves : kThreads) void
         // fp32 input (two loads per piece): cleared once all loads are out, since clearing a register that a load is still to
         // fill means waiting for that load (masked fp32 [16384, 2 x 2048] 40.3 -> 38.4 us; bf16 input, whose clearing the
         // compiler already places behind the loads, measured 21.0 -> 21.2 us on a ragged batch with it and keeps its place)
-        if constexpr (!(FULL && !MASK) && sizeof(InT) == 4) {
-#pragma unroll
-            for (int r = 0; r < RPW; ++r)
-                if (unused[r]) { rg[r].zero(); ru[r].zero(); }
-        }
-
         // (in this variant the fetch of the later arguments starts at the head of the kernel, where its paths part)
         if constexpr (TAILED != 0) fetch_late_arguments(p, CLAMP != 0, TAILED == 2, TILE != T_ROW);
-        if constexpr (FULL && XB != 0) {
+        if constexpr (XB != 0) {
 #pragma unroll
             for (int r = 0; r < RPW; ++r) {
                 rg[r].template settle<64>(xchg[wave], lane);
                 ru[r].template settle<64>(xchg[wave], lane);
             }
+        }
+        if constexpr (!(FULL && !MASK) && sizeof(InT) == 4) {
+#pragma unroll
+            for (int r = 0; r < RPW; ++r)
+                if (unused[r]) { rg[r].zero(); ru[r].zero(); }
         }
         float wrow = 0.0f;
         if constexpr (EARLY_WEIGHT) {
@@ -569,6 +576,9 @@ __global__ __launch_bounds__(kThreads) void swiglu_cast_flat_kernel(TK_SWIGLU_KE
     const int gpr = p.tiles_k;   // groups per row
     const InT *xb = reinterpret_cast<const InT *>(p.x);
     ClampCounter<CLAMP> counter;
+    // fp32 input: the lanes of a group read its 512 bytes as two runs and deal them out through LDS
+    constexpr int XB = Raw8<InT>::kXchgBytes;
+    __shared__ __attribute__((aligned(16))) uint8_t xchg[XB ? kThreads * XB : 16];
 
     // Mask entries and weight indices of all slots are asked for first, then the data of all slots, then the weights: a
     // load whose address hangs on a loaded value waits for every load issued before it, so with a slot's mask entry read
@@ -606,10 +616,25 @@ __global__ __launch_bounds__(kThreads) void swiglu_cast_flat_kernel(TK_SWIGLU_KE
         // no branch around the loads: a padding row, and a lane beyond the matrix, reads its first bytes and is cleared by value
         const bool ok = inside[r] && live[r];
         const InT *src = ok ? xb + (int64_t)row[r] * (2 * (int64_t)p.H) + col : xb;
-        rg[r].load(src);
+        if constexpr (XB != 0) {
+            const InT *run = src - own * 8;      // (not used where the row is not)
+            rg[r].template load_run_part<LPG>(run, own, ok ? 128 : 0, xb);
+            vmem_issue_gap();
+            ru[r].template load_run_part<LPG>(run + p.H, own, ok ? 128 : 0, xb);
+        } else {
+            rg[r].load(src);
+            vmem_issue_gap();
+            ru[r].load(ok ? src + p.H : src);
+        }
         vmem_issue_gap();
-        ru[r].load(ok ? src + p.H : src);
-        vmem_issue_gap();
+    }
+    if constexpr (XB != 0) {
+#pragma unroll
+        for (int r = 0; r < RPW; ++r) {
+            uint8_t *run_lds = xchg + (threadIdx.x / LPG) * (LPG * XB);
+            rg[r].template settle<LPG>(run_lds, own);
+            ru[r].template settle<LPG>(run_lds, own);
+        }
     }
 #pragma unroll
     for (int r = 0; r < RPW; ++r)      // (cleared once all loads are out)

@@ -134,6 +134,12 @@ __device__ __forceinline__ void st_stream4(void *p, uint32_t v) {
     __hip_atomic_store(reinterpret_cast<uint32_t *>(p), v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
+// Between LDS accesses of one wave that exchange data between its lanes: keeps the compiler from reordering them.
+__device__ __forceinline__ void wave_lds_fence() {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
+
 // 8 consecutive elements, as fp32.  `ok == false` yields zeros without touching memory.
 template <typename T> struct Raw8;
 template <> struct Raw8<bf16_t> {
@@ -164,7 +170,8 @@ template <> struct Raw8<bf16_t> {
 // half with the other, 16 consecutive bytes per lane; settle() then hands every lane its own 32 bytes through LDS (two
 // 16-byte writes, two 16-byte reads; the run's 32 * LANES bytes of LDS are private to its lanes, which belong to one wave,
 // so no barrier is involved).  Measured on MI355X, per-token cast of fp32 [4096, 7168]: 26.6 -> 23.5 us; fused SwiGLU cast of
-// fp32 [8192, 2 x 2048]: 27.6 -> 25.6 us (timed with the exchange left out).  All lanes of the run must be in range.
+// fp32 [8192, 2 x 2048]: 27.6 -> 25.6 us (timed with the exchange left out).  All lanes of the run must be in range
+// (load_run_part(): any number of them).
 template <> struct Raw8<float> {
     u32x4 a, b;
     static constexpr int kXchgBytes = 32;   // LDS bytes per lane of a run
@@ -180,13 +187,26 @@ template <> struct Raw8<float> {
         vmem_issue_gap();
         b = ld_stream16(q + 16 * LANES);
     }
+    // The same where only the first n of the run's elements exist (n a multiple of 8; none: n <= 0): the 16-byte pieces beyond
+    // them are read from `safe` instead, no lane branches, and settle() hands the lanes beyond the end something to be cleared.
+    // run: the first element of the run.
+    template <int LANES> __device__ __forceinline__ void load_run_part(const void *run, int i, int n, const void *safe) {
+        const uint8_t *q = reinterpret_cast<const uint8_t *>(run) + 16 * i;
+        a = ld_stream16(4 * i < n ? static_cast<const void *>(q) : safe);
+        vmem_issue_gap();
+        b = ld_stream16(4 * (LANES + i) < n ? static_cast<const void *>(q + 16 * LANES) : safe);
+    }
     // run_lds: the 32 * LANES bytes of LDS of this lane's run, 16-byte aligned
     template <int LANES> __device__ __forceinline__ void settle(uint8_t *run_lds, int i) {
         u32x4 *w = reinterpret_cast<u32x4 *>(run_lds);
+        // The words read were written by other lanes, which the compiler cannot see from one lane's addresses: without the fences it
+        // may move the first read in front of the second write (no instruction comes of them, LDS serves a wave in order).
         w[i] = a;
         w[LANES + i] = b;
+        wave_lds_fence();
         a = w[2 * i];
         b = w[2 * i + 1];
+        wave_lds_fence();
     }
     __device__ __forceinline__ void load_cached(const void *p) {
         a = *reinterpret_cast<const u32x4 *>(p);
