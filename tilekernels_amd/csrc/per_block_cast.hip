@@ -39,7 +39,7 @@ struct PerBlockParams {
 // THREADS: threads per tile.
 // FULL: the tile lies wholly inside the matrix, so no bounds checks are compiled in.
 template <typename InT, int FMT, int BM, int BK, int TW, int THREADS, bool FULL>
-__device__ __forceinline__ void per_block_cast_tile(const PerBlockParams &p) {
+__device__ __forceinline__ void per_block_cast_tile(const PerBlockParams &p, uint8_t *xchg) {
     constexpr int LPR = TW / 8;                                      // lanes along a row of the tile
     constexpr int SUBM = kBlockTile / BM, SUBK = TW / BK;            // scale blocks per tile
     constexpr int LPG = BK / 8;                                      // lanes sharing a block in one row
@@ -63,17 +63,31 @@ __device__ __forceinline__ void per_block_cast_tile(const PerBlockParams &p) {
     // fp32 input: the LPR lanes of a tile row read its 32 * LPR bytes as two whole-line loads and deal them out through LDS
     constexpr int XB = Raw8<InT>::kXchgBytes;
     constexpr int RUN = LPR < 64 ? LPR : 64;     // lanes of one run: a tile row, or the part of it that one wave holds
-    __shared__ __attribute__((aligned(16))) uint8_t xchg[XB ? THREADS * XB : 16];
     Raw8<InT> raw[NI];
 #pragma unroll
     for (int i = 0; i < NI; ++i) {
-        if (FULL) raw[i].template load_run<RUN>(x + (int64_t)(TR * i) * p.K, c % RUN);
-        else raw[i].load(x + (int64_t)(TR * i) * p.K, col_ok && row0 + TR * i < p.M);
+        if constexpr (FULL) {
+            raw[i].template load_run<RUN>(x + (int64_t)(TR * i) * p.K, c % RUN);
+        } else {
+            // No lane branches around its load: all loads of a lane go out together, where each one in a branch of its own is waited
+            // for before the next (the tiles at the lower edge then end the launch some 5 us after the others).  A lane beyond the
+            // last row reads that row, one beyond the last column the last columns (fp32: nothing, it is cleared): no maximum changes.
+            const InT *xr = reinterpret_cast<const InT *>(p.x) + (int64_t)min(row0 + TR * i, p.M - 1) * p.K;
+            if constexpr (XB != 0) {
+                const int first = col - (c % RUN) * 8;
+                raw[i].template load_run_part<RUN>(xr + first, c % RUN, p.K - first, p.x);
+            } else {
+                raw[i].load(xr + (col_ok ? col : p.K - 8));
+            }
+        }
         if (i + 1 < NI) vmem_issue_gap();
     }
-    if constexpr (FULL && XB != 0) {
+    if constexpr (XB != 0) {
 #pragma unroll
-        for (int i = 0; i < NI; ++i) raw[i].template settle<RUN>(xchg + (threadIdx.x / RUN) * (RUN * XB), c % RUN);
+        for (int i = 0; i < NI; ++i) {
+            raw[i].template settle<RUN>(xchg + (threadIdx.x / RUN) * (RUN * XB), c % RUN);
+            if (!col_ok) raw[i].zero();
+        }
     }
 
     float inv[SUBM];
@@ -163,13 +177,15 @@ __device__ __forceinline__ void per_block_cast_tile(const PerBlockParams &p) {
 template <typename InT, int FMT, int BM, int BK, int TW, int THREADS, bool FULL_GRID>
 __global__ __launch_bounds__(THREADS) void per_block_cast_kernel(TK_PB_KERNEL_ARGS) {
     TK_PB_KERNEL_UNPACK;
+    constexpr int XB = Raw8<InT>::kXchgBytes;
+    __shared__ __attribute__((aligned(16))) uint8_t xchg[XB ? THREADS * XB : 16];      // (one for both kinds of tile)
     if constexpr (FULL_GRID) {
-        per_block_cast_tile<InT, FMT, BM, BK, TW, THREADS, true>(p);
+        per_block_cast_tile<InT, FMT, BM, BK, TW, THREADS, true>(p, xchg);
     } else {
         if (((int)blockIdx.y + 1) * kBlockTile <= p.M && ((int)blockIdx.x + 1) * TW <= p.K)
-            per_block_cast_tile<InT, FMT, BM, BK, TW, THREADS, true>(p);
+            per_block_cast_tile<InT, FMT, BM, BK, TW, THREADS, true>(p, xchg);
         else
-            per_block_cast_tile<InT, FMT, BM, BK, TW, THREADS, false>(p);
+            per_block_cast_tile<InT, FMT, BM, BK, TW, THREADS, false>(p, xchg);
     }
 }
 
