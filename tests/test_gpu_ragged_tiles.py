@@ -65,3 +65,61 @@ def test_per_channel_gathered_codes(M, K):
     want = torch_ref.per_channel_cast_fused(codes, 128, 128, False, pos)
     assert_same(got[0], want[0], 'codes')
     assert_same(got[1], want[1], 'scales')
+
+
+@pytest.mark.parametrize('kind,transpose,gather', [('bf16', False, False), ('bf16', False, True), ('bf16', True, False), ('bf16', True, True),
+                                                   ('fp32', False, False), ('fp32', False, True), ('e4m3', False, False), ('e4m3', False, True),
+                                                   ('e4m3', True, False), ('e4m3', True, True), ('swiglu', False, False), ('swiglu', True, False)])
+@pytest.mark.parametrize('num_per_tokens', [32, 128])
+def test_per_channel_tile_widths_agree(kind, transpose, gather, num_per_tokens):
+    """One call on a matrix that takes wide tiles against calls on its pieces of 512 rows, which take narrow ones (no scale spans two
+    pieces): every form of tk_per_channel_cast, also those the Python functions do not ask for and codes aligned to 8 bytes."""
+    from tilekernels_amd import _ffi
+    lib = _ffi.load()
+    M, K = 2176, 8320 if kind == 'e4m3' and not transpose else 4224                # 289 wide tiles; 68 and fewer in a piece
+    g = torch.Generator(device='cuda').manual_seed(K)
+    width = 2 * K if kind == 'swiglu' else K
+    x = torch.randn((M, width), generator=g, device='cuda')
+    x = x if kind == 'fp32' else x.to(torch.bfloat16)
+    sf = None
+    if kind == 'e4m3':
+        x, sf = x.to(torch.float8_e4m3fn), torch.rand((M, K // 128), generator=g, device='cuda') + 0.1
+    pos = torch.randint(-1, M, (M,), generator=g, device='cuda', dtype=torch.int32) if gather else None
+    x = x.view(torch.uint8)
+
+    def cast(first, rows, shift):
+        lo = 0 if gather else first
+        data = torch.zeros((M - lo) * x.shape[1] + 16, dtype=torch.uint8, device='cuda')
+        data[shift:shift + (M - lo) * x.shape[1]] = x[lo:].reshape(-1)
+        out = torch.zeros(rows * K + 16, dtype=torch.uint8, device='cuda')
+        out_sf = torch.zeros((-(-rows // num_per_tokens), K), device='cuda')
+        sub_sf, sub_pos = None if sf is None else sf[lo:], None if pos is None else pos[first:]
+        rc = lib.tk_per_channel_cast(data.data_ptr() + shift, int(kind == 'fp32'), _ffi.ptr(sub_sf), M - lo, K, _ffi.ptr(sub_pos), rows,
+                                     out.data_ptr() + shift, out_sf.data_ptr(), num_per_tokens, 1, int(transpose), int(kind == 'swiglu'),
+                                     int(kind == 'swiglu'), 1.5 if kind == 'swiglu' else 0.0, _ffi.current_stream(x.device))
+        assert rc == 0, rc
+        out = out[shift:shift + rows * K]
+        return (out.view(K, rows).T if transpose else out.view(rows, K)), out_sf
+
+    for shift in (0, 8) if kind == 'e4m3' and not transpose else (0,):
+        codes, scales = cast(0, M, shift)
+        pieces = [cast(first, min(512, M - first), shift) for first in range(0, M, 512)]
+        assert torch.equal(codes, torch.cat([p[0] for p in pieces])) and torch.equal(scales, torch.cat([p[1] for p in pieces]))
+
+
+@pytest.mark.parametrize('clamp', [None, 1.5])
+@pytest.mark.parametrize('weighted', [False, True])
+@pytest.mark.parametrize('R,H', [(6145, 2048), (8190, 2048), (8191, 2048), (4099, 4096), (2051, 8192)])
+def test_swiglu_launches_that_end_in_smaller_waves_on_any_row_count(R, H, weighted, clamp):
+    """Row-major scales, rows that are no multiple of four: one call against calls on pieces of 999 rows, which are too small to end in
+    smaller waves."""
+    import tilekernels_amd as tk
+    g = torch.Generator(device='cuda').manual_seed(R)
+    x = (torch.randn((R, 2 * H), generator=g, device='cuda') * 2).to(torch.bfloat16)
+    slots = torch.randint(-1, R, (R,), generator=g, device='cuda', dtype=torch.int32) if weighted else None
+    weights = torch.rand((R, 1), generator=g, device='cuda') if weighted else None
+    op = tk.quant.swiglu_forward_and_per_token_cast
+    codes, sf = op(x, 'e4m3', 128, slots, weights, swiglu_clamp_value=clamp)
+    pieces = [op(x[i:i + 999], 'e4m3', 128, None if slots is None else slots[i:i + 999], weights, swiglu_clamp_value=clamp) for i in range(0, R, 999)]
+    assert torch.equal(codes.view(torch.uint8), torch.cat([p[0].view(torch.uint8) for p in pieces]))
+    assert torch.equal(sf, torch.cat([p[1] for p in pieces]))

@@ -265,7 +265,7 @@ __device__ __forceinline__ void swiglu_row_wave(SwigluParams p, int row0, int st
 enum { T_STACKED = 0, T_ROW = 2, T_ROWC = 3 };
 
 // ONECOL: the grid is known to be a single column of tiles (else it is found out at run time)
-// TAILED (tiles of four-piece waves, exact grids): the launch ends in finer-grained waves.  The grid's row tiles
+// TAILED (tiles of four-piece waves that fit the columns and, column-major scales, the rows): the launch ends in finer-grained waves.  The grid's row tiles
 // come in three runs: `yb` workgroups of one-row waves as described above, then `ym` workgroups whose waves take two
 // pieces, then workgroups whose waves take one; all cover the rows in order.  The requests of a launch are served
 // roughly in the order they were made, so what arrives last belongs to the last workgroups; with whole rows per wave
@@ -288,7 +288,7 @@ enum { T_STACKED = 0, T_ROW = 2, T_ROWC = 3 };
 // [16384, 2 x 2048] 27.53 / 27.13; packed UE8M0: 14.79 / 14.36, 14.70 / 14.47, 21.11 / 20.61, 27.18 / 26.88.
 template <typename InT, int CLAMP, int RPW, int TILE, bool FULL_GRID, bool MASK, bool ONECOL, int TAILED = 0>
 __global__ __launch_bounds__(TILE == T_ROW ? 64 * kMaxWideWaves : kThreads) void swiglu_cast_kernel(TK_SWIGLU_KERNEL_ARGS) {
-    static_assert(!TAILED || (FULL_GRID && !MASK && CLAMP != 2 && RPW == 4), "tail waves: exact unmasked grids of four-piece waves");
+    static_assert(!TAILED || (FULL_GRID && !MASK && CLAMP != 2 && RPW == 4), "tail waves: unmasked grids of four-piece waves without bounds checks");
     if constexpr (TAILED) {
         // a_nwaves: waves per workgroup (bits 0-3), column tiles (4-15), two-piece workgroups (16-31); a_tiles_k: one-row workgroups
         const int yb = a_tiles_k, ym = (int)((unsigned)a_nwaves >> 16);
@@ -832,10 +832,16 @@ static void launch_swiglu_tiled(SwigluParams &p, int max_blocks, hipStream_t str
         // [10240, 2 x 2048] 17.84 / 17.18, [16384, 2 x 2048] 26.92 / 26.50, [8192, 2 x 4096] 26.59 / 26.17, [2048, 2 x 8192]
         // 14.77 / 14.32, [24576, 2 x 2048] 42.92 / 42.54; smaller and larger launches lose with it ([4096, 2 x 2048] 8.11 / 8.48,
         // [32768, 2 x 2048] 57.37 / 57.71), and so does a masked batch ([48128, 2 x 2048], a third of the rows padding, 59.9 / 61.8).
+        // Row-major tiles take any number of rows this way ([8189, 2 x 2048] 14.4 / 13.75, [12345, 2 x 2048] 21.0 / 20.3, [4001, 2 x 4096]
+        // 14.0 / 13.6); the column-major ones need whole groups of four rows, whose scales leave together.
         const int64_t slots = wave_slots(), ppr = p.H / kStripCols, row_waves = (int64_t)p.R * ppr / RPW;
         int rs = (int)std::min<int64_t>((int64_t)p.R * 15 / 100, slots * 6 / 10 / ppr) / 4 * 4;
         int rm = (int)std::min<int64_t>((int64_t)p.R * 55 / 100, slots * 22 / 10 / ppr) / 4 * 4;
         int rb = p.R - rm - rs;
+        if constexpr (TILE == T_ROW) {      // the rows beyond the last four are among those of one-piece waves, a workgroup each
+            rb = rb / kWaves * kWaves;
+            rs = p.R - rm - rb;
+        }
         int64_t ym = (int64_t)rm * 2 / waves, ys = (int64_t)rs * 4 / waves, yb = rb / waves;
         if constexpr (TILE == T_STACKED) {
             // stacked tiles of 16 rows, then workgroups of 8 rows (two per wave), then of 4 rows, each on one strip of 512 columns
@@ -844,7 +850,7 @@ static void launch_swiglu_tiled(SwigluParams &p, int max_blocks, hipStream_t str
             rm = p.R - rb - rs;
             yb = rb / rows; ym = rm / (2 * kWaves); ys = rs / kWaves;
         }
-        if (full && !p.pos_to_expert && waves == kWaves && row_waves * 4 >= slots * 3 && row_waves * 2 <= slots * 7 && rs > 0 && p.tiles_k <= 0xFFF &&
+        if ((TILE == T_ROW ? p.H % cols == 0 : full) && !p.pos_to_expert && waves == kWaves && row_waves * 4 >= slots * 3 && row_waves * 2 <= slots * 7 && rs > 0 && p.tiles_k <= 0xFFF &&
             ym <= 0xFFFF) {
             const dim3 tgrid = tile_grid(p.tiles_k, (int)(yb + ym + ys));
             p.nwaves = waves | (p.tiles_k << 4) | ((int)ym << 16);
