@@ -198,8 +198,8 @@ __global__ __launch_bounds__(kThreads) void fused_mapping_table_kernel(const int
 // range, and one per slice of its own.  From these every workgroup derives the same expert offsets (a prefix sum over
 // the padded expert sizes) and its slices' first positions, hands out positions exactly as the assign launch does, and
 // marks its share of the padding positions: the ends of the experts e = workgroup, workgroup + gridDim, ... and its
-// stride of the unused tail of the buffers.  Measured on MI355X for 4096 tokens, top-8 of 256 experts: 9.1 us, of which
-// the counting pass is 4.2 (its LDS atomics), against 17.8 us for the three launches.
+// stride of the unused tail of the buffers.  Measured on MI355X for 4096 tokens, top-8 of 256 experts: 8.0 us, of which
+// about half is the counting pass (its LDS atomics), against 17.8 us for the three launches.
 constexpr int kSingleLaunchPairs = 64 * 1024 - 1;
 constexpr int kSingleWaves = 16;
 constexpr int kSingleSlice = 64;            // entries a wave hands out: 1024 per workgroup, so that the scattered stores of the
@@ -265,12 +265,13 @@ __global__ __launch_bounds__(64 * kSingleWaves) void fused_mapping_single_kernel
             if (i >= own_base && i < own_end) atomicAdd(&slice[((i - own_base) / kSingleSlice) * num_experts + e], 1);
         }
     };
-    // The list is read in 16-byte pieces (two ids), 16 of them per thread in flight at a time: with a load or four at a
-    // time the pass took as many memory round trips as it has iterations (24 us for 32 Ki pairs).
+    // The list is read in 16-byte pieces (two ids), 4 of them per thread in flight at a time.  A thread's loads beyond the end of the
+    // list read its first piece, and in a short list nearly all of them are beyond it: with 16 in flight, us for 512 / 2720 / 8000 /
+    // 32768 pairs: 5.06 / 5.31 / 5.70 / 8.67; 4: 3.65 / 3.93 / 4.40 / 8.01; 2: 3.47 / 3.79 / 4.39 / 8.26; 1: 3.49 / 3.86 / 4.50 / 8.81.
     const int head = TABLE ? 0 : (int)((reinterpret_cast<uintptr_t>(topk_idx) >> 3) & 1);      // ids before the first 16-byte boundary
     const int pairs = TABLE ? 0 : (numel - head) / 2;
     const u32x4 *wide = reinterpret_cast<const u32x4 *>(topk_idx + head);
-    constexpr int U = 16;
+    constexpr int U = 4;
     for (int p0 = 0; p0 < pairs; p0 += U * nthreads) {
         u32x4 w[U];
 #pragma unroll
