@@ -104,7 +104,7 @@ __global__ __launch_bounds__(LANES * kPcParts, 4) void per_channel_cast_kernel(T
             tile_m = (q / p.tiles_k) * 8 + (blockIdx.x & 7);
         }
     }
-    const int run = (int)threadIdx.x / LANES, hl = (int)threadIdx.x % LANES;
+    const int lane = threadIdx.x & 63, run = wave_id() * (64 / LANES) + lane / LANES, hl = lane % LANES;
     const int col0 = tile_k * kPcTileK, col = col0 + hl * 8;
     const bool col_ok = col < p.K;
     const int tok0 = tile_m * kPcTileM + run * kPcRows;
@@ -313,7 +313,7 @@ __global__ __launch_bounds__(LANES * kPcParts, 4) void per_channel_cast_fp8in_ke
         tile_k = q % p.tiles_k;
         tile_m = (q / p.tiles_k) * 8 + (blockIdx.x & 7);
     }
-    const int run = (int)threadIdx.x / LANES, hl = (int)threadIdx.x % LANES;
+    const int lane = threadIdx.x & 63, run = wave_id() * (64 / LANES) + lane / LANES, hl = lane % LANES;
     const int col0 = tile_k * kPcWideK, col = col0 + hl * 16;
     const bool col_ok = col < p.K;              // K is a multiple of 128: all 16 columns of a lane or none
     const int tok0 = tile_m * kPcTileM + run * kPcRows;
