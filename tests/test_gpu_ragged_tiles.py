@@ -109,9 +109,10 @@ def test_per_channel_tile_widths_agree(kind, transpose, gather, num_per_tokens):
 
 @pytest.mark.parametrize('clamp', [None, 1.5])
 @pytest.mark.parametrize('weighted', [False, True])
-@pytest.mark.parametrize('R,H', [(6145, 2048), (8190, 2048), (8191, 2048), (4099, 4096), (2051, 8192)])
+@pytest.mark.parametrize('R,H', [(6145, 2048), (8190, 2048), (8191, 2048), (4099, 4096), (2051, 8192), (8189, 2560), (6545, 2560), (10921, 1536), (2049, 7168),
+                                 (32771, 512)])
 def test_swiglu_launches_that_end_in_smaller_waves_on_any_row_count(R, H, weighted, clamp):
-    """Row-major scales, rows that are no multiple of four: one call against calls on pieces of 999 rows, which are too small to end in
+    """Row-major scales, rows that are no multiple of the tiles (H a multiple of 2048: row-wise tiles, else stacked): one call against calls on pieces of 999 rows, which are too small to end in
     smaller waves."""
     import tilekernels_amd as tk
     g = torch.Generator(device='cuda').manual_seed(R)

@@ -832,8 +832,9 @@ static void launch_swiglu_tiled(SwigluParams &p, int max_blocks, hipStream_t str
         // [10240, 2 x 2048] 17.84 / 17.18, [16384, 2 x 2048] 26.92 / 26.50, [8192, 2 x 4096] 26.59 / 26.17, [2048, 2 x 8192]
         // 14.77 / 14.32, [24576, 2 x 2048] 42.92 / 42.54; smaller and larger launches lose with it ([4096, 2 x 2048] 8.11 / 8.48,
         // [32768, 2 x 2048] 57.37 / 57.71), and so does a masked batch ([48128, 2 x 2048], a third of the rows padding, 59.9 / 61.8).
-        // Row-major tiles take any number of rows this way ([8189, 2 x 2048] 14.4 / 13.75, [12345, 2 x 2048] 21.0 / 20.3, [4001, 2 x 4096]
-        // 14.0 / 13.6); the column-major ones need whole groups of four rows, whose scales leave together.
+        // With row-major scales any number of rows may end this way ([8189, 2 x 2048] 14.4 / 13.75, [12345, 2 x 2048] 21.0 / 20.3, [4001, 2 x
+        // 4096] 14.0 / 13.6; stacked tiles [8189, 2 x 2560] 18.2 / 17.3, [2049, 2 x 7168] 13.8 / 12.7, [16381, 2 x 1536] 20.9 / 20.05);
+        // column-major scales need whole groups of four rows, whose scales leave together.
         const int64_t slots = wave_slots(), ppr = p.H / kStripCols, row_waves = (int64_t)p.R * ppr / RPW;
         int rs = (int)std::min<int64_t>((int64_t)p.R * 15 / 100, slots * 6 / 10 / ppr) / 4 * 4;
         int rm = (int)std::min<int64_t>((int64_t)p.R * 55 / 100, slots * 22 / 10 / ppr) / 4 * 4;
@@ -847,10 +848,13 @@ static void launch_swiglu_tiled(SwigluParams &p, int max_blocks, hipStream_t str
             // stacked tiles of 16 rows, then workgroups of 8 rows (two per wave), then of 4 rows, each on one strip of 512 columns
             rs = rs / 8 * 8;
             rb = (p.R - rm - rs) / rows * rows;
-            rm = p.R - rb - rs;
-            yb = rb / rows; ym = rm / (2 * kWaves); ys = rs / kWaves;
+            rm = (p.R - rb - rs) / 8 * 8;
+            rs = p.R - rb - rm;
+            yb = rb / rows; ym = rm / (2 * kWaves); ys = (rs + kWaves - 1) / kWaves;
         }
-        if ((TILE == T_ROW ? p.H % cols == 0 : full) && !p.pos_to_expert && waves == kWaves && row_waves * 4 >= slots * 3 && row_waves * 2 <= slots * 7 && rs > 0 && p.tiles_k <= 0xFFF &&
+        // row-major scales are stored by the waves themselves: a workgroup that overhangs the last row has no barrier to meet
+        const bool any_rows = TILE == T_ROW || (TILE == T_STACKED && p.sf.layout == TK_SF_ROW_F32 && tile_grid_exact(p.tiles_k, tiles_m));
+        if ((any_rows ? p.H % cols == 0 : full) && !p.pos_to_expert && waves == kWaves && row_waves * 4 >= slots * 3 && row_waves * 2 <= slots * 7 && rs > 0 && p.tiles_k <= 0xFFF &&
             ym <= 0xFFFF) {
             const dim3 tgrid = tile_grid(p.tiles_k, (int)(yb + ym + ys));
             p.nwaves = waves | (p.tiles_k << 4) | ((int)ym << 16);
