@@ -238,3 +238,42 @@ def test_masked_swiglu_with_more_rows_than_one_grid_plane(dtype, H, clamp):
     torch.cuda.synchronize()
     assert torch.equal(codes_buf[:R], codes.view(torch.uint8)) and torch.equal(sf2, sf)
     assert bool((codes_buf[R:] == 0x5A).all()), 'rows beyond the batch were written'
+
+
+@pytest.mark.parametrize('hidden,dtype,tokens', [(8, torch.bfloat16, 2 ** 26 + 5), (2048, torch.float32, 2 ** 24 + 3)], ids=['bf16', 'fp32'])
+def test_reduce_fused_of_more_tokens_than_one_launch_takes(hidden, dtype, tokens):
+    """Rows of one column of pieces put all their row tiles on grid.x, where HIP takes fewer than 2^32 threads: the tokens are
+    cut into launches.  One term per token, so that every row of the result is a row of a table."""
+    from tilekernels_amd import _ffi
+    x = (torch.randn((5, hidden), generator=torch.Generator().manual_seed(hidden)) * 20).to(dtype)
+    codes = torch.cat([torch.zeros((1, hidden), dtype=torch.uint8), x.to(torch.float8_e4m3fn).view(torch.uint8)]).cuda()
+    x = x.cuda()
+    t2p = (torch.arange(tokens, device='cuda') * 7 % 6 - 1).to(torch.int32)
+    out = torch.full((tokens + 1, hidden), 0x5A, dtype=torch.uint8, device='cuda')
+    rc = _ffi.load().tk_reduce_fused(x.data_ptr(), _ffi.dtype_code(x), 5, hidden, 0, 0, t2p.data_ptr(), tokens, 1, out.data_ptr(),
+                                     _ffi.TK_OUT_E4M3, 0, torch.cuda.current_stream().cuda_stream)
+    assert rc == 0, rc
+    step = 2 ** 31 // hidden
+    for a in range(0, tokens, step):
+        b = min(a + step, tokens)
+        assert torch.equal(out[a:b], codes[(t2p[a:b] + 1).long()]), (a, b)
+    assert bool((out[tokens:] == 0x5A).all())
+
+
+@pytest.mark.parametrize('hidden,dtype,rows', [(1536, torch.bfloat16, 4), (2048, torch.bfloat16, 2), (4096, torch.float32, 1)], ids=['4', '2', '1'])
+def test_reduce_fused_on_more_than_one_grid_plane(hidden, dtype, rows):
+    """Several columns of pieces and more than 32768 row tiles (of `rows` tokens): a second, partly empty plane."""
+    tk = _tk()
+    edge, R = 32768 * rows, 64
+    tokens = edge + 8 * rows + 3
+    g = torch.Generator().manual_seed(hidden)
+    x = torch.randn((R, hidden), generator=g).to(dtype)
+    t2p = torch.randint(-1, R, (tokens, 3), generator=g, dtype=torch.int32)
+    w = torch.rand((tokens, 3), generator=g)
+    got = tk.moe.reduce_fused(x.cuda(), w.cuda(), t2p.cuda())
+    for a, b in ((0, 16), (edge - 16, edge + 16), (tokens - 16, tokens)):
+        _same_bytes(got[a:b], torch_ref.reduce_fused(x, w[a:b].contiguous(), t2p[a:b].contiguous()), f'rows[{a}:{b}]')
+    for a in range(0, tokens, 16384):
+        b = min(a + 16384, tokens)
+        part = tk.moe.reduce_fused(x.cuda(), w[a:b].cuda(), t2p[a:b].cuda())
+        assert torch.equal(part.view(torch.uint8), got[a:b].view(torch.uint8)), (a, b)

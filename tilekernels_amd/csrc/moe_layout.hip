@@ -918,21 +918,29 @@ extern "C" int tk_reduce_fused(const void *x, int x_dtype, int64_t num_expanded,
     const int side_log2 = strips % 4 == 0 && x_dtype == TK_F32 ? 2 : (strips % 2 == 0 ? 1 : 0);
     const int64_t rows = kWaves >> side_log2;
     const int cols = strips >> side_log2;
-    const dim3 grid = tile_grid(cols, (int)((num_tokens + rows - 1) / rows));
+    // HIP takes fewer than 2^32 threads along a grid dimension, and the row tiles of a single column of pieces all ride on x:
+    // at most 2^23 row tiles (2^31 threads) per launch.
+    const int64_t step = rows << 23, out_bytes = out_dtype == TK_F32 ? 4 : (out_dtype == TK_BF16 ? 2 : 1);
+    for (int64_t t0 = 0; t0 < num_tokens; t0 += step) {
+        const int64_t tokens = std::min(num_tokens - t0, step);
+        const dim3 grid = tile_grid(cols, (int)((tokens + rows - 1) / rows));
+        const int32_t *pos = token_topk_to_pos + t0 * num_topk;
+        const float *weights = topk_weights ? topk_weights + t0 * num_topk : nullptr;
+        void *o = static_cast<uint8_t *>(out) + t0 * hidden * out_bytes;
 #define TK_REDUCE_LAUNCH(T, O)                                                                                              \
     hipLaunchKernelGGL((reduce_fused_kernel<T, O>), grid, dim3(kThreads), 0, s, static_cast<const ReduceIn<T>::elem *>(x),  \
-                       token_topk_to_pos, num_tokens, num_topk, (int)hidden, (int)num_expanded, side_log2, (int)(cols == 1), \
-                       topk_weights, x_sf, sf, out)
-    if (x_dtype == TK_BF16) {
-        if (out_dtype == TK_OUT_E4M3) TK_REDUCE_LAUNCH(bf16_t, 2);
-        else TK_REDUCE_LAUNCH(bf16_t, 0);
-    } else if (hidden % 512 == 0) {
-        if (out_dtype == TK_OUT_E4M3) TK_REDUCE_LAUNCH(SplitF32, 2);
-        else TK_REDUCE_LAUNCH(SplitF32, 1);
-    } else {
-        if (out_dtype == TK_OUT_E4M3) TK_REDUCE_LAUNCH(float, 2);
-        else TK_REDUCE_LAUNCH(float, 1);
-    }
+                       pos, tokens, num_topk, (int)hidden, (int)num_expanded, side_log2, (int)(cols == 1), weights, x_sf, sf, o)
+        if (x_dtype == TK_BF16) {
+            if (out_dtype == TK_OUT_E4M3) TK_REDUCE_LAUNCH(bf16_t, 2);
+            else TK_REDUCE_LAUNCH(bf16_t, 0);
+        } else if (hidden % 512 == 0) {
+            if (out_dtype == TK_OUT_E4M3) TK_REDUCE_LAUNCH(SplitF32, 2);
+            else TK_REDUCE_LAUNCH(SplitF32, 1);
+        } else {
+            if (out_dtype == TK_OUT_E4M3) TK_REDUCE_LAUNCH(float, 2);
+            else TK_REDUCE_LAUNCH(float, 1);
+        }
 #undef TK_REDUCE_LAUNCH
+    }
     return (int)hipGetLastError();
 }
