@@ -3,6 +3,8 @@ its host-side validation returns the documented status codes (no kernel is ever 
 import ctypes
 import os
 import re
+import subprocess
+import sys
 
 import pytest
 
@@ -314,3 +316,15 @@ def test_missing_library_fails_loudly(monkeypatch, tmp_path):
     monkeypatch.setattr(_ffi, 'LIB_PATH', str(tmp_path / 'nope.so'))
     with pytest.raises(ImportError):
         _ffi.load()
+
+
+@pytest.mark.parametrize('rows,hidden', [(2 ** 26 + 2 ** 20, 256), (2 ** 27 + 2 ** 20, 128), (2 ** 25 + 2 ** 24, 384)])
+def test_swiglu_launch_plan_of_very_many_short_rows(rows, hidden):
+    """Rows shorter than a piece of 512 columns, too many for the kernel that lays them end to end: the plan of the launch has no
+    piece per row to divide by.  In a process that sees no GPU, where the call ends with HIP's status for that."""
+    code = ('import sys, torch; from tilekernels_amd import _ffi; assert not torch.cuda.is_available(); P = 0x10000; rows, hidden = map(int, sys.argv[1:]); '
+            'rc = _ffi.load().tk_swiglu_per_token_cast(P, 0, rows, hidden, P, P, hidden // 128, 128, 0, 0, -1.0, 0, 0, 0, 0, 0, 0.0, 0, 0, 0); '
+            'assert rc == 100, rc')            # hipErrorNoDevice
+    done = subprocess.run([sys.executable, '-c', code, str(rows), str(hidden)], cwd=ROOT, capture_output=True, text=True,
+                          env=dict(os.environ, HIP_VISIBLE_DEVICES='-1'))
+    assert done.returncode == 0, (done.returncode, done.stderr[-2000:])

@@ -277,3 +277,21 @@ def test_reduce_fused_on_more_than_one_grid_plane(hidden, dtype, rows):
         b = min(a + 16384, tokens)
         part = tk.moe.reduce_fused(x.cuda(), w[a:b].cuda(), t2p[a:b].cuda())
         assert torch.equal(part.view(torch.uint8), got[a:b].view(torch.uint8)), (a, b)
+
+
+def test_swiglu_of_more_short_rows_than_lane_slots():
+    """Rows of 256 outputs, too many for the kernel that numbers lane slots in 32 bits: tiles of 512 columns.  1040 copies of one
+    block of rows, whose result is that of the block alone."""
+    tk = _tk()
+    n, block, H = 1040, 2 ** 16, 256
+    assert n * block * (H // 128) * 16 > LIMIT
+    x1 = _randn_bf16((block, 2 * H), 21)
+    want, want_sf = tk.quant.swiglu_forward_and_per_token_cast(x1, 'e4m3', 128)
+    check_fused((want[:32], want_sf[:32].contiguous()), torch_ref.swiglu_forward_and_per_token_cast(x1[:32].cpu(), 'e4m3', 128), H // 128, False, 'block')
+    x = torch.empty((n, block, 2 * H), dtype=torch.bfloat16, device='cuda')
+    x[:] = x1
+    codes, sf = tk.quant.swiglu_forward_and_per_token_cast(x.view(n * block, 2 * H), 'e4m3', 128)
+    del x
+    codes, sf = codes.view(torch.uint8).view(n, block, H), sf.view(n, block, H // 128)
+    for i in range(n):
+        assert torch.equal(codes[i], want.view(torch.uint8)) and torch.equal(sf[i], want_sf), i

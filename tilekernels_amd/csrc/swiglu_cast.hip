@@ -836,26 +836,31 @@ static void launch_swiglu_tiled(SwigluParams &p, int max_blocks, hipStream_t str
         // 4096] 14.0 / 13.6; stacked tiles [8189, 2 x 2560] 18.2 / 17.3, [2049, 2 x 7168] 13.8 / 12.7, [16381, 2 x 1536] 20.9 / 20.05);
         // column-major scales need whole groups of four rows, whose scales leave together.
         const int64_t slots = wave_slots(), ppr = p.H / kStripCols, row_waves = (int64_t)p.R * ppr / RPW;
-        int rs = (int)std::min<int64_t>((int64_t)p.R * 15 / 100, slots * 6 / 10 / ppr) / 4 * 4;
-        int rm = (int)std::min<int64_t>((int64_t)p.R * 55 / 100, slots * 22 / 10 / ppr) / 4 * 4;
-        int rb = p.R - rm - rs;
-        if constexpr (TILE == T_ROW) {      // the rows beyond the last four are among those of one-piece waves, a workgroup each
-            rb = rb / kWaves * kWaves;
-            rs = p.R - rm - rb;
-        }
-        int64_t ym = (int64_t)rm * 2 / waves, ys = (int64_t)rs * 4 / waves, yb = rb / waves;
-        if constexpr (TILE == T_STACKED) {
-            // stacked tiles of 16 rows, then workgroups of 8 rows (two per wave), then of 4 rows, each on one strip of 512 columns
-            rs = rs / 8 * 8;
-            rb = (p.R - rm - rs) / rows * rows;
-            rm = (p.R - rb - rs) / 8 * 8;
-            rs = p.R - rb - rm;
-            yb = rb / rows; ym = rm / (2 * kWaves); ys = (rs + kWaves - 1) / kWaves;
-        }
         // row-major scales are stored by the waves themselves: a workgroup that overhangs the last row has no barrier to meet
         const bool any_rows = TILE == T_ROW || (TILE == T_STACKED && p.sf.layout == TK_SF_ROW_F32 && tile_grid_exact(p.tiles_k, tiles_m));
-        if ((any_rows ? p.H % cols == 0 : full) && !p.pos_to_expert && waves == kWaves && row_waves * 4 >= slots * 3 && row_waves * 2 <= slots * 7 && rs > 0 && p.tiles_k <= 0xFFF &&
-            ym <= 0xFFFF) {
+        // (a row shorter than one piece has no strip to divide by below: it does not fit the columns)
+        const bool fits = any_rows ? p.H % cols == 0 : full;
+        int rs = 0, rm = 0, rb = 0;
+        int64_t ym = 0, ys = 0, yb = 0;
+        if (fits && !p.pos_to_expert && waves == kWaves && row_waves * 4 >= slots * 3 && row_waves * 2 <= slots * 7 && p.tiles_k <= 0xFFF) {
+            rs = (int)std::min<int64_t>((int64_t)p.R * 15 / 100, slots * 6 / 10 / ppr) / 4 * 4;
+            rm = (int)std::min<int64_t>((int64_t)p.R * 55 / 100, slots * 22 / 10 / ppr) / 4 * 4;
+            rb = p.R - rm - rs;
+            if constexpr (TILE == T_ROW) {      // the rows beyond the last four are among those of one-piece waves, a workgroup each
+                rb = rb / kWaves * kWaves;
+                rs = p.R - rm - rb;
+            }
+            ym = (int64_t)rm * 2 / waves; ys = (int64_t)rs * 4 / waves; yb = rb / waves;
+            if constexpr (TILE == T_STACKED) {
+                // stacked tiles of 16 rows, then workgroups of 8 rows (two per wave), then of 4 rows, each on one strip of 512 columns
+                rs = rs / 8 * 8;
+                rb = (p.R - rm - rs) / rows * rows;
+                rm = (p.R - rb - rs) / 8 * 8;
+                rs = p.R - rb - rm;
+                yb = rb / rows; ym = rm / (2 * kWaves); ys = (rs + kWaves - 1) / kWaves;
+            }
+        }
+        if (rs > 0 && ym <= 0xFFFF) {
             const dim3 tgrid = tile_grid(p.tiles_k, (int)(yb + ym + ys));
             p.nwaves = waves | (p.tiles_k << 4) | ((int)ym << 16);
             p.tiles_k = (int)yb;
