@@ -1,6 +1,7 @@
 """The native call path of the ops against their Python code: the same results in the same layout for every form both accept,
 and None (so that the Python code takes the call) for the forms it leaves alone."""
 import itertools
+import os
 
 import pytest
 import torch
@@ -180,3 +181,49 @@ def test_cpu_tensors_are_left_alone(op):
     assert fn(*[None] * len(args)) is None and fn(*[object()] * len(args)) is None
     with pytest.raises(TypeError):
         fn()
+
+
+def test_native_path_is_named_for_what_it_was_built_against():
+    import sysconfig
+    from tilekernels_amd import _ffi
+    name = os.path.basename(_ffi.HOST_PATH)
+    assert torch.__version__ in name and sysconfig.get_config_var('SOABI') in name
+    assert os.path.exists(_ffi.HOST_PATH)
+
+
+@pytest.mark.parametrize('content', [None, b'not a library'], ids=['missing', 'unusable'])
+def test_calls_without_a_native_path_are_left_to_python(monkeypatch, tmp_path, content):
+    """A library built for another torch or Python is not loaded: one warning, then every call is that of the Python code."""
+    import warnings
+    import tilekernels_amd as tk
+    from tilekernels_amd import _ffi
+    path = tmp_path / '_host.so'
+    if content is not None:
+        path.write_bytes(content)
+    monkeypatch.setattr(_ffi, 'HOST_PATH', str(path))
+    monkeypatch.setattr(_ffi, 'host', _ffi._UnloadedHost())
+    x = torch.zeros((4, 512), dtype=torch.bfloat16)
+    with pytest.warns(RuntimeWarning, match='native call path'):
+        with pytest.raises(_ffi.TkError, match='GPU only'):
+            tk.quant.per_token_cast(x, 'e4m3', 128)
+    with warnings.catch_warnings():
+        warnings.simplefilter('error')
+        with pytest.raises(_ffi.TkError, match='GPU only'):
+            tk.quant.per_block_cast(x, 'e4m3', (128, 128))
+        with pytest.raises(AssertionError):
+            tk.quant.per_token_cast(x, 'e4m3', 48)
+
+
+def test_native_path_is_loaded_once_by_threads(monkeypatch):
+    import threading
+    from tilekernels_amd import _ffi
+    loads, load_host = [], _ffi._load_host
+    monkeypatch.setattr(_ffi, '_load_host', lambda: loads.append(1) or load_host())
+    monkeypatch.setattr(_ffi, 'host', _ffi._UnloadedHost())
+    results = []
+    threads = [threading.Thread(target=lambda: results.append(_ffi.host.cast_back(None, None, None, None, None))) for _ in range(8)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert results == [None] * 8 and len(loads) == 1

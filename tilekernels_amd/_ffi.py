@@ -5,12 +5,17 @@ There is deliberately no fallback: if the library has not been built, importing 
 import ctypes
 import importlib.util
 import os
+import sysconfig
+import threading
+import warnings
 
 import torch  # noqa: F401  (loads the HIP runtime the library links against before the library itself)
 
 _PKG = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_PKG, 'lib', 'libtk_quant.so')
-HOST_PATH = os.path.join(_PKG, 'lib', '_host.so')
+# the native call path is compiled against torch's C++ headers and the CPython ABI, neither of which is stable: its name carries the
+# versions it was built for, so that a process with others does not load it
+HOST_PATH = os.path.join(_PKG, 'lib', f'_host.torch-{torch.__version__}.{sysconfig.get_config_var("SOABI")}.so')
 
 TK_BF16, TK_F32, TK_OUT_E4M3 = 0, 1, 2
 TK_E4M3, TK_E2M1, TK_E5M6 = 0, 1, 2
@@ -81,19 +86,46 @@ def load() -> ctypes.CDLL:
     return _lib
 
 
+_host_lock = threading.Lock()
+
+
+def _leave_to_python(*args):
+    return None
+
+
+class _NoHost:
+    """Stands in for a native call path that this process cannot load: every call is left to its Python code."""
+
+    def __getattr__(self, name):
+        if name.startswith('__'):
+            raise AttributeError(name)
+        return _leave_to_python
+
+
 class _UnloadedHost:
     """Stands in `host` until the first op is called: importing the package does not need the built libraries."""
 
     def __getattr__(self, name):
         global host
-        load()
-        if not os.path.exists(HOST_PATH):
-            raise ImportError(f'{HOST_PATH} not found: build it with `python -m tilekernels_amd.build`')
+        if name.startswith('__'):
+            raise AttributeError(name)
+        with _host_lock:
+            if host is self:
+                host = _load_host()
+        return getattr(host, name)
+
+
+def _load_host():
+    load()
+    try:
         spec = importlib.util.spec_from_file_location('tilekernels_amd._host', HOST_PATH)
         module = importlib.util.module_from_spec(spec)
         spec.loader.exec_module(module)
-        host = module
-        return getattr(module, name)
+        return module
+    except ImportError as e:
+        warnings.warn(f'no native call path for this torch and Python ({e}); every call of an op costs the host some 6 us more. '
+                      'Build it with `python -m tilekernels_amd.build`', RuntimeWarning, stacklevel=3)
+        return _NoHost()
 
 
 # the native call path (csrc/host.cpp): each function gives an op's result, or None for calls that its Python code is to take

@@ -1,4 +1,5 @@
-"""Ahead-of-time build of libtk_quant.so (hipcc, gfx950 only) and of _host.so, the ops' native call path (host code on torch).
+"""Ahead-of-time build of libtk_quant.so (hipcc, gfx950 only) and of _host.*.so, the ops' native call path (host code
+on torch, named for the torch and Python versions it is built against).
 
     python -m tilekernels_amd.build [--force]
 
@@ -11,11 +12,12 @@ import sys
 import sysconfig
 from concurrent.futures import ThreadPoolExecutor
 
+from ._ffi import HOST_PATH
+
 PKG = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(PKG, 'csrc')
 LIB_DIR = os.path.join(PKG, 'lib')
 LIB_PATH = os.path.join(LIB_DIR, 'libtk_quant.so')
-HOST_PATH = os.path.join(LIB_DIR, '_host.so')
 SOURCES = ['api.hip', 'per_token_cast.hip', 'per_block_cast.hip', 'swiglu_cast.hip', 'cast_back.hip', 'moe_layout.hip',
            'swiglu_backward.hip', 'per_channel_cast.hip', 'lossless_cast.hip', 'stream_floor.hip', 'swiglu_cast_variants.hip']
 
@@ -49,15 +51,16 @@ def _build_host() -> None:
     import torch
     root = os.path.dirname(torch.__file__)
     cmd = [os.environ.get('CXX', 'g++'), '-O2', '-std=c++17', '-fPIC', '-shared', '-Wall', '-D__HIP_PLATFORM_AMD__=1', '-DUSE_ROCM=1',
-           f'-I{root}/include', f'-I{sysconfig.get_paths()["include"]}', '-I/opt/rocm/include', os.path.join(CSRC, 'host.cpp'), '-o', HOST_PATH,
+           f'-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}', f'-I{root}/include', f'-I{sysconfig.get_paths()["include"]}',
+           '-I/opt/rocm/include', os.path.join(CSRC, 'host.cpp'), '-o', HOST_PATH,
            f'-L{LIB_DIR}', '-l:libtk_quant.so', f'-L{root}/lib', '-lc10', '-lc10_hip', '-ltorch_cpu', '-ltorch_python', '-Wl,-rpath,$ORIGIN']
     r = subprocess.run(cmd, capture_output=True, text=True)
     if r.returncode != 0:
-        raise RuntimeError(f'the build of _host.so failed:\n{r.stderr}')
+        raise RuntimeError(f'the build of {HOST_PATH} failed:\n{r.stderr}')
 
 
 def build_library(force: bool = True) -> str:
-    """Compile every HIP source, link libtk_quant.so and build _host.so beside it.  Returns the path of libtk_quant.so."""
+    """Compile every HIP source, link libtk_quant.so and build the native call path beside it.  Returns the path of libtk_quant.so."""
     if not force and os.path.exists(LIB_PATH) and os.path.exists(HOST_PATH):
         return LIB_PATH
     os.makedirs(LIB_DIR, exist_ok=True)
