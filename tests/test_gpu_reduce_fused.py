@@ -106,3 +106,26 @@ def test_reduce_fused_with_few_and_many_live_terms(T, K, dtype, hidden):
     w = torch.rand((T, K), generator=g)
     want = torch_ref.reduce_fused(x, w, t2p)
     assert_same(tk.moe.reduce_fused(x.cuda(), w.cuda(), t2p.cuda()), want, 'reduced')
+
+
+@pytest.mark.parametrize('dtype', [torch.float32, torch.bfloat16], ids=['f32', 'bf16'])
+@pytest.mark.parametrize('T,hidden', [(7, 256), (9, 512), (6, 768), (5, 1280), (3, 2048), (2060, 2048), (4, 2560), (1030, 4096), (3, 7168)])
+def test_reduce_fused_workgroup_shapes_and_dead_terms(T, hidden, dtype):
+    """Rows of one to fourteen pieces, launches below and above one round of wave slots, one to thirteen terms: lists that are all live,
+    and lists whose dead terms carry any position outside the rows, a NaN weight and no scale of their own."""
+    tk = _tk()
+    R = 40
+    g = torch.Generator().manual_seed(T + hidden)
+    x = torch.randn((R, hidden), generator=g).to(dtype)
+    x_sf = torch.rand((R,), generator=g)
+    for K in (1, 2, 3, 8, 13):
+        w = torch.rand((T, K), generator=g)
+        full = torch.randint(0, R, (T, K), generator=g, dtype=torch.int32)
+        dead = torch.rand((T, K), generator=g) < 0.5
+        some = full.masked_fill(dead, -1)
+        outside = torch.tensor([-1, -2 ** 31, R, 2 ** 31 - 1], dtype=torch.int32)[torch.randint(0, 4, (T, K), generator=g)]
+        xg, sg = x.cuda(), x_sf.cuda()
+        for xin, xgpu in ((x, xg), ((x, x_sf), (xg, sg))):
+            assert_same(tk.moe.reduce_fused(xgpu, w.cuda(), full.cuda()), torch_ref.reduce_fused(xin, w, full), f'{K} full')
+            got = tk.moe.reduce_fused(xgpu, w.masked_fill(dead, float('nan')).cuda(), torch.where(dead, outside, full).cuda())
+            assert_same(got, torch_ref.reduce_fused(xin, w, some), f'{K} some')

@@ -541,64 +541,103 @@ __global__ __launch_bounds__(kThreads) void expand_short_rows_kernel(const uint8
 // s = topk_weights[t, k] (or 1) times x_sf[pos] (if given); positions < 0 are skipped.  The sum is scaled by *sf (if
 // given) and rounded to the output type.
 //
-// What bounds it is the gather of whole rows from HBM.  A wave owns 512 columns of one token.  Lane k fetches position and
-// factor of term k, a ballot says which terms are live, and only those are loaded, 8 (fp32: 4) of them before the first
-// is used (v_readlane hands a live term's row and factor to the whole wave as scalars).  A rank of an expert-parallel
-// group holds few of a token's experts, one or two of eight on average; loading place-holders for the others (row 0, so
-// that there is no branch around a load) took as long as loading rows.  Measured on MI355X, us, place-holders / this:
-//   bf16 [34816, 7168] -> [21616, 7168], 1.6 live terms of 8: 226 / 130 (6.0 TB/s);  [.., 2560]: 102 / 44;  [.., 1280]: 39 / 26
-//   bf16 [48128, 4096] -> [4096, 4096], 8 of 8: 49.0 / 48.7;  [.., 1280], 8 of 8: 16.0 / 17.0;  [.., 2560], 6 of 6: 27.3 / 24.3
-//   fp32 [81792, 4096], 8 of 8: 209.9 / 211.4 (to E4M3 175.3 / 177.2);  [.., 2304], 9 of 9: 103 / 76
-// Positions and factors through the scalar path instead (eight loads each, put into lanes one by one): 163 and 54 us where 132
-// and 45; two pieces of 512 columns per wave and four terms at a time: 133 and 52.5 us, 8.0 instead of 4.4 us for 300 tokens.
+// What bounds it is the gather of whole rows from HBM.  A wave owns 512 columns of one token and asks for all its terms' pieces, up to
+// 8, before it uses the first.  Positions, weights and scales are the same for the whole wave and come through the scalar path.  A
+// rank of an expert-parallel group holds few of a token's experts, one or two of eight on average, and a term that is not live must
+// cost nothing: place-holders for it (row 0, so that there is no branch around a load) take as long as rows.  So a group of terms
+// that are all live loads without a branch, any other skips its dead terms by branches between the loads; that works because the
+// loads' addresses are buffers in scalar registers (see reduce_load).
+// us on MI355X, place-holders / live terms found by a ballot over positions that a vector load fetched, 512 columns of 4 tokens or
+// 1024 of 2 per workgroup / this, all with weights:
+//   bf16 1 of 8 live: [21537, 1280] -> [20000, 1280] 34.5 / 21.3 / 18.9;  [4096, 7168] into a worst-case buffer 40.5 / 21.3 / 19.7
+//   bf16 8 of 8: [4096, 512] 7.05 / 7.1 / 7.05;  [.., 1280] 15.9 / 17.0 / 16.1;  [.., 2048] 25.2 / 25.9 / 25.2;  [.., 2560] 35.3 / 31.4 / 31.1;
+//   [.., 4096] 50.1 / 49.2 / 49.2;  [.., 7168] 88.6 / 86.3 / 85.6;  340 tokens of 4096 5.07 / 5.4 / 5.1;  [8192, 1280], 2 of 2: 10.8 / 12.6 / 11.2
+//   fp32 8 of 8: [4096, 1280] 37.8 / 39.2 / 36.4;  [.., 2048] 50.5 / 51.2 / 50.2;  [.., 4096] 103.2 / 104.0 / 100.3;  64 tokens of 7168 4.1 / 4.9 / 4.2
 // fp32 rows whose length is a multiple of 512: a thread's 8 elements are two runs of 4, 256 columns apart, so that each
 // of its 16-byte loads (and of its fp32 stores) is, over the wave, 1024 consecutive bytes.  With the 8 elements in one
 // run, every instruction touches half of each cache line it names (fp32 [81792, 4096] -> fp32, top-8: 220 instead of 210 us).
 struct SplitF32 {};
-struct Raw8SplitF32 {
-    u32x4 a, b;
-    __device__ __forceinline__ void load(const float *p) { a = ld_stream16(p); vmem_issue_gap(); b = ld_stream16(p + 256); }
-    __device__ __forceinline__ void get(float (&v)[8]) const {
-        v[0] = u2f(a.x); v[1] = u2f(a.y); v[2] = u2f(a.z); v[3] = u2f(a.w);
-        v[4] = u2f(b.x); v[5] = u2f(b.y); v[6] = u2f(b.z); v[7] = u2f(b.w);
-    }
-};
 template <typename InT> struct ReduceIn;
-template <> struct ReduceIn<bf16_t> { typedef Raw8<bf16_t> raw; typedef bf16_t elem; static constexpr bool split = false; static constexpr int unroll = 8; };
-template <> struct ReduceIn<float> { typedef Raw8<float> raw; typedef float elem; static constexpr bool split = false; static constexpr int unroll = 4; };
-template <> struct ReduceIn<SplitF32> { typedef Raw8SplitF32 raw; typedef float elem; static constexpr bool split = true; static constexpr int unroll = 4; };
+template <> struct ReduceIn<bf16_t> { typedef Raw8<bf16_t> raw; typedef bf16_t elem; static constexpr int lane_bytes = 16, second = 0; };
+template <> struct ReduceIn<float> { typedef Raw8<float> raw; typedef float elem; static constexpr int lane_bytes = 32, second = 16; };
+template <> struct ReduceIn<SplitF32> { typedef Raw8<float> raw; typedef float elem; static constexpr int lane_bytes = 16, second = 1024; };
 
-// the first U terms of `live`, which has at least that many: all pieces are loaded before the first is used
-template <typename InT, int U>
-__device__ __forceinline__ void reduce_terms(float (&acc)[8], const typename ReduceIn<InT>::elem *x, int hidden, unsigned long long &live, int pos,
-                                             float factor) {
-    typename ReduceIn<InT>::raw raw[U];
-    float s[U];
-#pragma unroll
-    for (int j = 0; j < U; ++j) {
-        const int k = __builtin_ctzll(live);
-        live &= live - 1;
-        raw[j].load(x + (int64_t)__builtin_amdgcn_readlane(pos, k) * hidden);
+// One lane's 8 elements of a piece of 512 columns.  The piece is a buffer of its own, `bytes` long: lanes beyond the end of the row
+// read zeros and touch no memory, and no register of the lane holds an address (with addresses in registers a load behind a branch
+// waits for an earlier one whose target the address is formed in).
+template <typename InT>
+__device__ __forceinline__ void reduce_load(typename ReduceIn<InT>::raw &raw, const uint8_t *piece, uint32_t bytes, uint32_t lane_off) {
+    const __amdgpu_buffer_rsrc_t buf = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t *>(piece), 0, (int)bytes, 0x00020000);
+    constexpr int kNonTemporal = 2;
+    const auto at = [&](uint32_t off) { return __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(buf, off, 0, kNonTemporal)); };
+    if constexpr (ReduceIn<InT>::second != 0) {
+        raw.a = at(lane_off);
         vmem_issue_gap();
-        s[j] = u2f((uint32_t)__builtin_amdgcn_readlane((int)f2u(factor), k));
+        raw.b = at(lane_off + ReduceIn<InT>::second);
+    } else {
+        raw.w = at(lane_off);
     }
-    // without this the arithmetic on the first piece moves in front of the later loads, which then wait for it
-    // (bf16 [16384, 256], 8 of 8 terms: 20.2 -> 12.5 us)
+    vmem_issue_gap();
+}
+
+// U consecutive terms of a token, those in `live` only (ALL: every one).  Everything but the pieces comes through the scalar path.
+template <typename InT, int U, bool ALL>
+__device__ __forceinline__ void reduce_terms(float (&acc)[8], const uint8_t *x, uint32_t bytes, uint32_t lane_off, uint64_t row_bytes, uint32_t num_expanded,
+                                             const uint32_t (&pos)[U], const float *weights, const float *x_sf) {
+    typename ReduceIn<InT>::raw raw[U];
+    uint32_t live = 0;
+    float w[U], f[U];
+#pragma unroll
+    for (int j = 0; j < U; ++j)
+        if (ALL || pos[j] < num_expanded) {
+            live |= 1u << j;
+            reduce_load<InT>(raw[j], x + pos[j] * row_bytes, bytes, lane_off);
+        }
+    if constexpr (!ALL) {
+        // (behind this the compiler no longer knows that the conditions below are those above: it would sink each load to its use)
+        live = (uint32_t)__builtin_amdgcn_readfirstlane((int)live);
+        asm volatile("" : "+s"(live));
+    }
+#pragma unroll
+    for (int j = 0; j < U; ++j) w[j] = f[j] = 1.0f;
+    if (weights) {
+#pragma unroll
+        for (int j = 0; j < U; ++j) w[j] = uniform_load(weights + j);
+    }
+    if (x_sf) {
+#pragma unroll
+        for (int j = 0; j < U; ++j) f[j] = uniform_load(x_sf + (ALL || pos[j] < num_expanded ? pos[j] : 0u));
+    }
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
     for (int j = 0; j < U; ++j) {
+        if (!ALL && !(live >> j & 1)) continue;
         float v[8];
         raw[j].get(v);
+        const float s = w[j] * f[j];
 #pragma unroll
-        for (int i = 0; i < 8; ++i) acc[i] = __builtin_fmaf(v[i], s[j], acc[i]);
+        for (int i = 0; i < 8; ++i) acc[i] = __builtin_fmaf(v[i], s, acc[i]);
     }
+}
+
+template <typename InT, int U>
+__device__ __forceinline__ void reduce_group(float (&acc)[8], const uint8_t *x, uint32_t bytes, uint32_t lane_off, uint64_t row_bytes, uint32_t num_expanded,
+                                             const int32_t *list, const float *weights, const float *x_sf) {
+    uint32_t pos[U], last = 0;
+#pragma unroll
+    for (int j = 0; j < U; ++j) pos[j] = (uint32_t)uniform_load(list + j);
+    // (written out: the compiler takes the maximum of uniform values through the vector unit)
+#pragma unroll
+    for (int j = 0; j < U; ++j) asm("s_max_u32 %0, %1, %2" : "=s"(last) : "s"(last), "s"(pos[j]) : "scc");
+    if (last < num_expanded) reduce_terms<InT, U, true>(acc, x, bytes, lane_off, row_bytes, num_expanded, pos, weights, x_sf);
+    else reduce_terms<InT, U, false>(acc, x, bytes, lane_off, row_bytes, num_expanded, pos, weights, x_sf);
 }
 
 // OUT: 0 bf16, 1 fp32, 2 E4M3
 template <typename InT, int OUT>
 __device__ __forceinline__ void reduce_store(const float (&acc)[8], void *out, int64_t idx) {
     typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
-    constexpr bool SPLIT = ReduceIn<InT>::split;
+    constexpr bool SPLIT = ReduceIn<InT>::second > 16;
     if (OUT == 1) {
         u32x4 *o = reinterpret_cast<u32x4 *>(reinterpret_cast<float *>(out) + idx);
         __builtin_nontemporal_store(u32x4{f2u(acc[0]), f2u(acc[1]), f2u(acc[2]), f2u(acc[3])}, o);
@@ -621,50 +660,52 @@ __device__ __forceinline__ void reduce_store(const float (&acc)[8], void *out, i
     }
 }
 
-// (Registers for eight waves per SIMD: the gather needs them all in flight, bf16 [34816, 7168] at six waves 142 us.)
-// A workgroup is kWaves >> side_log2 tokens high and 1 << side_log2 pieces of 512 columns wide.
-template <typename InT, int OUT>
-__global__ __launch_bounds__(kThreads, 8) void reduce_fused_kernel(const typename ReduceIn<InT>::elem *x, const int32_t *token_topk_to_pos, int64_t num_tokens,
-                                                                int num_topk, int hidden, int num_expanded, int side_log2, int one_col,
+// A workgroup takes `side` pieces of one token, or (STACKED, side 1 or 2) those of 4 / side tokens.
+template <typename InT, int OUT, bool STACKED>
+__global__ __launch_bounds__(kThreads) void reduce_fused_kernel(const typename ReduceIn<InT>::elem *x, const int32_t *token_topk_to_pos, int num_tokens,
+                                                                int num_topk, int hidden, int num_expanded, int shape,
                                                                 const float *topk_weights, const float *x_sf, const float *sf, void *out) {
-    constexpr bool SPLIT = ReduceIn<InT>::split;
+    constexpr uint32_t kElem = sizeof(typename ReduceIn<InT>::elem);
+    const int side = shape & 7, one_col = shape >> 3;
     const int lane = threadIdx.x & 63, wave = wave_id();
-    const int64_t t = ((int64_t)tile_grid_row(one_col) << (2 - side_log2)) + (wave >> side_log2);
-    static_assert(kWaves == 4, "side_log2 is 0 to 2");
-    const int piece = (tile_grid_col(one_col) << side_log2) + (wave & ((1 << side_log2) - 1));
-    // SPLIT: elements col .. col + 3 and col + 256 .. col + 259
-    const int col = piece * kStripCols + lane * (SPLIT ? 4 : 8);
+    const int t = STACKED ? (tile_grid_row(one_col) << (3 - side)) + (wave >> (side - 1)) : tile_grid_row(one_col);
+    const int piece = tile_grid_col(one_col) * side + (STACKED ? wave & (side - 1) : wave);
     if (t >= num_tokens) return;
-    const bool inside = col < hidden;
-    x += inside ? col : 0;
+    const int cols = min(hidden - piece * kStripCols, kStripCols);
+    const uint32_t lane_off = (uint32_t)lane * ReduceIn<InT>::lane_bytes;
+    const uint8_t *xp = reinterpret_cast<const uint8_t *>(x) + (uint64_t)(uint32_t)piece * (kStripCols * kElem);
+    const uint64_t row_bytes = (uint64_t)(uint32_t)hidden * kElem;
     float acc[8];
 #pragma unroll
     for (int i = 0; i < 8; ++i) acc[i] = 0.0f;
-    for (int k0 = 0; k0 < num_topk; k0 += 64) {
-        const int k = k0 + lane;
-        const int64_t at = t * num_topk + (k < num_topk ? k : k0);
-        const int pos = token_topk_to_pos[at];
-        float factor = topk_weights ? topk_weights[at] : 1.0f;
-        const bool ok = k < num_topk && pos >= 0 && pos < num_expanded;
-        if (x_sf) factor = factor * x_sf[ok ? pos : 0];
-        unsigned long long live = __builtin_amdgcn_ballot_w64(ok);
-        int n = __popcll(live);
-        constexpr int U = ReduceIn<InT>::unroll;
-        for (; n >= U; n -= U) reduce_terms<InT, U>(acc, x, hidden, live, pos, factor);
-        if (U > 4 && (n & 4)) reduce_terms<InT, 4>(acc, x, hidden, live, pos, factor);
-        if (n & 2) reduce_terms<InT, 2>(acc, x, hidden, live, pos, factor);
-        if (n & 1) reduce_terms<InT, 1>(acc, x, hidden, live, pos, factor);
+    const int32_t *list = token_topk_to_pos + (int64_t)t * num_topk;
+    const float *weights = topk_weights ? topk_weights + (int64_t)t * num_topk : nullptr;
+    int left = num_topk;
+#define TK_REDUCE_TERMS(U)                                                                                                       \
+    do {                                                                                                                         \
+        reduce_group<InT, U>(acc, xp, (uint32_t)cols * kElem, lane_off, row_bytes, (uint32_t)num_expanded, list, weights, x_sf); \
+        list += U;                                                                                                               \
+        if (weights) weights += U;                                                                                               \
+    } while (0)
+    if constexpr (!STACKED) {      // (STACKED: one or two terms)
+        for (; left >= 8; left -= 8) TK_REDUCE_TERMS(8);
+        if (left & 4) TK_REDUCE_TERMS(4);
     }
+    if (left & 2) TK_REDUCE_TERMS(2);
+    if (left & 1) TK_REDUCE_TERMS(1);
+#undef TK_REDUCE_TERMS
     if (sf) {
         const float f = uniform_load(sf);
 #pragma unroll
         for (int i = 0; i < 8; ++i) acc[i] = acc[i] * f;
     }
-    if (inside) reduce_store<InT, OUT>(acc, out, t * hidden + col);
+    // the lane's first column; SPLIT: elements col .. col + 3 and col + 256 .. col + 259 (whole pieces only)
+    const int col = piece * kStripCols + lane * (int)(ReduceIn<InT>::lane_bytes / kElem);
+    if (col < hidden) reduce_store<InT, OUT>(acc, out, (int64_t)t * hidden + col);
 }
 
 // reduce_fused without a single expanded row: every term is skipped, the result is zeros.  (The reduction kernel
-// cannot run then: its skipped terms read row 0, which does not exist.)
+// reads the first row's scale in the place of a skipped term's, and there is none then.)
 __global__ __launch_bounds__(kThreads) void reduce_zero_kernel(uint64_t *out, int64_t words) {
     for (int64_t i = (int64_t)blockIdx.x * kThreads + threadIdx.x; i < words; i += (int64_t)gridDim.x * kThreads) out[i] = 0ull;
 }
@@ -912,15 +953,21 @@ extern "C" int tk_reduce_fused(const void *x, int x_dtype, int64_t num_expanded,
         return (int)hipGetLastError();
     }
     const int strips = (int)((hidden + kStripCols - 1) / kStripCols);
-    // Two pieces side by side where the row has an even number of them (300 tokens of 4096 columns 4.9 -> 4.3 us, nothing
-    // lost at larger sizes), four of fp32 (344 tokens of 4096 4.5 -> 3.7, 65536 terms of 4096 columns 213.5 -> 211); with an odd
-    // number the last workgroup of a row would be half idle (3 pieces: 26 -> 32 us).
-    const int side_log2 = strips % 4 == 0 && x_dtype == TK_F32 ? 2 : (strips % 2 == 0 ? 1 : 0);
-    const int64_t rows = kWaves >> side_log2;
-    const int cols = strips >> side_log2;
+    // Pieces side by side in a workgroup: whole rows of up to four, otherwise the largest number up to four that divides the row (five
+    // or seven waves 31.5 and 43.5 us instead of 31.0 and 42.8 for bf16 [4096, 2560] and [.., 3584], 8 of 8).  In launches that fill the
+    // GPU's wave slots more than once, with more than four terms, two instead of four (bf16 [4096, 4096], 8 of 8: 51.5 / 49.2 us; with
+    // two terms [32768, 2048] 61.5 / 63.5, and 340 tokens 5.2 / 5.5) and, fp32, one ([4096, 4096] 104.0 / 100.3).
+    int side = 4;
+    while (strips % side) --side;
+    if (side == 4 && num_topk > 4 && num_tokens * strips > 8192) side = x_dtype == TK_BF16 ? 2 : 1;
+    // One or two terms of short rows: four waves to a workgroup all the same, on further tokens, since workgroups of one wave are
+    // not started fast enough (bf16 [262144, 256], one term: 69.1 / 61.9 us; fp32 104.3 / 102.9, but [262144, 512] 180 / 186).
+    const bool stacked = num_topk <= 2 && (x_dtype == TK_BF16 ? side <= 2 : hidden <= 256);
     // HIP takes fewer than 2^32 threads along a grid dimension, and the row tiles of a single column of pieces all ride on x:
     // at most 2^23 row tiles (2^31 threads) per launch.
-    const int64_t step = rows << 23, out_bytes = out_dtype == TK_F32 ? 4 : (out_dtype == TK_BF16 ? 2 : 1);
+    const int64_t rows = stacked ? 4 / side : 1, step = rows << 23, out_bytes = out_dtype == TK_F32 ? 4 : (out_dtype == TK_BF16 ? 2 : 1);
+    const int cols = strips / side;
+    const dim3 block((unsigned)(64 * side * rows));
     for (int64_t t0 = 0; t0 < num_tokens; t0 += step) {
         const int64_t tokens = std::min(num_tokens - t0, step);
         const dim3 grid = tile_grid(cols, (int)((tokens + rows - 1) / rows));
@@ -928,8 +975,13 @@ extern "C" int tk_reduce_fused(const void *x, int x_dtype, int64_t num_expanded,
         const float *weights = topk_weights ? topk_weights + t0 * num_topk : nullptr;
         void *o = static_cast<uint8_t *>(out) + t0 * hidden * out_bytes;
 #define TK_REDUCE_LAUNCH(T, O)                                                                                              \
-    hipLaunchKernelGGL((reduce_fused_kernel<T, O>), grid, dim3(kThreads), 0, s, static_cast<const ReduceIn<T>::elem *>(x),  \
-                       pos, tokens, num_topk, (int)hidden, (int)num_expanded, side_log2, (int)(cols == 1), weights, x_sf, sf, o)
+    do {                                                                                                                    \
+        if (stacked) TK_REDUCE_LAUNCH_2(T, O, true);                                                                        \
+        else TK_REDUCE_LAUNCH_2(T, O, false);                                                                               \
+    } while (0)
+#define TK_REDUCE_LAUNCH_2(T, O, S)                                                                                         \
+    hipLaunchKernelGGL((reduce_fused_kernel<T, O, S>), grid, block, 0, s, static_cast<const ReduceIn<T>::elem *>(x), pos,   \
+                       (int)tokens, num_topk, (int)hidden, (int)num_expanded, side | (int)(cols == 1) << 3, weights, x_sf, sf, o)
         if (x_dtype == TK_BF16) {
             if (out_dtype == TK_OUT_E4M3) TK_REDUCE_LAUNCH(bf16_t, 2);
             else TK_REDUCE_LAUNCH(bf16_t, 0);
@@ -940,6 +992,7 @@ extern "C" int tk_reduce_fused(const void *x, int x_dtype, int64_t num_expanded,
             if (out_dtype == TK_OUT_E4M3) TK_REDUCE_LAUNCH(float, 2);
             else TK_REDUCE_LAUNCH(float, 1);
         }
+#undef TK_REDUCE_LAUNCH_2
 #undef TK_REDUCE_LAUNCH
     }
     return (int)hipGetLastError();
