@@ -158,3 +158,36 @@ def test_mapping_of_long_lists(T, K, E, drop, alignment):
             assert torch.equal(a.cpu()[:n], b[:n]) and bool((a.cpu()[n:] == -1).all()), (name, extra)
         for a, b, name in zip(got[3:7], want[3:7], ('token_topk_to_pos', 'expert_start', 'expert_end', 'num_tokens_per_expert')):
             assert_same(a, b, name)
+
+
+@pytest.mark.parametrize('col_major', [False, True], ids=['row', 'col'])
+@pytest.mark.parametrize('live', [0.2, 1.0])
+@pytest.mark.parametrize('T,K,row_bytes,sf_cols,pad', [(9, 8, 4096, 32, 40), (63, 8, 4096, 32, 300), (64, 4, 4096, 300, 300), (70, 3, 9216, 288, 9),
+                                                       (127, 8, 2048, 16, 600), (129, 8, 2048, 200, 600), (300, 2, 1024, 100, 500), (33, 70, 1040, 65, 0)])
+def test_expand_to_fused_scale_words(T, K, row_bytes, sf_cols, pad, live, col_major):
+    """A workgroup per list entry (few tokens, or much padding) and per token, with fewer and with more scale words than threads per row."""
+    from tilekernels_amd import _ffi
+    g = torch.Generator().manual_seed(T * K + sf_cols)
+    here = torch.rand((T, K), generator=g) < live
+    n = int(here.sum())
+    R = n + pad
+    t2p = torch.full((T, K), -1, dtype=torch.int32)
+    t2p[here] = torch.randperm(R, generator=g)[:n].to(torch.int32)
+    p2e = torch.full((R,), -1, dtype=torch.int32)
+    p2e[t2p[here].long()] = 1
+    x = torch.randint(0, 256, (T, row_bytes), generator=g, dtype=torch.uint8)
+    sf = torch.randint(-2 ** 31, 2 ** 31 - 1, (T, sf_cols), generator=g, dtype=torch.int32)
+    want, want_sf = torch.zeros((R, row_bytes), dtype=torch.uint8), torch.zeros((R, sf_cols), dtype=torch.int32)
+    token = torch.arange(T)[:, None].expand(T, K)[here]
+    want[t2p[here].long()], want_sf[t2p[here].long()] = x[token], sf[token]
+    xg, sg, tg, pg = x.cuda(), sf.cuda(), t2p.cuda(), p2e.cuda()
+    out = torch.full((R, row_bytes), 0x5A, dtype=torch.uint8, device='cuda')
+    ld = R + 3 if col_major else sf_cols + 3
+    out_sf = torch.full((sf_cols if col_major else R, ld), 0x5A5A5A5A, dtype=torch.int32, device='cuda')
+    rc = _ffi.load().tk_expand_to_fused(xg.data_ptr(), T, row_bytes, tg.data_ptr(), K, pg.data_ptr(), R, out.data_ptr(), sg.data_ptr(), sf_cols,
+                                        out_sf.data_ptr(), ld, int(col_major), torch.cuda.current_stream().cuda_stream)
+    assert rc == 0, rc
+    assert torch.equal(out.cpu(), want)
+    got = out_sf.cpu()
+    assert bool((got[:, -3:] == 0x5A5A5A5A).all())
+    assert torch.equal(got[:, :-3].T.contiguous() if col_major else got[:, :-3], want_sf)

@@ -426,10 +426,12 @@ __device__ __forceinline__ void expand_zero_padding(int pb, int pad_rows, int nu
 // ballot says which entries have a position, and there is one store per thread for each of them.  What bounds an
 // expert-parallel rank's expansion with EVERY is the dispatch of workgroups that find no position (0.7 ns each, whatever
 // they do).  us per call on MI355X, EVERY / one per token (codes with scales, top-8 unless said):
-//   [4096, 7168] of 8 ranks, [21504] tokens -> [34816]  218 / 62      340 tokens -> [3232, 4096] (worst-case buffer)  5.4 / 4.4
-//   [512, 4096] -> [6144]   7.0 / 6.2                  [2048, 7168] -> [18432]  30.6 / 28.5       top-2 of [4096, 7168]  17.3 / 17.3
-//   [4096, 4096] -> [48128]  38.1 / 39.2               bf16 [4096, 4096] -> [48128]  64.4 / 73.5
-template <bool EVERY>
+//   one of 8 ranks: 21504 tokens -> [24064, 7168]  214 / 59.5      340 tokens -> [6784, 4096] (worst-case buffer)  6.7 / 5.4
+//   full lists: [512, 4096] -> [5120]  6.6 / 4.7      [2048, 7168] -> [17536]  31.3 / 27.9      top-2 of [8192, 7168]  32.1 / 29.5
+//   bf16 -> rows of 4096, 110 MB 25.6 / 22.8, 132 MB 30.3 / 27.2, 154 MB 35.4 / 32.9;  7168, 160 MB 36.8 / 33.9;  from 160 MB on EVERY:
+//   [4096, 4096] codes -> 197 MB 38.1 / 39.2, bf16 -> 394 MB 64.4 / 73.5
+// SF: there may be scales (else nothing of them is looked at; x_sf may be null all the same)
+template <bool EVERY, bool SF>
 __global__ __launch_bounds__(kThreads) void expand_to_fused_kernel(const uint8_t *x, int64_t row_bytes, const int32_t *token_topk_to_pos,
                                                                    int num_topk, int chunks, int copy_blocks, int num_tokens,
                                                                    int num_expanded, uint8_t *out, const int32_t *pos_to_expert,
@@ -446,24 +448,37 @@ __global__ __launch_bounds__(kThreads) void expand_to_fused_kernel(const uint8_t
         const u32x4 *src = reinterpret_cast<const u32x4 *>(x + (int64_t)t * row_bytes + off);
         const int32_t *list = token_topk_to_pos + (int64_t)t * num_topk;
         u32x4 v = u32x4{0u, 0u, 0u, 0u};
-        auto copy_to = [&](int p) {
+        if constexpr (EVERY) {
+            const int p = uniform_load(list + k);
+            if (off < row_bytes) v = *src;   // cached: read num_topk times
+            if (p < 0 || p >= num_expanded) return;
             if (off < row_bytes) expand_store16(out + (int64_t)p * row_bytes + off, v);
             if (x_sf && c == 0)
                 for (int j = threadIdx.x; j < sf_cols; j += kThreads)
                     out_sf[sf_col_major ? (int64_t)j * out_sf_ld + p : (int64_t)p * out_sf_ld + j] = x_sf[(int64_t)t * sf_cols + j];
-        };
-        if (EVERY) {
-            const int p = uniform_load(list + k);
-            if (off < row_bytes) v = *src;   // cached: read num_topk times
-            if (p >= 0 && p < num_expanded) copy_to(p);
             return;
         }
+        // the thread's first scale word is loaded once, with the row: loaded at each copy it is waited for at each copy
+        const bool scales = SF && x_sf && c == 0, scale_word = scales && (int)threadIdx.x < sf_cols;
+        const uint32_t *sf_row = x_sf + (int64_t)t * sf_cols;
+        const int64_t sf_step = sf_col_major ? 1 : out_sf_ld, sf_word = sf_col_major ? out_sf_ld : 1;
+        uint32_t *sf_dst = out_sf + (int64_t)threadIdx.x * sf_word;
+        uint32_t sf0 = 0;
         for (int k0 = 0; k0 < num_topk; k0 += 64) {
             const int kk = k0 + (threadIdx.x & 63);
             const int pos = list[kk < num_topk ? kk : 0];
-            if (k0 == 0 && off < row_bytes) v = *src;      // a token without any position is rare: not waited for
+            if (k0 == 0) {      // a token without any position is rare: not waited for
+                if (off < row_bytes) v = *src;
+                if (scales) sf0 = sf_row[scale_word ? threadIdx.x : 0];
+            }
             unsigned long long live = __builtin_amdgcn_ballot_w64(kk < num_topk && pos >= 0 && pos < num_expanded);
-            for (; live; live &= live - 1) copy_to(__builtin_amdgcn_readlane(pos, __builtin_ctzll(live)));
+            for (; live; live &= live - 1) {
+                const int64_t p = __builtin_amdgcn_readlane(pos, __builtin_ctzll(live));
+                if (off < row_bytes) expand_store16(out + p * row_bytes + off, v);
+                if (scale_word) sf_dst[p * sf_step] = sf0;
+                if (scales && sf_cols > kThreads)
+                    for (int j = threadIdx.x + kThreads; j < sf_cols; j += kThreads) out_sf[j * sf_word + p * sf_step] = sf_row[j];
+            }
         }
     } else {
         const int r0 = (b - copy_blocks) * pad_rows;
@@ -483,7 +498,7 @@ __global__ __launch_bounds__(kThreads) void expand_to_fused_kernel(const uint8_t
 // threads had nothing to copy: bf16 [32768, 1024], top-8: 198.7 us, 124.6 us this way.)
 // EVERY as above; without it kpw counts tokens, and group g serves all entries of token b * kpw + g (us, EVERY / per token:
 // codes [21504, 1280] of 8 ranks 47 / 17.5; top-8 of [8192, 1024] codes 26.2 / 24.8; of bf16 [32768, 1024] 133.5 / 138.9).
-template <bool EVERY>
+template <bool EVERY, bool SF>
 __global__ __launch_bounds__(kThreads) void expand_short_rows_kernel(const uint8_t *x, int64_t row_bytes, const int32_t *token_topk_to_pos,
                                                                      int num_topk, int kpw, int tpr, int copy_blocks, int num_tokens,
                                                                      int num_expanded, uint8_t *out, const int32_t *pos_to_expert,
@@ -507,27 +522,35 @@ __global__ __launch_bounds__(kThreads) void expand_short_rows_kernel(const uint8
         const u32x4 *src = reinterpret_cast<const u32x4 *>(x + (int64_t)t * row_bytes + off);
         const int32_t *list = token_topk_to_pos + (int64_t)t * num_topk;
         u32x4 v = u32x4{0u, 0u, 0u, 0u};
-        auto copy_to = [&](int p) {
+        if constexpr (EVERY) {
+            const int p = list[k];
+            if (off < row_bytes) v = *src;   // cached: read num_topk times
             if (p < 0 || p >= num_expanded) return;
             if (off < row_bytes) expand_store16(out + (int64_t)p * row_bytes + off, v);
             if (x_sf)
                 for (int j = i; j < sf_cols; j += tpr)
                     out_sf[sf_col_major ? (int64_t)j * out_sf_ld + p : (int64_t)p * out_sf_ld + j] = x_sf[(int64_t)t * sf_cols + j];
-        };
-        if (EVERY) {
-            const int p = list[k];
-            if (off < row_bytes) v = *src;   // cached: read num_topk times
-            copy_to(p);
             return;
         }
+        const bool scales = SF && x_sf, scale_word = scales && i < sf_cols;      // (see expand_to_fused_kernel)
+        const uint32_t *sf_row = x_sf + (int64_t)t * sf_cols;
+        const int64_t sf_step = sf_col_major ? 1 : out_sf_ld, sf_word = sf_col_major ? out_sf_ld : 1;
+        uint32_t *sf_dst = out_sf + (int64_t)i * sf_word;
+        uint32_t sf0 = 0;
         if (off < row_bytes) v = *src;
+        if (scales) sf0 = sf_row[scale_word ? i : 0];
         for (int k0 = 0; k0 < num_topk; k0 += 8) {
             int p[8];
 #pragma unroll
             for (int j = 0; j < 8; ++j) p[j] = list[k0 + j < num_topk ? k0 + j : k0];
 #pragma unroll
-            for (int j = 0; j < 8; ++j)
-                if (k0 + j < num_topk) copy_to(p[j]);
+            for (int j = 0; j < 8; ++j) {
+                if (k0 + j >= num_topk || (unsigned)p[j] >= (unsigned)num_expanded) continue;
+                if (off < row_bytes) expand_store16(out + (int64_t)p[j] * row_bytes + off, v);
+                if (scale_word) sf_dst[p[j] * sf_step] = sf0;
+                if (scales && sf_cols > tpr)
+                    for (int w = i + tpr; w < sf_cols; w += tpr) out_sf[w * sf_word + p[j] * sf_step] = sf_row[w];
+            }
         }
     } else {
         expand_zero_padding(b - copy_blocks, pad_rows, num_expanded, row_bytes, out, pos_to_expert, x_sf != nullptr, sf_cols, out_sf, out_sf_ld,
@@ -884,23 +907,29 @@ extern "C" int tk_expand_to_fused(const void *x, int64_t num_tokens, int64_t row
                                             x_sf, sf_cols, out_sf, out_sf_ld, sf_col_major);
     if (rc != TK_OK) return rc;
     const int64_t chunks = (row_bytes + kExpandChunk - 1) / kExpandChunk;
-    // A workgroup per list entry only for long outputs with many positions per token, see the kernel's comment.  num_expanded
-    // bounds the live entries; a buffer sized for the worst case looks like a full list here and loses nothing against before.
+    // A workgroup per list entry only for long outputs with many positions per token (see the kernel's comment) and for so few tokens
+    // that a workgroup each leaves most compute units without work (full lists of codes with scales, us, EVERY / per token: 32 tokens of
+    // 4096 2.9 / 3.2, 64 of 2048, two to a workgroup, 2.75 / 3.0; 64 of 4096 3.1 / 3.3, but 3.2 / 3.05 with one entry of eight live).
+    // num_expanded bounds the live entries; a buffer sized for the worst case looks like a full list here.
     const bool many = num_expanded >= 4 * num_tokens;
-    const bool every = many && num_expanded * row_bytes >= (int64_t)160 << 20;
     // rows of at most half a chunk: several positions of a token, or several tokens, per workgroup
     const int tpr = (int)((row_bytes + 15) / 16);
     const bool short_rows = tpr * 2 <= kThreads;
-    const int kpw = !short_rows ? 1 : (every && kThreads / tpr > num_topk ? num_topk : kThreads / tpr);
     const int64_t token_groups = (num_tokens + 7) / 8 * 8;
-    const int64_t copy_blocks = every ? token_groups * (short_rows ? (num_topk + kpw - 1) / kpw : num_topk * chunks)
-                                      : (short_rows ? (num_tokens + kpw - 1) / kpw : token_groups * chunks);
+    const int64_t token_blocks = short_rows ? (num_tokens + kThreads / tpr - 1) / (kThreads / tpr) : token_groups * chunks;
+    // With few positions per token, long rows and a quarter or more of the output certainly padding, too (codes [10000, 7168], top-2,
+    // -> [30000]: 40.6 / 43.5, -> [20400] 36.1 / 32.5 for rows of 4096).
+    const bool every = many ? num_expanded * row_bytes >= (int64_t)160 << 20 || token_blocks < 64
+                            : !short_rows && num_expanded * 3 >= num_tokens * num_topk * 4;
+    const int kpw = !short_rows ? 1 : (every && kThreads / tpr > num_topk ? num_topk : kThreads / tpr);
+    const int64_t copy_blocks = !every ? token_blocks : token_groups * (short_rows ? (num_topk + kpw - 1) / kpw : num_topk * chunks);
     // padding workgroups take 8 KB of consecutive rows each, two stores per thread.  Measured (us per call, 1 / 2 / 4
     // rows per workgroup): 8 KB rows 64.4 / 69.7 / 71.0; 4 KB rows with scales 41.4 / 36.0 / 37.0
     int pad_rows = row_bytes >= 8192 ? 1 : (int)(8192 / row_bytes > 8 ? 8 : 8192 / row_bytes);
-    // Most rows of a long buffer are live where tokens have few positions: four times the rows per padding workgroup (codes
-    // of [34816, 7168]: 68.7 -> 62.2 us; with a third of the rows padding it costs 1 to 3 %, and below 16384 rows nothing is won)
-    if (!many && num_expanded >= 16384) pad_rows *= 4;
+    // Most rows of a long buffer are live where tokens have few positions: four times the rows per padding workgroup (us, 1 / 2 / 4
+    // times: codes -> [24064, 7168] of 8 ranks 61.5 / 58.9 / 57.7, bf16 -> [33408, 4096], top-2, 76.7 / 72.3 / 70.8; with a third of
+    // rows of 2048 padding 18.3 / 17.6 / 17.7; below 16384 rows nothing is won)
+    if (!many && !every && num_expanded >= 16384) pad_rows *= 4;
     const int64_t grid = copy_blocks + (num_expanded + pad_rows - 1) / pad_rows;
     if (grid == 0) return TK_OK;
     hipStream_t s = static_cast<hipStream_t>(stream);
@@ -910,11 +939,13 @@ extern "C" int tk_expand_to_fused(const void *x, int64_t num_tokens, int64_t row
                        static_cast<uint8_t *>(out), pos_to_expert, static_cast<const uint32_t *>(x_sf), sf_cols,            \
                        static_cast<uint32_t *>(out_sf), out_sf_ld, sf_col_major, pad_rows)
     if (short_rows) {
-        if (every) TK_EXPAND_LAUNCH(expand_short_rows_kernel<true>, kpw, tpr);
-        else TK_EXPAND_LAUNCH(expand_short_rows_kernel<false>, kpw, tpr);
+        if (every) TK_EXPAND_LAUNCH((expand_short_rows_kernel<true, true>), kpw, tpr);
+        else if (x_sf) TK_EXPAND_LAUNCH((expand_short_rows_kernel<false, true>), kpw, tpr);
+        else TK_EXPAND_LAUNCH((expand_short_rows_kernel<false, false>), kpw, tpr);
     } else {
-        if (every) TK_EXPAND_LAUNCH(expand_to_fused_kernel<true>, (int)chunks);
-        else TK_EXPAND_LAUNCH(expand_to_fused_kernel<false>, (int)chunks);
+        if (every) TK_EXPAND_LAUNCH((expand_to_fused_kernel<true, true>), (int)chunks);
+        else if (x_sf) TK_EXPAND_LAUNCH((expand_to_fused_kernel<false, true>), (int)chunks);
+        else TK_EXPAND_LAUNCH((expand_to_fused_kernel<false, false>), (int)chunks);
     }
 #undef TK_EXPAND_LAUNCH
     return (int)hipGetLastError();
