@@ -141,9 +141,10 @@ def test_expand_to_fused_long_output_with_full_lists(dim):
 
 
 @pytest.mark.parametrize('T,K,E,drop,alignment', [(65536, 1, 1, 0.0, 128), (65537, 1, 512, 0.0, 16), (8200, 8, 3, 0.9, 128), (12000, 6, 9, 1.0, 16),
-                                                  (95000, 8, 256, 0.9, 128), (100001, 9, 4, 0.5, 64)])
+                                                  (95000, 8, 256, 0.9, 128), (100001, 9, 4, 0.5, 64), (230400, 8, 1, 0.3, 128), (230401, 8, 1, 0.3, 16)])
 def test_mapping_of_long_lists(T, K, E, drop, alignment):
-    """Lists from 64 Ki pairs on, which are counted into a table first (95000 x 8 of 256 experts: too long for it, three launches);
+    """Lists from 64 Ki pairs on, which are counted into a table first (95000 x 8 of 256 experts, and
+    230401 x 8 of one: too long for it, three launches);
     buffers that are longer, and shorter, than the expanded rows."""
     tk = _tk()
     g = torch.Generator().manual_seed(T)

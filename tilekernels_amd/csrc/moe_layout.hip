@@ -764,9 +764,12 @@ extern "C" int tk_check_get_fused_mapping(const int64_t *topk_idx, int64_t num_t
 
 // Whether the two launches around a table (a row per 1024 pairs) beat the three: every workgroup reads the whole table, groups^2 *
 // experts words in all.  us on MI355X, three launches / table: 172160 pairs of 32 experts (0.9 Mi words) 15.5 / 8.5, 73728 of 256
-// (1.3 Mi) 23.0 / 10.2, 1048576 of 64 (64 Mi) 64 / 30, 2097152 of 32 (128 Mi) 56 / 45; beyond that not measured.
+// (1.3 Mi) 23.0 / 10.2, 1048576 of 64 (64 Mi) 64 / 30, 2080000 of 32 (128 Mi) 71 / 50, 720000 of 256 (128 Mi) 130 / 44, 524288 of 512
+// (128 Mi) 172 / 43; beyond that not measured.  With very few experts the columns are long: one expert, 524288 pairs (512 groups) 26 / 12,
+// 2000000 (1954) 40.4 / 41.8, 4000000 60 / 82; two, 4800000 (4688) 77 / 70, 6400000 (6250) 95 / 97, 8000000 112 / 119;
+// four, 5600000 (5469) 80 / 76.
 static bool table_mapping_pays(int64_t groups, int64_t num_experts) {
-    return num_experts <= kSingleMaxExperts && groups <= (1 << 13) && groups * groups * num_experts <= (1 << 27);
+    return num_experts <= kSingleMaxExperts && groups <= (1 << 13) && groups * groups * num_experts <= (1 << 27) && groups <= 1800 * (2 * num_experts - 1);
 }
 
 // `ws` holds at least tk_fused_mapping_workspace_bytes() bytes
