@@ -417,14 +417,23 @@ __global__ __launch_bounds__(LANES * kPcParts, 4) void per_channel_cast_fp8in_ke
     }
 }
 
-// Narrow tiles (16 lanes per run, twice as many workgroups of half the size) where wide ones leave compute units without
-// work; from one wide tile per compute unit on their longer rows are the better traffic.  Measured on MI355X, us per call, wide / narrow:
-//   SwiGLU transposed [128, 4096] 7.4 / 5.1, [1024, 2048] (64 wide tiles) 7.9 / 5.6, [4096, 1408] (192) 9.0 / 8.9, [16256, 1024] (508)
-//   16.6 / 16.4, [12800, 3072] (1200) 37.4 / 39.9; bf16 transposed [1024, 7168] (224) 5.3 / 4.65, [2304, 2560] (180) 5.05 / 4.45,
-//   [16256, 1024] (508) 9.2 / 9.65; E4M3 input [4608, 1408] (108) 6.2 / 5.1, [2048, 7168] (224) 6.7 / 6.6, [4096, 4096] (256) 7.25 / 7.6,
-//   [13120, 2560] (515) 13.8 / 15.0.
+// Wide tiles from which on a launch takes them; with fewer it takes narrow ones (16 lanes per run, twice as many workgroups of half the
+// size).  An MI355X has 256 compute units.  What computes more per byte (the SwiGLU, E4M3 input, the turn of a transposed output,
+// gathered bf16 rows) is better off in narrow tiles as long as wide ones leave compute units without work; where loads and stores are
+// all there is, narrow tiles lose already where some units hold two of them and others one, fp32 (a wide tile is 128 KB) as soon as any
+// unit does.  Measured on MI355X, us per call, wide / narrow:
+//   SwiGLU transposed [128, 4096] 7.4 / 5.1, [1024, 2048] (64 wide tiles) 7.9 / 5.6, [4096, 1408] (192) 8.8 / 8.5, [896, 8192] (224) 9.15 / 9.1,
+//   [16256, 1024] (508) 16.6 / 16.4, [12800, 3072] (1200) 37.4 / 39.9; bf16 transposed [1024, 7168] (224) 5.3 / 4.85, [2304, 2560] (180)
+//   5.05 / 4.45, [16256, 1024] (508) 9.2 / 9.65; E4M3 input [4608, 1408] (108) 6.2 / 5.1, [2048, 7168] (224) 6.7 / 6.6, [4096, 4096] (256)
+//   7.25 / 7.6, [13120, 2560] (515) 13.8 / 15.0; bf16 gathered [2048, 3072] (192) 4.3 / 3.9, [1152, 7168] (252) 4.6 / 4.2;
+//   bf16 [2048, 2048] (128) 3.5 / 2.95, [4096, 1280] (160) 4.2 / 4.1, [3072, 1792] (168) 4.2 / 4.05, [1024, 5632] (176) 4.34 / 4.41,
+//   [4096, 1536] (192) 4.4 / 4.7, [2048, 3584] (224) 4.6 / 5.3; fp32, gathered or not, [2048, 2048] (128) 7.0 / 5.3, [512, 8448] (132) 7.4 / 7.9,
+//   [1024, 5120] (160) 7.2 / 8.1, [2048, 3584] (224) 8.0 / 9.2.
 // (Runs of 8 lanes: [128, 4096] 4.9, [1024, 7168] 5.7; 4 tokens per lane instead of 8, E4M3 input: [10112, 7168] 29.0 / 32.0.)
-constexpr int64_t kPcWideMinTiles = 256;      // the compute units of an MI355X
+template <int MODE> static int64_t wide_tiles_from(bool transpose, bool gather) {
+    if (MODE == PC_F32) return 129;
+    return MODE != PC_BF16 || transpose || gather ? 256 : 176;
+}
 
 template <int MODE, int NPT, int LANES>
 static void launch_per_channel_3(const PerChannelParams &a, bool transpose, hipStream_t stream) {
@@ -466,7 +475,7 @@ template <int MODE, int NPT>
 static void launch_per_channel_2(const PerChannelParams &p, bool transpose, hipStream_t stream) {
     const int wide_cols = MODE == PC_E4M3 && !transpose ? 512 : 256;
     const int64_t tiles = (int64_t)((p.M + kPcTileM - 1) / kPcTileM) * ((p.K + wide_cols - 1) / wide_cols);
-    if (tiles < kPcWideMinTiles) launch_per_channel_3<MODE, NPT, 16>(p, transpose, stream);
+    if (tiles < wide_tiles_from<MODE>(transpose, p.pos_to_token != nullptr)) launch_per_channel_3<MODE, NPT, 16>(p, transpose, stream);
     else launch_per_channel_3<MODE, NPT, 32>(p, transpose, stream);
 }
 
