@@ -124,3 +124,77 @@ def test_swiglu_launches_that_end_in_smaller_waves_on_any_row_count(R, H, weight
     pieces = [op(x[i:i + 999], 'e4m3', 128, None if slots is None else slots[i:i + 999], weights, swiglu_clamp_value=clamp) for i in range(0, R, 999)]
     assert torch.equal(codes.view(torch.uint8), torch.cat([p[0].view(torch.uint8) for p in pieces]))
     assert torch.equal(sf, torch.cat([p[1] for p in pieces]))
+
+
+# fp32 tiles that overhang the matrix: launches of fewer than 256 workgroups load each lane's elements directly, larger ones deal whole-line
+# loads out between the lanes.  4101 rows of each length here are more than that and 499 rows fewer, in the tiles they take.
+FEW, MANY = 499, 4101
+
+
+def _both_sides(cast, x):
+    whole = cast(x)
+    pieces = [cast(x[i:i + FEW]) for i in range(0, MANY, FEW)]
+    for i, part in enumerate(whole):
+        assert torch.equal(part.contiguous().view(torch.uint8), torch.cat([p[i] for p in pieces]).contiguous().view(torch.uint8)), f'output {i}'
+    return pieces[-1], x[MANY // FEW * FEW:]
+
+
+@pytest.mark.parametrize('group', [16, 32, 64, 128])
+@pytest.mark.parametrize('fmt', ['e4m3', 'e2m1'])
+@pytest.mark.parametrize('K', [512, 896, 1408, 1536, 320, 640])       # one strip, two, three (one wide tile; ragged, whole), short rows end to end
+def test_per_token_fp32_few_and_many_workgroups(K, fmt, group):
+    import tilekernels_amd as tk
+    if K % group:
+        pytest.skip('rows are whole groups')
+    x = _matrix(MANY, K, torch.float32).cuda()
+    last, rows = _both_sides(lambda v: tk.quant.per_token_cast(v, fmt, group), x)
+    want = torch_ref.cast(rows.cpu(), fmt, (1, group))
+    assert_same(last[0], want[0], 'codes')
+    assert_same(last[1], want[1], 'scales')
+    _both_sides(lambda v: (tk.quant.per_token_cast_with_sf_only(v, fmt, group),), x)
+    sf = torch.rand((1, K // group), device='cuda') + 0.5
+    _both_sides(lambda v: (tk.quant.per_token_cast_with_precomputed_sf(v, fmt, group, sf.repeat(v.shape[0], 1)),), x)
+    assert_same(tk.quant.per_token_cast_with_sf_only(rows, fmt, group), want[1], 'scales alone')
+
+
+@pytest.mark.parametrize('with_mask', [False, True])
+@pytest.mark.parametrize('mode', ['plain', 'clamp', 'count'])
+@pytest.mark.parametrize('H', [512, 896, 2560, 640])
+def test_swiglu_fp32_few_and_many_workgroups(H, mode, with_mask):
+    import tilekernels_amd as tk
+    from tests.test_gpu_swiglu import check_fused
+    g = torch.Generator().manual_seed(H)
+    x = torch.randn((MANY, 2 * H), generator=g) * 2
+    pe = torch.randint(-1, 4, (MANY,), generator=g, dtype=torch.int32)
+    clamp = None if mode == 'plain' else 1.0
+
+    def run(v, first, rows):
+        count = torch.zeros(3, dtype=torch.int64, device=v.device) if mode == 'count' else None
+        kw = dict(swiglu_clamp_value=clamp, clamped_count=count)
+        m = pe[first:first + rows].to(v.device) if with_mask else None
+        return (tk.quant if v.is_cuda else torch_ref).swiglu_forward_and_per_token_cast(v[first:first + rows], 'e4m3', 128, pos_to_expert=m, **kw), count
+
+    xd = x.cuda()
+    (codes, sf), count = run(xd, 0, MANY)
+    pieces = [run(xd, i, FEW) for i in range(0, MANY, FEW)]
+    live = (pe >= 0).cuda() if with_mask else torch.ones(MANY, dtype=torch.bool, device='cuda')     # (what padding rows hold is not defined)
+    for got, parts in ((codes.view(torch.uint8), [p[0][0].view(torch.uint8) for p in pieces]), (sf, [p[0][1] for p in pieces])):
+        assert torch.equal(got[live], torch.cat(parts)[live])
+    if count is not None:
+        assert torch.equal(count, sum(p[1] for p in pieces)) and count.sum() > 0
+    first = MANY // FEW * FEW
+    rows = live[first:].cpu()
+    got, want = pieces[-1][0], run(x, first, FEW)[0]
+    check_fused((got[0][rows.cuda()], got[1][rows.cuda()]), (want[0][rows], want[1][rows]), H // 128, False)
+
+
+@pytest.mark.parametrize('fmt', ['e4m3', 'e2m1'])
+@pytest.mark.parametrize('block', [(128, 128), (32, 32), (128, 32)])
+@pytest.mark.parametrize('M', [1, 31, 32, 63, 64, 65])
+def test_per_block_fp32_few_rows(M, block, fmt):
+    import tilekernels_amd as tk
+    for K in (64, 192, 2560):
+        x = _matrix(M, K, torch.float32)
+        got, want = tk.quant.per_block_cast(x.cuda(), fmt, block), torch_ref.cast(x, fmt, block)
+        assert_same(got[0], want[0], 'codes')
+        assert_same(got[1], want[1], 'scales')

@@ -8,6 +8,8 @@
 // LDS exchange (a partial per 16-lane row, one barrier, vector reads).
 //
 // Reference semantics: tile_kernels/quant/per_block_cast_kernel.py:52-136.
+#include <type_traits>
+
 #include "tk_device.hpp"
 #include "tk_host.hpp"
 
@@ -38,7 +40,8 @@ struct PerBlockParams {
 // TW: columns of a tile (128, 256 or 512); a tile is 128 rows x TW columns.
 // THREADS: threads per tile.
 // FULL: the tile lies wholly inside the matrix, so no bounds checks are compiled in.
-template <typename InT, int FMT, int BM, int BK, int TW, int THREADS, bool FULL>
+// FEW: of a matrix of few rows, see the launch code.
+template <typename InT, int FMT, int BM, int BK, int TW, int THREADS, bool FULL, bool FEW = false>
 __device__ __forceinline__ void per_block_cast_tile(const PerBlockParams &p, uint8_t *xchg) {
     constexpr int LPR = TW / 8;                                      // lanes along a row of the tile
     constexpr int SUBM = kBlockTile / BM, SUBK = TW / BK;            // scale blocks per tile
@@ -61,13 +64,15 @@ __device__ __forceinline__ void per_block_cast_tile(const PerBlockParams &p, uin
     const int64_t out_ld = FMT == TK_E4M3 ? p.K : p.K / 2;
 
     // fp32 input: the LPR lanes of a tile row read its 32 * LPR bytes as two whole-line loads and deal them out through LDS
-    constexpr int XB = Raw8<InT>::kXchgBytes;
+    constexpr int XB = FEW ? 0 : Raw8<InT>::kXchgBytes;
     constexpr int RUN = LPR < 64 ? LPR : 64;     // lanes of one run: a tile row, or the part of it that one wave holds
     Raw8<InT> raw[NI];
 #pragma unroll
     for (int i = 0; i < NI; ++i) {
         if constexpr (FULL) {
             raw[i].template load_run<RUN>(x + (int64_t)(TR * i) * p.K, c % RUN);
+        } else if constexpr (FEW) {
+            raw[i].load(x + (int64_t)(TR * i) * p.K, col_ok && row0 + TR * i < p.M);
         } else {
             // No lane branches around its load: all loads of a lane go out together, where each one in a branch of its own is waited
             // for before the next (the tiles at the lower edge then end the launch some 5 us after the others).  A lane beyond the
@@ -174,13 +179,15 @@ __device__ __forceinline__ void per_block_cast_tile(const PerBlockParams &p, uin
 // FULL_GRID: M and K are multiples of 128.  Otherwise only the tiles on the lower and right edges take the
 // bounds-checked path; the choice is uniform over the workgroup.  (With every tile checked, bf16 [32767, 4096] took
 // 63.9 us against 59.1 us for [32768, 4096].)
-template <typename InT, int FMT, int BM, int BK, int TW, int THREADS, bool FULL_GRID>
+template <typename InT, int FMT, int BM, int BK, int TW, int THREADS, bool FULL_GRID, bool FEW = false>
 __global__ __launch_bounds__(THREADS) void per_block_cast_kernel(TK_PB_KERNEL_ARGS) {
     TK_PB_KERNEL_UNPACK;
-    constexpr int XB = Raw8<InT>::kXchgBytes;
+    constexpr int XB = FEW ? 0 : Raw8<InT>::kXchgBytes;
     __shared__ __attribute__((aligned(16))) uint8_t xchg[XB ? THREADS * XB : 16];      // (one for both kinds of tile)
     if constexpr (FULL_GRID) {
         per_block_cast_tile<InT, FMT, BM, BK, TW, THREADS, true>(p, xchg);
+    } else if constexpr (FEW) {
+        per_block_cast_tile<InT, FMT, BM, BK, TW, THREADS, false, true>(p, xchg);
     } else {
         if (((int)blockIdx.y + 1) * kBlockTile <= p.M && ((int)blockIdx.x + 1) * TW <= p.K)
             per_block_cast_tile<InT, FMT, BM, BK, TW, THREADS, true>(p, xchg);
@@ -205,6 +212,15 @@ constexpr int64_t kWideMinTiles = 512, kWideMaxTiles = 1280;     // in 128 x 128
 template <typename InT, int FMT, int BM, int BK, int TW, int THREADS>
 static void launch_per_block_3(const PerBlockParams &p, hipStream_t stream) {
     const dim3 grid((unsigned)((p.K + TW - 1) / TW), (unsigned)p.tiles_m), block(THREADS);
+    // fp32 of at most 64 rows: each lane loads what it has, in a branch.  With few loads per lane the waits in between cost less than
+    // loads of rows that do not exist and the exchange between lanes (us, without branches / this, blocks of 128 and of 32: 1 row of
+    // 2560 3.05 / 2.55, 4.0 / 3.35; 40 rows 3.2 / 3.15, 4.2 / 3.75; 64 of 2816 3.3 / 3.35, 4.15 / 3.9; but 65 of 2560 3.65 / 4.4, 4.65 / 5.1).
+    if constexpr (std::is_same<InT, float>::value && TW == kBlockTile) {
+        if (p.M <= 64) {
+            hipLaunchKernelGGL((per_block_cast_kernel<InT, FMT, BM, BK, TW, THREADS, false, true>), grid, block, 0, stream, TK_PB_LAUNCH_ARGS(p));
+            return;
+        }
+    }
     if (p.M % kBlockTile == 0 && p.K % TW == 0)
         hipLaunchKernelGGL((per_block_cast_kernel<InT, FMT, BM, BK, TW, THREADS, true>), grid, block, 0, stream, TK_PB_LAUNCH_ARGS(p));
     else

@@ -56,6 +56,7 @@ struct PerTokenParams {
 //             wave; the scales a wave produces are neighbours in the scale row and it stores them itself: no LDS
 //             stage and no barrier
 // FULL_GRID: the tile grid covers the matrix exactly, so no bounds checks are compiled in.
+// RUNS: fp32 input of tiles that overhang the matrix arrives as whole-line loads too, see few_workgroups.
 enum { T_STACKED = 0, T_WIDE = 1, T_ROWWISE = 2 };
 
 // Waves per workgroup of the row-wise tiles (their waves share nothing, so this only sets how many rows are dispatched
@@ -68,7 +69,7 @@ template <typename InT, int FMT> constexpr int rowwise_waves() {
     return Elem<InT>::quantised ? kWaves : (sizeof(InT) == 4 ? 1 : (FMT == TK_E2M1 ? 2 : kWaves));
 }
 
-template <typename InT, int G, int FMT, int RPW, int TILE, bool FULL_GRID, bool GIVEN = false>
+template <typename InT, int G, int FMT, int RPW, int TILE, bool FULL_GRID, bool GIVEN = false, bool RUNS = true>
 __global__ __launch_bounds__(TILE == T_WIDE ? 64 * kMaxWideWaves : kThreads) void per_token_cast_kernel(TK_PT_KERNEL_ARGS) {
     TK_PT_KERNEL_UNPACK;
     // GIVEN: the cast with caller-supplied scales, chosen at the launch (row-wise tiles).  The mode argument lies beyond the
@@ -87,7 +88,7 @@ __global__ __launch_bounds__(TILE == T_WIDE ? 64 * kMaxWideWaves : kThreads) voi
     using RS = RowScales<Fmt<FMT>::qmax, RPW, LPG>;
     __shared__ uint32_t stage[ROWW ? 1 : ROWS][ROWW ? 1 : SGPR];
     // fp32 input: a wave's 2 KB of one row arrive as two whole-line loads and are dealt out to their lanes through LDS
-    constexpr int XB = Raw8<InT>::kXchgBytes;
+    constexpr int XB = FULL || RUNS ? Raw8<InT>::kXchgBytes : 0;
     __shared__ __attribute__((aligned(16))) uint8_t xchg[XB ? (WIDE ? kMaxWideWaves : kWaves) : 1][XB ? 64 * XB : 16];
 
     // wide tiles: the waves of one tile cover a whole row; row-wise: one wave does
@@ -389,7 +390,7 @@ static void launch_per_token_rowgroup(PerTokenParams &p, hipStream_t stream) {
 // can be partly empty (576 columns in groups of 128: 72 of 80 lanes).  A wave holds RPW slots of 64 lanes; every group
 // is complete inside one slot, so the reductions and the shared scale arithmetic are those of the tiled kernel.  Each
 // scale is stored by one lane (all three layouts).
-template <typename InT, int G, int FMT, int RPW>
+template <typename InT, int G, int FMT, int RPW, bool RUNS = true>
 __global__ __launch_bounds__(kThreads) void per_token_cast_flat_kernel(TK_PT_KERNEL_ARGS) {
     TK_PT_KERNEL_UNPACK;
     constexpr int LPG = G / 8;
@@ -400,7 +401,7 @@ __global__ __launch_bounds__(kThreads) void per_token_cast_flat_kernel(TK_PT_KER
     const int own = lane % LPG;
     // fp32 input: the lanes of a group read its 32 * LPG bytes as two runs and deal them out through LDS.  With fewer than 8 lanes
     // a run's instructions span no whole line either ([8001, 576] in groups of 64: 5.93 -> 5.06 us; [16001, 1216] of 32: 16.8 -> 17.5).
-    constexpr int XB = LPG >= 8 ? Raw8<InT>::kXchgBytes : 0;
+    constexpr int XB = RUNS && LPG >= 8 ? Raw8<InT>::kXchgBytes : 0;
     __shared__ __attribute__((aligned(16))) uint8_t xchg[XB ? kThreads * XB : 16];
 
     int row[RPW], grp[RPW];
@@ -483,6 +484,11 @@ __global__ __launch_bounds__(kThreads) void per_token_cast_flat_kernel(TK_PT_KER
 // its fixed work; E4M3 1x128 [8192, 4096] -> E2M1 1x32: 14.3 / 12.0 / 12.2 for 2 / 4 / 8 rows.
 template <typename InT> constexpr int rows_per_wave() { return Elem<InT>::quantised ? 4 : 2; }
 
+// Launches that leave compute units without work: there the exchange of whole-line loads between lanes is latency and saves nothing
+// (fp32, ragged, us with the exchange / without: 1 row of 2560 2.2 / 2.1, [64, 2816] 2.5 / 2.35, [333, 768] 2.6 / 2.5; from about 256
+// workgroups on it pays: [4001, 2560] 9.2 / 10.7).
+static bool few_workgroups(int64_t n) { return n < 256; }
+
 template <typename InT, int G, int FMT, int TILE>
 static void launch_per_token_tiled(PerTokenParams &p, hipStream_t stream) {
     constexpr int RPW = rows_per_wave<InT>();
@@ -500,6 +506,12 @@ static void launch_per_token_tiled(PerTokenParams &p, hipStream_t stream) {
         if (p.mode == TK_CAST_GIVEN_SF) {
             if (exact) hipLaunchKernelGGL((per_token_cast_kernel<InT, G, FMT, RPW, TILE, true, true>), grid, block, 0, stream, TK_PT_LAUNCH_ARGS(p));
             else hipLaunchKernelGGL((per_token_cast_kernel<InT, G, FMT, RPW, TILE, false, true>), grid, block, 0, stream, TK_PT_LAUNCH_ARGS(p));
+            return;
+        }
+    }
+    if constexpr (std::is_same<InT, float>::value && !ROWW) {
+        if (!exact && few_workgroups((int64_t)tiles_m * tiles_k)) {
+            hipLaunchKernelGGL((per_token_cast_kernel<InT, G, FMT, RPW, TILE, false, false, false>), grid, block, 0, stream, TK_PT_LAUNCH_ARGS(p));
             return;
         }
     }
@@ -525,6 +537,13 @@ static void launch_per_token_group(PerTokenParams &p, hipStream_t stream) {
             if (lanes < INT32_MAX - 2 * kThreads * RPW) {   // lane slots are numbered in 32 bits
             p.geom = (int)gpr;
             p.in_bm = (int)(uint32_t)(gpr == 1 ? 0xFFFFFFFFull : (1ull << 32) / (uint64_t)gpr);   // plain input: the field carries the reciprocal of gpr
+            if constexpr (std::is_same<InT, float>::value && G >= 64) {      // (smaller groups have no exchange)
+                if (few_workgroups(blocks)) {
+                    hipLaunchKernelGGL((per_token_cast_flat_kernel<InT, G, FMT, RPW, false>), dim3((unsigned)blocks), dim3(kThreads), 0, stream,
+                                       TK_PT_LAUNCH_ARGS(p));
+                    return;
+                }
+            }
             hipLaunchKernelGGL((per_token_cast_flat_kernel<InT, G, FMT, RPW>), dim3((unsigned)blocks), dim3(kThreads), 0, stream,
                                TK_PT_LAUNCH_ARGS(p));
             return;

@@ -286,7 +286,8 @@ enum { T_STACKED = 0, T_ROW = 2, T_ROWC = 3 };
 // 14.42 / 14.20, 20.78 / 20.39, 13.12 / 12.83, 20.95 / 20.47).  bf16, us per call without / with,
 // column-major fp32 scales: [8192, 2 x 2048] 15.39 / 14.74, [4096, 2 x 4096] 15.34 / 14.86, [12288, 2 x 2048] 21.40 / 20.89,
 // [16384, 2 x 2048] 27.53 / 27.13; packed UE8M0: 14.79 / 14.36, 14.70 / 14.47, 21.11 / 20.61, 27.18 / 26.88.
-template <typename InT, int CLAMP, int RPW, int TILE, bool FULL_GRID, bool MASK, bool ONECOL, int TAILED = 0>
+// RUNS: fp32 input of tiles that overhang the matrix arrives as whole-line loads too (launches of more than a few workgroups, see there)
+template <typename InT, int CLAMP, int RPW, int TILE, bool FULL_GRID, bool MASK, bool ONECOL, int TAILED = 0, bool RUNS = true>
 __global__ __launch_bounds__(TILE == T_ROW ? 64 * kMaxWideWaves : kThreads) void swiglu_cast_kernel(TK_SWIGLU_KERNEL_ARGS) {
     static_assert(!TAILED || (FULL_GRID && !MASK && CLAMP != 2 && RPW == 4), "tail waves: unmasked grids of four-piece waves without bounds checks");
     if constexpr (TAILED) {
@@ -361,7 +362,7 @@ __global__ __launch_bounds__(TILE == T_ROW ? 64 * kMaxWideWaves : kThreads) void
     using RS = RowScales<448, RPW, 16>;
     __shared__ uint32_t stage[DIRECT ? 1 : ROWS][DIRECT ? 1 : SGPR];
     // fp32 input: a wave's 2 KB of one row arrive as two whole-line loads and are dealt out to their lanes through LDS
-    constexpr int XB = Raw8<InT>::kXchgBytes;
+    constexpr int XB = FULL || RUNS ? Raw8<InT>::kXchgBytes : 0;
     __shared__ __attribute__((aligned(16))) uint8_t xchg[XB ? kWaves : 1][XB ? 64 * XB : 16];
 
     const int total = LOOP ? ((p.R + rows - 1) / rows) * p.tiles_k : 1;
@@ -474,9 +475,6 @@ __global__ __launch_bounds__(TILE == T_ROW ? 64 * kMaxWideWaves : kThreads) void
                 }
             }
         }
-        // fp32 input (two loads per piece): cleared once all loads are out, since clearing a register that a load is still to
-        // fill means waiting for that load (masked fp32 [16384, 2 x 2048] 40.3 -> 38.4 us; bf16 input, whose clearing the
-        // compiler already places behind the loads, measured 21.0 -> 21.2 us on a ragged batch with it and keeps its place)
         // (in this variant the fetch of the later arguments starts at the head of the kernel, where its paths part)
         if constexpr (TAILED != 0) fetch_late_arguments(p, CLAMP != 0, TAILED == 2, TILE != T_ROW);
         if constexpr (XB != 0) {
@@ -486,6 +484,9 @@ __global__ __launch_bounds__(TILE == T_ROW ? 64 * kMaxWideWaves : kThreads) void
                 ru[r].template settle<64>(xchg[wave], lane);
             }
         }
+        // fp32 input (two loads per piece): cleared once all loads are out, since clearing a register that a load is still to
+        // fill means waiting for that load (masked fp32 [16384, 2 x 2048] 40.3 -> 38.4 us; bf16 input, whose clearing the
+        // compiler already places behind the loads, measured 21.0 -> 21.2 us on a ragged batch with it and keeps its place)
         if constexpr (!(FULL && !MASK) && sizeof(InT) == 4) {
 #pragma unroll
             for (int r = 0; r < RPW; ++r)
@@ -567,7 +568,7 @@ __global__ __launch_bounds__(TILE == T_ROW ? 64 * kMaxWideWaves : kThreads) void
 // a row can be partly empty.  Every group is complete inside 64 lanes, so the reduction and the shared scale arithmetic
 // are those of the tiled kernel; rows differ from lane to lane, so mask and weight are read per lane, and each scale is
 // stored by one lane (all three layouts).  CLAMP: 0 none, 1 clamp (the counting variant stays with the tiled kernel).
-template <typename InT, int CLAMP, int RPW>
+template <typename InT, int CLAMP, int RPW, bool RUNS = true>
 __global__ __launch_bounds__(kThreads) void swiglu_cast_flat_kernel(TK_SWIGLU_KERNEL_ARGS) {
     TK_SWIGLU_KERNEL_UNPACK;
     constexpr int LPG = 16;
@@ -577,7 +578,7 @@ __global__ __launch_bounds__(kThreads) void swiglu_cast_flat_kernel(TK_SWIGLU_KE
     const InT *xb = reinterpret_cast<const InT *>(p.x);
     ClampCounter<CLAMP> counter;
     // fp32 input: the lanes of a group read its 512 bytes as two runs and deal them out through LDS
-    constexpr int XB = Raw8<InT>::kXchgBytes;
+    constexpr int XB = RUNS ? Raw8<InT>::kXchgBytes : 0;
     __shared__ __attribute__((aligned(16))) uint8_t xchg[XB ? kThreads * XB : 16];
 
     // Mask entries and weight indices of all slots are asked for first, then the data of all slots, then the weights: a
@@ -799,6 +800,11 @@ static int64_t wave_slots() {
     return (int64_t)cus * 32;
 }
 
+// Launches that leave compute units without work: there the exchange of whole-line loads between lanes is latency and saves nothing
+// (fp32, ragged, us with the exchange / without: 1 row of 2560 2.8 / 2.65, [65, 2 x 2560] 3.25 / 3.05, [333, 2 x 2560] (210 workgroups) 3.4 /
+// 3.3, [700, 2 x 768] (131) 3.7 / 3.5; [450, 2 x 2560] (285) 3.9 / 4.2, [4001, 2 x 2560] 16.0 / 18.7).
+static bool few_workgroups(int64_t n) { return n < 256; }
+
 template <typename InT, int CLAMP, int RPW, int TILE>
 static void launch_swiglu_tiled(SwigluParams &p, int max_blocks, hipStream_t stream) {
     // T_ROW, rows per workgroup (= waves), us per call at [8192, 4096] dense / [48128, 4096] with a third of the rows
@@ -880,6 +886,15 @@ static void launch_swiglu_tiled(SwigluParams &p, int max_blocks, hipStream_t str
             return;
         }
     }
+    if constexpr (sizeof(InT) == 4 && TILE != T_ROW) {
+        if (!full && few_workgroups(CLAMP == 2 ? (int64_t)grid.x : (int64_t)tiles_m * p.tiles_k)) {
+            if (p.pos_to_expert)
+                hipLaunchKernelGGL((swiglu_cast_kernel<InT, CLAMP, RPW, TILE, false, true, false, 0, false>), grid, block, 0, stream, TK_SWIGLU_LAUNCH_ARGS(p));
+            else
+                hipLaunchKernelGGL((swiglu_cast_kernel<InT, CLAMP, RPW, TILE, false, false, false, 0, false>), grid, block, 0, stream, TK_SWIGLU_LAUNCH_ARGS(p));
+            return;
+        }
+    }
 #define TK_SWIGLU_LAUNCH(FULL_, MASK_)                                                                                          \
     do {                                                                                                                        \
         if (onecol)                                                                                                             \
@@ -915,8 +930,15 @@ static hipError_t launch_swiglu_2(SwigluParams &p, bool row_group, int max_block
             static_assert(RowScales<448, RPW, 16>::A == 2, "the flat kernel selects between two slots");
             p.tiles_k = (int)gpr;
             p.nwaves = (int)(uint32_t)(gpr == 1 ? 0xFFFFFFFFull : (1ull << 32) / (uint64_t)gpr);   // reciprocal of gpr for the kernel's divisions
-            hipLaunchKernelGGL((swiglu_cast_flat_kernel<InT, CLAMP, RPW>), dim3((unsigned)((lanes + kThreads * RPW - 1) / (kThreads * RPW))),
-                               dim3(kThreads), 0, stream, TK_SWIGLU_LAUNCH_ARGS(p));
+            const int64_t blocks = (lanes + kThreads * RPW - 1) / (kThreads * RPW);
+            if constexpr (sizeof(InT) == 4) {
+                if (few_workgroups(blocks)) {
+                    hipLaunchKernelGGL((swiglu_cast_flat_kernel<InT, CLAMP, RPW, false>), dim3((unsigned)blocks), dim3(kThreads), 0, stream,
+                                       TK_SWIGLU_LAUNCH_ARGS(p));
+                    return hipGetLastError();
+                }
+            }
+            hipLaunchKernelGGL((swiglu_cast_flat_kernel<InT, CLAMP, RPW>), dim3((unsigned)blocks), dim3(kThreads), 0, stream, TK_SWIGLU_LAUNCH_ARGS(p));
             return hipGetLastError();
         }
     }
