@@ -167,6 +167,92 @@ def test_calls_the_python_code_takes(monkeypatch):
         q.per_token_cast(_x(8, 513)[:, 1:], 'e4m3', 128)
 
 
+@pytest.mark.gpu
+def test_watched_and_wrapped_calls_are_left_alone():
+    """Tracing, function transforms, function modes and tensors that are more than their storage: the native functions return None."""
+    from torch.overrides import TorchFunctionMode
+    from tilekernels_amd import _ffi
+    x = _x(8, 512, torch.float32)
+    seen = []
+
+    def native(v):
+        seen.append(_ffi.host.per_token_cast(v, 'e4m3', 128, None, False, False, False))
+        return v.sum()
+
+    class Mode(TorchFunctionMode):
+        def __torch_function__(self, func, types, args=(), kwargs=None):
+            return func(*args, **(kwargs or {}))
+
+    class Sub(torch.Tensor):
+        pass
+
+    def in_mode():
+        with Mode():
+            seen.append(_ffi.host.per_token_cast(x, 'e4m3', 128, None, False, False, False))
+
+    def outer(v):       # a tensor from outside the transform
+        seen.append(_ffi.host.per_token_cast(x, 'e4m3', 128, None, False, False, False))
+        return v.sum()
+
+    sub, negative = x.as_subclass(Sub), torch._neg_view(x)
+    assert type(sub) is Sub and negative.is_neg()
+    cases = {'trace': lambda: torch.jit.trace(native, x, check_trace=False), 'vmap': lambda: torch.func.vmap(native)(x[None]),
+             'grad': lambda: torch.func.grad(native)(x), 'jvp': lambda: torch.func.jvp(native, (x,), (x,)),
+             'functionalize': lambda: torch.func.functionalize(native)(x), 'inside vmap': lambda: torch.func.vmap(outer)(x),
+             'inside grad': lambda: torch.func.grad(outer)(x), 'function mode': in_mode, 'subclass': lambda: native(sub),
+             'negated view': lambda: native(negative), 'zero tensor': lambda: native(torch._efficientzerotensor((8, 512), device='cuda'))}
+    for name, run in cases.items():
+        seen.clear()
+        native(x)
+        run()
+        native(x)
+        assert len(seen) >= 3 and seen[0] is not None and seen[-1] is not None, name
+        assert all(r is None for r in seen[1:-1]), name
+
+
+@pytest.mark.gpu
+def test_threads_on_their_own_streams():
+    """The lock is released around each launch: threads that call at the same time get the results each would get alone."""
+    import threading
+    import tilekernels_amd as tk
+    g = torch.Generator().manual_seed(5)
+    inputs, wants = [], []
+
+    def calls(x, idx):
+        m = tk.moe.get_fused_mapping(idx, 8, 1024, 16)
+        e = tk.moe.expand_to_fused(x, m[3], m[0])
+        c = tk.quant.per_token_cast(x, 'e4m3', 128, None, True, True, True)
+        s = tk.quant.swiglu_forward_and_per_token_cast(e, 'e4m3', 128, pos_to_expert=m[0])
+        r = tk.moe.reduce_fused(e, None, m[3])
+        live = m[0] >= 0
+        return [m[0], m[1], m[3], *c, s[0].view(torch.uint8)[live], s[1][live], e[live], r]
+
+    for i in range(4):
+        x = torch.randn((200 + i, 512), generator=g).to(torch.bfloat16).cuda()
+        idx = torch.randint(-1, 8, (200 + i, 4), generator=g).cuda()
+        inputs.append((x, idx))
+        wants.append([_bytes(t) for t in calls(x, idx)])
+    torch.cuda.synchronize()
+    start, failed, finished = threading.Barrier(4), [], []
+
+    def work(i):
+        stream = torch.cuda.Stream()
+        with torch.cuda.stream(stream):
+            start.wait()
+            for n in range(20):
+                got = calls(*inputs[i])
+                stream.synchronize()
+                failed.extend((i, n, j) for j, (a, b) in enumerate(zip(got, wants[i])) if not torch.equal(_bytes(a), b))
+        finished.append(i)
+
+    threads = [threading.Thread(target=work, args=(i,)) for i in range(4)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert sorted(finished) == [0, 1, 2, 3] and not failed, failed[:10]
+
+
 @pytest.mark.parametrize('op', ['per_token_cast', 'per_block_cast', 'cast_back', 'swiglu_forward', 'reduce_fused', 'expand_to_fused', 'get_fused_mapping'])
 def test_cpu_tensors_are_left_alone(op):
     from tilekernels_amd import _ffi
