@@ -192,3 +192,24 @@ def test_expand_to_fused_scale_words(T, K, row_bytes, sf_cols, pad, live, col_ma
     got = out_sf.cpu()
     assert bool((got[:, -3:] == 0x5A5A5A5A).all())
     assert torch.equal(got[:, :-3].T.contiguous() if col_major else got[:, :-3], want_sf)
+
+
+@pytest.mark.parametrize('T,K,E', [(1, 1, 1), (2, 1, 3), (3, 1, 2), (1, 4, 4), (5, 3, 8), (1365, 3, 32), (4097, 4, 64), (5462, 3, 72),      # one workgroup per expert
+                                   (65537, 1, 512), (16500, 4, 9), (230401, 8, 1)])                                                   # a table; three launches
+def test_mapping_of_a_list_between_16_byte_boundaries(T, K, E):
+    """A contiguous list that starts 8 bytes off (a slice of a longer one): the kernels read pairs from the boundary on, and the first
+    (and, of an even number, the last) entry by itself."""
+    tk = _tk()
+    g = torch.Generator().manual_seed(T + K)
+    idx = torch.randint(-1, E, (T, K), generator=g)
+    idx[0, 0] = idx[-1, -1] = E - 1
+    want = torch_ref.get_fused_mapping(idx, E, 16)
+    buf = torch.empty((T * K + 1,), dtype=torch.int64, device='cuda')
+    buf[0] = 0                      # an entry in front of the list that would count
+    view = buf[1:].view(T, K)
+    view.copy_(idx)
+    assert view.data_ptr() % 16 == 8 and view.is_contiguous()
+    for got in (tk.moe.get_fused_mapping(view, E, 0, 16), tk.moe.get_fused_mapping(view, E, want[0].numel(), 16)):
+        for name, a, b in zip(('pos_to_expert', 'pos_to_token', 'pos_to_token_topk', 'token_topk_to_pos', 'expert_start', 'expert_end',
+                               'num_tokens_per_expert'), got[:7], want):
+            assert_same(a, b, name)
