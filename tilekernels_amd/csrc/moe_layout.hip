@@ -1020,8 +1020,8 @@ extern "C" int tk_reduce_fused(const void *x, int x_dtype, int64_t num_expanded,
             if (out_dtype == TK_OUT_E4M3) TK_REDUCE_LAUNCH(bf16_t, 2);
             else TK_REDUCE_LAUNCH(bf16_t, 0);
         } else if (hidden % 512 == 0) {
-            if (out_dtype == TK_OUT_E4M3) TK_REDUCE_LAUNCH(SplitF32, 2);
-            else TK_REDUCE_LAUNCH(SplitF32, 1);
+            if (out_dtype == TK_OUT_E4M3) TK_REDUCE_LAUNCH_2(SplitF32, 2, false);      // (never stacked: rows of 512 and more)
+            else TK_REDUCE_LAUNCH_2(SplitF32, 1, false);
         } else {
             if (out_dtype == TK_OUT_E4M3) TK_REDUCE_LAUNCH(float, 2);
             else TK_REDUCE_LAUNCH(float, 1);
