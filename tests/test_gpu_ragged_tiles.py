@@ -159,8 +159,8 @@ def test_per_token_fp32_few_and_many_workgroups(K, fmt, group):
 
 @pytest.mark.parametrize('with_mask', [False, True])
 @pytest.mark.parametrize('mode', ['plain', 'clamp', 'count'])
-@pytest.mark.parametrize('H', [512, 896, 2560, 640])
-def test_swiglu_fp32_few_and_many_workgroups(H, mode, with_mask):
+@pytest.mark.parametrize('H,layout', [(512, 'row'), (896, 'row'), (2560, 'row'), (640, 'row'), (1024, 'col'), (2048, 'packed')])
+def test_swiglu_fp32_few_and_many_workgroups(H, layout, mode, with_mask):
     import tilekernels_amd as tk
     from tests.test_gpu_swiglu import check_fused
     g = torch.Generator().manual_seed(H)
@@ -170,26 +170,23 @@ def test_swiglu_fp32_few_and_many_workgroups(H, mode, with_mask):
 
     def run(v, first, rows):
         count = torch.zeros(3, dtype=torch.int64, device=v.device) if mode == 'count' else None
-        kw = dict(swiglu_clamp_value=clamp, clamped_count=count)
+        kw = dict(swiglu_clamp_value=clamp, clamped_count=count, **LAYOUTS[layout])
         m = pe[first:first + rows].to(v.device) if with_mask else None
         return (tk.quant if v.is_cuda else torch_ref).swiglu_forward_and_per_token_cast(v[first:first + rows], 'e4m3', 128, pos_to_expert=m, **kw), count
 
     xd = x.cuda()
     (codes, sf), count = run(xd, 0, MANY)
     pieces = [run(xd, i, FEW) for i in range(0, MANY, FEW)]
-    live = (pe >= 0).cuda() if with_mask else torch.ones(MANY, dtype=torch.bool, device='cuda')     # (what padding rows hold is not defined)
-    for got, parts in ((codes.view(torch.uint8), [p[0][0].view(torch.uint8) for p in pieces]), (sf, [p[0][1] for p in pieces])):
-        assert torch.equal(got[live], torch.cat(parts)[live])
+    assert torch.equal(codes.view(torch.uint8), torch.cat([p[0][0].view(torch.uint8) for p in pieces]))
+    assert torch.equal(sf, torch.cat([p[0][1] for p in pieces]))
     if count is not None:
         assert torch.equal(count, sum(p[1] for p in pieces)) and count.sum() > 0
     first = MANY // FEW * FEW
-    rows = live[first:].cpu()
-    got, want = pieces[-1][0], run(x, first, FEW)[0]
-    check_fused((got[0][rows.cuda()], got[1][rows.cuda()]), (want[0][rows], want[1][rows]), H // 128, False)
+    check_fused(pieces[-1][0], run(x, first, FEW)[0], H // 128, layout == 'packed')
 
 
 @pytest.mark.parametrize('fmt', ['e4m3', 'e2m1'])
-@pytest.mark.parametrize('block', [(128, 128), (32, 32), (128, 32)])
+@pytest.mark.parametrize('block', [(128, 128), (32, 32), (128, 32), (32, 128)])
 @pytest.mark.parametrize('M', [1, 31, 32, 63, 64, 65])
 def test_per_block_fp32_few_rows(M, block, fmt):
     import tilekernels_amd as tk
