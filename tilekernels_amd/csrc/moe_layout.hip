@@ -428,8 +428,10 @@ __device__ __forceinline__ void expand_zero_padding(int pb, int pad_rows, int nu
 // they do).  us per call on MI355X, EVERY / one per token (codes with scales, top-8 unless said):
 //   one of 8 ranks: 21504 tokens -> [24064, 7168]  214 / 59.5      340 tokens -> [6784, 4096] (worst-case buffer)  6.7 / 5.4
 //   full lists: [512, 4096] -> [5120]  6.6 / 4.7      [2048, 7168] -> [17536]  31.3 / 27.9      top-2 of [8192, 7168]  32.1 / 29.5
-//   bf16 -> rows of 4096, 110 MB 25.6 / 22.8, 132 MB 30.3 / 27.2, 154 MB 35.4 / 32.9;  7168, 160 MB 36.8 / 33.9;  from 160 MB on EVERY:
-//   [4096, 4096] codes -> 197 MB 38.1 / 39.2, bf16 -> 394 MB 64.4 / 73.5
+//   bf16 -> rows of 4096, 110 MB 25.6 / 22.8, 132 MB 30.3 / 27.2, 154 MB 35.4 / 32.9, 184 MB 42.0 / 40.2, 203 MB 46.4 / 48.1, 234 MB 53.2 / 54.5,
+//   304 MB 68.3 / 70.6, 404 MB 90.9 / 95.4 (2048 and codes of 4096 the same);  7168, 168 MB 38.3 / 35.6, 236 MB 54.6 / 51.0, 407 MB 92.5 / 89.9;
+//   a third of [48128] rows of 4096 padding: codes with scales, 197 MB 38.1 / 39.2, bf16, 394 MB 64.4 / 73.5
+// The line lies at 160 MB for all of them, so that no output beyond it is slower than entry by entry.
 // SF: there may be scales (else nothing of them is looked at; x_sf may be null all the same)
 template <bool EVERY, bool SF>
 __global__ __launch_bounds__(kThreads) void expand_to_fused_kernel(const uint8_t *x, int64_t row_bytes, const int32_t *token_topk_to_pos,
