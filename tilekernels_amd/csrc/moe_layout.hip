@@ -432,7 +432,7 @@ __device__ __forceinline__ void expand_zero_padding(int pb, int pad_rows, int nu
 //   304 MB 68.3 / 70.6, 404 MB 90.9 / 95.4 (2048 and codes of 4096 the same);  7168, 168 MB 38.3 / 35.6, 236 MB 54.6 / 51.0, 407 MB 92.5 / 89.9;
 //   a third of [48128] rows of 4096 padding: codes with scales, 197 MB 38.1 / 39.2, bf16, 394 MB 64.4 / 73.5
 // The line lies at 160 MB for all of them, so that no output beyond it is slower than entry by entry.
-// SF: there may be scales (else nothing of them is looked at; x_sf may be null all the same)
+// SF: there are scales (with EVERY there may be); otherwise nothing of them is looked at.
 template <bool EVERY, bool SF>
 __global__ __launch_bounds__(kThreads) void expand_to_fused_kernel(const uint8_t *x, int64_t row_bytes, const int32_t *token_topk_to_pos,
                                                                    int num_topk, int chunks, int copy_blocks, int num_tokens,
@@ -460,26 +460,31 @@ __global__ __launch_bounds__(kThreads) void expand_to_fused_kernel(const uint8_t
                     out_sf[sf_col_major ? (int64_t)j * out_sf_ld + p : (int64_t)p * out_sf_ld + j] = x_sf[(int64_t)t * sf_cols + j];
             return;
         }
-        // the thread's first scale word is loaded once, with the row: loaded at each copy it is waited for at each copy
-        const bool scales = SF && x_sf && c == 0, scale_word = scales && (int)threadIdx.x < sf_cols;
-        const uint32_t *sf_row = x_sf + (int64_t)t * sf_cols;
-        const int64_t sf_step = sf_col_major ? 1 : out_sf_ld, sf_word = sf_col_major ? out_sf_ld : 1;
-        uint32_t *sf_dst = out_sf + (int64_t)threadIdx.x * sf_word;
+        // The thread's first scale word is loaded once, with the row: loaded at each copy it is waited for at each copy.  Where its copies go is
+        // worked out behind the ballot, once there is one: in front of it a workgroup without a position did all of that, too (codes with
+        // scales, one of 8 ranks, us: top-1 of [8192, 2048] 5.8 / 5.1, [21504, 2048] 11.4 / 9.8, top-2 of [8192, 7168] 13.3 / 12.6).
         uint32_t sf0 = 0;
         for (int k0 = 0; k0 < num_topk; k0 += 64) {
             const int kk = k0 + (threadIdx.x & 63);
             const int pos = list[kk < num_topk ? kk : 0];
             if (k0 == 0) {      // a token without any position is rare: not waited for
                 if (off < row_bytes) v = *src;
-                if (scales) sf0 = sf_row[scale_word ? threadIdx.x : 0];
+                if (SF && c == 0) sf0 = x_sf[(int64_t)t * sf_cols + ((int)threadIdx.x < sf_cols ? threadIdx.x : 0)];
             }
             unsigned long long live = __builtin_amdgcn_ballot_w64(kk < num_topk && pos >= 0 && pos < num_expanded);
+            if (!live) continue;
+            int i = threadIdx.x, token = t, turned = sf_col_major;
+            if constexpr (SF) asm volatile("" : "+v"(i), "+s"(token), "+s"(turned));      // (opaque, or the compiler computes all of this in front of the loop)
+            const bool scales = SF && c == 0, scale_word = scales && i < sf_cols;
+            const uint32_t *sf_row = x_sf + (int64_t)token * sf_cols;
+            const int64_t sf_step = turned ? 1 : out_sf_ld, sf_word = turned ? out_sf_ld : 1;
+            uint32_t *sf_dst = out_sf + (int64_t)i * sf_word;
             for (; live; live &= live - 1) {
                 const int64_t p = __builtin_amdgcn_readlane(pos, __builtin_ctzll(live));
                 if (off < row_bytes) expand_store16(out + p * row_bytes + off, v);
                 if (scale_word) sf_dst[p * sf_step] = sf0;
                 if (scales && sf_cols > kThreads)
-                    for (int j = threadIdx.x + kThreads; j < sf_cols; j += kThreads) out_sf[j * sf_word + p * sf_step] = sf_row[j];
+                    for (int j = i + kThreads; j < sf_cols; j += kThreads) out_sf[j * sf_word + p * sf_step] = sf_row[j];
             }
         }
     } else {
@@ -534,24 +539,31 @@ __global__ __launch_bounds__(kThreads) void expand_short_rows_kernel(const uint8
                     out_sf[sf_col_major ? (int64_t)j * out_sf_ld + p : (int64_t)p * out_sf_ld + j] = x_sf[(int64_t)t * sf_cols + j];
             return;
         }
-        const bool scales = SF && x_sf, scale_word = scales && i < sf_cols;      // (see expand_to_fused_kernel)
-        const uint32_t *sf_row = x_sf + (int64_t)t * sf_cols;
-        const int64_t sf_step = sf_col_major ? 1 : out_sf_ld, sf_word = sf_col_major ? out_sf_ld : 1;
-        uint32_t *sf_dst = out_sf + (int64_t)i * sf_word;
-        uint32_t sf0 = 0;
         if (off < row_bytes) v = *src;
-        if (scales) sf0 = sf_row[scale_word ? i : 0];
+        uint32_t sf0 = 0;
+        if (SF) sf0 = x_sf[(int64_t)t * sf_cols + (i < sf_cols ? i : 0)];
         for (int k0 = 0; k0 < num_topk; k0 += 8) {
             int p[8];
 #pragma unroll
             for (int j = 0; j < 8; ++j) p[j] = list[k0 + j < num_topk ? k0 + j : k0];
+            bool live = false;
+#pragma unroll
+            for (int j = 0; j < 8; ++j) live |= (unsigned)p[j] < (unsigned)num_expanded;
+            if (!live) continue;
+            // (as in expand_to_fused_kernel)
+            int word = i, token = t, turned = sf_col_major;
+            if constexpr (SF) asm volatile("" : "+v"(word), "+v"(token), "+s"(turned));
+            const bool scale_word = SF && word < sf_cols;
+            const uint32_t *sf_row = x_sf + (int64_t)token * sf_cols;
+            const int64_t sf_step = turned ? 1 : out_sf_ld, sf_word = turned ? out_sf_ld : 1;
+            uint32_t *sf_dst = out_sf + (int64_t)word * sf_word;
 #pragma unroll
             for (int j = 0; j < 8; ++j) {
                 if (k0 + j >= num_topk || (unsigned)p[j] >= (unsigned)num_expanded) continue;
                 if (off < row_bytes) expand_store16(out + (int64_t)p[j] * row_bytes + off, v);
                 if (scale_word) sf_dst[p[j] * sf_step] = sf0;
-                if (scales && sf_cols > tpr)
-                    for (int w = i + tpr; w < sf_cols; w += tpr) out_sf[w * sf_word + p[j] * sf_step] = sf_row[w];
+                if (SF && sf_cols > tpr)
+                    for (int w = word + tpr; w < sf_cols; w += tpr) out_sf[w * sf_word + p[j] * sf_step] = sf_row[w];
             }
         }
     } else {
