@@ -166,7 +166,7 @@ def test_mapping_of_long_lists(T, K, E, drop, alignment):
 @pytest.mark.parametrize('T,K,row_bytes,sf_cols,pad', [(9, 8, 4096, 32, 40), (63, 8, 4096, 32, 300), (64, 4, 4096, 300, 300), (70, 3, 9216, 288, 9),
                                                        (127, 8, 2048, 16, 600), (129, 8, 2048, 200, 600), (300, 2, 1024, 100, 500), (33, 70, 1040, 65, 0)])
 def test_expand_to_fused_scale_words(T, K, row_bytes, sf_cols, pad, live, col_major):
-    """A workgroup per list entry (few tokens, or much padding) and per token, with fewer and with more scale words than threads per row."""
+    """A workgroup per list entry (few tokens) and per token, with fewer and with more scale words than threads per row."""
     from tilekernels_amd import _ffi
     g = torch.Generator().manual_seed(T * K + sf_cols)
     here = torch.rand((T, K), generator=g) < live

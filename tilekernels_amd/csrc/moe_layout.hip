@@ -428,6 +428,8 @@ __device__ __forceinline__ void expand_zero_padding(int pb, int pad_rows, int nu
 // they do).  us per call on MI355X, EVERY / one per token (codes with scales, top-8 unless said):
 //   one of 8 ranks: 21504 tokens -> [24064, 7168]  214 / 59.5      340 tokens -> [6784, 4096] (worst-case buffer)  6.7 / 5.4
 //   full lists: [512, 4096] -> [5120]  6.6 / 4.7      [2048, 7168] -> [17536]  31.3 / 27.9      top-2 of [8192, 7168]  32.1 / 29.5
+//   with much padding, top-2: bf16 [3000, 2560] -> [8192]  12.9 / 10.4, codes [10000, 7168] -> [30000]  43.2 / 44.2; worst-case buffers of one of
+//   8 ranks, bf16 [3000, 2560] -> [9984]  15.0 / 10.7, [5000, 7168] -> [13952]  56.2 / 44.1
 //   bf16 -> rows of 4096, 110 MB 25.6 / 22.8, 132 MB 30.3 / 27.2, 154 MB 35.4 / 32.9, 184 MB 42.0 / 40.2, 203 MB 46.4 / 48.1, 234 MB 53.2 / 54.5,
 //   304 MB 68.3 / 70.6, 404 MB 90.9 / 95.4 (2048 and codes of 4096 the same);  7168, 168 MB 38.3 / 35.6, 236 MB 54.6 / 51.0, 407 MB 92.5 / 89.9;
 //   a third of [48128] rows of 4096 padding: codes with scales, 197 MB 38.1 / 39.2, bf16, 394 MB 64.4 / 73.5
@@ -934,19 +936,18 @@ extern "C" int tk_expand_to_fused(const void *x, int64_t num_tokens, int64_t row
     const bool short_rows = tpr * 2 <= kThreads;
     const int64_t token_groups = (num_tokens + 7) / 8 * 8;
     const int64_t token_blocks = short_rows ? (num_tokens + kThreads / tpr - 1) / (kThreads / tpr) : token_groups * chunks;
-    // With few positions per token, long rows and a quarter or more of the output certainly padding, too (codes [10000, 7168], top-2,
-    // -> [30000]: 40.6 / 43.5, -> [20400] 36.1 / 32.5 for rows of 4096).
-    const bool every = many ? num_expanded * row_bytes >= (int64_t)160 << 20 || token_blocks < 64
-                            : !short_rows && num_expanded * 3 >= num_tokens * num_topk * 4;
+    const bool every = many && (num_expanded * row_bytes >= (int64_t)160 << 20 || token_blocks < 64);
     const int kpw = !short_rows ? 1 : (every && kThreads / tpr > num_topk ? num_topk : kThreads / tpr);
     const int64_t copy_blocks = !every ? token_blocks : token_groups * (short_rows ? (num_topk + kpw - 1) / kpw : num_topk * chunks);
     // padding workgroups take 8 KB of consecutive rows each, two stores per thread.  Measured (us per call, 1 / 2 / 4
     // rows per workgroup): 8 KB rows 64.4 / 69.7 / 71.0; 4 KB rows with scales 41.4 / 36.0 / 37.0
     int pad_rows = row_bytes >= 8192 ? 1 : (int)(8192 / row_bytes > 8 ? 8 : 8192 / row_bytes);
-    // Most rows of a long buffer are live where tokens have few positions: four times the rows per padding workgroup (us, 1 / 2 / 4
-    // times: codes -> [24064, 7168] of 8 ranks 61.5 / 58.9 / 57.7, bf16 -> [33408, 4096], top-2, 76.7 / 72.3 / 70.8; with a third of
-    // rows of 2048 padding 18.3 / 17.6 / 17.7; below 16384 rows nothing is won)
-    if (!many && !every && num_expanded >= 16384) pad_rows *= 4;
+    // Most rows of a long buffer are live where tokens have few positions and it is not much longer than the list: four times the rows per
+    // padding workgroup (us, 1 / 2 / 4 times: codes -> [24064, 7168] of 8 ranks 61.5 / 58.9 / 57.7, bf16 -> [33408, 4096], top-2, 76.7 / 72.3 /
+    // 70.8; with a third of rows of 2048 padding 18.3 / 17.6 / 17.7; below 16384 rows nothing is won).  With a quarter of the rows certainly
+    // padding that many zeros in one place cost more (1 / 4 times: top-2 of bf16 [5000, 7168] -> [16384] 46.2 / 48.6, codes of 4096 14.0 / 16.1; a
+    // worst-case buffer of one of 8 ranks, bf16 [8192, 2560] -> [24448], 26.5 / 30.1).
+    if (!many && !every && num_expanded >= 16384 && num_expanded * 3 < num_tokens * num_topk * 4) pad_rows *= 4;
     const int64_t grid = copy_blocks + (num_expanded + pad_rows - 1) / pad_rows;
     if (grid == 0) return TK_OK;
     hipStream_t s = static_cast<hipStream_t>(stream);
