@@ -109,10 +109,11 @@ def test_reduce_fused_with_few_and_many_live_terms(T, K, dtype, hidden):
 
 
 @pytest.mark.parametrize('dtype', [torch.float32, torch.bfloat16], ids=['f32', 'bf16'])
-@pytest.mark.parametrize('T,hidden', [(7, 256), (9, 512), (6, 768), (5, 1280), (3, 2048), (2060, 2048), (4, 2560), (1030, 4096), (3, 7168)])
+@pytest.mark.parametrize('T,hidden', [(7, 256), (9, 512), (6, 768), (5, 1280), (3, 2048), (2060, 2048), (4, 2560), (1030, 4096), (3, 7168),
+                                      (2048, 256), (2051, 256), (2050, 512), (409, 2560), (411, 2560), (2053, 4096)])
 def test_reduce_fused_workgroup_shapes_and_dead_terms(T, hidden, dtype):
-    """Rows of one to fourteen pieces, launches below and above one round of wave slots, one to thirteen terms: lists that are all live,
-    and lists whose dead terms carry any position outside the rows, a NaN weight and no scale of their own."""
+    """Rows of one to fourteen pieces, launches below and above one round of wave slots, workgroups of one token and of several, one to thirteen
+    terms: lists that are all live, and lists whose dead terms carry any position outside the rows, a NaN weight and no scale of their own."""
     tk = _tk()
     R = 40
     g = torch.Generator().manual_seed(T + hidden)

@@ -699,8 +699,8 @@ __device__ __forceinline__ void reduce_store(const float (&acc)[8], void *out, i
     }
 }
 
-// A workgroup takes `side` pieces of one token, or (STACKED, side 1 or 2) those of 4 / side tokens.
-template <typename InT, int OUT, bool STACKED>
+// A workgroup takes `side` pieces of one token, or (STACKED, side 1 or 2) those of 4 / side tokens.  FEW: one or two terms.
+template <typename InT, int OUT, bool STACKED, bool FEW>
 __global__ __launch_bounds__(kThreads) void reduce_fused_kernel(const typename ReduceIn<InT>::elem *x, const int32_t *token_topk_to_pos, int num_tokens,
                                                                 int num_topk, int hidden, int num_expanded, int shape,
                                                                 const float *topk_weights, const float *x_sf, const float *sf, void *out) {
@@ -726,7 +726,7 @@ __global__ __launch_bounds__(kThreads) void reduce_fused_kernel(const typename R
         list += U;                                                                                                               \
         if (weights) weights += U;                                                                                               \
     } while (0)
-    if constexpr (!STACKED) {      // (STACKED: one or two terms)
+    if constexpr (!FEW) {
         for (; left >= 8; left -= 8) TK_REDUCE_TERMS(8);
         if (left & 4) TK_REDUCE_TERMS(4);
     }
@@ -1003,15 +1003,20 @@ extern "C" int tk_reduce_fused(const void *x, int x_dtype, int64_t num_expanded,
     }
     const int strips = (int)((hidden + kStripCols - 1) / kStripCols);
     // Pieces side by side in a workgroup: whole rows of up to four, otherwise the largest number up to four that divides the row (five
-    // or seven waves 31.5 and 43.5 us instead of 31.0 and 42.8 for bf16 [4096, 2560] and [.., 3584], 8 of 8).  In launches that fill the
-    // GPU's wave slots more than once, with more than four terms, two instead of four (bf16 [4096, 4096], 8 of 8: 51.5 / 49.2 us; with
-    // two terms [32768, 2048] 61.5 / 63.5, and 340 tokens 5.2 / 5.5) and, fp32, one ([4096, 4096] 104.0 / 100.3).
+    // or seven waves 31.5 and 43.5 us instead of 31.0 and 42.8 for bf16 [4096, 2560] and [.., 3584], 8 of 8).  Large launches take two instead
+    // of four with more than four terms (bf16 [4096, 4096], 8 of 8: 51.5 / 49.2 us), larger ones with three or four (bf16 [16384, 4096], 3 of 3:
+    // 86.8 / 80.9, [8192, 8192] 84.8 / 80.8, but [4500, 8192] 47.8 / 54.9, 4 of 4 58.2 / 56.0; with two terms [32768, 2048] 61.5 / 63.5) and, fp32, one ([4096, 4096]
+    // 104.0 / 100.3, but [1100, 4096], 6 of 6, 23.2 / 24.3).
+    const int64_t waves = num_tokens * strips;
+    const bool bf16 = x_dtype == TK_BF16, few = num_topk <= 2;
     int side = 4;
     while (strips % side) --side;
-    if (side == 4 && num_topk > 4 && num_tokens * strips > 8192) side = x_dtype == TK_BF16 ? 2 : 1;
-    // One or two terms of short rows: four waves to a workgroup all the same, on further tokens, since workgroups of one wave are
-    // not started fast enough (bf16 [262144, 256], one term: 69.1 / 61.9 us; fp32 104.3 / 102.9, but [262144, 512] 180 / 186).
-    const bool stacked = num_topk <= 2 && (x_dtype == TK_BF16 ? side <= 2 : hidden <= 256);
+    if (side == 4 && !few && (num_topk > 4 ? waves > (bf16 ? 8192 : 16384) : bf16 && waves >= (num_topk == 4 ? 65536 : 98304))) side = bf16 ? 2 : 1;
+    // Four waves to a workgroup all the same, on further tokens, since workgroups of one wave are not started fast enough: with one or two
+    // terms (bf16 [262144, 256], one term: 69.1 / 61.9 us; fp32 104.3 / 102.9, but [262144, 512] 180 / 186), and with more where there is one
+    // piece side by side and the launch is not all latency (one of 8 ranks, 8 terms: bf16 [8192, 2560] 20.7 / 14.8, [8192, 3584] 27.8 / 20.6,
+    // [512, 2560] 3.4 / 2.9, 8 of 8 the same within 2 %; but 8 of 8 of fp32 [512, 256] 2.8 / 3.3, [64, 2560] 2.9 / 3.5).
+    const bool stacked = few ? (bf16 ? side <= 2 : hidden <= 256) : side == 1 && waves > 2048;
     // HIP takes fewer than 2^32 threads along a grid dimension, and the row tiles of a single column of pieces all ride on x:
     // at most 2^23 row tiles (2^31 threads) per launch.
     const int64_t rows = stacked ? 4 / side : 1, step = rows << 23, out_bytes = out_dtype == TK_F32 ? 4 : (out_dtype == TK_BF16 ? 2 : 1);
@@ -1025,23 +1030,29 @@ extern "C" int tk_reduce_fused(const void *x, int x_dtype, int64_t num_expanded,
         void *o = static_cast<uint8_t *>(out) + t0 * hidden * out_bytes;
 #define TK_REDUCE_LAUNCH(T, O)                                                                                              \
     do {                                                                                                                    \
-        if (stacked) TK_REDUCE_LAUNCH_2(T, O, true);                                                                        \
-        else TK_REDUCE_LAUNCH_2(T, O, false);                                                                               \
+        if (stacked && few) TK_REDUCE_LAUNCH_2(T, O, true, true);                                                           \
+        else TK_REDUCE_LAUNCH_MANY(T, O);                                                                                   \
     } while (0)
-#define TK_REDUCE_LAUNCH_2(T, O, S)                                                                                         \
-    hipLaunchKernelGGL((reduce_fused_kernel<T, O, S>), grid, block, 0, s, static_cast<const ReduceIn<T>::elem *>(x), pos,   \
+#define TK_REDUCE_LAUNCH_MANY(T, O)                                                                                         \
+    do {                                                                                                                    \
+        if (stacked) TK_REDUCE_LAUNCH_2(T, O, true, false);                                                                 \
+        else TK_REDUCE_LAUNCH_2(T, O, false, false);                                                                        \
+    } while (0)
+#define TK_REDUCE_LAUNCH_2(T, O, S, F)                                                                                      \
+    hipLaunchKernelGGL((reduce_fused_kernel<T, O, S, F>), grid, block, 0, s, static_cast<const ReduceIn<T>::elem *>(x), pos, \
                        (int)tokens, num_topk, (int)hidden, (int)num_expanded, side | (int)(cols == 1) << 3, weights, x_sf, sf, o)
         if (x_dtype == TK_BF16) {
             if (out_dtype == TK_OUT_E4M3) TK_REDUCE_LAUNCH(bf16_t, 2);
             else TK_REDUCE_LAUNCH(bf16_t, 0);
         } else if (hidden % 512 == 0) {
-            if (out_dtype == TK_OUT_E4M3) TK_REDUCE_LAUNCH_2(SplitF32, 2, false);      // (never stacked: rows of 512 and more)
-            else TK_REDUCE_LAUNCH_2(SplitF32, 1, false);
+            if (out_dtype == TK_OUT_E4M3) TK_REDUCE_LAUNCH_MANY(SplitF32, 2);      // (with one or two terms never stacked: rows of 512 and more)
+            else TK_REDUCE_LAUNCH_MANY(SplitF32, 1);
         } else {
             if (out_dtype == TK_OUT_E4M3) TK_REDUCE_LAUNCH(float, 2);
             else TK_REDUCE_LAUNCH(float, 1);
         }
 #undef TK_REDUCE_LAUNCH_2
+#undef TK_REDUCE_LAUNCH_MANY
 #undef TK_REDUCE_LAUNCH
     }
     return (int)hipGetLastError();
