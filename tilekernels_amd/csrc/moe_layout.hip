@@ -1005,13 +1005,14 @@ extern "C" int tk_reduce_fused(const void *x, int x_dtype, int64_t num_expanded,
     // Pieces side by side in a workgroup: whole rows of up to four, otherwise the largest number up to four that divides the row (five
     // or seven waves 31.5 and 43.5 us instead of 31.0 and 42.8 for bf16 [4096, 2560] and [.., 3584], 8 of 8).  Large launches take two instead
     // of four with more than four terms (bf16 [4096, 4096], 8 of 8: 51.5 / 49.2 us), larger ones with three or four (bf16 [16384, 4096], 3 of 3:
-    // 86.8 / 80.9, [8192, 8192] 84.8 / 80.8, but [4500, 8192] 47.8 / 54.9, 4 of 4 58.2 / 56.0; with two terms [32768, 2048] 61.5 / 63.5) and, fp32, one ([4096, 4096]
-    // 104.0 / 100.3, but [1100, 4096], 6 of 6, 23.2 / 24.3).
+    // 86.8 / 80.9, [8192, 8192] 84.8 / 80.8, but [4500, 8192] 47.8 / 54.9, 4 of 4 58.2 / 56.0; with two terms [32768, 2048] 61.5 / 63.5)
+    // and, fp32, one ([8192, 2048], 8 of 8: 102.9 / 99.9; but not rows of a multiple of 16 KB, where some lists lose more than others win:
+    // [4500, 4096], 8 of 8, 114.3 / 108.4, [2200, 4096], 7 of 7, 50.8 / 56.0, [8192, 4096], 7 terms of one of 4 ranks, 59.8 / 66.4).
     const int64_t waves = num_tokens * strips;
     const bool bf16 = x_dtype == TK_BF16, few = num_topk <= 2;
     int side = 4;
     while (strips % side) --side;
-    if (side == 4 && !few && (num_topk > 4 ? waves > (bf16 ? 8192 : 16384) : bf16 && waves >= (num_topk == 4 ? 65536 : 98304))) side = bf16 ? 2 : 1;
+    if (side == 4 && !few && (num_topk > 4 ? waves > 8192 && (bf16 || hidden % 4096 != 0) : bf16 && waves >= (num_topk == 4 ? 65536 : 98304))) side = bf16 ? 2 : 1;
     // Four waves to a workgroup all the same, on further tokens, since workgroups of one wave are not started fast enough: with one or two
     // terms (bf16 [262144, 256], one term: 69.1 / 61.9 us; fp32 104.3 / 102.9, but [262144, 512] 180 / 186), and with more where there is one
     // piece side by side and the launch is not all latency (one of 8 ranks, 8 terms: bf16 [8192, 2560] 20.7 / 14.8, [8192, 3584] 27.8 / 20.6,
