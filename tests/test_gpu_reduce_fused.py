@@ -119,7 +119,7 @@ def test_reduce_fused_workgroup_shapes_and_dead_terms(T, hidden, dtype):
     g = torch.Generator().manual_seed(T + hidden)
     x = torch.randn((R, hidden), generator=g).to(dtype)
     x_sf = torch.rand((R,), generator=g)
-    for K in (1, 2, 3, 8, 13):
+    for K in (1, 2, 3, 6, 8, 13):
         w = torch.rand((T, K), generator=g)
         full = torch.randint(0, R, (T, K), generator=g, dtype=torch.int32)
         dead = torch.rand((T, K), generator=g) < 0.5

@@ -622,7 +622,7 @@ __device__ __forceinline__ void reduce_load(typename ReduceIn<InT>::raw &raw, co
 // U consecutive terms of a token, those in `live` only (ALL: every one).  Everything but the pieces comes through the scalar path.
 template <typename InT, int U, bool ALL>
 __device__ __forceinline__ void reduce_terms(float (&acc)[8], const uint8_t *x, uint32_t bytes, uint32_t lane_off, uint64_t row_bytes, uint32_t num_expanded,
-                                             const uint32_t (&pos)[U], const float *weights, const float *x_sf) {
+                                             const uint32_t (&pos)[U], const float *weights, const float *x_sf, int left = U) {
     typename ReduceIn<InT>::raw raw[U];
     uint32_t live = 0;
     float w[U], f[U];
@@ -641,7 +641,7 @@ __device__ __forceinline__ void reduce_terms(float (&acc)[8], const uint8_t *x, 
     for (int j = 0; j < U; ++j) w[j] = f[j] = 1.0f;
     if (weights) {
 #pragma unroll
-        for (int j = 0; j < U; ++j) w[j] = uniform_load(weights + j);
+        for (int j = 0; j < U; ++j) w[j] = uniform_load(weights + (ALL ? j : min(j, left - 1)));
     }
     if (x_sf) {
 #pragma unroll
@@ -670,6 +670,29 @@ __device__ __forceinline__ void reduce_group(float (&acc)[8], const uint8_t *x, 
     for (int j = 0; j < U; ++j) asm("s_max_u32 %0, %1, %2" : "=s"(last) : "s"(last), "s"(pos[j]) : "scc");
     if (last < num_expanded) reduce_terms<InT, U, true>(acc, x, bytes, lane_off, row_bytes, num_expanded, pos, weights, x_sf);
     else reduce_terms<InT, U, false>(acc, x, bytes, lane_off, row_bytes, num_expanded, pos, weights, x_sf);
+}
+
+// The last five to seven terms.  Of a list with dead terms all live ones together: four and then the rest are two round trips (one of 8
+// ranks, 6 terms: bf16 [512, 4096] 3.4 / 3.2 us, [1100, 7168] 7.6 / 7.0, [8192, 4096] 21.0 / 19.8).  A full list is better off in steps, which
+// hold fewer loads (6 of 6: bf16 [4500, 2048] 22.5 together / in steps 21.85).
+template <typename InT>
+__device__ __forceinline__ void reduce_rest(float (&acc)[8], const uint8_t *x, uint32_t bytes, uint32_t lane_off, uint64_t row_bytes, uint32_t num_expanded,
+                                            const int32_t *list, const float *weights, const float *x_sf, int left) {
+    uint32_t pos[8], last = 0;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) pos[j] = (uint32_t)uniform_load(list + min(j, left - 1));
+#pragma unroll
+    for (int j = 0; j < 7; ++j) asm("s_max_u32 %0, %1, %2" : "=s"(last) : "s"(last), "s"(pos[j]) : "scc");
+    if (last < num_expanded) {
+        reduce_terms<InT, 4, true>(acc, x, bytes, lane_off, row_bytes, num_expanded, {pos[0], pos[1], pos[2], pos[3]}, weights, x_sf);
+        if (left & 2) reduce_terms<InT, 2, true>(acc, x, bytes, lane_off, row_bytes, num_expanded, {pos[4], pos[5]}, weights ? weights + 4 : weights, x_sf);
+        if (left & 1) reduce_terms<InT, 1, true>(acc, x, bytes, lane_off, row_bytes, num_expanded, {pos[7]}, weights ? weights + (left - 1) : weights, x_sf);
+    } else {
+#pragma unroll
+        for (int j = 5; j < 8; ++j)
+            if (j >= left) pos[j] = 0xFFFFFFFFu;
+        reduce_terms<InT, 8, false>(acc, x, bytes, lane_off, row_bytes, num_expanded, pos, weights, x_sf, left);
+    }
 }
 
 // OUT: 0 bf16, 1 fp32, 2 E4M3
@@ -728,6 +751,10 @@ __global__ __launch_bounds__(kThreads) void reduce_fused_kernel(const typename R
     } while (0)
     if constexpr (!FEW) {
         for (; left >= 8; left -= 8) TK_REDUCE_TERMS(8);
+        if (left > 4) {
+            reduce_rest<InT>(acc, xp, (uint32_t)cols * kElem, lane_off, row_bytes, (uint32_t)num_expanded, list, weights, x_sf, left);
+            left = 0;
+        }
         if (left & 4) TK_REDUCE_TERMS(4);
     }
     if (left & 2) TK_REDUCE_TERMS(2);
