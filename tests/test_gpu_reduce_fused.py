@@ -130,3 +130,5 @@ def test_reduce_fused_workgroup_shapes_and_dead_terms(T, hidden, dtype):
             assert_same(tk.moe.reduce_fused(xgpu, w.cuda(), full.cuda()), torch_ref.reduce_fused(xin, w, full), f'{K} full')
             got = tk.moe.reduce_fused(xgpu, w.masked_fill(dead, float('nan')).cuda(), torch.where(dead, outside, full).cuda())
             assert_same(got, torch_ref.reduce_fused(xin, w, some), f'{K} some')
+        one = torch.full((1,), 0.5)
+        assert_same(tk.moe.reduce_fused(xg, w.cuda(), some.cuda(), 'e4m3', one.cuda()), torch_ref.reduce_fused(x, w, some, 'e4m3', one), f'{K} e4m3')
