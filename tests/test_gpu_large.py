@@ -8,6 +8,7 @@ import torch
 
 from oracle import torch_ref
 from tests._util import dense_bytes
+from tests.test_gpu_per_channel import gathered_fp8_rows
 from tests.test_gpu_swiglu import check_fused
 from tests.test_gpu_swiglu_backward import check_backward
 
@@ -295,3 +296,24 @@ def test_swiglu_of_more_short_rows_than_lane_slots():
     codes, sf = codes.view(torch.uint8).view(n, block, H), sf.view(n, block, H // 128)
     for i in range(n):
         assert torch.equal(codes[i], want.view(torch.uint8)) and torch.equal(sf[i], want_sf), i
+
+
+@pytest.mark.parametrize('N', [32, 128])
+def test_gathered_fp8_rows_beyond_4_gb(N):
+    # more input than a 32-bit offset reaches: every gathered row against the oracle
+    T, K, M = 600_000, 7168, 2560
+    assert T * K > 2 * LIMIT
+    g = torch.Generator(device='cuda').manual_seed(3)
+    codes = torch.empty((T, K), dtype=torch.uint8, device='cuda')
+    for a in range(0, T, 100_000):
+        codes[a:a + 100_000] = torch.randint(0, 0x7F, (100_000, K), generator=g, device='cuda', dtype=torch.uint8)
+    codes = codes.view(torch.float8_e4m3fn)
+    sf = torch.rand((T, K // 128), generator=g, device='cuda') + 0.01
+    pos = torch.randint(0, T, (M,), generator=g, device='cuda', dtype=torch.int32)
+    pos[7], pos[100], pos[-1] = -1, 0, T - 1
+    out, out_sf = gathered_fp8_rows(codes, sf, pos, N)
+    rows = pos.clamp(min=0).long()
+    local = torch.where(pos >= 0, torch.arange(M, device='cuda', dtype=torch.int32), -1).to(torch.int32)
+    want = torch_ref.per_channel_cast_fused((codes.view(torch.uint8)[rows].view(torch.float8_e4m3fn).cpu(), sf[rows].cpu()), N, 128, False, local.cpu())
+    _same_bytes(out, want[0], 'codes')
+    _same_bytes(out_sf, want[1], 'sf')

@@ -219,3 +219,35 @@ def test_fp8_input_with_buffers_that_are_only_8_byte_aligned(x_shift, out_shift)
     assert_same(got, want_codes, 'codes')
     assert_same(out_sf, want_sf, 'scales')
     assert int(obuf[:out_shift].sum()) == 0 and int(obuf[out_shift + T * K:].sum()) == 0
+
+
+def gathered_fp8_rows(codes, sf, pos, N):
+    """The per-channel cast of gathered E4M3 rows with one scale per N tokens (the Python function takes 128 only)."""
+    from tilekernels_amd import _ffi
+    (T, K), M = codes.shape, pos.shape[0]
+    out = torch.empty((M, K), dtype=torch.float8_e4m3fn, device='cuda')
+    out_sf = torch.empty((-(-M // N), K), dtype=torch.float32, device='cuda')
+    rc = _ffi.load().tk_per_channel_cast(codes.data_ptr(), 0, sf.data_ptr(), T, K, pos.data_ptr(), M, out.data_ptr(), out_sf.data_ptr(),
+                                         N, 0, 0, 0, 0, 0.0, _ffi.current_stream(out.device))
+    assert rc == 0, rc
+    torch.cuda.synchronize()
+    return out, out_sf
+
+
+# (tokens, rows, columns): few tokens and much padding; column order with a last tile that is partly beyond the matrix, at both ends of its
+# range of tokens; rows about as many as tokens; wide tiles, written through and not; each with rows of -1 and of the last token
+@pytest.mark.parametrize('N', [32, 128])
+@pytest.mark.parametrize('T,M,K', [(1, 16, 128), (100, 2064, 640), (4095, 7184, 384), (4096, 7168, 384), (16383, 28672, 128), (16384, 28688, 640),
+                                   (3000, 2992, 1408), (6553, 8192, 2048), (6600, 8192, 2048), (6000, 8320, 2176)])
+def test_gathered_fp8_rows_by_tokens_and_rows(T, M, K, N):
+    g = torch.Generator().manual_seed(T + K)
+    x = torch_ref.cast(torch.randn((T, K), generator=g).to(torch.bfloat16), 'e4m3', (1, 128))
+    pos = torch.randint(0, T, (M,), generator=g, dtype=torch.int32)
+    pos[torch.rand((M,), generator=g) < 0.2] = -1
+    pos[-1], pos[0] = T - 1, -1
+    if M > 256:
+        pos[128:256] = -1                           # a whole tile of padding
+    want = torch_ref.per_channel_cast_fused(x, N, 128, False, pos)
+    got = gathered_fp8_rows(x[0].cuda(), x[1].cuda(), pos.cuda(), N)
+    assert_same(got[0], want[0], 'codes')
+    assert_same(got[1], want[1], 'scales')

@@ -290,15 +290,58 @@ __global__ __launch_bounds__(LANES * kPcParts, 4) void per_channel_cast_kernel(T
     }
 }
 
+// Gathered E4M3 rows: whether most of the output is padding or tokens that other rows repeat.  Narrow tiles serve that better, wide ones
+// the rest (figures at the kernel; from 9100 tokens [13120, 2560] wide / narrow 12.5 / 11.4 us, cold 14.3 / 15.2; 21520 -> [33792, 7168] 85.4 / 90.5).
+__host__ __device__ inline bool gather_repeats(int num_tokens, int M) { return 4 * (int64_t)M >= 7 * (int64_t)num_tokens; }
+// and whether its tiles then go in column order, each XCD down a column of its own: a column tile of all tokens (256 bytes of each) stays in
+// the XCD's 4 MB L2 until the next expert's rows ask for it ([10112, 7168] from 5401 tokens 21.6 / 19.2 us, [18432, 7168] from 8192 37.1 / 33.0).
+// So few tokens that all of their rows stay in the caches need no order (88 -> [31616, 7168] 41.5 / 42.9, 928 -> [32768, 3712] 24.4 / 25.2).
+__host__ __device__ inline bool gather_by_columns(int num_tokens, int M) { return gather_repeats(num_tokens, M) && num_tokens >= 4096 && num_tokens < 16384; }
+
+// Offset beyond the end of any buffer, also with a lane's part of up to 496 bytes added to it.
+constexpr uint32_t kPcNowhere = 0xFFFFFC00u;
+
+// out[r] = v of lane 8 g + r, in every lane of lanes 8 g .. 8 g + 7
+__device__ __forceinline__ void deal_rows(uint32_t (&out)[kPcRows], uint32_t v) {
+#define TK_PC_DEAL(r) out[r] = (uint32_t)__builtin_amdgcn_ds_swizzle((int)v, (r) << 5 | 0x18)
+    TK_PC_DEAL(0); TK_PC_DEAL(1); TK_PC_DEAL(2); TK_PC_DEAL(3);
+    TK_PC_DEAL(4); TK_PC_DEAL(5); TK_PC_DEAL(6); TK_PC_DEAL(7);
+#undef TK_PC_DEAL
+}
+
+// Write-through store of 16 codes.  (The conversion that makes a code fills half a register, and what reads it next has to stay one wait
+// state away; the compiler keeps that distance from instructions it knows, this one keeps it by itself.)
+__device__ __forceinline__ void st_codes16(void *p, u32x4 v) {
+    asm volatile("s_nop 0" : "+v"(v));
+    st_stream16(p, v);
+}
+
 // E4M3 input with 1 x 128 scales, plain (not transposed) output, with 16 codes per lane instead of 8: a workgroup of 512
 // threads owns 128 tokens x 512 columns, half a wave (32 lanes x 16 columns) takes 8 consecutive tokens, and every
 // load and store instruction of a lane moves 16 bytes (8 bytes per lane make a half-wave's instruction 256 bytes
 // long; measured on MI355X at [8192, 4096]: 13.8 us that way, 12.8 us this way).  The rest is the kernel above: maxima down the lane's columns, the 16 partial maxima per column meet in LDS,
 // thread c derives the scale(s) of column c and hands the multipliers back.
-// LANES = 16: 256 threads, 128 x 256 tiles, where the wide tiles are too few for the GPU.
-template <int NPT, bool GATHER, int LANES>
+// LANES = 16: 256 threads, 128 x 256 tiles, where the wide tiles are too few for the GPU and for gathers with much reuse or padding.
+//
+// Gathered rows.  What bounds a gather is its reads of rows that other tiles read too: every token is fetched once per expert it went to,
+// and non-temporal loads fetch it from HBM each time; with ordinary loads the second read is served by a cache.  Padding rows read nothing:
+// the input is a buffer in scalar registers, their offset lies beyond its end, and what is read there is zero (reads of some row in their
+// place all went to the same lines).  A half-wave's scales and source rows come with one load each, lane (group, row) holding row `row`'s,
+// and are dealt out within the half-wave.  us on MI355X, all rows by non-temporal loads, padding from row 0 / this, three sets of inputs in
+// rotation (twelve, which no cache holds):
+//   experts' rows of 7168 from 5401 tokens, [10112] 29.1 / 19.2 (29.8 / 28.5);  two copies each of 8192 tokens, [18432] 49.5 / 33.0 (49.7 / 47.7)
+//   mostly padding: 244 tokens -> [32768, 3968] 40.9 / 25.8 (43.0 / 25.7), 1202 -> [18048, 6144] 41.0 / 23.9 (40.2 / 24.0), 928 -> [32768, 3712]
+//   42.6 / 24.4 (43.6 / 24.0);  little of either: 16600 -> [17408, 6144] 42.6 / 42.6 (43.0 / 44.4), 19800 -> [28800, 4096] 43.8 / 42.4 (44.1 / 43.3)
+// So rows that are about as many as the tokens, each read about once, keep the non-temporal loads.
+// SRC: where rows come from.  PC_IN_ORDER: those of the output; PC_GATHERED; PC_GATHERED_ONCE: with non-temporal loads; PC_GATHERED_FAR:
+// from more than a buffer's 4 GB, by addresses.
+// THROUGH: write-through stores.  Where the output is short, nothing is left to be written back when the launch ends ([4096, 4096] 6.2 / 5.4
+// us, [16384, 1024] 6.1 / 5.4, but [8128, 2560] from cold inputs 8.7 / 10.9, [10112, 7168] 21.6 / 30.5).
+enum { PC_IN_ORDER = 0, PC_GATHERED = 1, PC_GATHERED_ONCE = 2, PC_GATHERED_FAR = 3 };
+template <int NPT, int SRC, int LANES, bool THROUGH>
 __global__ __launch_bounds__(LANES * kPcParts, 4) void per_channel_cast_fp8in_kernel(TK_PC_KERNEL_ARGS) {
     TK_PC_KERNEL_UNPACK;
+    constexpr bool GATHER = SRC != PC_IN_ORDER, BUFFER = SRC == PC_GATHERED || SRC == PC_GATHERED_ONCE;
     constexpr int kPcWideK = LANES * 16;
     constexpr int NB = kPcTileM / NPT;
     __shared__ __attribute__((aligned(16))) float part[kPcParts][kPcWideK];
@@ -306,9 +349,15 @@ __global__ __launch_bounds__(LANES * kPcParts, 4) void per_channel_cast_fp8in_ke
 
     // the tiles of one token range share the 128-byte lines of the input scales: 8 token ranges advance side by
     // side, one per XCD (workgroups are dealt to the XCDs round-robin)
+    const int tiles_m = (p.M + kPcTileM - 1) / kPcTileM;
     int tile_m = blockIdx.x / p.tiles_k, tile_k = blockIdx.x - tile_m * p.tiles_k;
-    const int tiles_m = (p.M + kPcTileM - 1) / kPcTileM, striped = (tiles_m / 8) * 8 * p.tiles_k;
-    if ((int)blockIdx.x < striped) {
+    if (SRC == PC_GATHERED && LANES == 16 && gather_by_columns(p.num_tokens, p.M)) {
+        // the tiles in column order, cut into one consecutive eighth per XCD
+        const int tiles = (int)gridDim.x, xcd = blockIdx.x & 7;
+        const int at = xcd * (tiles >> 3) + min(xcd, tiles & 7) + (int)(blockIdx.x >> 3);
+        tile_k = at / tiles_m;
+        tile_m = at - tile_k * tiles_m;
+    } else if (const int striped = (tiles_m / 8) * 8 * p.tiles_k; (int)blockIdx.x < striped) {
         const int q = blockIdx.x >> 3;
         tile_k = q % p.tiles_k;
         tile_m = (q / p.tiles_k) * 8 + (blockIdx.x & 7);
@@ -320,36 +369,65 @@ __global__ __launch_bounds__(LANES * kPcParts, 4) void per_channel_cast_fp8in_ke
     const bool rows_ok = tok0 < p.M;            // M is a multiple of 16: all 8 tokens of a lane or none
 
     Raw8<e4m3in_t> lo[kPcRows], hi[kPcRows];
-#pragma unroll
-    for (int r = 0; r < kPcRows; ++r) { lo[r].zero(); hi[r].zero(); }
-    if (rows_ok && col_ok) {
-        // (gather indices of all rows first: see per_channel_cast_kernel)
-        int gathered[kPcRows];
-        if constexpr (GATHER) {
-#pragma unroll
-            for (int r = 0; r < kPcRows; ++r) gathered[r] = p.pos_to_token[tok0 + r];
-        }
+    if constexpr (BUFFER) {
+        constexpr int kHint = SRC == PC_GATHERED_ONCE ? 2 : 0;      // 2: non-temporal
+        const uint32_t row_bytes = (uint32_t)p.K, sf_bytes = (uint32_t)(p.K >> 7) * 4u;
+        const __amdgpu_buffer_rsrc_t x = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t *>(reinterpret_cast<const uint8_t *>(p.x)) + col0, 0,
+                                                                           (int)((uint32_t)p.num_tokens * row_bytes - (uint32_t)col0), 0x00020000);
+        const __amdgpu_buffer_rsrc_t x_sf = __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(p.x_sf), 0, (int)((uint32_t)p.num_tokens * sf_bytes), 0x00020000);
+        // lane (g, r) of the run: row r, and the scale of its columns 128 g ..; whether there are such columns is the same for its 8 lanes
+        const int src = p.pos_to_token[rows_ok ? tok0 + (hl & 7) : 0];
+        const bool live = rows_ok && col_ok && src >= 0 && src < p.num_tokens;
+        uint32_t offs[kPcRows];
+        deal_rows(offs, live ? (uint32_t)src * row_bytes : kPcNowhere);
+        u32x4 w[kPcRows];
 #pragma unroll
         for (int r = 0; r < kPcRows; ++r) {
-            int src = tok0 + r;
-            bool valid = true;
-            if constexpr (GATHER) {
-                src = gathered[r];
-                valid = src >= 0 && src < p.num_tokens;
-                src = valid ? src : 0;
-            }
-            const u32x4 w = ld_stream16(reinterpret_cast<const uint8_t *>(p.x) + (int64_t)src * p.K + col);
+            w[r] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(x, offs[r] + (uint32_t)(hl * 16), 0, kHint));
             vmem_issue_gap();
-            lo[r].w = u32x2{w.x, w.y};
-            hi[r].w = u32x2{w.z, w.w};
-            lo[r].s = hi[r].s = p.x_sf[(int64_t)src * (p.K >> 7) + (col >> 7)];
-            vmem_issue_gap();
-            gathered[r] = valid ? 1 : 0;
         }
-        if constexpr (GATHER) {      // (cleared once all loads are out)
+        const uint32_t s = __builtin_amdgcn_raw_buffer_load_b32(x_sf, live ? (uint32_t)src * sf_bytes + (uint32_t)(col >> 7) * 4u : kPcNowhere, 0, 0);
+        __builtin_amdgcn_sched_barrier(0);
+        uint32_t scales[kPcRows];
+        deal_rows(scales, s);
 #pragma unroll
-            for (int r = 0; r < kPcRows; ++r)
-                if (!gathered[r]) { lo[r].zero(); hi[r].zero(); }
+        for (int r = 0; r < kPcRows; ++r) {
+            lo[r].w = u32x2{w[r].x, w[r].y};
+            hi[r].w = u32x2{w[r].z, w[r].w};
+            lo[r].s = hi[r].s = u2f(scales[r]);
+        }
+    } else {
+#pragma unroll
+        for (int r = 0; r < kPcRows; ++r) { lo[r].zero(); hi[r].zero(); }
+        if (rows_ok && col_ok) {
+            // (gather indices of all rows first: see per_channel_cast_kernel)
+            int gathered[kPcRows];
+            if constexpr (GATHER) {
+#pragma unroll
+                for (int r = 0; r < kPcRows; ++r) gathered[r] = p.pos_to_token[tok0 + r];
+            }
+#pragma unroll
+            for (int r = 0; r < kPcRows; ++r) {
+                int src = tok0 + r;
+                bool valid = true;
+                if constexpr (GATHER) {
+                    src = gathered[r];
+                    valid = src >= 0 && src < p.num_tokens;
+                    src = valid ? src : 0;
+                }
+                const u32x4 w = ld_stream16(reinterpret_cast<const uint8_t *>(p.x) + (int64_t)src * p.K + col);
+                vmem_issue_gap();
+                lo[r].w = u32x2{w.x, w.y};
+                hi[r].w = u32x2{w.z, w.w};
+                lo[r].s = hi[r].s = p.x_sf[(int64_t)src * (p.K >> 7) + (col >> 7)];
+                vmem_issue_gap();
+                gathered[r] = valid ? 1 : 0;
+            }
+            if constexpr (GATHER) {      // (cleared once all loads are out)
+#pragma unroll
+                for (int r = 0; r < kPcRows; ++r)
+                    if (!gathered[r]) { lo[r].zero(); hi[r].zero(); }
+            }
         }
     }
 
@@ -412,8 +490,11 @@ __global__ __launch_bounds__(LANES * kPcParts, 4) void per_channel_cast_fp8in_ke
             b[j] = b[j] * inv[8 + j];
         }
         const u32x2 x0 = pack_e4m3x8<false>(a), x1 = pack_e4m3x8<false>(b);
-        if (rows_ok && col_ok)
-            __builtin_nontemporal_store(u32x4{x0.x, x0.y, x1.x, x1.y}, reinterpret_cast<u32x4 *>(p.out + (int64_t)(tok0 + r) * p.K + col));
+        if (rows_ok && col_ok) {
+            uint8_t *dst = p.out + (int64_t)(tok0 + r) * p.K + col;
+            if constexpr (THROUGH) st_codes16(dst, u32x4{x0.x, x0.y, x1.x, x1.y});
+            else __builtin_nontemporal_store(u32x4{x0.x, x0.y, x1.x, x1.y}, reinterpret_cast<u32x4 *>(dst));
+        }
     }
 }
 
@@ -435,6 +516,11 @@ template <int MODE> static int64_t wide_tiles_from(bool transpose, bool gather) 
     return MODE != PC_BF16 || transpose || gather ? 256 : 176;
 }
 
+constexpr int64_t kPcThrough = 16 << 20;      // bytes of output up to which gathered codes are written through
+// More input than a buffer can hold, and rows that are read about once (see the kernel).
+static bool gather_far(const PerChannelParams &p) { return (int64_t)p.num_tokens * p.K > (int64_t)kPcNowhere; }
+static bool gather_once(const PerChannelParams &p) { return 4 * (int64_t)p.M < 5 * (int64_t)p.num_tokens; }
+
 template <int MODE, int NPT, int LANES>
 static void launch_per_channel_3(const PerChannelParams &a, bool transpose, hipStream_t stream) {
     PerChannelParams p = a;
@@ -444,8 +530,14 @@ static void launch_per_channel_3(const PerChannelParams &a, bool transpose, hipS
         if (!transpose && aligned_to(p.x, 16) && aligned_to(p.out, 16)) {
             p.tiles_k = (p.K + LANES * 16 - 1) / (LANES * 16);
             const dim3 grid((unsigned)(tiles_m * p.tiles_k));
-            if (p.pos_to_token) hipLaunchKernelGGL((per_channel_cast_fp8in_kernel<NPT, true, LANES>), grid, block, 0, stream, TK_PC_LAUNCH_ARGS(p));
-            else hipLaunchKernelGGL((per_channel_cast_fp8in_kernel<NPT, false, LANES>), grid, block, 0, stream, TK_PC_LAUNCH_ARGS(p));
+#define TK_PC_FP8_LAUNCH(SRC, T) \
+    hipLaunchKernelGGL((per_channel_cast_fp8in_kernel<NPT, SRC, LANES, T>), grid, block, 0, stream, TK_PC_LAUNCH_ARGS(p))
+            if (!p.pos_to_token) TK_PC_FP8_LAUNCH(PC_IN_ORDER, false);
+            else if (LANES == 32 && gather_far(p)) TK_PC_FP8_LAUNCH(LANES == 32 ? PC_GATHERED_FAR : PC_GATHERED, false);
+            else if (LANES == 32 && gather_once(p)) TK_PC_FP8_LAUNCH(LANES == 32 ? PC_GATHERED_ONCE : PC_GATHERED, false);
+            else if ((int64_t)p.M * p.K <= kPcThrough) TK_PC_FP8_LAUNCH(PC_GATHERED, true);
+            else TK_PC_FP8_LAUNCH(PC_GATHERED, false);
+#undef TK_PC_FP8_LAUNCH
             return;
         }
     }
@@ -475,7 +567,10 @@ template <int MODE, int NPT>
 static void launch_per_channel_2(const PerChannelParams &p, bool transpose, hipStream_t stream) {
     const int wide_cols = MODE == PC_E4M3 && !transpose ? 512 : 256;
     const int64_t tiles = (int64_t)((p.M + kPcTileM - 1) / kPcTileM) * ((p.K + wide_cols - 1) / wide_cols);
-    if (tiles < wide_tiles_from<MODE>(transpose, p.pos_to_token != nullptr)) launch_per_channel_3<MODE, NPT, 16>(p, transpose, stream);
+    bool narrow = tiles < wide_tiles_from<MODE>(transpose, p.pos_to_token != nullptr);
+    if (MODE == PC_E4M3 && !transpose && p.pos_to_token && aligned_to(p.x, 16) && aligned_to(p.out, 16))
+        narrow = !gather_far(p) && (narrow || gather_repeats(p.num_tokens, p.M));
+    if (narrow) launch_per_channel_3<MODE, NPT, 16>(p, transpose, stream);
     else launch_per_channel_3<MODE, NPT, 32>(p, transpose, stream);
 }
 
