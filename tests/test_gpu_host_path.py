@@ -135,6 +135,20 @@ def test_expanded_ops(monkeypatch, tokens, hidden):
 
 
 @pytest.mark.gpu
+def test_uninitialised_memory_is_filled_where_torch_is_told_to():
+    """Three rows of column-major scales are stored in columns of four: the fourth is written by nobody but torch.empty."""
+    import tilekernels_amd as tk
+    x = _x(3, 512)
+    torch.use_deterministic_algorithms(True)
+    try:
+        _, sf = tk.quant.per_token_cast(x, 'e4m3', 128, use_tma_aligned_col_major_sf=True)
+    finally:
+        torch.use_deterministic_algorithms(False)
+    stored = torch.as_strided(sf, (4, 4), (4, 1))
+    assert bool(stored[:, 3].isnan().all()) and torch.equal(stored[:, :3].T, sf)
+
+
+@pytest.mark.gpu
 def test_calls_the_python_code_takes(monkeypatch):
     """Empty inputs, modes, number types and options the native path leaves alone: the result is that of the Python code."""
     import tilekernels_amd as tk

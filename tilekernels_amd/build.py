@@ -53,7 +53,7 @@ def _build_host() -> None:
     cmd = [os.environ.get('CXX', 'g++'), '-O2', '-std=c++17', '-fPIC', '-shared', '-Wall', '-D__HIP_PLATFORM_AMD__=1', '-DUSE_ROCM=1',
            f'-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}', f'-I{root}/include', f'-I{sysconfig.get_paths()["include"]}',
            '-I/opt/rocm/include', os.path.join(CSRC, 'host.cpp'), '-o', HOST_PATH,
-           f'-L{LIB_DIR}', '-l:libtk_quant.so', f'-L{root}/lib', '-lc10', '-lc10_hip', '-ltorch_cpu', '-ltorch_python', '-Wl,-rpath,$ORIGIN']
+           f'-L{LIB_DIR}', '-l:libtk_quant.so', f'-L{root}/lib', '-lc10', '-lc10_hip', '-ltorch_cpu', '-ltorch_hip', '-ltorch_python', '-Wl,-rpath,$ORIGIN']
     r = subprocess.run(cmd, capture_output=True, text=True)
     if r.returncode != 0:
         raise RuntimeError(f'the build of {HOST_PATH} failed:\n{r.stderr}')

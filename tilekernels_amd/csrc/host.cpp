@@ -11,6 +11,7 @@
 
 #include <ATen/ATen.h>
 #include <ATen/PythonTorchFunctionTLS.h>
+#include <ATen/hip/EmptyTensor.h>
 #include <c10/core/impl/LocalDispatchKeySet.h>
 #include <c10/core/impl/TorchDispatchModeTLS.h>
 #include <c10/hip/HIPFunctions.h>
@@ -126,8 +127,21 @@ int64_t align(int64_t a, int64_t b) { return ceil_div(a, b) * b; }
 
 void *stream() { return static_cast<void *>(c10::hip::getCurrentHIPStream().stream()); }
 
+// torch.empty on the device of `like`, without the dispatcher (0.70 -> 0.35 us, and up to eight of them in a call), which need_plain_thread()
+// and tensor() have found nothing to do for.  Where torch is told to fill what it leaves uninitialised, it does so.
 at::Tensor empty(at::IntArrayRef sizes, at::ScalarType type, const at::Tensor &like) {
-    return at::empty(sizes, at::TensorOptions().dtype(type).device(like.device()));
+    const at::Context &context = at::globalContext();
+    if (context.deterministicAlgorithms() && context.deterministicFillUninitializedMemory())
+        return at::empty(sizes, at::TensorOptions().dtype(type).device(like.device()));
+    return at::detail::empty_cuda(sizes, type, like.device(), c10::nullopt);
+}
+
+// The first rows x cols elements of a matrix of `ld` x cols that is stored column after column.
+at::Tensor empty_columns(int64_t rows, int64_t cols, int64_t ld, at::ScalarType type, const at::Tensor &like) {
+    at::Tensor t = empty({cols, ld}, type, like);
+    const int64_t sizes[] = {rows, cols}, strides[] = {1, ld};
+    t.unsafeGetTensorImpl()->set_sizes_and_strides(c10::IntArrayRef(sizes), c10::IntArrayRef(strides));
+    return t;
 }
 
 at::Tensor empty_codes(int64_t rows, int64_t cols, int fmt, const at::Tensor &like) {
@@ -153,7 +167,7 @@ struct Scales {
         // columns are stored one after the other, padded to 16 bytes: four fp32 scales, or four words of four exponent bytes
         const bool packed = layout == TK_SF_COL_UE8M0;
         const int64_t cols = packed ? ceil_div(nk, 4) : nk, rows = align(nm, 4);
-        out = empty({cols, rows}, packed ? at::kInt : at::kFloat, like).as_strided({nm, cols}, {1, rows});
+        out = empty_columns(nm, cols, rows, packed ? at::kInt : at::kFloat, like);
         ld = packed ? rows * 4 : rows;
     }
 };
@@ -420,7 +434,7 @@ PyObject *get_fused_mapping(PyObject *const *a) {
             counts_host = counts.cpu();
             int64_t rows = 0;
             for (int e = 0; e < experts; ++e) rows += counts_host.const_data_ptr<int32_t>()[e];
-            for (at::Tensor *t : {&pos_to_expert, &pos_to_token, &pos_to_token_topk}) *t = t->slice(0, 0, rows);
+            for (at::Tensor *t : {&pos_to_expert, &pos_to_token, &pos_to_token_topk}) t->unsafeGetTensorImpl()->set_sizes_contiguous({rows});
         }
     }
     PyObject *list = PyList_New(sync ? experts : 0);
@@ -455,7 +469,7 @@ PyObject *expand_to_fused(PyObject *const *a) {
         int64_t ld = 0;
         if (x_sf) {
             ld = col_major ? align(rows, 4) : sf_cols;
-            out_sf = col_major ? empty({sf_cols, ld}, x_sf->scalar_type(), x).as_strided({rows, sf_cols}, {1, ld})
+            out_sf = col_major ? empty_columns(rows, sf_cols, ld, x_sf->scalar_type(), x)
                                : empty({rows, sf_cols}, x_sf->scalar_type(), x);
         }
         launched(tk_expand_to_fused(x.const_data_ptr(), tokens, hidden * x.element_size(), t2p.const_data_ptr<int32_t>(), (int)t2p.size(1),
