@@ -213,3 +213,42 @@ def test_mapping_of_a_list_between_16_byte_boundaries(T, K, E):
         for name, a, b in zip(('pos_to_expert', 'pos_to_token', 'pos_to_token_topk', 'token_topk_to_pos', 'expert_start', 'expert_end',
                                'num_tokens_per_expert'), got[:7], want):
             assert_same(a, b, name)
+
+
+# one launch, two around a table, three; behind an idle stream and behind work that takes longer than the wait in a loop
+@pytest.mark.parametrize('busy', [False, True])
+@pytest.mark.parametrize('T,K,E', [(1, 1, 1), (700, 6, 512), (11000, 8, 32), (90, 5, 700), (0, 4, 8)])
+def test_segment_lengths_on_the_host(T, K, E, busy):
+    from tilekernels_amd import _ffi
+    tk = _tk()
+    g = torch.Generator().manual_seed(T + E)
+    idx = torch.randint(-1, E, (T, K), generator=g)
+    want = torch_ref.get_fused_mapping(idx, E, 16) if T else None
+    idx = idx.cuda()
+    if busy:
+        torch.cuda._sleep(5_000_000)
+    got = tk.moe.get_fused_mapping(idx, E, 0, 16)
+    assert got[7] == got[6].tolist() and got[0].shape[0] == sum(got[7])
+    if T == 0:
+        return
+    for a, b in zip(got[:7], want[:7]):
+        assert torch.equal(a.cpu(), b)
+    lib, i32 = _ffi.load(), dict(dtype=torch.int32, device='cuda')
+    rows = (T * K + 15 * E) // 16 * 16
+    out = [torch.empty((max(rows, T * K, E),), **i32) for _ in range(7)]
+    ws = torch.empty((lib.tk_fused_mapping_workspace_bytes(T, K, E) // 4,), **i32)
+    host = torch.empty((E,), dtype=torch.int32, pin_memory=True)
+
+    def call(counts, stream):
+        return lib.tk_get_fused_mapping_with_counts(idx.data_ptr(), T, K, E, 16, rows, *(t.data_ptr() for t in out), ws.data_ptr(), ws.numel() * 4,
+                                                    counts, stream)
+    if busy:
+        torch.cuda._sleep(5_000_000)
+    assert call(host.data_ptr(), _ffi.current_stream(idx.device)) == 0
+    assert host.tolist() == got[7]
+    assert call(None, _ffi.current_stream(idx.device)) == -1                    # null pointer
+    graph = torch.cuda.CUDAGraph()
+    torch.cuda.synchronize()
+    with torch.cuda.graph(graph):
+        rc = call(host.data_ptr(), torch.cuda.current_stream().cuda_stream)
+    assert rc == -7                                                             # nothing runs during a capture: no lengths to wait for

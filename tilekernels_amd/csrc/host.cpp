@@ -424,14 +424,18 @@ PyObject *get_fused_mapping(PyObject *const *a) {
         counts = empty({experts}, at::kInt, idx);
         const int64_t words = std::max<int64_t>(tk_fused_mapping_workspace_bytes(tokens, (int)topk, experts), 4) / 4;
         const at::Tensor workspace = empty({words}, at::kInt, idx);
-        launched(tk_get_fused_mapping(idx.const_data_ptr<int64_t>(), tokens, (int)topk, experts, alignment, expanded,
-                                      pos_to_expert.mutable_data_ptr<int32_t>(), pos_to_token.mutable_data_ptr<int32_t>(),
-                                      pos_to_token_topk.mutable_data_ptr<int32_t>(), token_topk_to_pos.mutable_data_ptr<int32_t>(),
-                                      expert_start.mutable_data_ptr<int32_t>(), expert_end.mutable_data_ptr<int32_t>(),
-                                      counts.mutable_data_ptr<int32_t>(), workspace.mutable_data_ptr(), words * 4, stream()),
-                 "tk_get_fused_mapping");
-        if (sync) {
-            counts_host = counts.cpu();
+        const auto launch = [&](auto f, auto... more) {
+            return f(idx.const_data_ptr<int64_t>(), tokens, (int)topk, experts, alignment, expanded, pos_to_expert.mutable_data_ptr<int32_t>(),
+                     pos_to_token.mutable_data_ptr<int32_t>(), pos_to_token_topk.mutable_data_ptr<int32_t>(),
+                     token_topk_to_pos.mutable_data_ptr<int32_t>(), expert_start.mutable_data_ptr<int32_t>(),
+                     expert_end.mutable_data_ptr<int32_t>(), counts.mutable_data_ptr<int32_t>(), workspace.mutable_data_ptr(), words * 4, more...,
+                     stream());
+        };
+        if (!sync) {
+            launched(launch(tk_get_fused_mapping), "tk_get_fused_mapping");
+        } else {
+            counts_host = at::empty({experts}, at::TensorOptions().dtype(at::kInt).pinned_memory(true));
+            launched(launch(tk_get_fused_mapping_with_counts, counts_host.mutable_data_ptr<int32_t>()), "tk_get_fused_mapping_with_counts");
             int64_t rows = 0;
             for (int e = 0; e < experts; ++e) rows += counts_host.const_data_ptr<int32_t>()[e];
             for (at::Tensor *t : {&pos_to_expert, &pos_to_token, &pos_to_token_topk}) t->unsafeGetTensorImpl()->set_sizes_contiguous({rows});
