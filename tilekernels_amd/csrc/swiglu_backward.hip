@@ -7,7 +7,7 @@
 //          x_grad codes[R, 2H] E4M3 with scales [R, 2H/N] fp32, quantised from the fp32 gradient
 //          weight_grad[T*K] fp32   = sum_c grad_out * silu(g) * u per routed row, 0 for unrouted pairs
 //
-// A workgroup owns RPW whole rows: its W waves stand side by side, 512 columns each, and step along
+// A workgroup owns RPW (one or two) whole rows: its W waves stand side by side, 512 columns each, and step along
 // the row together, so the row's dot product for weight_grad is finished inside the workgroup (lane
 // partials, a wave reduction, one LDS exchange) and written exactly once, in a fixed order.  A lane
 // holds 8 consecutive gate columns and the 8 matching up columns: two 8-byte code loads, one 16-byte
@@ -200,7 +200,17 @@ __global__ __launch_bounds__(64 * kBwdMaxWaves) void swiglu_backward_kernel(TK_B
     }
 }
 
-constexpr int kBwdRowsPerGroup = 2;
+// Whether a workgroup takes one row or two.  With two, a wave has twice the loads in flight but holds 96 to 106 registers: four or five
+// waves per SIMD, of workgroups as many waves wide as the row has strips, so that from five strips on only one or two workgroups fit a CU
+// with waves to spare.  With one it is 60 registers and eight waves.  us on MI355X, two rows / one:
+//   five strips and more: [3072, 2560] 24.3 / 18.9, [10112, 2560] 65.1 / 49.2, [10112, 3072] 70.1 / 59.6, [10112, 7168] 164.8 / 160.8, [39000, 4096] 326 / 321
+//   launches that two rows to a workgroup leave short of waves: [1130, 512] 4.3 / 3.7, [1130, 1024] 5.8 / 5.0, [2130, 1024] 7.4 / 7.0, [1130, 1536]
+//   7.1 / 6.0, but [2130, 1536] 8.9 / 9.0, [4130, 1024] 9.5 / 10.6, [6130, 512] 7.8 / 9.4, [9216, 896] 20.5 / 20.9
+//   four whole strips: [2130, 2048] 11.5 / 11.2, [6130, 2048] 27.1 / 26.8, [9130, 2048] 38.0 / 38.2, [25000, 2048] 108.0 / 110.1
+static bool backward_single_rows(int64_t R, int64_t H) {
+    const int64_t strips = (H + kStripCols - 1) / kStripCols;
+    return strips > 4 || R * strips <= 5000 || (H == 4 * kStripCols && R <= 6144);
+}
 
 struct BackwardArgs {
     const uint8_t *x;
@@ -219,9 +229,8 @@ struct BackwardArgs {
     int64_t num_weights;
 };
 
-template <int N, bool CLAMP>
-static hipError_t launch_backward(const BackwardArgs &a, hipStream_t stream) {
-    constexpr int RPW = kBwdRowsPerGroup;
+template <int N, bool CLAMP, int RPW>
+static hipError_t launch_backward_2(const BackwardArgs &a, hipStream_t stream) {
     const int strips = (a.H + kStripCols - 1) / kStripCols;
     const int waves = backward_waves(strips);
     const int blocks = a.R > 0 ? (a.R + RPW - 1) / RPW : 1;
@@ -235,6 +244,11 @@ static hipError_t launch_backward(const BackwardArgs &a, hipStream_t stream) {
     else TK_BWD_LAUNCH(false);
 #undef TK_BWD_LAUNCH
     return hipGetLastError();
+}
+
+template <int N, bool CLAMP>
+static hipError_t launch_backward(const BackwardArgs &a, hipStream_t stream) {
+    return backward_single_rows(a.R, a.H) ? launch_backward_2<N, CLAMP, 1>(a, stream) : launch_backward_2<N, CLAMP, 2>(a, stream);
 }
 
 }  // namespace tk
