@@ -457,6 +457,21 @@ def test_smallest_shapes():
     f.check(300)
 
 
+# (rows, columns) in and around the ranges of the tile shapes: 256 columns by 1024 threads, 512 columns, 256 columns by 512 threads (bf16 to
+# E2M1), and 128 columns; whole and with edge tiles below and, where columns allow it, to the right
+@pytest.mark.parametrize('block', [(128, 128), (32, 32), (128, 32), (32, 128)])
+@pytest.mark.parametrize('fmt', ['e4m3', 'e2m1'])
+@pytest.mark.parametrize('dtype', [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize('M,K', [(3072, 2048), (3841, 1280), (4096, 2048), (4481, 2048), (8192, 2048), (8193, 2048), (16385, 1280), (16640, 1024), (900, 704)])
+def test_per_block_cast_tile_shapes(M, K, dtype, fmt, block):
+    tk = _tk()
+    x = _randn((M, K), dtype, M + K, 2.0)
+    want = torch_ref.cast(x, fmt, block)
+    got = tk.quant.per_block_cast(x.cuda(), fmt, block)
+    assert_same(got[0], want[0], 'codes')
+    assert_same(got[1], want[1], 'sf')
+
+
 @pytest.mark.parametrize('fmt', ['e4m3', 'e2m1'])
 def test_per_block_cast_into_a_buffer_that_is_only_8_byte_aligned(fmt):
     """The wide tiles of mid-sized matrices store 16 codes per lane; the entry point only asks for 8-byte alignment of the codes."""

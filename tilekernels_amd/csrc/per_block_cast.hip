@@ -1,6 +1,6 @@
 // Per-block (bm x bk, bm/bk in {32, 128}) block-scaled cast to E4M3 / E2M1 for gfx950.
 //
-// A workgroup owns one tile of 128 rows x TW columns (TW = 128 with 512 threads, or 512 with 1024 threads: see the
+// A workgroup owns one tile of 128 rows x TW columns (TW = 128 or 256 with 512 threads, 256 or 512 with 1024 threads: see the
 // table at the launch code), i.e. 1 to 64 scale blocks.  With TW = 128, thread (t, c) = (tid / 16, tid % 16) holds
 // the 8 elements at columns 8c.. of rows t, t+32, t+64, t+96: four 16-byte streaming loads per thread (bf16), all
 // issued up front; the tile stays in registers between the amax reduction and the conversion, so HBM is read once.  The amax of a block is
@@ -16,7 +16,7 @@
 namespace tk {
 
 constexpr int kBlockTile = 128;
-constexpr int kPerBlockThreads = 512, kWideTile = 512, kWideThreads = 1024;   // the two tile shapes: see the table at the launch code
+constexpr int kPerBlockThreads = 512, kMidTile = 256, kWideTile = 512, kWideThreads = 1024;   // the tile shapes: see the table at the launch code
 
 struct PerBlockParams {
     const void *x;
@@ -40,8 +40,9 @@ struct PerBlockParams {
 // TW: columns of a tile (128, 256 or 512); a tile is 128 rows x TW columns.
 // THREADS: threads per tile.
 // FULL: the tile lies wholly inside the matrix, so no bounds checks are compiled in.
+// FULL_GRID: so do all tiles of the launch.
 // FEW: of a matrix of few rows, see the launch code.
-template <typename InT, int FMT, int BM, int BK, int TW, int THREADS, bool FULL, bool FEW = false>
+template <typename InT, int FMT, int BM, int BK, int TW, int THREADS, bool FULL, bool FULL_GRID, bool FEW = false>
 __device__ __forceinline__ void per_block_cast_tile(const PerBlockParams &p, uint8_t *xchg) {
     constexpr int LPR = TW / 8;                                      // lanes along a row of the tile
     constexpr int SUBM = kBlockTile / BM, SUBK = TW / BK;            // scale blocks per tile
@@ -136,14 +137,15 @@ __device__ __forceinline__ void per_block_cast_tile(const PerBlockParams &p, uin
     }
     if (p.mode == TK_SF_ONLY) return;
 
-    // Wide tiles: the two lanes that hold 16 neighbouring columns exchange the codes of two row slots, so that each stores
-    // 16 consecutive codes of one row with one instruction: half as many store instructions, each twice as wide.  A launch of
-    // wide tiles fits the GPU in one round, all its workgroups finish loading at about the same time (measured: the last load
-    // of every workgroup of [7168, 2048] arrives between 3.4 and 4.7 us after the start) and the rest of the launch is one
-    // burst of stores, which drains faster in fewer, wider instructions: bf16 [7168, 2048] -> E4M3 8.54 -> 8.20 us,
-    // [4096, 4096] 9.22 -> 8.66, [8192, 2048] 9.94 -> 9.07.  (128-column tiles, whose workgroups finish at different times so
-    // that loads and stores overlap, do not gain: [8192, 4096] 17.43 -> 17.65 us.)
-    constexpr bool PAIRED = FULL && TW == kWideTile && NI % 2 == 0;
+    // The two lanes that hold 16 neighbouring columns exchange the codes of two row slots, so that each stores 16 consecutive codes of
+    // one row with one instruction: half as many store instructions, each twice as wide.  A launch of wide tiles fits the GPU in one
+    // round, all its workgroups finish loading at about the same time (measured: the last load of every workgroup of [7168, 2048]
+    // arrives between 3.4 and 4.7 us after the start) and the rest of the launch is one burst of stores, which drains faster in fewer,
+    // wider instructions: bf16 [7168, 2048] -> E4M3 8.54 -> 8.20 us, [4096, 4096] 9.22 -> 8.66, [8192, 2048] 9.94 -> 9.07.
+    // (128-column tiles gain to E2M1 where the matrix is ragged, bf16 [3666, 576] 3.38 -> 3.09, [7830, 960] 6.0 -> 5.5; not where all tiles
+    // are whole, [1536, 2048] 2.92 -> 3.23, nor fp32, [2560, 2048] 6.45 -> 6.54, nor, of more than some 1000 tiles, E4M3, whose workgroups
+    // finish loading at different times so that loads and stores overlap: [3589, 6144] 12.54 -> 12.75.)
+    constexpr bool PAIRED = !FEW && NI % 2 == 0 && (TW > kBlockTile || (!FULL_GRID && FMT == TK_E2M1 && std::is_same<InT, bf16_t>::value));
     if constexpr (PAIRED) {
         const bool odd = threadIdx.x & 1;
 #pragma unroll
@@ -157,7 +159,9 @@ __device__ __forceinline__ void per_block_cast_tile(const PerBlockParams &p, uin
             const u32x2 send = odd ? a : b;
             const u32x2 recv = {dpp_u32<kDppXor1>(send.x), FMT == TK_E4M3 ? dpp_u32<kDppXor1>(send.y) : 0u};
             const u32x2 lo = odd ? recv : a, hi = odd ? b : recv;
-            uint8_t *out_row = p.out + (int64_t)(row0 + TR * (i + (odd ? 1 : 0))) * out_ld;
+            const int row = row0 + TR * (i + (odd ? 1 : 0));
+            if (!FULL && (!col_ok || row >= p.M)) continue;      // (K is a multiple of 64: both lanes have columns, or neither)
+            uint8_t *out_row = p.out + (int64_t)row * out_ld;
             if (FMT == TK_E4M3) st_stream16(out_row + (col & ~15), u32x4{lo.x, lo.y, hi.x, hi.y});
             else st_stream8(out_row + ((col & ~15) >> 1), u32x2{lo.x, hi.x});
         }
@@ -185,14 +189,14 @@ __global__ __launch_bounds__(THREADS) void per_block_cast_kernel(TK_PB_KERNEL_AR
     constexpr int XB = FEW ? 0 : Raw8<InT>::kXchgBytes;
     __shared__ __attribute__((aligned(16))) uint8_t xchg[XB ? THREADS * XB : 16];      // (one for both kinds of tile)
     if constexpr (FULL_GRID) {
-        per_block_cast_tile<InT, FMT, BM, BK, TW, THREADS, true>(p, xchg);
+        per_block_cast_tile<InT, FMT, BM, BK, TW, THREADS, true, true>(p, xchg);
     } else if constexpr (FEW) {
-        per_block_cast_tile<InT, FMT, BM, BK, TW, THREADS, false, true>(p, xchg);
+        per_block_cast_tile<InT, FMT, BM, BK, TW, THREADS, false, false, true>(p, xchg);
     } else {
         if (((int)blockIdx.y + 1) * kBlockTile <= p.M && ((int)blockIdx.x + 1) * TW <= p.K)
-            per_block_cast_tile<InT, FMT, BM, BK, TW, THREADS, true>(p, xchg);
+            per_block_cast_tile<InT, FMT, BM, BK, TW, THREADS, true, false>(p, xchg);
         else
-            per_block_cast_tile<InT, FMT, BM, BK, TW, THREADS, false>(p, xchg);
+            per_block_cast_tile<InT, FMT, BM, BK, TW, THREADS, false, false>(p, xchg);
     }
 }
 
@@ -203,11 +207,18 @@ __global__ __launch_bounds__(THREADS) void per_block_cast_kernel(TK_PB_KERNEL_AR
 //   128 x 512, 512 threads (16 rows/thread)    6.31         8.87         9.82        16.59        20.37        58.8
 //   128 x 256, 1024 threads                    4.72         9.30        10.57        16.39        18.06
 // (128 x 128 with 256 threads: 9.4 at [7168,2048], with 1024: 9.8.)  A wave of a 512-column tile reads 1 KB of one
-// row per load instruction instead of 256 bytes of four rows, which pays while the matrix has too few 128 x 128
-// tiles to fill the GPU several times over (here 896 and 1024 tiles: 3.5 and 4 workgroups per CU) and costs where it
-// has many, or so few that whole CUs would stay empty.  The wide tile is used inside that window (with the paired
-// 16-byte stores: [7168,2048] 8.24).  fp32 input, same window: [7168,2048] 13.58 -> 12.31, [8192,4096] 30.16 -> 29.96.
-constexpr int64_t kWideMinTiles = 512, kWideMaxTiles = 1280;     // in 128 x 128 tiles
+// row per load instruction instead of 256 bytes of four rows.  Its workgroup of 1024 threads at 96 registers has a CU to itself, so
+// that the launch is as long as the CU with the most tiles: the wide tile pays where there are at most 256 of them and not much fewer
+// than 140, and 256 columns with 1024 threads where there are 192 to 256 of those.  us, 128 / 256 (1024 threads) / 512 columns:
+//   E4M3 bf16 [3072,2048] 4.85 / 4.79 / 6.30, [3584,2048] 5.30 / 4.97 / 6.50, [4096,2048] 5.66 / 5.22 / 6.62, [2100,4096] 5.94 / 6.46 / 6.47,
+//   [4608,2048] 6.78 / 7.61 / 6.75, [6144,2048] 7.82 / 8.33 / 7.44, [7168,2048] 8.90 / 9.17 / 8.29, [8192,2048] 9.74 / 10.12 / 9.23, [8704,2048]
+//   10.79 / 11.83 / 11.93, [9044,2048] 11.0 / 12.1 / 13.3, [4100,4096] 9.90 / 10.5 / 10.8, [5000,4096] 11.9 / 12.5 / 13.75
+//   fp32 [2560,2048] 6.39 / 6.17 / 8.38, [4096,2048] 8.39 / 7.61 / 9.03, [4608,2048] 9.74 / 10.90 / 9.30, [8192,2048] 14.98 / 15.22 / 13.98,
+//   [9044,2048] 16.5 / 18.4 / 20.0
+// More tiles than that to E2M1, whose stores of a lane's 8 codes are 4 bytes in a 128-column tile and 8 in a wider one, go with 256 columns
+// and 512 threads (bf16, 128 / 256 columns: [9044,2048] 10.9 / 10.6, [12352,2048] 13.6 / 12.7, [5000,4096] 11.7 / 10.6, [3000,7168] 12.0 / 10.9,
+// [16384,7168] 48.5 / 45.8, but [8704,2048] 10.0 / 10.35; fp32 [16384,7168] 86.5 / 82.6, but [8192,8192] 47.6 / 53.7).
+constexpr int64_t kWideMinTiles = 561, kWideMaxTiles = 1024, kMidMinTiles = 384, kMidMinTilesF32 = 300, kMidMaxTiles = 512;     // in 128 x 128 tiles
 
 template <typename InT, int FMT, int BM, int BK, int TW, int THREADS>
 static void launch_per_block_3(const PerBlockParams &p, hipStream_t stream) {
@@ -230,10 +241,22 @@ static void launch_per_block_3(const PerBlockParams &p, hipStream_t stream) {
 template <typename InT, int FMT, int BM, int BK>
 static void launch_per_block_2(const PerBlockParams &p, hipStream_t stream) {
     const int64_t tiles = (int64_t)p.tiles_m * p.tiles_k;
-    if (p.K % kWideTile == 0 && tiles >= kWideMinTiles && tiles <= kWideMaxTiles)
+    constexpr bool F32 = std::is_same<InT, float>::value;
+    if (p.K % kWideTile == 0 && tiles >= kWideMinTiles && tiles <= kWideMaxTiles) {
         launch_per_block_3<InT, FMT, BM, BK, kWideTile, kWideThreads>(p, stream);
-    else
-        launch_per_block_3<InT, FMT, BM, BK, kBlockTile, kPerBlockThreads>(p, stream);
+        return;
+    }
+    if (p.K % kMidTile == 0 && tiles >= (F32 ? kMidMinTilesF32 : kMidMinTiles) && tiles <= kMidMaxTiles) {
+        launch_per_block_3<InT, FMT, BM, BK, kMidTile, kWideThreads>(p, stream);
+        return;
+    }
+    if constexpr (FMT == TK_E2M1 && !F32) {
+        if (p.K % kMidTile == 0 && tiles > kWideMaxTiles) {
+            launch_per_block_3<InT, FMT, BM, BK, kMidTile, kPerBlockThreads>(p, stream);
+            return;
+        }
+    }
+    launch_per_block_3<InT, FMT, BM, BK, kBlockTile, kPerBlockThreads>(p, stream);
 }
 
 template <typename InT, int FMT>
