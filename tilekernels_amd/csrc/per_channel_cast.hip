@@ -62,6 +62,12 @@ struct PerChannelParams {
 #define TK_PC_LAUNCH_ARGS(p) \
     (p).x, (p).out, (p).out_sf, (p).x_sf, (p).pos_to_token, (p).num_tokens, (p).K, (p).M, (p).tiles_k, (p).round_sf, (p).use_clamp, (p).clamp
 
+// What bounds the SwiGLU form is half memory, half arithmetic: 1077 vector instructions per lane (64 elements), 128 of them exponentials and
+// reciprocals.  They were 1402 while the clamp was compiled in for every call (at infinity where there was none), the rounded
+// activations were unpacked again for their maxima, registers were cleared for lanes beyond the matrix, and every row's address was a
+// product.  us on MI355X, before / after, SwiGLU and bf16 operand together: [768, 2 x 3456] and [768, 3328] 9.3 / 8.65, [2560, 2 x 2560] and
+// [2560, 4096] 16.1 / 15.1, [8064, 2 x 2048] and [8064, 4096] 35.0 / 34.3.  (With fewer workgroups resident, so that one's stores meet
+// another's loads: 39 to 42.)
 template <int MODE> struct PcRaw { typedef Raw8<bf16_t> type; };
 template <> struct PcRaw<PC_E4M3> { typedef Raw8<e4m3in_t> type; };
 template <> struct PcRaw<PC_F32> { typedef Raw8<float> type; };
@@ -76,7 +82,8 @@ __device__ __forceinline__ uint32_t pack_bf16x2(float a, float b) {
     return __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2{a, b}), bf16x2));
 }
 
-template <int MODE, int NPT, bool TRANS, bool GATHER, int LANES>
+// CLAMP: of the SwiGLU's inputs.
+template <int MODE, int NPT, bool TRANS, bool GATHER, int LANES, bool CLAMP = false>
 __global__ __launch_bounds__(LANES * kPcParts, 4) void per_channel_cast_kernel(TK_PC_KERNEL_ARGS) {
     TK_PC_KERNEL_UNPACK;
     constexpr int kPcTileK = LANES * 8, kPcThreads = LANES * kPcParts;
@@ -111,103 +118,105 @@ __global__ __launch_bounds__(LANES * kPcParts, 4) void per_channel_cast_kernel(T
     const bool rows_ok = tok0 < p.M;            // M is a multiple of 16: all 8 tokens of a lane or none
     const int64_t in_ld = MODE == PC_SWIGLU ? 2 * (int64_t)p.K : p.K;
 
-    // ---- load (and, for SwiGLU, activate) 8 tokens x 8 columns.  Whether a lane has anything to load
-    // does not depend on the token (M is a multiple of 16), so the loads sit in straight-line code
-    // under one branch; a gathered row with a negative index is read from row 0 and zeroed by value.
+    // ---- load (and, for SwiGLU, activate) 8 tokens x 8 columns.  No lane branches around its loads: one beyond the last token reads
+    // the last 8 tokens, whose scale block is its own or one that is not stored, one beyond the last column the last 8 columns.  (M is a
+    // multiple of 16, K of 8.)  A gathered row with a negative index is read from row 0 and zeroed by value.
+    const int tok_in = min(tok0, p.M - kPcRows), col_in = min(col, p.K - 8);
     Raw raw[kPcRows];
-#pragma unroll
-    for (int r = 0; r < kPcRows; ++r) raw[r].zero();
-    if (rows_ok && col_ok) {
-        if constexpr (MODE == PC_SWIGLU) {
-            // all sixteen loads of the lane go out before the first activation is evaluated (issuing them in batches of
-            // 4 or 2 tokens brings the kernel from 92 to 67 / 61 VGPRs and more waves per SIMD, but measured 18-19 us
-            // against 16.8 us for bf16 [8192, 4096])
-            Raw8<bf16_t> rg[kPcRows], ru[kPcRows];
-#pragma unroll
-            for (int r = 0; r < kPcRows; ++r) {
-                const uint16_t *xr = reinterpret_cast<const uint16_t *>(p.x) + (int64_t)(tok0 + r) * in_ld + col;
-                rg[r].load(xr);
-                vmem_issue_gap();
-                ru[r].load(xr + p.K);
-                vmem_issue_gap();
-            }
-            __builtin_amdgcn_sched_barrier(0);
-            // the clamp arguments lie beyond the preloaded ones: touched only now, behind the loads.
-            // No clamp = clamp at infinity, so there is no branch in the hot loop.
-            float clamp_arg = p.clamp;
-            int use_clamp = p.use_clamp;
-            asm volatile("" : "+s"(clamp_arg), "+s"(use_clamp));
-            const float cl = use_clamp ? clamp_arg : __builtin_inff();
-            const float lo = cl >= 0.0f ? -cl : cl;      // (a negative limit makes every element the limit, as the two-step form does)
-#pragma unroll
-            for (int r = 0; r < kPcRows; ++r) {
-                float g[8], u[8], a[8];
-                rg[r].get(g);
-                ru[r].get(u);
-#pragma unroll
-                for (int i = 0; i < 8; ++i) {
-                    g[i] = __builtin_fminf(g[i], cl);
-                    u[i] = __builtin_amdgcn_fmed3f(u[i], lo, cl);      // min(max(u, -cl), cl) in one instruction
-                    a[i] = silu_mul<bf16_t>(g[i], u[i]);
-                }
-                // the activation is rounded to bf16 before it is quantised, as in the reference
-                raw[r].w = u32x4{pack_bf16x2(a[0], a[1]), pack_bf16x2(a[2], a[3]), pack_bf16x2(a[4], a[5]), pack_bf16x2(a[6], a[7])};
-            }
-        } else {
-            // (the gather indices of all rows are asked for before the first row's data: a load whose address hangs on a loaded value
-            // waits for every load issued before it)
-            int gathered[kPcRows];
-            bool valid[kPcRows];
-            if constexpr (GATHER) {
-#pragma unroll
-                for (int r = 0; r < kPcRows; ++r) gathered[r] = p.pos_to_token[tok0 + r];
-            }
-#pragma unroll
-            for (int r = 0; r < kPcRows; ++r) {
-                int src = tok0 + r;
-                valid[r] = true;
-                if constexpr (GATHER) {
-                    src = gathered[r];
-                    valid[r] = src >= 0 && src < p.num_tokens;
-                    src = valid[r] ? src : 0;
-                }
-                if constexpr (MODE == PC_E4M3) {
-                    raw[r].load(reinterpret_cast<const uint8_t *>(p.x) + (int64_t)src * in_ld + col);
-                    vmem_issue_gap();
-                    raw[r].s = p.x_sf[(int64_t)src * (p.K >> 7) + (col >> 7)];
-                    vmem_issue_gap();
-                } else if constexpr (MODE == PC_F32) {
-                    raw[r].load(reinterpret_cast<const float *>(p.x) + (int64_t)src * in_ld + col);
-                    vmem_issue_gap();
-                } else {
-                    raw[r].load(reinterpret_cast<const uint16_t *>(p.x) + (int64_t)src * in_ld + col);
-                    vmem_issue_gap();
-                }
-            }
-            // (rows without a source are cleared once all loads are out: clearing a register a load is still to fill means waiting for it)
-            if constexpr (GATHER) {
-#pragma unroll
-                for (int r = 0; r < kPcRows; ++r)
-                    if (!valid[r]) raw[r].zero();
-            }
-        }
-    }
-
-    // ---- |x| maxima down this lane's 8 columns
-    float m[8];
+    float m[8];          // |x| maxima down this lane's 8 columns
 #pragma unroll
     for (int j = 0; j < 8; ++j) m[j] = 0.0f;
+    if constexpr (MODE == PC_SWIGLU) {
+        // all sixteen loads of the lane go out before the first activation is evaluated (issuing them in batches of
+        // 4 or 2 tokens brings the kernel from 92 to 67 / 61 VGPRs and more waves per SIMD, but measured 18-19 us
+        // against 16.8 us for bf16 [8192, 4096])
+        Raw8<bf16_t> rg[kPcRows], ru[kPcRows];
+        const uint16_t *xr = reinterpret_cast<const uint16_t *>(p.x) + tok_in * in_ld + col_in;
 #pragma unroll
-    for (int r = 0; r < kPcRows; ++r) {
-        float v[8];
-        raw[r].get(v);
+        for (int r = 0; r < kPcRows; ++r, xr += in_ld) {
+            rg[r].load(xr);
+            vmem_issue_gap();
+            ru[r].load(xr + p.K);
+            vmem_issue_gap();
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        float cl = 0.0f, lo = 0.0f;
+        if constexpr (CLAMP) {
+            // the clamp lies beyond the preloaded arguments: touched only now, behind the loads
+            cl = p.clamp;
+            asm volatile("" : "+s"(cl));
+            lo = cl >= 0.0f ? -cl : cl;      // (a negative limit makes every element the limit, as the two-step form does)
+        }
 #pragma unroll
-        for (int j = 0; j < 8; ++j) m[j] = __builtin_fmaxf(m[j], __builtin_fabsf(v[j]));
+        for (int r = 0; r < kPcRows; ++r) {
+            float g[8], u[8], a[8];
+            rg[r].get(g);
+            ru[r].get(u);
+#pragma unroll
+            for (int i = 0; i < 8; ++i) {
+                if constexpr (CLAMP) {
+                    g[i] = __builtin_fminf(g[i], cl);
+                    u[i] = __builtin_amdgcn_fmed3f(u[i], lo, cl);      // min(max(u, -cl), cl) in one instruction
+                }
+                a[i] = silu_mul<bf16_t>(g[i], u[i]);
+                m[i] = __builtin_fmaxf(m[i], __builtin_fabsf(a[i]));
+            }
+            // the activation is rounded to bf16 before it is quantised, as in the reference
+            raw[r].w = u32x4{pack_bf16x2(a[0], a[1]), pack_bf16x2(a[2], a[3]), pack_bf16x2(a[4], a[5]), pack_bf16x2(a[6], a[7])};
+        }
+        // the largest rounded magnitude is the rounded largest one
+        Raw8<bf16_t> rounded;
+        rounded.w = u32x4{pack_bf16x2(m[0], m[1]), pack_bf16x2(m[2], m[3]), pack_bf16x2(m[4], m[5]), pack_bf16x2(m[6], m[7])};
+        rounded.get(m);
+    } else {
+        // (the gather indices of all rows are asked for before the first row's data: a load whose address hangs on a loaded value
+        // waits for every load issued before it)
+        int gathered[kPcRows];
+        bool valid[kPcRows];
+        if constexpr (GATHER) {
+#pragma unroll
+            for (int r = 0; r < kPcRows; ++r) gathered[r] = p.pos_to_token[tok_in + r];
+        }
+#pragma unroll
+        for (int r = 0; r < kPcRows; ++r) {
+            int src = tok_in + r;
+            valid[r] = true;
+            if constexpr (GATHER) {
+                src = gathered[r];
+                valid[r] = src >= 0 && src < p.num_tokens;
+                src = valid[r] ? src : 0;
+            }
+            if constexpr (MODE == PC_E4M3) {
+                raw[r].load(reinterpret_cast<const uint8_t *>(p.x) + (int64_t)src * in_ld + col_in);
+                vmem_issue_gap();
+                raw[r].s = p.x_sf[(int64_t)src * (p.K >> 7) + (col_in >> 7)];
+                vmem_issue_gap();
+            } else if constexpr (MODE == PC_F32) {
+                raw[r].load(reinterpret_cast<const float *>(p.x) + (int64_t)src * in_ld + col_in);
+                vmem_issue_gap();
+            } else {
+                raw[r].load(reinterpret_cast<const uint16_t *>(p.x) + (int64_t)src * in_ld + col_in);
+                vmem_issue_gap();
+            }
+        }
+        // (rows without a source are cleared once all loads are out: clearing a register a load is still to fill means waiting for it)
+        if constexpr (GATHER) {
+#pragma unroll
+            for (int r = 0; r < kPcRows; ++r)
+                if (!valid[r]) raw[r].zero();
+        }
+#pragma unroll
+        for (int r = 0; r < kPcRows; ++r) {
+            float v[8];
+            raw[r].get(v);
+#pragma unroll
+            for (int j = 0; j < 8; ++j) m[j] = __builtin_fmaxf(m[j], __builtin_fabsf(v[j]));
+        }
+        // the tile is unpacked a second time after the scales are known; without this the compiler keeps
+        // all 64 unpacked values alive across the two barriers instead
+#pragma unroll
+        for (int r = 0; r < kPcRows; ++r) forget_unpacked(raw[r]);
     }
-    // the tile is unpacked a second time after the scales are known; without this the compiler keeps
-    // all 64 unpacked values alive across the two barriers instead
-#pragma unroll
-    for (int r = 0; r < kPcRows; ++r) forget_unpacked(raw[r]);
     {
         u32x4 *dst = reinterpret_cast<u32x4 *>(&part[run][hl * 8]);
         dst[0] = u32x4{f2u(m[0]), f2u(m[1]), f2u(m[2]), f2u(m[3])};
@@ -260,7 +269,8 @@ __global__ __launch_bounds__(LANES * kPcParts, 4) void per_channel_cast_kernel(T
             raw[4 * d + 3].get(v3);
 #pragma unroll
             for (int j = 0; j < 8; ++j) {
-                const int lo = __builtin_amdgcn_cvt_pk_fp8_f32(v0[j] * inv[j], v1[j] * inv[j], 0, false);
+                const float a = v0[j] * inv[j], b = v1[j] * inv[j];
+                const int lo = __builtin_amdgcn_cvt_pk_fp8_f32(a, b, (int)f2u(a), false);      // (any register serves as the half that the next one fills)
                 acc[j][d] = (uint32_t)__builtin_amdgcn_cvt_pk_fp8_f32(v2[j] * inv[j], v3[j] * inv[j], lo, true);
             }
         }
@@ -545,20 +555,22 @@ static void launch_per_channel_3(const PerChannelParams &a, bool transpose, hipS
     // (token tiles on x, so that successive workgroups write neighbouring pieces of the same transposed rows,
     // measured slower: 19.7 -> 21.1 us transposed, 17.4 -> 20.3 us with SwiGLU)
     const dim3 grid = MODE == PC_E4M3 ? dim3((unsigned)(tiles_m * p.tiles_k)) : dim3((unsigned)p.tiles_k, (unsigned)tiles_m);
-#define TK_PC_LAUNCH(T, G) \
-    hipLaunchKernelGGL((per_channel_cast_kernel<MODE, NPT, T, G, LANES>), grid, block, 0, stream, TK_PC_LAUNCH_ARGS(p))
+#define TK_PC_LAUNCH(T, ...) \
+    hipLaunchKernelGGL((per_channel_cast_kernel<MODE, NPT, T, __VA_ARGS__>), grid, block, 0, stream, TK_PC_LAUNCH_ARGS(p))
     if constexpr (MODE == PC_SWIGLU) {
-        if (transpose) TK_PC_LAUNCH(true, false);
-        else TK_PC_LAUNCH(false, false);
+        if (transpose && p.use_clamp) TK_PC_LAUNCH(true, false, LANES, true);
+        else if (transpose) TK_PC_LAUNCH(true, false, LANES);
+        else if (p.use_clamp) TK_PC_LAUNCH(false, false, LANES, true);
+        else TK_PC_LAUNCH(false, false, LANES);
     } else if constexpr (MODE == PC_F32) {   // checked before: no transposed output from fp32
-        if (p.pos_to_token) TK_PC_LAUNCH(false, true);
-        else TK_PC_LAUNCH(false, false);
+        if (p.pos_to_token) TK_PC_LAUNCH(false, true, LANES);
+        else TK_PC_LAUNCH(false, false, LANES);
     } else if (p.pos_to_token) {
-        if (transpose) TK_PC_LAUNCH(true, true);
-        else TK_PC_LAUNCH(false, true);
+        if (transpose) TK_PC_LAUNCH(true, true, LANES);
+        else TK_PC_LAUNCH(false, true, LANES);
     } else {
-        if (transpose) TK_PC_LAUNCH(true, false);
-        else TK_PC_LAUNCH(false, false);
+        if (transpose) TK_PC_LAUNCH(true, false, LANES);
+        else TK_PC_LAUNCH(false, false, LANES);
     }
 #undef TK_PC_LAUNCH
 }
