@@ -202,3 +202,28 @@ def test_swiglu_rows_that_share_one_gate_value(gate):
     want = torch_ref.swiglu_forward_and_per_token_cast(x, 'e4m3', 128)
     got = tk.quant.swiglu_forward_and_per_token_cast(x.cuda(), 'e4m3', 128)
     check_fused(got, want, H // 128, False, f'gate {gate} everywhere')
+
+
+@pytest.mark.parametrize('mode', [(False, False, False), (True, False, False), (True, True, True)], ids=lambda m: 'col%d-round%d-packed%d' % tuple(int(v) for v in m))
+@pytest.mark.parametrize('with_weights,clamp', [(False, None), (True, 1.0)])
+@pytest.mark.parametrize('R,H', [(1024, 1664), (1021, 1664), (1024, 3072), (1022, 3072), (1024, 2048), (1021, 2048), (640, 1408), (100, 4096)])
+def test_mostly_padding(R, H, with_weights, clamp, mode):
+    """Long runs of padding between few live rows, whose waves write zeros without a look at their data (here NaN), and shorter runs next to
+    live rows, which take the usual way; the first and the last row in and out of a run; a batch of nothing but padding."""
+    tk = _tk()
+    col, round_sf, packed = mode
+    g = torch.Generator().manual_seed(R + H)
+    x = (torch.randn((R, 2 * H), generator=g) * 2).to(torch.bfloat16)
+    w = torch.rand((R, 2), generator=g)
+    for rows in ([0, 1, 130, 400, R - 200], [50, 51, 52, 163, 300, R - 1], []):
+        rows = [r for r in rows if 0 <= r < R]
+        p2e = torch.full((R,), -1, dtype=torch.int32)
+        p2e[rows] = 3
+        ptt = torch.where(p2e >= 0, 2 * torch.arange(R, dtype=torch.int32) + 1, -1).to(torch.int32)
+        xm = x.clone()
+        xm[p2e < 0] = float('nan')
+        weights = (ptt, w) if with_weights else (None, None)
+        want = torch_ref.swiglu_forward_and_per_token_cast(x, 'e4m3', 128, *weights, p2e, col, round_sf, packed, swiglu_clamp_value=clamp)
+        dev = [t.cuda() if t is not None else None for t in weights]
+        got = tk.quant.swiglu_forward_and_per_token_cast(xm.cuda(), 'e4m3', 128, *dev, p2e.cuda(), col, round_sf, packed, swiglu_clamp_value=clamp)
+        check_fused(got, want, H // 128, packed, f'{rows}')

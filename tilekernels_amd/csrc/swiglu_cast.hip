@@ -250,6 +250,25 @@ __device__ __forceinline__ void swiglu_row_wave(SwigluParams p, int row0, int st
     }
 }
 
+// Zero codes for a wave's RPW pieces: non-temporal stores of 16 bytes that cover whole lines (512 bytes of one row by 32 lanes).
+template <int RPW, bool ROW, bool FULL>
+__device__ __forceinline__ void zero_dead_wave(const SwigluParams &p, int row0, int strip, int lane) {
+    const bool wide = RPW % 2 == 0 && (reinterpret_cast<uintptr_t>(p.out) & 15) == 0;
+#pragma unroll
+    for (int r = 0; r < RPW; r += 2) {
+        if (wide) {
+            const int piece = r + (lane >> 5), row = row0 + (ROW ? 0 : piece), col = (strip + (ROW ? piece : 0)) * kStripCols + (lane & 31) * 16;
+            if (FULL || (row < p.R && col < p.H)) __builtin_nontemporal_store(u32x4{0u, 0u, 0u, 0u}, reinterpret_cast<u32x4 *>(p.out + (int64_t)row * p.H + col));
+            continue;
+        }
+#pragma unroll
+        for (int q = r; q < r + 2 && q < RPW; ++q) {
+            const int row = row0 + (ROW ? 0 : q), col = (strip + (ROW ? q : 0)) * kStripCols + lane * 8;
+            if (FULL || (row < p.R && col < p.H)) __builtin_nontemporal_store(u32x2{0u, 0u}, reinterpret_cast<u32x2 *>(p.out + (int64_t)row * p.H + col));
+        }
+    }
+}
+
 // Tile shapes (a wave always holds RPW pieces of 512 output columns, each with its gate and its up half):
 //   T_ROW     (row-major scales, H a multiple of RPW*512): W rows x (RPW*512) columns, one row per wave.  The RPW*4
 //             scales a wave produces are neighbours in the scale row, so the wave stores them itself as one
@@ -395,17 +414,39 @@ __global__ __launch_bounds__(TILE == T_ROW ? 64 * kMaxWideWaves : kThreads) void
 #pragma unroll
         for (int r = 0; r < RPW; ++r)
             expert[r] = (MASK && (FULL || row0 + r * kRowStep < p.R)) ? uniform_load(p.pos_to_expert + row0 + r * kRowStep) : 0;
-        if constexpr (MASK && RPW == 4 && !ROW)   // all four values must exist here, so their loads are issued together above
-            asm volatile("" ::"s"(expert[0]), "s"(expert[1]), "s"(expert[2]), "s"(expert[3]));
-        // A masked row-wise wave with routing weights asks for its row's slot in the weight list together with its mask entry
-        // (one scalar round trip for both) and for the weight itself right behind its vector loads, so that neither is waited
-        // for once the data is there.  Fetched where they are used, after the data, they cost [48128, 2 x 2048] with 32768 live
-        // rows 0.6 us of 61 on MI355X (2.6 us of 59 when the input is still in the last-level cache).
-        constexpr bool EARLY_WEIGHT = MASK && ROW;
-        int wpos = -1;
-        if constexpr (EARLY_WEIGHT) {
-            if (has_weight && (FULL || row0 < p.R)) wpos = uniform_load(p.pos_to_token_topk + row0);
+        // rows around the wave's own, in the segments next to its own too (segments are usually multiples of 128 rows)
+        constexpr bool RUN_OF_PADDING = MASK && !DIRECT && CLAMP != 2 && sizeof(InT) == 2;
+        int around[4] = {0, 0, 0, 0};
+        if constexpr (RUN_OF_PADDING) {
+            around[0] = uniform_load(p.pos_to_expert + max(row0 - 112, 0));
+            around[1] = uniform_load(p.pos_to_expert + max(row0 - 48, 0));
+            around[2] = uniform_load(p.pos_to_expert + min(row0 + 48, p.R - 1));
+            around[3] = uniform_load(p.pos_to_expert + min(row0 + 112, p.R - 1));
         }
+        // all these values must exist here, so that their loads are issued together above; and, so that neither path behind the branch
+        // below waits for them in front of its loads or stores, the later arguments
+        if constexpr (MASK && RPW == 4 && !ROW)
+            asm volatile("" ::"s"(expert[0]), "s"(expert[1]), "s"(expert[2]), "s"(expert[3]));
+        if constexpr (RUN_OF_PADDING)
+            asm volatile("" ::"s"(expert[0]), "s"(around[0]), "s"(around[1]), "s"(around[2]), "s"(around[3]), "s"(p.pos_to_token_topk), "s"(p.topk_weights), "s"(p.num_weights),
+                         "s"(p.sf.layout), "s"(p.sf.nk), "s"(p.clamp));
+        // Routing weights of a masked wave.  One of T_ROW asks for its row's slot in the weight list together with its mask entry (one scalar
+        // round trip for both), the others behind their vector loads, and all for the weights themselves right after, so that neither
+        // is waited for once the data is there.  Fetched where they are used, after the data, they cost [48128, 2 x 2048] with 32768 live
+        // rows 0.6 us of 61 on MI355X (2.6 us of 59 when the input is still in the last-level cache), stacked tiles of one of 8 ranks
+        // [35328, 2 x 1664] 47.8 / 46.4, [720, 2 x 2560] 3.9 / 3.7 (fp32 input 1 to 3 % slower: not there).
+        constexpr bool EARLY_WEIGHT = MASK && (ROW || sizeof(InT) == 2);
+        constexpr int WROWS = ROW ? 1 : RPW;      // rows of the wave
+        int wpos[WROWS];
+#pragma unroll
+        for (int r = 0; r < WROWS; ++r) wpos[r] = -1;
+        const auto ask_for_weights = [&] {
+            if (!has_weight) return;
+#pragma unroll
+            for (int r = 0; r < WROWS; ++r)
+                if (FULL || row0 + r < p.R) wpos[r] = uniform_load(p.pos_to_token_topk + row0 + r);
+        };
+        if constexpr (EARLY_WEIGHT && DIRECT) ask_for_weights();
         // A wave whose row is padding writes the row's zeros and leaves: no loads, no arithmetic.  The zeros go out as
         // non-temporal 16-byte stores that cover whole lines.  Measured on MI355X, bf16, us per call, padding rows flowing
         // through the arithmetic as zeros / this way: configuration with runs of padding (32768 live rows of 47488, H = 2048)
@@ -428,130 +469,160 @@ __global__ __launch_bounds__(TILE == T_ROW ? 64 * kMaxWideWaves : kThreads) void
                 else return;
             }
         }
+        // Tiles that stage their scales: in a long run of padding (few tokens, many experts, the end of a buffer for the worst case), a wave
+        // without a live row writes its zeros, stages zeros and goes to the barrier.  Elsewhere padding rows read the matrix's first
+        // bytes and flow through the arithmetic as zeros: where most waves do that, they all ask for one line.  us per call on MI355X,
+        // bf16, 513 live rows of 28544, through the arithmetic / this: H = 1664 32.4 / 22.9, H = 3072 45.7 / 31.0, column-major scales, H = 4096
+        // 62.6 / 45.0.  Short runs are better paced by the arithmetic than written in bursts between the live rows' requests: with every
+        // wave of padding done this way, 6824 live rows of 8192 in segments of a multiple of 128, column-major scales, H = 2048 13.8 / 14.8.
+        // (fp32 input is left as it was: 1 to 5 % slower on small batches.)
+        bool dead = false;
+        if constexpr (RUN_OF_PADDING) {
+            dead = (around[0] & around[1] & around[2] & around[3]) < 0;
 #pragma unroll
-        for (int r = 0; r < RPW; ++r) {
-            live[r] = (FULL || row0 + r * kRowStep < p.R) && expert[r] >= 0;
-            const InT *xr = x + (uint64_t)(uint32_t)(r * kRowStep) * (2u * uh) + r * kColStep;
-            const bool piece_ok = FULL || col + r * kColStep < p.H;
-            if (FULL && !MASK) {
-                // (a wave-uniform 64-bit base plus a 32-bit byte offset per lane: see swiglu_row_wave)
-                const uint8_t *xg = reinterpret_cast<const uint8_t *>(p.x) + (uint64_t)(uint32_t)(row0 + r * kRowStep) * (2u * uh * (uint32_t)sizeof(InT)) +
-                                    (uint32_t)(r * kColStep) * (uint32_t)sizeof(InT);
-                const uint32_t lane_off = (uint32_t)strip * (uint32_t)(kStripCols * sizeof(InT)) + (uint32_t)lane * (uint32_t)(8 * sizeof(InT));
-                rg[r].template load_run<64>(xg + lane_off, lane);
-                vmem_issue_gap();
-                ru[r].template load_run<64>(xg + uh * (uint32_t)sizeof(InT) + lane_off, lane);
-                if (r + 1 < RPW) vmem_issue_gap();
-            } else if (FULL && XB != 0) {
-                // (a padding row reads the first 2 KB of the matrix, as one run)
-                const bool ok = live[r];
-                const InT *src = ok ? xr : reinterpret_cast<const InT *>(p.x) + lane * 8;
-                rg[r].template load_run<64>(src, lane);
-                vmem_issue_gap();
-                ru[r].template load_run<64>(ok ? xr + uh : src, lane);
-                if (r + 1 < RPW) vmem_issue_gap();
-                unused[r] = !ok;
-            } else {
-                // no branch around the loads (a branch would make the compiler wait for all eight loads
-                // before the first row is evaluated): a padding row, and a lane beyond the last row or column,
-                // reads the first bytes of the matrix, which every wave shares, and is cleared by value
-                const bool ok = live[r] && piece_ok;
-                if constexpr (XB != 0) {      // (whole lines: fp32 [4001, 2 x 2560] 18.5 us with each lane reading its own bytes)
-                    const int first = (strip + r * (ROW ? 1 : 0)) * kStripCols, n = live[r] ? p.H - first : 0;
-                    const InT *run = xr - lane * 8;
-                    rg[r].template load_run_part<64>(run, lane, n, p.x);
-                    vmem_issue_gap();
-                    ru[r].template load_run_part<64>(run + uh, lane, n, p.x);
-                } else {
-                    const InT *src = ok ? xr : reinterpret_cast<const InT *>(p.x);
-                    rg[r].load(src);
-                    vmem_issue_gap();
-                    ru[r].load(ok ? xr + uh : src);
-                }
-                if (r + 1 < RPW) vmem_issue_gap();
-                unused[r] = !ok;
-                if constexpr (sizeof(InT) != 4) {
-                    if (!ok) { rg[r].zero(); ru[r].zero(); }
+            for (int r = 0; r < RPW; ++r) dead = dead && ((!FULL && row0 + r * kRowStep >= p.R) || expert[r] < 0);
+            if (dead) zero_dead_wave<RPW, ROW, FULL>(p, row0, strip, lane);
+            if (dead && own < RS::A) {
+#pragma unroll
+                for (int c = 0; c < RS::NC; ++c) {
+                    if (ROWC) stage[srow][(c * RS::A + own) * GPS + (lane >> 4)] = 0u;
+                    else stage[srow + c * RS::A + own][lane >> 4] = 0u;
                 }
             }
         }
-        // (in this variant the fetch of the later arguments starts at the head of the kernel, where its paths part)
-        if constexpr (TAILED != 0) fetch_late_arguments(p, CLAMP != 0, TAILED == 2, TILE != T_ROW);
-        if constexpr (XB != 0) {
+        if (!dead) {
 #pragma unroll
             for (int r = 0; r < RPW; ++r) {
-                rg[r].template settle<64>(xchg[wave], lane);
-                ru[r].template settle<64>(xchg[wave], lane);
-            }
-        }
-        // fp32 input (two loads per piece): cleared once all loads are out, since clearing a register that a load is still to
-        // fill means waiting for that load (masked fp32 [16384, 2 x 2048] 40.3 -> 38.4 us; bf16 input, whose clearing the
-        // compiler already places behind the loads, measured 21.0 -> 21.2 us on a ragged batch with it and keeps its place)
-        if constexpr (!(FULL && !MASK) && sizeof(InT) == 4) {
-#pragma unroll
-            for (int r = 0; r < RPW; ++r)
-                if (unused[r]) { rg[r].zero(); ru[r].zero(); }
-        }
-        float wrow = 0.0f;
-        if constexpr (EARLY_WEIGHT) {
-            if (has_weight && live[0] && wpos >= 0 && wpos < p.num_weights) wrow = uniform_load(p.topk_weights + wpos);
-        }
-        // dead rows hold zeros, so they flow through as v = 0 and only their scale is overridden
-        float v[RPW][8], amax[RPW];
-#pragma unroll
-        for (int r = 0; r < RPW; ++r) {
-            float g[8], u[8];
-            rg[r].get(g);
-            ru[r].get(u);
-            counter.apply8(g, u, p.clamp);
-#pragma unroll
-            for (int i = 0; i < 8; ++i) v[r][i] = silu_mul<InT>(g[i], u[i]);
-            if (has_weight) {
-                const float w = EARLY_WEIGHT ? wrow : (live[r] ? row_weight(p, row0 + r * kRowStep) : 0.0f);
-#pragma unroll
-                for (int i = 0; i < 8; ++i) v[r][i] = v[r][i] * w;
-            }
-            amax[r] = group_allmax<16>(absmax8(v[r]));
-        }
-        RS rs;
-        rs.compute(amax, p.floor_, p.round_sf != 0, lane);
-        if (MASK) {
-#pragma unroll
-            for (int c = 0; c < RS::NC; ++c) {
-                const int pick = lane & (RS::A - 1);
-                const bool l0 = live[c * RS::A];
-                const bool l1 = RS::A >= 2 ? live[c * RS::A + (RS::A >= 2 ? 1 : 0)] : false;
-                const bool l2 = RS::A >= 4 ? live[c * RS::A + (RS::A >= 4 ? 2 : 0)] : false;
-                const bool l3 = RS::A >= 4 ? live[c * RS::A + (RS::A >= 4 ? 3 : 0)] : false;
-                bool mine = l0;
-                if (RS::A >= 2) mine = pick == 1 ? l1 : mine;
-                if (RS::A >= 4) { mine = pick == 2 ? l2 : mine; mine = pick == 3 ? l3 : mine; }
-                if (!mine) { rs.own[c].sf = 0.0f; rs.own[c].e8 = 0u; }
-            }
-#pragma unroll
-            for (int r = 0; r < RPW; ++r) rs.inv[r] = live[r] ? rs.inv[r] : 0.0f;
-        }
-        // lane j (< A) of a group computed the scale of piece c*A + j
-        if (own < RS::A) {
-#pragma unroll
-            for (int c = 0; c < RS::NC; ++c) {
-                if constexpr (ROWC) {
-                    stage[srow][(c * RS::A + own) * GPS + (lane >> 4)] = p.sf.layout == TK_SF_COL_UE8M0 ? rs.own[c].e8 : f2u(rs.own[c].sf);
-                } else if constexpr (DIRECT) {
-                    // group (lane >> 4) of piece c*A + own: the wave's scales form one run of RPW * 4 floats
-                    const int k = (strip + c * RS::A + own) * GPS + (lane >> 4);
-                    if (FULL || (row0 < p.R && k < p.sf.nk))
-                        st_stream4(reinterpret_cast<float *>(p.sf.base) + (int64_t)row0 * p.sf.ld + k, f2u(rs.own[c].sf));
+                live[r] = (FULL || row0 + r * kRowStep < p.R) && expert[r] >= 0;
+                const InT *xr = x + (uint64_t)(uint32_t)(r * kRowStep) * (2u * uh) + r * kColStep;
+                const bool piece_ok = FULL || col + r * kColStep < p.H;
+                if (FULL && !MASK) {
+                    // (a wave-uniform 64-bit base plus a 32-bit byte offset per lane: see swiglu_row_wave)
+                    const uint8_t *xg = reinterpret_cast<const uint8_t *>(p.x) + (uint64_t)(uint32_t)(row0 + r * kRowStep) * (2u * uh * (uint32_t)sizeof(InT)) +
+                                        (uint32_t)(r * kColStep) * (uint32_t)sizeof(InT);
+                    const uint32_t lane_off = (uint32_t)strip * (uint32_t)(kStripCols * sizeof(InT)) + (uint32_t)lane * (uint32_t)(8 * sizeof(InT));
+                    rg[r].template load_run<64>(xg + lane_off, lane);
+                    vmem_issue_gap();
+                    ru[r].template load_run<64>(xg + uh * (uint32_t)sizeof(InT) + lane_off, lane);
+                    if (r + 1 < RPW) vmem_issue_gap();
+                } else if (FULL && XB != 0) {
+                    // (a padding row reads the first 2 KB of the matrix, as one run)
+                    const bool ok = live[r];
+                    const InT *src = ok ? xr : reinterpret_cast<const InT *>(p.x) + lane * 8;
+                    rg[r].template load_run<64>(src, lane);
+                    vmem_issue_gap();
+                    ru[r].template load_run<64>(ok ? xr + uh : src, lane);
+                    if (r + 1 < RPW) vmem_issue_gap();
+                    unused[r] = !ok;
                 } else {
-                    stage[srow + c * RS::A + own][lane >> 4] =
-                        p.sf.layout == TK_SF_COL_UE8M0 ? rs.own[c].e8 : f2u(rs.own[c].sf);
+                    // no branch around the loads (a branch would make the compiler wait for all eight loads
+                    // before the first row is evaluated): a padding row, and a lane beyond the last row or column,
+                    // reads the first bytes of the matrix, which every wave shares, and is cleared by value
+                    const bool ok = live[r] && piece_ok;
+                    if constexpr (XB != 0) {      // (whole lines: fp32 [4001, 2 x 2560] 18.5 us with each lane reading its own bytes)
+                        const int first = (strip + r * (ROW ? 1 : 0)) * kStripCols, n = live[r] ? p.H - first : 0;
+                        const InT *run = xr - lane * 8;
+                        rg[r].template load_run_part<64>(run, lane, n, p.x);
+                        vmem_issue_gap();
+                        ru[r].template load_run_part<64>(run + uh, lane, n, p.x);
+                    } else {
+                        const InT *src = ok ? xr : reinterpret_cast<const InT *>(p.x);
+                        rg[r].load(src);
+                        vmem_issue_gap();
+                        ru[r].load(ok ? xr + uh : src);
+                    }
+                    if (r + 1 < RPW) vmem_issue_gap();
+                    unused[r] = !ok;
+                    if constexpr (sizeof(InT) != 4) {
+                        if (!ok) { rg[r].zero(); ru[r].zero(); }
+                    }
                 }
             }
-        }
+            // (in this variant the fetch of the later arguments starts at the head of the kernel, where its paths part)
+            if constexpr (TAILED != 0) fetch_late_arguments(p, CLAMP != 0, TAILED == 2, TILE != T_ROW);
+            if constexpr (XB != 0) {
 #pragma unroll
-        for (int r = 0; r < RPW; ++r)
-            if ((FULL || col + r * kColStep < p.H) && (FULL || row0 + r * kRowStep < p.R))
-                quantise_store8<TK_E4M3, false>(v[r], rs.inv[r], p.out + (int64_t)(row0 + r * kRowStep) * p.H, col + r * kColStep);
+                for (int r = 0; r < RPW; ++r) {
+                    rg[r].template settle<64>(xchg[wave], lane);
+                    ru[r].template settle<64>(xchg[wave], lane);
+                }
+            }
+            // fp32 input (two loads per piece): cleared once all loads are out, since clearing a register that a load is still to
+            // fill means waiting for that load (masked fp32 [16384, 2 x 2048] 40.3 -> 38.4 us; bf16 input, whose clearing the
+            // compiler already places behind the loads, measured 21.0 -> 21.2 us on a ragged batch with it and keeps its place)
+            if constexpr (!(FULL && !MASK) && sizeof(InT) == 4) {
+#pragma unroll
+                for (int r = 0; r < RPW; ++r)
+                    if (unused[r]) { rg[r].zero(); ru[r].zero(); }
+            }
+            if constexpr (EARLY_WEIGHT && !DIRECT) ask_for_weights();
+            float wrow[WROWS];
+#pragma unroll
+            for (int r = 0; r < WROWS; ++r) wrow[r] = 0.0f;
+            if constexpr (EARLY_WEIGHT) {
+                if (has_weight) {
+#pragma unroll
+                    for (int r = 0; r < WROWS; ++r)
+                        if (live[r] && wpos[r] >= 0 && wpos[r] < p.num_weights) wrow[r] = uniform_load(p.topk_weights + wpos[r]);
+                }
+            }
+            // dead rows hold zeros, so they flow through as v = 0 and only their scale is overridden
+            float v[RPW][8], amax[RPW];
+#pragma unroll
+            for (int r = 0; r < RPW; ++r) {
+                float g[8], u[8];
+                rg[r].get(g);
+                ru[r].get(u);
+                counter.apply8(g, u, p.clamp);
+#pragma unroll
+                for (int i = 0; i < 8; ++i) v[r][i] = silu_mul<InT>(g[i], u[i]);
+                if (has_weight) {
+                    const float w = EARLY_WEIGHT ? wrow[ROW ? 0 : r] : (live[r] ? row_weight(p, row0 + r * kRowStep) : 0.0f);
+#pragma unroll
+                    for (int i = 0; i < 8; ++i) v[r][i] = v[r][i] * w;
+                }
+                amax[r] = group_allmax<16>(absmax8(v[r]));
+            }
+            RS rs;
+            rs.compute(amax, p.floor_, p.round_sf != 0, lane);
+            if (MASK) {
+#pragma unroll
+                for (int c = 0; c < RS::NC; ++c) {
+                    const int pick = lane & (RS::A - 1);
+                    const bool l0 = live[c * RS::A];
+                    const bool l1 = RS::A >= 2 ? live[c * RS::A + (RS::A >= 2 ? 1 : 0)] : false;
+                    const bool l2 = RS::A >= 4 ? live[c * RS::A + (RS::A >= 4 ? 2 : 0)] : false;
+                    const bool l3 = RS::A >= 4 ? live[c * RS::A + (RS::A >= 4 ? 3 : 0)] : false;
+                    bool mine = l0;
+                    if (RS::A >= 2) mine = pick == 1 ? l1 : mine;
+                    if (RS::A >= 4) { mine = pick == 2 ? l2 : mine; mine = pick == 3 ? l3 : mine; }
+                    if (!mine) { rs.own[c].sf = 0.0f; rs.own[c].e8 = 0u; }
+                }
+#pragma unroll
+                for (int r = 0; r < RPW; ++r) rs.inv[r] = live[r] ? rs.inv[r] : 0.0f;
+            }
+            // lane j (< A) of a group computed the scale of piece c*A + j
+            if (own < RS::A) {
+#pragma unroll
+                for (int c = 0; c < RS::NC; ++c) {
+                    if constexpr (ROWC) {
+                        stage[srow][(c * RS::A + own) * GPS + (lane >> 4)] = p.sf.layout == TK_SF_COL_UE8M0 ? rs.own[c].e8 : f2u(rs.own[c].sf);
+                    } else if constexpr (DIRECT) {
+                        // group (lane >> 4) of piece c*A + own: the wave's scales form one run of RPW * 4 floats
+                        const int k = (strip + c * RS::A + own) * GPS + (lane >> 4);
+                        if (FULL || (row0 < p.R && k < p.sf.nk))
+                            st_stream4(reinterpret_cast<float *>(p.sf.base) + (int64_t)row0 * p.sf.ld + k, f2u(rs.own[c].sf));
+                    } else {
+                        stage[srow + c * RS::A + own][lane >> 4] =
+                            p.sf.layout == TK_SF_COL_UE8M0 ? rs.own[c].e8 : f2u(rs.own[c].sf);
+                    }
+                }
+            }
+#pragma unroll
+            for (int r = 0; r < RPW; ++r)
+                if ((FULL || col + r * kColStep < p.H) && (FULL || row0 + r * kRowStep < p.R))
+                    quantise_store8<TK_E4M3, false>(v[r], rs.inv[r], p.out + (int64_t)(row0 + r * kRowStep) * p.H, col + r * kColStep);
+        }
         if constexpr (!DIRECT) {
             __syncthreads();
             if (ROWC) sf_store_tile_colmajor<ROWS, SGPR>(p.sf, stage, tile_m * ROWS, tile_k * SGPR);
