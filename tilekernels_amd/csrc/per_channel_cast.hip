@@ -284,6 +284,12 @@ __global__ __launch_bounds__(LANES * kPcParts, 4) void per_channel_cast_kernel(T
         // 8 lanes x 16 bytes = the 128 tokens of one output row; a wave stores 8 rows per step
         const int chunk = threadIdx.x & 7;
         const int tok = tile_m * kPcTileM + chunk * 16;
+        // Behind the SwiGLU a launch of more tiles than fit the GPU at a time (two to a CU) writes through: 128-byte pieces of its output rows
+        // that stay behind in the L2 leave it in no order.  us, non-temporal / write-through, three sets of inputs in rotation (twelve):
+        // [8192, 2 x 8320] 65.2 / 58.8 (66.0 / 66.8), [16384, 2 x 2048] 31.6 / 30.4 (32.2 / 30.7), [12288, 2 x 2560] 29.5 / 28.0 (30.0 / 28.1), [4480,
+        // 2 x 6144] 26.4 / 25.8 (26.7 / 25.9); in one round [8064, 2 x 2048] 16.4 / 16.2 (16.5 / 18.1).  (Neighbouring token tiles side by side in
+        // the grid, 2, 4 or 8, on neighbouring XCDs or on one, so that pieces of one row meet: 1 to 5 % slower.)
+        const bool through = MODE == PC_SWIGLU && LANES == 32 && p.tiles_k * ((p.M + kPcTileM - 1) / kPcTileM) > 512;
 #pragma unroll
         for (int i = 0; i < kPcTileK / (kPcThreads / 8); ++i) {
             const int h = (threadIdx.x >> 3) + (kPcThreads / 8) * i;
@@ -291,9 +297,9 @@ __global__ __launch_bounds__(LANES * kPcParts, 4) void per_channel_cast_kernel(T
                 const int unit = (chunk + (h >> 4)) & 7;
                 u32x4 d = *reinterpret_cast<const u32x4 *>(&turned[h * kPcPitch + unit * 16]);
                 if (LANES == 32 && i >= 2) d = u32x4{d.z, d.w, d.x, d.y};          // rows of the lanes hl >= 16: h >= 128
-                // (write-through stores against non-temporal ones, bf16 [8192, 4096] on MI355X: plain and FP8 input 19.6 -> 19.2 us,
-                // behind the SwiGLU 16.7 -> 16.9 us; ordinary stores 19.6 and 18.4 us)
-                if constexpr (MODE != PC_SWIGLU) st_stream16(p.out + (int64_t)(col0 + h) * p.M + tok, d);
+                // (write-through stores against non-temporal ones, bf16 [8192, 4096] on MI355X: plain and FP8 input 19.6 -> 19.2 us, ordinary
+                // stores 19.6 and 18.4 us; behind the SwiGLU see `through`)
+                if (MODE != PC_SWIGLU || through) st_stream16(p.out + (int64_t)(col0 + h) * p.M + tok, d);
                 else __builtin_nontemporal_store(d, reinterpret_cast<u32x4 *>(p.out + (int64_t)(col0 + h) * p.M + tok));
             }
         }
