@@ -215,6 +215,25 @@ def test_mapping_of_a_list_between_16_byte_boundaries(T, K, E):
             assert_same(a, b, name)
 
 
+@pytest.mark.parametrize('T,K,E,alignment', [(57, 9, 256, 128), (1, 1, 512, 128), (300, 8, 512, 128), (3, 2, 64, 1024)])
+def test_mapping_of_short_lists_into_long_buffers(T, K, E, alignment):
+    """More workgroups than the list has pairs for: they mark the padding of experts and of the buffer's end."""
+    tk = _tk()
+    g = torch.Generator().manual_seed(T * E)
+    idx = torch.randint(-1, E, (T, K), generator=g)
+    want = torch_ref.get_fused_mapping(idx, E, alignment)
+    rows = want[0].numel()
+    got = tk.moe.get_fused_mapping(idx.cuda(), E, 0, alignment)
+    for a, b in zip(got[:7], want[:7]):
+        assert torch.equal(a.cpu(), b)
+    for extra in (1, 70_001):
+        got = tk.moe.get_fused_mapping(idx.cuda(), E, rows + extra, alignment)
+        for a, b in zip(got[:3], want[:3]):
+            assert torch.equal(a[:rows].cpu(), b) and bool((a[rows:] == -1).all())
+        for a, b in zip(got[3:7], want[3:7]):
+            assert torch.equal(a.cpu(), b)
+
+
 # one launch, two around a table, three; behind an idle stream and behind work that takes longer than the wait in a loop
 @pytest.mark.parametrize('busy', [False, True])
 @pytest.mark.parametrize('T,K,E', [(1, 1, 1), (700, 6, 512), (11000, 8, 32), (90, 5, 700), (0, 4, 8)])
