@@ -457,6 +457,22 @@ def test_smallest_shapes():
     f.check(300)
 
 
+# bf16 rows that leave part of their last 512 columns empty, on both sides of the size from which they are laid end to end; rows apart
+@pytest.mark.parametrize('fmt,group', [('e4m3', 16), ('e4m3', 64), ('e4m3', 128), ('e2m1', 32), ('e2m1', 128)])
+@pytest.mark.parametrize('M,K', [(1736, 2304), (1737, 2304), (2831, 1416), (1789, 2808), (700, 6600)])
+def test_per_token_cast_of_ragged_rows(M, K, fmt, group):
+    tk = _tk()
+    x = _randn((M, K), torch.bfloat16, M + K, 2.0)
+    for round_sf in (False, True):
+        want = torch_ref.cast(x, fmt, (1, group), round_sf=round_sf)
+        apart = torch.zeros((M, K + 72), dtype=torch.bfloat16, device='cuda')[:, :K]
+        apart.copy_(x)
+        for xd in (x.cuda(), apart):
+            got = tk.quant.per_token_cast(xd, fmt, group, None, False, round_sf)
+            assert_same(got[0], want[0], 'codes')
+            assert_same(got[1], want[1], 'sf')
+
+
 # (rows, columns) in and around the ranges of the tile shapes: 256 columns by 1024 threads, 512 columns, 256 columns by 512 threads (bf16 to
 # E2M1), and 128 columns; whole and with edge tiles below and, where columns allow it, to the right
 @pytest.mark.parametrize('block', [(128, 128), (32, 32), (128, 32), (32, 128)])
