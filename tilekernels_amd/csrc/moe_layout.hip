@@ -908,7 +908,10 @@ extern "C" int tk_get_fused_mapping_with_counts(const int64_t *topk_idx, int64_t
     rc = launch_fused_mapping(topk_idx, num_tokens, num_topk, num_experts, alignment, num_expanded, pos_to_expert, pos_to_token,
                               pos_to_token_topk, token_topk_to_pos, expert_start, expert_end, num_tokens_per_expert,
                               static_cast<int32_t *>(workspace), s, static_cast<int32_t *>(device));
-    if (rc != TK_OK) return rc;
+    if (rc != TK_OK) {
+        (void)hipStreamSynchronize(s);      // what was launched all the same may still write to host_counts
+        return rc;
+    }
     // Longer than this and there is other work in front of the kernels, or they have failed: hipStreamSynchronize waits without a busy
     // loop, and behind it the words are there.
     const auto give_up = std::chrono::steady_clock::now() + std::chrono::microseconds(200);
