@@ -527,11 +527,13 @@ inline bool short_rows_pay(int64_t K, int G) {
     return K * 5 < strips * kStripCols * 4 && groups * G < strips * kStripCols;
 }
 
-// bf16 rows that leave part of their last strip empty, row-major scales: laid end to end too, from some 4 million elements on.  Their tiles
-// are checked for their edges everywhere, and the last wave of a row is partly idle.  us, tiles / laid end to end, three sets of
-// inputs in rotation (twelve): E4M3 1 x 128 [2000, 2304] 4.0 / 3.9 (4.45 / 4.0), [5290, 2304] 7.7 / 7.35 (8.6 / 8.0), [16000, 1408] 12.7 / 12.1, [1500, 5888]
-// 6.1 / 5.7, [9000, 7232] 30.2 / 29.8 (33.0 / 32.2), 1 x 32 [5290, 2304] 8.0 / 7.4, E2M1 [3000, 2688] 5.3 / 4.7 (6.4 / 5.3); but [1000, 1664] 2.68 / 2.71, [500, 7232] 3.5 / 3.4 (3.7 / 4.0).  (Column-
-// major scales, which the tiles store as runs down their rows: 1 x 32 [5290, 2304] 8.15 / 10.8; fp32 [4500, 3840] 14.7 / 14.7.)
+// bf16 rows that leave part of their last strip empty, row-major scales: laid end to end too, from some 4 million elements on.  As tiles
+// they are checked for edges everywhere, and the last wave of a row is partly idle.  us on MI355X, tiles / laid end to end, three sets of
+// inputs in rotation (twelve):
+//   E4M3 1 x 128 [2000, 2304] 4.1 / 3.9 (4.4 / 4.0), [5290, 2304] 7.7 / 7.35 (8.6 / 8.0), [16000, 1408] 12.7 / 12.1, [1500, 5888] 6.1 / 5.7,
+//   [9000, 7232] 30.2 / 29.8 (33.0 / 32.2);  1 x 32 [5290, 2304] 8.0 / 7.4;  E2M1 1 x 64 [3000, 2688] 5.4 / 4.7 (6.4 / 5.3)
+//   but [1000, 1664] 2.68 / 2.71, [500, 7232] 3.5 / 3.4 (3.7 / 4.0);  fp32 [4500, 3840] 14.7 / 14.7;  column-major scales, which tiles store
+//   as runs down their rows, 1 x 32 [5290, 2304] 8.15 / 10.8.
 template <typename InT, int G> static bool ragged_rows_pay(const PerTokenParams &p) {
     const int64_t strips = (p.K + kStripCols - 1) / kStripCols, groups = (p.K + G - 1) / G;
     return std::is_same<InT, bf16_t>::value && p.sf.layout == TK_SF_ROW_F32 && p.mode == TK_CAST_AND_SF && groups * G < strips * kStripCols &&
