@@ -241,6 +241,26 @@ def test_masked_swiglu_with_more_rows_than_one_grid_plane(dtype, H, clamp):
     assert bool((codes_buf[R:] == 0x5A).all()), 'rows beyond the batch were written'
 
 
+@pytest.mark.parametrize('R,H,col', [(4 * 32768 + 4 * 700 + 3, 4096, True), (16 * 32768 + 16 * 40 + 5, 896, False)], ids=['whole-rows', 'stacked'])
+def test_masked_swiglu_tiles_with_staged_scales_on_more_than_one_grid_plane(R, H, col):
+    """Masked tiles that stage their scales, 4 or 16 rows each, two columns of them: most workgroups of the second plane lie wholly beyond the last
+    row, where there is no mask to read, neither their own rows' nor of the rows around.  Long runs of padding, one at the end, and short ones."""
+    tk = _tk()
+    g = torch.Generator(device='cuda').manual_seed(14)
+    x = torch.randn((R, 2 * H), generator=g, device='cuda', dtype=torch.bfloat16) * 2
+    pe = torch.zeros((R,), dtype=torch.int32, device='cuda')
+    pe[3::5] = -1
+    pe[1000:70000] = -1
+    pe[R - 300:] = -1
+    got = tk.quant.swiglu_forward_and_per_token_cast(x, 'e4m3', 128, pos_to_expert=pe, use_tma_aligned_col_major_sf=col)
+    for a, b in [(0, 32), (990, 1010), (R // 2, R // 2 + 32), (R - 320, R)]:
+        xw, pw = x[a:b].cpu(), pe[a:b].cpu()
+        want = torch_ref.swiglu_forward_and_per_token_cast(xw, 'e4m3', 128, pos_to_expert=pw, use_tma_aligned_col_major_sf=col)
+        live = pw >= 0
+        assert torch.all(got[0][a:b].cpu().view(torch.uint8)[~live] == 0) and torch.all(got[1][a:b].cpu()[~live] == 0)
+        check_fused((got[0][a:b].cpu()[live], got[1][a:b].cpu()[live].contiguous()), (want[0][live], want[1][live].contiguous()), H // 128, False, f'rows[{a}:{b}]')
+
+
 @pytest.mark.parametrize('hidden,dtype,tokens', [(8, torch.bfloat16, 2 ** 26 + 5), (2048, torch.float32, 2 ** 24 + 3)], ids=['bf16', 'fp32'])
 def test_reduce_fused_of_more_tokens_than_one_launch_takes(hidden, dtype, tokens):
     """Rows of one column of pieces put all their row tiles on grid.x, where HIP takes fewer than 2^32 threads: the tokens are

@@ -418,10 +418,12 @@ __global__ __launch_bounds__(TILE == T_ROW ? 64 * kMaxWideWaves : kThreads) void
         constexpr bool RUN_OF_PADDING = MASK && !DIRECT && CLAMP != 2 && sizeof(InT) == 2;
         int around[4] = {0, 0, 0, 0};
         if constexpr (RUN_OF_PADDING) {
-            around[0] = uniform_load(p.pos_to_expert + max(row0 - 112, 0));
-            around[1] = uniform_load(p.pos_to_expert + max(row0 - 48, 0));
-            around[2] = uniform_load(p.pos_to_expert + min(row0 + 48, p.R - 1));
-            around[3] = uniform_load(p.pos_to_expert + min(row0 + 112, p.R - 1));
+            // (a grid of several planes of row tiles may have whole planes beyond the last row: row0 may lie anywhere behind it)
+            const int inside = FULL ? row0 : min(row0, p.R - 1);
+            around[0] = uniform_load(p.pos_to_expert + max(inside - 112, 0));
+            around[1] = uniform_load(p.pos_to_expert + max(inside - 48, 0));
+            around[2] = uniform_load(p.pos_to_expert + min(inside + 48, p.R - 1));
+            around[3] = uniform_load(p.pos_to_expert + min(inside + 112, p.R - 1));
         }
         // all these values must exist here, so that their loads are issued together above; and, so that neither path behind the branch
         // below waits for them in front of its loads or stores, the later arguments
