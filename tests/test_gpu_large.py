@@ -261,6 +261,19 @@ def test_masked_swiglu_tiles_with_staged_scales_on_more_than_one_grid_plane(R, H
         check_fused((got[0][a:b].cpu()[live], got[1][a:b].cpu()[live].contiguous()), (want[0][live], want[1][live].contiguous()), H // 128, False, f'rows[{a}:{b}]')
 
 
+def test_mapping_of_a_short_list_into_the_longest_buffers():
+    """2^31 - 1025 positions: the workgroups' next position beyond the end does not fit 32 bits."""
+    tk = _tk()
+    idx = torch.tensor([[0, 2], [2, -1], [1, 2]], device='cuda')
+    n = 2 ** 31 - 1025
+    maps = tk.moe.get_fused_mapping(idx, 3, n, 16)
+    want = torch_ref.get_fused_mapping(idx.cpu(), 3, 16)
+    for got, ref in zip(maps[:3], want[:3]):
+        assert torch.equal(got[:48].cpu(), ref)
+        assert all(bool((part == -1).all()) for part in got[48:].split(2 ** 28))
+    assert torch.equal(maps[3].cpu(), want[3])
+
+
 @pytest.mark.parametrize('hidden,dtype,tokens', [(8, torch.bfloat16, 2 ** 26 + 5), (2048, torch.float32, 2 ** 24 + 3)], ids=['bf16', 'fp32'])
 def test_reduce_fused_of_more_tokens_than_one_launch_takes(hidden, dtype, tokens):
     """Rows of one column of pieces put all their row tiles on grid.x, where HIP takes fewer than 2^32 threads: the tokens are

@@ -36,7 +36,8 @@ __global__ __launch_bounds__(kThreads) void fused_mapping_count_kernel(const int
     int32_t *h = hist + wave * num_experts;
     for (int e = lane; e < num_experts; e += 64) h[e] = 0;
     // padding positions keep -1; the assign launch overwrites the live ones
-    for (int i = blockIdx.x * kThreads + threadIdx.x; i < num_expanded; i += gridDim.x * kThreads) {
+    // (64 bits: buffers of nearly 2^31 positions plus a stride of all workgroups)
+    for (int64_t i = (int64_t)blockIdx.x * kThreads + threadIdx.x; i < num_expanded; i += (int64_t)gridDim.x * kThreads) {
         pos_to_expert[i] = -1;
         pos_to_token[i] = -1;
         pos_to_token_topk[i] = -1;
@@ -363,7 +364,7 @@ __global__ __launch_bounds__(64 * kSingleWaves) void fused_mapping_single_kernel
         }
     }
     // positions beyond the last expert
-    for (int i = total + (int)blockIdx.x * nthreads + tid; i < num_expanded; i += (int)gridDim.x * nthreads) {
+    for (int64_t i = (int64_t)total + (int)blockIdx.x * nthreads + tid; i < num_expanded; i += (int)gridDim.x * nthreads) {      // (64 bits: as in the count kernel)
         pos_to_expert[i] = -1;
         pos_to_token[i] = -1;
         pos_to_token_topk[i] = -1;
