@@ -225,6 +225,28 @@ def test_watched_and_wrapped_calls_are_left_alone():
 
 
 @pytest.mark.gpu
+def test_the_wait_for_segment_lengths_is_seen_by_sync_debug_mode():
+    """A call that trims waits for the stream: torch refuses or reports that where it is told to, and has nothing to say to calls that do not wait."""
+    import tilekernels_amd as tk
+    from tilekernels_amd import _ffi
+    idx = torch.randint(0, 8, (64, 4), generator=torch.Generator().manual_seed(3)).cuda()
+    want = tk.moe.get_fused_mapping(idx, 8, 0, 16)
+    assert _ffi.host.get_fused_mapping(idx, 8, 0, 16, False) is not None
+    try:
+        torch.cuda.set_sync_debug_mode('error')
+        with pytest.raises(RuntimeError, match='synchroniz'):
+            tk.moe.get_fused_mapping(idx, 8, 0, 16)
+        for args in ((idx, 8, 512, 16, False), (idx, 8, 0, 16, True)):
+            assert _ffi.host.get_fused_mapping(*args) is not None
+        torch.cuda.set_sync_debug_mode('warn')
+        with pytest.warns(UserWarning, match='synchroniz'):
+            got = tk.moe.get_fused_mapping(idx, 8, 0, 16)
+    finally:
+        torch.cuda.set_sync_debug_mode('default')
+    assert got[7] == want[7] and all(torch.equal(a, b) for a, b in zip(got[:7], want[:7]))
+
+
+@pytest.mark.gpu
 def test_threads_on_their_own_streams():
     """The lock is released around each launch: threads that call at the same time get the results each would get alone."""
     import threading

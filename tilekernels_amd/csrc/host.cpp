@@ -12,6 +12,7 @@
 #include <ATen/ATen.h>
 #include <ATen/PythonTorchFunctionTLS.h>
 #include <ATen/hip/EmptyTensor.h>
+#include <c10/core/impl/GPUTrace.h>
 #include <c10/core/impl/LocalDispatchKeySet.h>
 #include <c10/core/impl/TorchDispatchModeTLS.h>
 #include <c10/hip/HIPFunctions.h>
@@ -407,6 +408,8 @@ PyObject *get_fused_mapping(PyObject *const *a) {
     const int experts = small(a[1]), alignment = small(a[3]);
     int64_t expanded = integer(a[2]);
     const bool sync = expanded == 0 && !boolean(a[4]);
+    // (the wait is the library's own: where torch is told to warn of waits, refuse or report them, Python's is the one it knows of)
+    if (sync) need(c10::hip::warning_state().get_sync_debug_mode() == c10::hip::SyncDebugMode::L_DISABLED && !c10::impl::GPUTrace::get_trace());
     need(is_matrix(idx) && idx.is_contiguous() && idx.scalar_type() == at::kLong && experts > 0 && alignment > 0 && expanded >= 0);
     need(idx.size(0) <= INT32_MAX && idx.size(1) <= INT32_MAX);
     const int64_t tokens = idx.size(0), topk = idx.size(1);
