@@ -292,9 +292,8 @@ int tk_check_get_fused_mapping(const int64_t *topk_idx, int64_t num_tokens, int 
 
 /*
  * tk_get_fused_mapping_with_counts: tk_get_fused_mapping, which also stores num_tokens_per_expert in host_counts, num_experts words of
- * host memory that the GPU can write (hipHostMalloc), and returns once they are there; the other outputs are ordered by the stream as
- * usual.  It waits for the work in front of it on the stream.  Rejected with TK_ERR_BAD_MODE on a stream that is being captured, and with
- * TK_ERR_BAD_VALUE where host_counts is no such memory.
+ * host memory that the GPU can write (hipHostMalloc), and returns once the stream is through, so that all outputs may be used on any
+ * stream.  Rejected with TK_ERR_BAD_MODE on a stream that is being captured, and with TK_ERR_BAD_VALUE where host_counts is no such memory.
  */
 int tk_get_fused_mapping_with_counts(const int64_t *topk_idx, int64_t num_tokens, int num_topk, int num_experts, int alignment,
                                      int64_t num_expanded, int32_t *pos_to_expert, int32_t *pos_to_token, int32_t *pos_to_token_topk,

@@ -266,8 +266,28 @@ def test_segment_lengths_on_the_host(T, K, E, busy):
     assert call(host.data_ptr(), _ffi.current_stream(idx.device)) == 0
     assert host.tolist() == got[7]
     assert call(None, _ffi.current_stream(idx.device)) == -1                    # null pointer
+    assert call(torch.empty((E,), dtype=torch.int32).data_ptr(), _ffi.current_stream(idx.device)) == -11        # memory the GPU cannot write
     graph = torch.cuda.CUDAGraph()
     torch.cuda.synchronize()
     with torch.cuda.graph(graph):
         rc = call(host.data_ptr(), torch.cuda.current_stream().cuda_stream)
     assert rc == -7                                                             # nothing runs during a capture: no lengths to wait for
+
+
+# one launch, two around a table, three
+@pytest.mark.parametrize('T,K,E', [(700, 6, 512), (50_000, 8, 32), (400_000, 8, 700)])
+def test_a_trimming_call_returns_when_the_stream_is_through(T, K, E):
+    """As behind a copy of the lengths to the host, the lists may be read on another stream without an event."""
+    tk = _tk()
+    idx = torch.randint(-1, E, (T, K), generator=torch.Generator().manual_seed(T)).cuda()
+    want = tk.moe.get_fused_mapping(idx, E, (T * K + 15 * E) // 16 * 16, 16)
+    torch.cuda.synchronize()
+    side = torch.cuda.Stream()
+    for _ in range(3):
+        got = tk.moe.get_fused_mapping(idx, E, 0, 16)
+        assert torch.cuda.current_stream().query()
+        with torch.cuda.stream(side):
+            there = [t.clone() for t in got[:7]]
+        torch.cuda.synchronize()
+        for a, b in zip(there, want[:7]):
+            assert torch.equal(a, b[:len(a)])

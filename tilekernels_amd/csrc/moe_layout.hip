@@ -7,7 +7,6 @@
 // tile_kernels/moe/reduce_fused_kernel.py:12-135, tile_kernels/torch/reduce_fused.py.
 #include <atomic>
 #include <algorithm>
-#include <chrono>
 
 #include "tk_device.hpp"
 #include "tk_host.hpp"
@@ -299,7 +298,7 @@ __global__ __launch_bounds__(64 * kSingleWaves) void fused_mapping_single_kernel
     int32_t mine = 0, incl = 0;
     if (tid < kSingleMaxExperts) {
         mine = tid < num_experts ? (int32_t)(((uint32_t)all_of(tid) + alignment - 1) / alignment * alignment) : 0;
-        if (host_counts && blockIdx.x == 0 && tid < num_experts) st_stream4(host_counts + tid, (uint32_t)mine);      // the host goes on while positions are handed out
+        if (host_counts && blockIdx.x == 0 && tid < num_experts) st_stream4(host_counts + tid, (uint32_t)mine);
         incl = mine;
 #pragma unroll
         for (int d = 1; d < 64; d <<= 1) {
@@ -881,10 +880,11 @@ extern "C" int tk_get_fused_mapping(const int64_t *topk_idx, int64_t num_tokens,
                                 static_cast<int32_t *>(workspace), static_cast<hipStream_t>(stream));
 }
 
-// The mapping for a caller that needs the segment lengths on the host.  A copy of num_tokens_per_expert behind the kernels and the wait for
-// the stream took some 13 us more than this; here the workgroup that has counted writes the lengths to host memory by itself, each a
-// word that was negative before, so that no order between them matters, and the calling thread reads on until it has them all.
-// us per call of get_fused_mapping on MI355X, copy and wait / this: 329 tokens, top-8, 32 experts 26.6 / 13.9; 21520 tokens 32.7 / 19.3.
+// The mapping for a caller that needs the segment lengths on the host.  The workgroup that has counted writes them to host memory by itself,
+// which saves a copy of num_tokens_per_expert behind the kernels, and the call returns when the stream is through: its caller may go on
+// with the lists on any stream, as behind a copy to the host.  us per call of get_fused_mapping on MI355X, copy and wait / this: 329 tokens, top-8,
+// 32 experts 26.6 / 20.7; 21520 tokens 32.7 / 27.2.  (Reading on until the words are there and returning then, while positions are still being
+// handed out, takes 13.8 and 18.8, and the lists are then in order on this stream only; a loop over hipStreamQuery 32.2 and 39.1.)
 extern "C" int tk_get_fused_mapping_with_counts(const int64_t *topk_idx, int64_t num_tokens, int num_topk, int num_experts, int alignment,
                                                 int64_t num_expanded, int32_t *pos_to_expert, int32_t *pos_to_token,
                                                 int32_t *pos_to_token_topk, int32_t *token_topk_to_pos, int32_t *expert_start,
@@ -905,28 +905,11 @@ extern "C" int tk_get_fused_mapping_with_counts(const int64_t *topk_idx, int64_t
         (void)hipGetLastError();
         return TK_ERR_BAD_VALUE;
     }
-    for (int i = 0; i < num_experts; ++i) host_counts[i] = -1;
     rc = launch_fused_mapping(topk_idx, num_tokens, num_topk, num_experts, alignment, num_expanded, pos_to_expert, pos_to_token,
                               pos_to_token_topk, token_topk_to_pos, expert_start, expert_end, num_tokens_per_expert,
                               static_cast<int32_t *>(workspace), s, static_cast<int32_t *>(device));
-    if (rc != TK_OK) {
-        (void)hipStreamSynchronize(s);      // what was launched all the same may still write to host_counts
-        return rc;
-    }
-    // Longer than this and there is other work in front of the kernels, or they have failed: hipStreamSynchronize waits without a busy
-    // loop, and behind it the words are there.
-    const auto give_up = std::chrono::steady_clock::now() + std::chrono::microseconds(200);
-    const volatile int32_t *counts = host_counts;
-    for (int i = 0, spins = 0; i < num_experts;) {
-        if (counts[i] >= 0) {
-            ++i;
-        } else if ((++spins & 63) == 0 && std::chrono::steady_clock::now() > give_up) {
-            e = hipStreamSynchronize(s);
-            break;
-        }
-    }
-    std::atomic_thread_fence(std::memory_order_acquire);
-    return (int)e;
+    e = hipStreamSynchronize(s);      // (also where a launch failed: what was launched all the same may still write to host_counts)
+    return rc != TK_OK ? rc : (int)e;
 }
 
 // ------------------------------------------------------------------------------------------------
