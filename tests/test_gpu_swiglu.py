@@ -227,3 +227,29 @@ def test_mostly_padding(R, H, with_weights, clamp, mode):
         dev = [t.cuda() if t is not None else None for t in weights]
         got = tk.quant.swiglu_forward_and_per_token_cast(xm.cuda(), 'e4m3', 128, *dev, p2e.cuda(), col, round_sf, packed, swiglu_clamp_value=clamp)
         check_fused(got, want, H // 128, packed, f'{rows}')
+
+
+# workgroups of 16 rows x 512 columns or of 4 rows x 2048, just beyond one round of the GPU and just below the line: whole and ragged tiles
+@pytest.mark.parametrize('mode', [(False, False, False), (True, False, False), (True, True, True)], ids=lambda m: 'col%d-round%d-packed%d' % tuple(int(v) for v in m))
+@pytest.mark.parametrize('with_weights,clamp', [(False, None), (True, 1.0)])
+@pytest.mark.parametrize('R,H', [(12304, 1536), (12289, 1408), (12288, 1536), (9220, 2048), (9219, 2048), (9216, 2048), (4612, 4096)])
+def test_mostly_padding_in_launches_of_about_one_round(R, H, with_weights, clamp, mode):
+    """Rows of padding hold NaN and come out as zeros whether or not their waves look at the mask around them; live rows come out as alone."""
+    tk = _tk()
+    col, round_sf, packed = mode
+    g = torch.Generator().manual_seed(R + H)
+    rows = torch.tensor([0, 1, 130, 400, 2000, 2001, 2050, R // 2, R - 300, R - 200, R - 1])
+    x = torch.full((R, 2 * H), float('nan'), dtype=torch.bfloat16)
+    live = (torch.randn((len(rows), 2 * H), generator=g) * 2).to(torch.bfloat16)
+    x[rows] = live
+    w = torch.rand((R, 2), generator=g)
+    p2e = torch.full((R,), -1, dtype=torch.int32)
+    p2e[rows] = 3
+    ptt = torch.where(p2e >= 0, 2 * torch.arange(R, dtype=torch.int32) + 1, -1).to(torch.int32)
+    weights = (ptt.cuda(), w.cuda()) if with_weights else (None, None)
+    want = torch_ref.swiglu_forward_and_per_token_cast(live, 'e4m3', 128, *((ptt[rows], w) if with_weights else (None, None)), p2e[rows], col, round_sf,
+                                                       packed, swiglu_clamp_value=clamp)
+    codes, sf = tk.quant.swiglu_forward_and_per_token_cast(x.cuda(), 'e4m3', 128, *weights, p2e.cuda(), col, round_sf, packed, swiglu_clamp_value=clamp)
+    codes, sf = codes.cpu(), sf.cpu()
+    check_fused((codes[rows], sf[rows].contiguous()), (want[0], want[1].contiguous()), H // 128, packed, 'live rows')
+    assert int((codes.view(torch.uint8) != 0).any(1).sum()) == len(rows) and bool((sf[p2e < 0] == 0).all())

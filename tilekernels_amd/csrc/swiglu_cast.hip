@@ -306,8 +306,10 @@ enum { T_STACKED = 0, T_ROW = 2, T_ROWC = 3 };
 // column-major fp32 scales: [8192, 2 x 2048] 15.39 / 14.74, [4096, 2 x 4096] 15.34 / 14.86, [12288, 2 x 2048] 21.40 / 20.89,
 // [16384, 2 x 2048] 27.53 / 27.13; packed UE8M0: 14.79 / 14.36, 14.70 / 14.47, 21.11 / 20.61, 27.18 / 26.88.
 // RUNS: fp32 input of tiles that overhang the matrix arrives as whole-line loads too (launches of more than a few workgroups, see there)
-template <typename InT, int CLAMP, int RPW, int TILE, bool FULL_GRID, bool MASK, bool ONECOL, int TAILED = 0, bool RUNS = true>
+// PADDING: waves look whether they lie in a long run of padding rows (long_padding_pays)
+template <typename InT, int CLAMP, int RPW, int TILE, bool FULL_GRID, bool MASK, bool ONECOL, int TAILED = 0, bool RUNS = true, bool PADDING = false>
 __global__ __launch_bounds__(TILE == T_ROW ? 64 * kMaxWideWaves : kThreads) void swiglu_cast_kernel(TK_SWIGLU_KERNEL_ARGS) {
+    static_assert(!PADDING || (MASK && TILE != T_ROW && CLAMP != 2 && sizeof(InT) == 2), "runs of padding: masked bf16 tiles that stage their scales");
     static_assert(!TAILED || (FULL_GRID && !MASK && CLAMP != 2 && RPW == 4), "tail waves: unmasked grids of four-piece waves without bounds checks");
     if constexpr (TAILED) {
         // a_nwaves: waves per workgroup (bits 0-3), column tiles (4-15), two-piece workgroups (16-31); a_tiles_k: one-row workgroups
@@ -415,9 +417,8 @@ __global__ __launch_bounds__(TILE == T_ROW ? 64 * kMaxWideWaves : kThreads) void
         for (int r = 0; r < RPW; ++r)
             expert[r] = (MASK && (FULL || row0 + r * kRowStep < p.R)) ? uniform_load(p.pos_to_expert + row0 + r * kRowStep) : 0;
         // rows around the wave's own, in the segments next to its own too (segments are usually multiples of 128 rows)
-        constexpr bool RUN_OF_PADDING = MASK && !DIRECT && CLAMP != 2 && sizeof(InT) == 2;
         int around[4] = {0, 0, 0, 0};
-        if constexpr (RUN_OF_PADDING) {
+        if constexpr (PADDING) {
             // (a grid of several planes of row tiles may have whole planes beyond the last row: row0 may lie anywhere behind it)
             const int inside = FULL ? row0 : min(row0, p.R - 1);
             around[0] = uniform_load(p.pos_to_expert + max(inside - 112, 0));
@@ -429,7 +430,7 @@ __global__ __launch_bounds__(TILE == T_ROW ? 64 * kMaxWideWaves : kThreads) void
         // below waits for them in front of its loads or stores, the later arguments
         if constexpr (MASK && RPW == 4 && !ROW)
             asm volatile("" ::"s"(expert[0]), "s"(expert[1]), "s"(expert[2]), "s"(expert[3]));
-        if constexpr (RUN_OF_PADDING)
+        if constexpr (PADDING)
             asm volatile("" ::"s"(expert[0]), "s"(around[0]), "s"(around[1]), "s"(around[2]), "s"(around[3]), "s"(p.pos_to_token_topk), "s"(p.topk_weights), "s"(p.num_weights),
                          "s"(p.sf.layout), "s"(p.sf.nk), "s"(p.clamp));
         // Routing weights of a masked wave.  One of T_ROW asks for its row's slot in the weight list together with its mask entry (one scalar
@@ -471,7 +472,7 @@ __global__ __launch_bounds__(TILE == T_ROW ? 64 * kMaxWideWaves : kThreads) void
                 else return;
             }
         }
-        // Tiles that stage their scales: in a long run of padding (few tokens, many experts, the end of a buffer for the worst case), a wave
+        // Tiles that stage their scales, in launches of more than one round: in a long run of padding (few tokens, many experts, the end of a buffer for the worst case), a wave
         // without a live row writes its zeros, stages zeros and goes to the barrier.  Elsewhere padding rows read the matrix's first
         // bytes and flow through the arithmetic as zeros: where most waves do that, they all ask for one line.  us per call on MI355X,
         // bf16, 513 live rows of 28544, through the arithmetic / this: H = 1664 32.4 / 22.9, H = 3072 45.7 / 31.0, column-major scales, H = 4096
@@ -479,7 +480,7 @@ __global__ __launch_bounds__(TILE == T_ROW ? 64 * kMaxWideWaves : kThreads) void
         // wave of padding done this way, 6824 live rows of 8192 in segments of a multiple of 128, column-major scales, H = 2048 13.8 / 14.8.
         // (fp32 input is left as it was: 1 to 5 % slower on small batches.)
         bool dead = false;
-        if constexpr (RUN_OF_PADDING) {
+        if constexpr (PADDING) {
             dead = (around[0] & around[1] & around[2] & around[3]) < 0;
 #pragma unroll
             for (int r = 0; r < RPW; ++r) dead = dead && ((!FULL && row0 + r * kRowStep >= p.R) || expert[r] < 0);
@@ -878,6 +879,16 @@ static int64_t wave_slots() {
 // 3.3, [700, 2 x 768] (131) 3.7 / 3.5; [450, 2 x 2560] (285) 3.9 / 4.2, [4001, 2 x 2560] 16.0 / 18.7).
 static bool few_workgroups(int64_t n) { return n < 256; }
 
+// Whether the waves of a masked launch look for long runs of padding.  A wave that looks waits in front of its loads for the entries around
+// its rows and for the later arguments, which come from host memory: 0.2 to 1.1 us where the first round of workgroups starts, which a launch
+// of more rounds than one hides.  bf16, us on MI355X, without / with, 83 % live rows in segments of 128 | 2 % live rows, the rest one run:
+//   up to one round: [1024, 2 x 1664] 3.74 / 4.03 | 3.70 / 2.95, [4096, 2 x 1664] 6.97 / 7.27 | 6.40 / 5.17, [8192, 2 x 1664] 11.96 / 13.08 | 10.3 / 6.8,
+//   [11008, 2 x 1408] 12.87 / 13.39 | 11.1 / 6.8, column-major scales, [1024, 2 x 4096] 4.43 / 4.69 | 4.43 / 3.01, [8192, 2 x 2048] 13.97 / 14.28 | 10.1 / 9.5
+//   more than one: [12672, 2 x 1408] 15.3 / 15.5 | 12.2 / 7.1, [13696, 2 x 1408] 16.6 / 16.3 | 12.8 / 7.3, [12288, 2 x 1664] 17.4 / 17.7 | 14.1 / 8.4,
+//   [28544, 2 x 1664] 38.2 / 35.8 | 29.4 / 14.9, column-major scales, [16384, 2 x 2048] 24.6 / 24.7 | 18.2 / 13.2
+// A batch of up to one round is a trimmed one more often than a worst-case buffer, and its rows are live: it does not look.
+static bool long_padding_pays(int64_t workgroups) { return workgroups * kWaves * 8 > wave_slots() * 9; }
+
 template <typename InT, int CLAMP, int RPW, int TILE>
 static void launch_swiglu_tiled(SwigluParams &p, int max_blocks, hipStream_t stream) {
     // T_ROW, rows per workgroup (= waves), us per call at [8192, 4096] dense / [48128, 4096] with a third of the rows
@@ -968,26 +979,33 @@ static void launch_swiglu_tiled(SwigluParams &p, int max_blocks, hipStream_t str
             return;
         }
     }
-#define TK_SWIGLU_LAUNCH(FULL_, MASK_)                                                                                          \
+#define TK_SWIGLU_LAUNCH(FULL_, MASK_, PADDING_)                                                                                     \
     do {                                                                                                                        \
         if (onecol)                                                                                                             \
-            hipLaunchKernelGGL((swiglu_cast_kernel<InT, CLAMP, RPW, TILE, FULL_, MASK_, ROWWISE>), grid, block, 0, stream,      \
+            hipLaunchKernelGGL((swiglu_cast_kernel<InT, CLAMP, RPW, TILE, FULL_, MASK_, ROWWISE, 0, true, PADDING_>), grid, block, 0, stream, \
                                TK_SWIGLU_LAUNCH_ARGS(p));                                                                       \
         else                                                                                                                    \
-            hipLaunchKernelGGL((swiglu_cast_kernel<InT, CLAMP, RPW, TILE, FULL_, MASK_, false>), grid, block, 0, stream,        \
+            hipLaunchKernelGGL((swiglu_cast_kernel<InT, CLAMP, RPW, TILE, FULL_, MASK_, false, 0, true, PADDING_>), grid, block, 0, stream,   \
                                TK_SWIGLU_LAUNCH_ARGS(p));                                                                       \
     } while (0)
     if (p.pos_to_expert) {
         // A masked batch in row-wise tiles takes one row per workgroup, so its grid fits unless it has more than one plane of
         // row tiles (several columns of tiles, more than 32768 rows); the counting variant's grid is flat and always fits.
         constexpr bool kAlwaysExact = TILE == T_ROW && CLAMP == 2;
-        if (full || kAlwaysExact) TK_SWIGLU_LAUNCH(true, true);
+        if constexpr (TILE != T_ROW && CLAMP != 2 && sizeof(InT) == 2) {
+            if (long_padding_pays((int64_t)tiles_m * p.tiles_k)) {
+                if (full) TK_SWIGLU_LAUNCH(true, true, true);
+                else TK_SWIGLU_LAUNCH(false, true, true);
+                return;
+            }
+        }
+        if (full || kAlwaysExact) TK_SWIGLU_LAUNCH(true, true, false);
         else if constexpr (TILE == T_ROW && !kAlwaysExact)
             hipLaunchKernelGGL((swiglu_cast_kernel<InT, CLAMP, RPW, TILE, false, true, false>), grid, block, 0, stream, TK_SWIGLU_LAUNCH_ARGS(p));
-        else if constexpr (!kAlwaysExact) TK_SWIGLU_LAUNCH(false, true);
+        else if constexpr (!kAlwaysExact) TK_SWIGLU_LAUNCH(false, true, false);
     } else {
-        if (full) TK_SWIGLU_LAUNCH(true, false);
-        else TK_SWIGLU_LAUNCH(false, false);
+        if (full) TK_SWIGLU_LAUNCH(true, false, false);
+        else TK_SWIGLU_LAUNCH(false, false, false);
     }
 #undef TK_SWIGLU_LAUNCH
 }
