@@ -306,13 +306,20 @@ __global__ __launch_bounds__(LANES * kPcParts, 4) void per_channel_cast_kernel(T
     }
 }
 
-// Gathered E4M3 rows: whether most of the output is padding or tokens that other rows repeat.  Narrow tiles serve that better, wide ones
-// the rest (figures at the kernel; from 9100 tokens [13120, 2560] wide / narrow 12.5 / 11.4 us, cold 14.3 / 15.2; 21520 -> [33792, 7168] 85.4 / 90.5).
-__host__ __device__ inline bool gather_repeats(int num_tokens, int M) { return 4 * (int64_t)M >= 7 * (int64_t)num_tokens; }
-// and whether its tiles then go in column order, each XCD down a column of its own: a column tile of all tokens (256 bytes of each) stays in
-// the XCD's 4 MB L2 until the next expert's rows ask for it ([10112, 7168] from 5401 tokens 21.6 / 19.2 us, [18432, 7168] from 8192 37.1 / 33.0).
-// So few tokens that all of their rows stay in the caches need no order (88 -> [31616, 7168] 41.5 / 42.9, 928 -> [32768, 3712] 24.4 / 25.2).
-__host__ __device__ inline bool gather_by_columns(int num_tokens, int M) { return gather_repeats(num_tokens, M) && num_tokens >= 4096 && num_tokens < 16384; }
+// Gathered E4M3 rows: whether a launch whose output is mostly padding or tokens that other rows repeat takes narrow tiles.  Up to 16383 tokens,
+// where narrow tiles can go in column order (below): from 9100 tokens [13120, 2560] wide / narrow 12.5 / 11.4 us, cold 14.3 / 15.2.  Beyond that
+// they would not, and wide tiles with ordinary loads serve repeated rows better; us, narrow / wide (wide with non-temporal loads), three sets of inputs in
+// rotation | twelve:  16384 tokens twice each, K = 2048 23.6 / 23.9 (28.5) | 29.8 / 27.4 (29.0), K = 7168 90.0 / 83.1 (88.5) | 91.5 / 84.9 (88.7);  eight times
+// each, K = 2048 72.4 / 71.7 (91.9) | 80.6 / 77.4 (91.5), K = 7168 295 / 286 (323) | 295 / 287 (324);  32768 twice, K = 2048 42.3 / 43.0 (51.1) | 52.8 / 49.6 (51.0),
+// K = 7168 179 / 167 (170) | 179 / 167 (171);  20000 once each among 65536 rows, K = 2048 29.3 / 30.0 (33.5) | 36.3 / 34.9 (34.2)
+__host__ __device__ inline bool gather_repeats(int num_tokens, int M) { return num_tokens < 16384 && 4 * (int64_t)M >= 7 * (int64_t)num_tokens; }
+// and whether those tiles go in column order, each XCD down a column of its own: a column tile of all tokens (256 bytes of each, so up to 16383 of
+// them) stays in the XCD's 4 MB L2 until the next expert's rows ask for it.  us, striped / in column order, three sets | twelve:  5401 tokens -> [10112,
+// 7168] 21.6 / 19.2, 8192 -> [18432, 7168] 37.1 / 33.0, 14336 six times each, K = 2048 54.4 / 41.9 | 59.1 / 54.8;  narrow rows, 6000 twice, K = 512 4.7 / 4.4 | 5.4 /
+// 5.3, 8192 twice 5.8 / 5.9 | 6.6 / 6.8.  Fewer tokens than 4096 gain by it where they are repeated (3000 twice, K = 7168 16.0 / 13.6 | 19.7 / 19.3; 1024 twice 8.5 /
+// 7.7 | 8.5 / 8.2) and lose where they stand between padding, which for so few tokens of several experts is the rule, whatever their bytes (88 -> [31616, 7168]
+// 40.4 / 47.4, 1202 -> [18048, 6144] 22.2 / 24.9 | 22.4 / 25.6, 3000 -> [32768, 7168], 21 MB of rows, 42.8 / 47.3 | 44.1 / 51.0; 6000 -> [32768, 4096] 27.1 / 26.9 | 29.7 / 30.3).
+__host__ __device__ inline bool gather_by_columns(int num_tokens, int M) { return gather_repeats(num_tokens, M) && num_tokens >= 4096; }
 
 // Offset beyond the end of any buffer, also with a lane's part of up to 496 bytes added to it.
 constexpr uint32_t kPcNowhere = 0xFFFFFC00u;
