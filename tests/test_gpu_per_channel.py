@@ -225,8 +225,8 @@ def gathered_fp8_rows(codes, sf, pos, N):
     """The per-channel cast of gathered E4M3 rows with one scale per N tokens (the Python function takes 128 only)."""
     from tilekernels_amd import _ffi
     (T, K), M = codes.shape, pos.shape[0]
-    out = torch.empty((M, K), dtype=torch.float8_e4m3fn, device='cuda')
-    out_sf = torch.empty((-(-M // N), K), dtype=torch.float32, device='cuda')
+    out = torch.full((M, K), 0x5A, dtype=torch.uint8, device='cuda').view(torch.float8_e4m3fn)      # (so that a tile nobody writes shows)
+    out_sf = torch.full((-(-M // N), K), -1.0, dtype=torch.float32, device='cuda')
     rc = _ffi.load().tk_per_channel_cast(codes.data_ptr(), 0, sf.data_ptr(), T, K, pos.data_ptr(), M, out.data_ptr(), out_sf.data_ptr(),
                                          N, 0, 0, 0, 0, 0.0, _ffi.current_stream(out.device))
     assert rc == 0, rc
@@ -234,11 +234,12 @@ def gathered_fp8_rows(codes, sf, pos, N):
     return out, out_sf
 
 
-# (tokens, rows, columns): few tokens and much padding; column order with a last tile that is partly beyond the matrix, at both ends of its
-# range of tokens; rows about as many as tokens; wide tiles, written through and not; each with rows of -1 and of the last token
+# (tokens, rows, columns): few tokens and much padding; column order with whole eighths of the tiles and without, with a last token tile and a last column
+# tile partly beyond the matrix and without, and the nearest sizes on either side of its range of tokens; rows about as many as tokens; wide tiles,
+# written through and not; each with rows of -1 and of the last token
 @pytest.mark.parametrize('N', [32, 128])
-@pytest.mark.parametrize('T,M,K', [(1, 16, 128), (100, 2064, 640), (4095, 7184, 384), (4096, 7168, 384), (16383, 28672, 128), (16384, 28688, 640),
-                                   (3000, 2992, 1408), (6553, 8192, 2048), (6600, 8192, 2048), (6000, 8320, 2176)])
+@pytest.mark.parametrize('T,M,K', [(1, 16, 128), (100, 2064, 640), (4095, 7184, 384), (4096, 7168, 384), (4096, 7184, 640), (5401, 10112, 1152), (16383, 28672, 128),
+                                   (16383, 28688, 384), (16384, 28688, 640), (3000, 2992, 1408), (6553, 8192, 2048), (6600, 8192, 2048), (6000, 8320, 2176)])
 def test_gathered_fp8_rows_by_tokens_and_rows(T, M, K, N):
     g = torch.Generator().manual_seed(T + K)
     x = torch_ref.cast(torch.randn((T, K), generator=g).to(torch.bfloat16), 'e4m3', (1, 128))
