@@ -205,11 +205,13 @@ __global__ __launch_bounds__(64 * kBwdMaxWaves) void swiglu_backward_kernel(TK_B
 // with waves to spare.  With one it is 60 registers and eight waves.  us on MI355X, two rows / one:
 //   five strips and more: [3072, 2560] 24.3 / 18.9, [10112, 2560] 65.1 / 49.2, [10112, 3072] 70.1 / 59.6, [10112, 7168] 164.8 / 160.8, [39000, 4096] 326 / 321
 //   launches that two rows to a workgroup leave short of waves: [1130, 512] 4.3 / 3.7, [1130, 1024] 5.8 / 5.0, [2130, 1024] 7.4 / 7.0, [1130, 1536]
-//   7.1 / 6.0, but [2130, 1536] 8.9 / 9.0, [4130, 1024] 9.5 / 10.6, [6130, 512] 7.8 / 9.4, [9216, 896] 20.5 / 20.9
-//   four whole strips: [2130, 2048] 11.5 / 11.2, [6130, 2048] 27.1 / 26.8, [9130, 2048] 38.0 / 38.2, [25000, 2048] 108.0 / 110.1
+//   7.1 / 6.0, [1152, 1664] 7.7 / 6.9, [1152, 2048] 7.6 / 7.0, but [2130, 1536] 8.9 / 9.0, [4130, 1024] 9.5 / 10.6, [6130, 512] 7.8 / 9.4, [9216, 896] 20.5 / 20.9
+//   four strips: [1536, 1664] 7.9 / 8.6, [6144, 1664] 25.0 / 25.3, [20480, 1664] 69.2 / 73.5, [1536, 1792] 7.9 / 8.6, [9216, 1792] 35.1 / 36.6, [20480, 1792]
+//   71.5 / 77.0, [6144, 1920] 26.6 / 27.2, [20480, 1920] 75.6 / 78.7; whole strips, [1536, 2048] 7.8 / 7.5, [2176, 2048] 11.9 / 11.6, [6144, 2048] 27.6 / 27.3,
+//   [9216, 2048] 38.9 / 38.7, [20480, 2048] 78.8 / 78.5, [25000, 2048] 108.0 / 110.1
 static bool backward_single_rows(int64_t R, int64_t H) {
     const int64_t strips = (H + kStripCols - 1) / kStripCols;
-    return strips > 4 || R * strips <= 5000 || (H == 4 * kStripCols && R <= 6144);
+    return strips > 4 || R * strips <= 5000;
 }
 
 struct BackwardArgs {
