@@ -478,7 +478,8 @@ def test_per_token_cast_of_ragged_rows(M, K, fmt, group):
 @pytest.mark.parametrize('block', [(128, 128), (32, 32), (128, 32), (32, 128)])
 @pytest.mark.parametrize('fmt', ['e4m3', 'e2m1'])
 @pytest.mark.parametrize('dtype', [torch.bfloat16, torch.float32])
-@pytest.mark.parametrize('M,K', [(3072, 2048), (3841, 1280), (4096, 2048), (4481, 2048), (8192, 2048), (8193, 2048), (16385, 1280), (16640, 1024), (900, 704)])
+@pytest.mark.parametrize('M,K', [(2433, 2048), (3072, 2048), (3841, 1280), (4096, 2048), (4481, 2048), (6785, 2048), (8192, 2048), (8193, 2048), (9984, 2048), (16385, 1280),
+                                 (16640, 1024), (900, 704)])
 def test_per_block_cast_tile_shapes(M, K, dtype, fmt, block):
     tk = _tk()
     x = _randn((M, K), dtype, M + K, 2.0)

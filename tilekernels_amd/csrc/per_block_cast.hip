@@ -209,16 +209,28 @@ __global__ __launch_bounds__(THREADS) void per_block_cast_kernel(TK_PB_KERNEL_AR
 // (128 x 128 with 256 threads: 9.4 at [7168,2048], with 1024: 9.8.)  A wave of a 512-column tile reads 1 KB of one
 // row per load instruction instead of 256 bytes of four rows.  Its workgroup of 1024 threads at 96 registers has a CU to itself, so
 // that the launch is as long as the CU with the most tiles: the wide tile pays where there are at most 256 of them and not much fewer
-// than 140, and 256 columns with 1024 threads where there are 192 to 256 of those.  us, 128 / 256 (1024 threads) / 512 columns:
+// than 140, and 256 columns with 1024 threads where there are at most 256 of those and not fewer than 192, to E4M3 from fp32 150.  us, 128 / 256
+// (1024 threads) / 512 columns:
 //   E4M3 bf16 [3072,2048] 4.85 / 4.79 / 6.30, [3584,2048] 5.30 / 4.97 / 6.50, [4096,2048] 5.66 / 5.22 / 6.62, [2100,4096] 5.94 / 6.46 / 6.47,
 //   [4608,2048] 6.78 / 7.61 / 6.75, [6144,2048] 7.82 / 8.33 / 7.44, [7168,2048] 8.90 / 9.17 / 8.29, [8192,2048] 9.74 / 10.12 / 9.23, [8704,2048]
 //   10.79 / 11.83 / 11.93, [9044,2048] 11.0 / 12.1 / 13.3, [4100,4096] 9.90 / 10.5 / 10.8, [5000,4096] 11.9 / 12.5 / 13.75
 //   fp32 [2560,2048] 6.39 / 6.17 / 8.38, [4096,2048] 8.39 / 7.61 / 9.03, [4608,2048] 9.74 / 10.90 / 9.30, [8192,2048] 14.98 / 15.22 / 13.98,
 //   [9044,2048] 16.5 / 18.4 / 20.0
+// To E2M1 the wide tile begins to pay later, from 160 of them for bf16 and 208 for fp32 (there for two widths of three):
+//   bf16 [3072,2048] 4.63 / 4.55 / 5.99, [3584,2048] 5.35 / 4.84 / 6.57, [4096,2048] 5.54 / 5.08 / 6.76, [2304,4096] 6.52 / 6.60 / 6.47, [4608,2048] 6.58 / 6.67 /
+//   6.91, [5376,2048] 7.16 / 6.97 / 6.91, [2688,4096] 7.16 / 7.02 / 6.70, [7168,2048] 8.80 / 7.82 / 7.76, [8192,2048] 9.14 / 8.60 / 8.77, [4096,4096] 9.22 / 8.73 / 8.03
+//   fp32 [1408,4096] 6.83 / 6.97 / 8.98, [3072,2048] 6.51 / 6.49 / 8.76, [3584,2048] 7.15 / 6.93 / 8.65, [1152,7168] 7.74 / 7.42 / 9.40, [4096,2048] 8.02 / 7.39 / 10.2,
+//   but [2048,4096] 8.31 / 9.15 / 9.32;  [4608,2048] 9.61 / 10.18 / 10.82, [6144,2048] 11.18 / 10.91 / 11.89, [3072,4096] 11.43 / 13.14 / 11.40, [3584,4096] 13.78 / 13.92 /
+//   12.81, [4096,4096] 15.34 / 16.18 / 14.44, [2048,7168] 13.04 / 11.76 / 11.95, [2304,7168] 14.02 / 12.76 / 13.04, [7168,2048] 13.34 / 11.61 / 13.58, but [8192,2048]
+//   14.52 / 12.88 / 17.10
 // More tiles than that to E2M1, whose stores of a lane's 8 codes are 4 bytes in a 128-column tile and 8 in a wider one, go with 256 columns
-// and 512 threads (bf16, 128 / 256 columns: [9044,2048] 10.9 / 10.6, [12352,2048] 13.6 / 12.7, [5000,4096] 11.7 / 10.6, [3000,7168] 12.0 / 10.9,
-// [16384,7168] 48.5 / 45.8, but [8704,2048] 10.0 / 10.35; fp32 [16384,7168] 86.5 / 82.6, but [8192,8192] 47.6 / 53.7).
-constexpr int64_t kWideMinTiles = 561, kWideMaxTiles = 1024, kMidMinTiles = 384, kMidMinTilesF32 = 300, kMidMaxTiles = 512;     // in 128 x 128 tiles
+// and 512 threads from 1233 on (bf16, 128 / 256 columns: [10240,2048] 11.35 / 10.94, [2816,7168] 10.70 / 10.75, [5120,4096] 11.37 / 10.67, [12352,2048] 13.6 / 12.7,
+// [16384,7168] 48.5 / 45.8, but [8704,2048] 9.95 / 10.30, [9216,2048] 10.30 / 10.67, [4608,4096] 10.15 / 10.42, [2560,7168] 10.22 / 10.44; fp32 [16384,7168] 86.5 / 82.6, but
+// [8192,8192] 47.6 / 53.7).
+// Bounds in 128 x 128 tiles:
+constexpr int64_t kWideMaxTiles = 1024, kMidMaxTiles = 512, kManyMinTiles = 1233;
+template <bool F32, int FMT> constexpr int64_t kWideMinTiles = FMT != TK_E2M1 ? 561 : F32 ? 833 : 641;
+template <bool F32, int FMT> constexpr int64_t kMidMinTiles = F32 && FMT != TK_E2M1 ? 300 : 384;
 
 template <typename InT, int FMT, int BM, int BK, int TW, int THREADS>
 static void launch_per_block_3(const PerBlockParams &p, hipStream_t stream) {
@@ -242,16 +254,16 @@ template <typename InT, int FMT, int BM, int BK>
 static void launch_per_block_2(const PerBlockParams &p, hipStream_t stream) {
     const int64_t tiles = (int64_t)p.tiles_m * p.tiles_k;
     constexpr bool F32 = std::is_same<InT, float>::value;
-    if (p.K % kWideTile == 0 && tiles >= kWideMinTiles && tiles <= kWideMaxTiles) {
+    if (p.K % kWideTile == 0 && tiles >= kWideMinTiles<F32, FMT> && tiles <= kWideMaxTiles) {
         launch_per_block_3<InT, FMT, BM, BK, kWideTile, kWideThreads>(p, stream);
         return;
     }
-    if (p.K % kMidTile == 0 && tiles >= (F32 ? kMidMinTilesF32 : kMidMinTiles) && tiles <= kMidMaxTiles) {
+    if (p.K % kMidTile == 0 && tiles >= kMidMinTiles<F32, FMT> && tiles <= kMidMaxTiles) {
         launch_per_block_3<InT, FMT, BM, BK, kMidTile, kWideThreads>(p, stream);
         return;
     }
     if constexpr (FMT == TK_E2M1 && !F32) {
-        if (p.K % kMidTile == 0 && tiles > kWideMaxTiles) {
+        if (p.K % kMidTile == 0 && tiles >= kManyMinTiles) {
             launch_per_block_3<InT, FMT, BM, BK, kMidTile, kPerBlockThreads>(p, stream);
             return;
         }
