@@ -433,12 +433,15 @@ __global__ __launch_bounds__(TILE == T_ROW ? 64 * kMaxWideWaves : kThreads) void
         if constexpr (PADDING)
             asm volatile("" ::"s"(expert[0]), "s"(around[0]), "s"(around[1]), "s"(around[2]), "s"(around[3]), "s"(p.pos_to_token_topk), "s"(p.topk_weights), "s"(p.num_weights),
                          "s"(p.sf.layout), "s"(p.sf.nk), "s"(p.clamp));
-        // Routing weights of a masked wave.  One of T_ROW asks for its row's slot in the weight list together with its mask entry (one scalar
-        // round trip for both), the others behind their vector loads, and all for the weights themselves right after, so that neither
+        // Routing weights of a masked wave.  One that holds one row asks for the row's slot in the weight list together with its mask entry (one
+        // scalar round trip for both), the others behind their vector loads, and all for the weights themselves right after, so that neither
         // is waited for once the data is there.  Fetched where they are used, after the data, they cost [48128, 2 x 2048] with 32768 live
         // rows 0.6 us of 61 on MI355X (2.6 us of 59 when the input is still in the last-level cache), stacked tiles of one of 8 ranks
-        // [35328, 2 x 1664] 47.8 / 46.4, [720, 2 x 2560] 3.9 / 3.7 (fp32 input 1 to 3 % slower: not there).
+        // [35328, 2 x 1664] 47.8 / 46.4, [720, 2 x 2560] 3.9 / 3.7 (fp32 input 1 to 3 % slower: not there).  (T_ROWC, slot behind the loads / with the
+        // mask entry: bf16 [1024, 2 x 2048] 3.94 / 3.84, [1024, 2 x 4096] 4.91 / 4.82, but fp32 [4096, 2 x 2048] 12.2 / 12.4, and a wave that looks for a run
+        // of padding has the mask entries around its row to wait for.)
         constexpr bool EARLY_WEIGHT = MASK && (ROW || sizeof(InT) == 2);
+        constexpr bool WITH_ENTRY = EARLY_WEIGHT && (DIRECT || (ROW && !PADDING && sizeof(InT) == 2));
         constexpr int WROWS = ROW ? 1 : RPW;      // rows of the wave
         int wpos[WROWS];
 #pragma unroll
@@ -449,7 +452,7 @@ __global__ __launch_bounds__(TILE == T_ROW ? 64 * kMaxWideWaves : kThreads) void
             for (int r = 0; r < WROWS; ++r)
                 if (FULL || row0 + r < p.R) wpos[r] = uniform_load(p.pos_to_token_topk + row0 + r);
         };
-        if constexpr (EARLY_WEIGHT && DIRECT) ask_for_weights();
+        if constexpr (WITH_ENTRY) ask_for_weights();
         // A wave whose row is padding writes the row's zeros and leaves: no loads, no arithmetic.  The zeros go out as
         // non-temporal 16-byte stores that cover whole lines.  Measured on MI355X, bf16, us per call, padding rows flowing
         // through the arithmetic as zeros / this way: configuration with runs of padding (32768 live rows of 47488, H = 2048)
@@ -558,7 +561,7 @@ __global__ __launch_bounds__(TILE == T_ROW ? 64 * kMaxWideWaves : kThreads) void
                 for (int r = 0; r < RPW; ++r)
                     if (unused[r]) { rg[r].zero(); ru[r].zero(); }
             }
-            if constexpr (EARLY_WEIGHT && !DIRECT) ask_for_weights();
+            if constexpr (EARLY_WEIGHT && !WITH_ENTRY) ask_for_weights();
             float wrow[WROWS];
 #pragma unroll
             for (int r = 0; r < WROWS; ++r) wrow[r] = 0.0f;
