@@ -10,7 +10,8 @@ def get_fused_mapping(topk_idx: torch.Tensor, num_experts: int, num_expanded_tok
     """Mappings between the (token, k) routing list and the expert-major expanded layout.
 
     ``num_expanded_tokens == 0`` (without ``force_no_sync``) sizes the buffers for the worst case, then
-    trims them to the real padded length, which needs a host synchronisation.
+    trims them to the real padded length, which needs a host synchronisation: the call returns when the
+    current stream is through, and its results may be used on any stream.  Other calls only enqueue.
 
     Returns ``(pos_to_expert, pos_to_token, pos_to_token_topk, token_topk_to_pos, expert_start, expert_end,
     num_tokens_per_expert, num_tokens_per_expert_list)``; the list is empty unless a sync happened.
